@@ -49,6 +49,14 @@ SIGNATURES = {
                               _i32, _pf64, _i64, _i64, _i64, _vp],
     "cc_stage3_plan_apply": [_vp, _vp, _vp, _vp],
     "cc_stage3_plan_destroy": [_vp],
+    "cc_slab_join_f64": [_vp, _i32, _pvp, _pf64, _i64, _i64, _i64, _i64, _vp, _vp],
+    "cc_form_work_size": [_i32, _i32, _i64, _i64, _i64, _pi64],
+    "cc_form_f64": [_vp, _i32, _pi32, _pvp, _pvp, _i64, _i64, _i64, _vp, _vp],
+    "cc_whiten_f64": [_vp, _i64, _i32, _vp, _vp, _vp, _vp],
+    "cc_formed_plan_create": [ctypes.POINTER(ctypes.c_void_p), _i64, _i64, _i32, _pvp, _pf64, _vp],
+    "cc_formed_plan_apply": [_vp, _vp, _vp, _vp],
+    "cc_formed_plan_destroy": [_vp],
+    "cc_lanczos_formed_f64": [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _f64, _f64, _i32, _i32, _vp, _vp, _pf64],
     "cc_profile_begin": [],
     "cc_profile_begin_sampled": [_i32],
     "cc_profile_end": [_i32, _pf64, _pi64],
@@ -91,6 +99,7 @@ SIGNATURES = {
     "cc_mlp_forward": [_vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp],
     "cc_mlp_backward": [_vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "cc_mlp_adam": [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _f64, _f64, _f64, _f64, _i64],
+    "cc_stage3_pack_sum_f64": [_vp, _i32, _pvp, _pf64, _i64, _i64, _i64, _i64, _vp, _vp],
     "cc_stage3_matvec_fused_f64": [_vp, _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32, _i32, _pf64, _i64, _i64,
                                    _i64, _vp, _vp, _vp],
     "cc_stage3_matvec_fused_f64_noalloc": [_vp, _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32, _i32, _pf64, _i64,

@@ -44,6 +44,12 @@ int cc_internal_stage3_apply(hipStream_t st, const void* plan, const double* x, 
 int64_t cc_internal_stage3_n(const void* plan);
 int cc_internal_lp_apply(hipStream_t st, const void* plan, const double* x, double* y);
 int64_t cc_internal_lp_n(const void* plan);
+int cc_internal_formed_apply(hipStream_t st, const void* plan, const double* x, double* y);
+int64_t cc_internal_formed_n(const void* plan);
+// C[b][m][j] = sum over k <= j of A[b][m][k] B[k][j] for n x n matrices: B upper triangular (row-major), C row-major,
+// A with element strides sAm, sAk.  Half the work of the full product.
+int cc_internal_gemm_upper(hipStream_t st, int64_t batch, int64_t n, const double* A, int64_t sAb, int64_t sAm, int64_t sAk,
+                           const double* B, int64_t ldb, double* C, int64_t sCb);
 
 // Launch timing (between cc_profile_begin[_sampled] and cc_profile_end, single-threaded use): a kernel
 // launch is bracketed by cc_prof_start / cc_prof_stop, which record HIP events on its stream when timing
@@ -122,6 +128,66 @@ __device__ inline void cc_slab_load_d(const CCSlabGather& g, const double* __res
 #pragma unroll
   for (int u = 0; u < NE; ++u)
     if (threadIdx.x + NTH * u < n) lds[at[u]] = v[u] * mul;
+}
+// A channel given as a weighted sum of tensors with the same legs and strides.
+constexpr int CC_SLAB_SOURCES = 8;
+struct CCSlabSum {
+  int n;
+  const double* p[CC_SLAB_SOURCES];
+  double c[CC_SLAB_SOURCES];
+};
+static inline CCSlabSum cc_slab_sum(int n, const double* const* src, const double* coef) {
+  CCSlabSum s;
+  s.n = n;
+  for (int i = 0; i < CC_SLAB_SOURCES; ++i) {
+    s.p[i] = src[i < n ? i : 0];
+    s.c[i] = i < n ? coef[i] : 0.0;
+  }
+  return s;
+}
+// cc_slab_load_d of the sum: lds[row * ld + col] = sum_i c_i src_i, each source's loads in flight together.
+template <int D, int NTH>
+__device__ inline void cc_slab_load_sum_d(const CCSlabGather& g, const CCSlabSum& src, int64_t al, double* lds, int ld) {
+  constexpr int n = D * D * D * D, NE = (n + NTH - 1) / NTH;
+  const int64_t a0 = al / g.na1, a1 = al - a0 * g.na1, base = a0 * g.sa0 + a1 * g.sa1;
+  double v[NE];
+  int at[NE];
+  int64_t off[NE];
+#pragma unroll
+  for (int u = 0; u < NE; ++u) {
+    const int e = threadIdx.x + NTH * u, ec = e < n ? e : 0;  // clamped: every load in bounds
+    const int k3 = ec % D, k2 = (ec / D) % D, k1 = (ec / (D * D)) % D, k0 = ec / (D * D * D);
+    off[u] = base + k0 * g.st[0] + k1 * g.st[1] + k2 * g.st[2] + k3 * g.st[3];
+    at[u] = (k0 * g.rw[0] + k1 * g.rw[1] + k2 * g.rw[2] + k3 * g.rw[3]) * ld + k0 * g.cw[0] + k1 * g.cw[1] + k2 * g.cw[2] +
+            k3 * g.cw[3];
+    v[u] = src.c[0] * src.p[0][off[u]];
+  }
+  for (int i = 1; i < src.n; ++i)
+#pragma unroll
+    for (int u = 0; u < NE; ++u) v[u] += src.c[i] * src.p[i][off[u]];
+#pragma unroll
+  for (int u = 0; u < NE; ++u)
+    if (threadIdx.x + NTH * u < n) lds[at[u]] = v[u];
+}
+// The same for any leg sizes.
+__device__ inline void cc_slab_load_sum(const CCSlabGather& g, const CCSlabSum& src, int64_t al, double* lds, int ld) {
+  const int64_t a0 = al / g.na1, a1 = al - a0 * g.na1, base = a0 * g.sa0 + a1 * g.sa1;
+  const int n = g.P * g.P;
+  for (int e = threadIdx.x; e < n; e += blockDim.x) {
+    int k = e;
+    const int k3 = k % g.sz[3];
+    k /= g.sz[3];
+    const int k2 = k % g.sz[2];
+    k /= g.sz[2];
+    const int k1 = k % g.sz[1];
+    const int k0 = k / g.sz[1];
+    const int64_t off = base + k0 * g.st[0] + k1 * g.st[1] + k2 * g.st[2] + k3 * g.st[3];
+    const int row = k0 * g.rw[0] + k1 * g.rw[1] + k2 * g.rw[2] + k3 * g.rw[3];
+    const int col = k0 * g.cw[0] + k1 * g.cw[1] + k2 * g.cw[2] + k3 * g.cw[3];
+    double v = src.c[0] * src.p[0][off];
+    for (int i = 1; i < src.n; ++i) v += src.c[i] * src.p[i][off];
+    lds[row * ld + col] = v;
+  }
 }
 // Loads slab alpha into lds[row * ld + col] (row, col < P) with all threads of the block.
 __device__ inline void cc_slab_load(const CCSlabGather& g, const double* __restrict__ src, int64_t al, double* lds, int ld,

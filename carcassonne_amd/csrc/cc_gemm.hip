@@ -19,6 +19,7 @@ struct GemmArgs {
   const double* B; int64_t sBb, sBk, sBn;
   double* C; int64_t sCb, sCm, sCn;
   int64_t batch0;
+  int upper;   // B is upper triangular: columns up to n0 + T - 1 of C take k < n0 + T only
 };
 
 // The operand tile of one K step (T rows or columns x BK) in LDS, in the order its loader writes without
@@ -49,7 +50,9 @@ __global__ void __launch_bounds__(256) gemm_f64_kernel(GemmArgs g) {
   const int wr = wave >> 1, wc = wave & 1;
   const int64_t bz = g.batch0 + blockIdx.z;
   double* C = g.C + bz * g.sCb;
-  const int64_t m0 = (int64_t)blockIdx.y * T, n0 = (int64_t)blockIdx.x * T;
+  // an upper-triangular B: the last columns have the longest sums and start first
+  const int64_t m0 = (int64_t)blockIdx.y * T, n0 = (int64_t)(g.upper ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * T;
+  const int64_t K = g.upper && n0 + T < g.K ? n0 + T : g.K;
 
   f64x4 acc[TM][TM];
 #pragma unroll
@@ -102,7 +105,7 @@ __global__ void __launch_bounds__(256) gemm_f64_kernel(GemmArgs g) {
 
   // Two LDS buffers and one barrier per K step: the next step's loads are in flight during a step's products,
   // and a buffer is written again only after every wave passed the barrier of the step in between.
-  const int full = (int)(g.K / BK), rest = (int)(g.K % BK);
+  const int full = (int)(K / BK), rest = (int)(K % BK);
   if (full > 0) load();
   for (int s = 0; s < full; ++s) {
     store(s & 1);
@@ -152,7 +155,7 @@ extern "C" int cc_gemm_f64(void* stream, int64_t batch, int64_t M, int64_t N, in
                            double* C, int64_t sCb, int64_t sCm, int64_t sCn) {
   if (batch < 0 || M < 0 || N < 0 || K < 0) { cc_set_last_error("cc_gemm_f64: negative size"); return CC_ERR_ARG; }
   if (batch == 0 || M == 0 || N == 0) return CC_OK;
-  GemmArgs g{M, N, K, alpha, beta, A, sAb, sAm, sAk, B, sBb, sBk, sBn, C, sCb, sCm, sCn, 0};
+  GemmArgs g{M, N, K, alpha, beta, A, sAb, sAm, sAk, B, sBb, sBk, sBn, C, sCb, sCm, sCn, 0, 0};
   // 64-wide tiles unless that grid would leave most of the 256 CUs idle
   const int64_t tiles64 = ((N + 63) / 64) * ((M + 63) / 64) * batch;
   const int T = tiles64 < 160 ? 32 : 64;
@@ -169,5 +172,19 @@ extern "C" int cc_gemm_f64(void* stream, int64_t batch, int64_t M, int64_t N, in
     else launch_gemm<64>(g, grid, a_k_fast, b_n_fast, st);
     CC_LAUNCH_CHECK();
   }
+  return CC_OK;
+}
+
+int cc_internal_gemm_upper(hipStream_t st, int64_t batch, int64_t n, const double* A, int64_t sAb, int64_t sAm, int64_t sAk,
+                           const double* B, int64_t ldb, double* C, int64_t sCb) {
+  GemmArgs g{n, n, n, 1.0, 0.0, A, sAb, sAm, sAk, B, 0, ldb, 1, C, sCb, n, 1, 0, 1};
+  const int64_t tiles64 = ((n + 63) / 64) * ((n + 63) / 64) * batch;
+  const int T = tiles64 < 160 ? 32 : 64;
+  const int64_t t = (n + T - 1) / T;
+  if (t > 65535 || batch > 65535) { cc_set_last_error("gemm: matrix too large for one launch"); return CC_ERR_UNSUPPORTED; }
+  const dim3 grid((unsigned)t, (unsigned)t, (unsigned)batch);
+  if (T == 32) launch_gemm<32>(g, grid, sAk == 1, true, st);
+  else launch_gemm<64>(g, grid, sAk == 1, true, st);
+  CC_LAUNCH_CHECK();
   return CC_OK;
 }

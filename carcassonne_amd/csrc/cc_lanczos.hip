@@ -281,8 +281,10 @@ struct Whitening {
 
 typedef int (*ApplyFn)(hipStream_t, const void*, const double*, double*);
 
+// w = W H W^T q; a formed operator (apply == cc_internal_formed_apply) holds the whitened matrices already
 int op_whitened(hipStream_t st, ApplyFn apply, const void* plan, const Whitening& wh, const double* q, double* t1, double* t2,
                 double* w) {
+  if (apply == cc_internal_formed_apply) return apply(st, plan, q, w);
   int rc = cc_skinny_f64(st, wh.n_env, 2, wh.Wt, (int)wh.d, q, t1);  // t1 = W^T q
   if (rc) return rc;
   rc = apply(st, plan, t1, t2);                                      // t2 = H t1
@@ -318,6 +320,15 @@ extern "C" int cc_lanczos_lp(void* stream, const void* lp_plan, int64_t n_env, i
   if (cc_internal_lp_n(lp_plan) != n_env * d) { cc_set_last_error("lanczos: operator size does not match the whitening"); return CC_ERR_DIM; }
   return lanczos_driver(cc_stream(stream), cc_internal_lp_apply, lp_plan, n_env, d, L, Lt, W, Wt, x0, tol_residual,
                         tol_energy, max_iter, check_every, work, x_out, host_result);
+}
+
+extern "C" int cc_lanczos_formed_f64(void* stream, const void* formed_plan, int64_t n_env, int64_t d, const double* Lt,
+                                     const double* Wt, const double* x0, double tol_residual, double tol_energy,
+                                     int max_iter, int check_every, double* work, double* x_out, double* host_result) {
+  if (!formed_plan || n_env * d <= 0 || max_iter < 1 || check_every < 0) { cc_set_last_error("lanczos: bad arguments"); return CC_ERR_ARG; }
+  if (cc_internal_formed_n(formed_plan) != n_env * d) { cc_set_last_error("lanczos: operator size does not match the whitening"); return CC_ERR_DIM; }
+  return lanczos_driver(cc_stream(stream), cc_internal_formed_apply, formed_plan, n_env, d, nullptr, Lt, nullptr, Wt, x0,
+                        tol_residual, tol_energy, max_iter, check_every, work, x_out, host_result);
 }
 
 static int lanczos_driver(hipStream_t st, ApplyFn apply, const void* plan, int64_t n_env, int64_t d, const double* L,

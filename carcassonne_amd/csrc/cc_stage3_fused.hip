@@ -2,25 +2,24 @@
 //
 //   Y[p'][q'][s'] = sum_t sum_alpha sum_{p,q,s} A_a(t)[alpha][p'][p] B_b(t)[alpha][q'][q] O_o(t)[s'][s] v[p][q][s]
 //
-// One wave owns a contiguous range of alpha.  Per alpha and per distinct A channel a:
-//   stage A   W_a[idx = s*P4 + q][p'] = sum_p V^T[idx][p] A_a[p'][p]      (V^T operands stay in registers)
+// A team of waves (one per 16-row p' tile) owns a contiguous range of alpha.  Per alpha and per distinct A channel a:
+//   stage A   W_a[idx = s*P4 + q][p'] = sum_p V^T[idx][p] A_a[p'][p]
 // and per term t of that channel:
 //   stage B   Y[p'][q'][s'] += sum_q (sum_s O[s'][s] W_a[s*P4+q][p']) B_b[q'][q]
+// where the terms of one B channel (the hub) are added up before their common stage B.
 // The f64 MFMA result layout (D[i][j] in lane j + 16(i%4), register i/4) puts W_a[s*P4 + 4u + lane/16][p']
 // in the lane/register that stage B needs as its A operand X[p' = lane%16][q = 4u + lane/16], so the
 // intermediate never leaves registers.  Slabs are pre-packed in MFMA-operand order
 // (packed[alpha][u][n][lane] = S[16n + lane%16][4u + lane/16], zero-padded), so each operand load is one
-// coalesced 512-byte read.  Each 4-wave workgroup reduces its waves' Y through LDS in a fixed order and
-// writes one partial; a second kernel sums the partials in a fixed order.
+// coalesced 512-byte read.  Each workgroup reduces its teams' Y through LDS in a fixed order and writes
+// one partial; a second kernel sums the partials in a fixed order.
 #include "cc_common.h"
 
 #include <mutex>
 #include <vector>
 
 namespace {
-// Optional timing of every fused-kernel launch (HIP events on the launch stream).
-
-constexpr int MAX_CH = 16, MAX_TERMS = 48, MAX_OPS = 16, MAX_D = 4;
+constexpr int MAX_CH = 16, MAX_TERMS = 48, MAX_OPS = 16, MAX_D = 4, MAX_VEC = 4;
 
 struct FusedPlan {
   const double* A[MAX_CH];
@@ -29,7 +28,13 @@ struct FusedPlan {
   int ta[MAX_TERMS], tb[MAX_TERMS], to[MAX_TERMS];  // terms sorted by channel a; to = -1 -> identity
   double ops[MAX_OPS][MAX_D * MAX_D];
   int64_t n_alpha;
+  // the same terms as the FP64 kernel takes them (fill_plan): the terms of B channel hub_b, each an A channel and a
+  // vector V O^T, summed before one stage B; and the others, sorted by A channel
+  int n_hub, hub_b, ha[MAX_TERMS], hv[MAX_TERMS];
+  int n_vec, vec_op[MAX_VEC];   // the vectors' operators (-1: identity; vector 0 is always v itself)
+  int n_direct, da[MAX_TERMS], db[MAX_TERMS], dop[MAX_TERMS];
 };
+
 
 template <int P, int DP>
 struct Shape {
@@ -39,18 +44,20 @@ struct Shape {
   static constexpr int IDX = DP * P4;              // stage-A rows idx = s*P4 + q
   static constexpr int MT = (IDX + 15) / 16;       // stage-A row tiles
   static constexpr int SLAB = KS * NT * 64;        // packed doubles per alpha
+  static constexpr int TEAMS = NT == 2 ? 6 : 4;    // teams of NT waves in a workgroup of the FP64 kernel
+  static constexpr int THREADS = 64 * TEAMS * NT;  // (at NT = 2 and 3 one workgroup is a CU's twelve waves)
 };
 
 constexpr int PACK_MAX_P = 64;
 // One alpha per workgroup step: the slab is gathered into LDS in source order (coalesced reads), then
 // written in MFMA-operand order (packed[alpha][u][n][lane] = S[16n + lane%16][4u + lane/16], zero padded).
-__global__ void __launch_bounds__(256) pack_kernel(int64_t n_alpha, int NT, int KS, CCSlabGather g,
-                                                   const double* __restrict__ src, double* __restrict__ dst) {
+__global__ void __launch_bounds__(256) pack_kernel(int64_t n_alpha, int NT, int KS, CCSlabGather g, CCSlabSum src,
+                                                   double* __restrict__ dst) {
   extern __shared__ double s[];  // P x (P + 1)
   const int P = g.P, ld = P + 1;
   const int per = KS * NT * 64;
   for (int64_t al = blockIdx.x; al < n_alpha; al += gridDim.x) {
-    cc_slab_load(g, src, al, s, ld, 1.0);
+    cc_slab_load_sum(g, src, al, s, ld);
     __syncthreads();
     double* out = dst + al * per;
     for (int r = threadIdx.x; r < per; r += blockDim.x) {
@@ -64,12 +71,11 @@ __global__ void __launch_bounds__(256) pack_kernel(int64_t n_alpha, int NT, int 
 
 // The same for slabs whose four legs all have extent D (constant index arithmetic).
 template <int D>
-__global__ void __launch_bounds__(256) pack_kernel_d(int64_t n_alpha, CCSlabGather g, const double* __restrict__ src,
-                                                     double* __restrict__ dst) {
+__global__ void __launch_bounds__(256) pack_kernel_d(int64_t n_alpha, CCSlabGather g, CCSlabSum src, double* __restrict__ dst) {
   constexpr int P = D * D, NT = (P + 15) / 16, KS = (P + 3) / 4, per = KS * NT * 64, ld = P + 1;
   __shared__ double s[P * ld];
   for (int64_t al = blockIdx.x; al < n_alpha; al += gridDim.x) {
-    cc_slab_load_d<D, 256>(g, src, al, s, ld, 1.0);
+    cc_slab_load_sum_d<D, 256>(g, src, al, s, ld);
     __syncthreads();
     double* out = dst + al * per;
     for (int r = threadIdx.x; r < per; r += blockDim.x) {
@@ -81,118 +87,147 @@ __global__ void __launch_bounds__(256) pack_kernel_d(int64_t n_alpha, CCSlabGath
   }
 }
 
-template <int P, int DP>
-__global__ void __launch_bounds__(256) fused_f64_kernel(const FusedPlan plan, const double* __restrict__ v,
-                                                        double* __restrict__ partial) {
-  using S = Shape<P, DP>;
-  constexpr int P4 = S::P4, NT = S::NT, KS = S::KS, MT = S::MT, SLAB = S::SLAB;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t gw = (int64_t)blockIdx.x * 4 + wave, nw = (int64_t)gridDim.x * 4;
-  const int64_t a0 = plan.n_alpha * gw / nw, a1 = plan.n_alpha * (gw + 1) / nw;
+// Y += X B_b for one B channel at one alpha: X[s'](p' tile, q) against all q' tiles.
+template <int P, int DP, typename F>
+__device__ __forceinline__ void fused_product(const double* __restrict__ Bp, int lane, f64x4 (&y)[Shape<P, DP>::NT][DP], F x) {
+  constexpr int NT = Shape<P, DP>::NT, KS = Shape<P, DP>::KS;
+  // B operands one K step ahead; the barrier keeps the scheduler from starting every step's loads at once, which
+  // would take more registers than three waves per SIMD leave
+  double bop[2][NT];
+#pragma unroll
+  for (int nq = 0; nq < NT; ++nq) bop[0][nq] = Bp[nq * 64 + lane];
+#pragma unroll
+  for (int u = 0; u < KS; ++u) {
+    if (u + 1 < KS) {
+#pragma unroll
+      for (int nq = 0; nq < NT; ++nq) bop[(u + 1) & 1][nq] = Bp[((u + 1) * NT + nq) * 64 + lane];
+    }
+#pragma unroll
+    for (int sp = 0; sp < DP; ++sp) {
+      const double xs = x(sp, u);
+#pragma unroll
+      for (int nq = 0; nq < NT; ++nq) y[nq][sp] = __builtin_amdgcn_mfma_f64_16x16x4f64(xs, bop[u & 1][nq], y[nq][sp], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
 
-  // stage-A A operands V^T[idx][p] (idx = 16m + lane%16, p = 4u + lane/16), stored in LDS in lane order so
-  // each read is conflict-free; the same LDS is reused for the final reduction.
+// Stage A: w[m] += V^T[16m.., :] A_a^T[:, 16np..] for one A channel at one alpha (V^T operands in LDS).
+template <int P, int DP>
+__device__ __forceinline__ void fused_stage_a(const double* __restrict__ Ap, const double* vt, int np, int lane,
+                                              f64x4 (&w)[Shape<P, DP>::MT]) {
+  constexpr int NT = Shape<P, DP>::NT, KS = Shape<P, DP>::KS, MT = Shape<P, DP>::MT;
+  double aop[KS];
+#pragma unroll
+  for (int u = 0; u < KS; ++u) aop[u] = Ap[(u * NT + np) * 64 + lane];
+#pragma unroll
+  for (int u = 0; u < KS; ++u) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      w[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(vt[(m * KS + u) * 64 + lane], aop[u], w[m], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Bound by the FP64 matrix cores.  A workgroup is TEAMS teams of NT waves; a team walks its own alpha range and wave
+// np of it owns the 16-row p' tile np, so a wave carries 2 NT accumulator tiles and three waves fit a SIMD (the loads
+// of one hide behind the products of the others; slabs are read by a team's waves at about the same time, so the
+// second and third read hit the cache).  The terms of B channel hub_b (the one with the most) take one stage B
+// together: sum_t O_t V A_t^T is stage A with the vector V O_t^T in place of V, accumulated over the terms, so it
+// costs neither vector work nor registers.  D = 6, chi = 64, transverse-field Ising: 1026 MFMAs per alpha (1674 with a
+// stage B per term of the unsummed channels), 282 -> 146 us per application (109 us at the matrix rate); Heisenberg at
+// D = 5, chi = 37: 230 -> 44 us (there the earlier fixed sixteen alpha per workgroup left two thirds of the CUs idle).
+template <int P, int DP>
+__global__ void __launch_bounds__((Shape<P, DP>::THREADS), 3) fused_f64_kernel(const FusedPlan plan, int per,
+                                                                                       const double* __restrict__ v,
+                                                                                       double* __restrict__ partial) {
+  using S = Shape<P, DP>;
+  constexpr int P4 = S::P4, NT = S::NT, KS = S::KS, MT = S::MT, SLAB = S::SLAB, TEAMS = S::TEAMS, NTH = S::THREADS;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), np = wave % NT, team = wave / NT;
+  const int64_t a0 = ((int64_t)blockIdx.x * TEAMS + team) * per, a1 = a0 + per < plan.n_alpha ? a0 + per : plan.n_alpha;
+
+  // stage-A A operands (V O^T)^T[idx][p] (idx = 16m + lane%16, p = 4u + lane/16) of every vector, stored in LDS in
+  // lane order so each read is conflict-free; the same LDS is reused for the final reduction.
   constexpr int NY = P * P * DP;
   constexpr int NVT = MT * KS * 64;
-  constexpr int NLDS = (NVT > 4 * NY) ? NVT : 4 * NY;
+  constexpr int NLDS = (MAX_VEC * NVT > TEAMS * NY) ? MAX_VEC * NVT : TEAMS * NY;
   __shared__ double lds[NLDS];
-  for (int e = threadIdx.x; e < NVT; e += 256) {
-    int l = e & 63, mu = e >> 6, u = mu % KS, m = mu / KS;
-    int idx = 16 * m + (l & 15), p = 4 * u + (l >> 4);
-    int s = idx / P4, q = idx % P4;
-    lds[e] = (s < DP && q < P && p < P) ? v[(p * P + q) * DP + s] : 0.0;
+  for (int e = threadIdx.x; e < NVT; e += NTH) {
+    const int l = e & 63, mu = e >> 6, u = mu % KS, m = mu / KS;
+    const int idx = 16 * m + (l & 15), p = 4 * u + (l >> 4), s = idx / P4, q = idx % P4;
+    const bool in = s < DP && q < P && p < P;
+    double x[DP];
+#pragma unroll
+    for (int j = 0; j < DP; ++j) x[j] = in ? v[(p * P + q) * DP + j] : 0.0;
+    for (int k = 0; k < plan.n_vec; ++k) {
+      const int o = plan.vec_op[k];
+      double t = 0.0;
+#pragma unroll
+      for (int j = 0; j < DP; ++j) t += (o < 0 ? (j == s ? 1.0 : 0.0) : in ? plan.ops[o < 0 ? 0 : o][s * DP + j] : 0.0) * x[j];
+      lds[k * NVT + e] = t;
+    }
   }
   __syncthreads();
 
-  f64x4 y[NT][NT][DP];
+  f64x4 y[NT][DP];
 #pragma unroll
-  for (int i = 0; i < NT; ++i)
+  for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int s = 0; s < DP; ++s) y[i][j][s] = (f64x4){0.0, 0.0, 0.0, 0.0};
+    for (int s = 0; s < DP; ++s) y[j][s] = (f64x4){0.0, 0.0, 0.0, 0.0};
 
   for (int64_t al = a0; al < a1; ++al) {
-    int t = 0;
-    while (t < plan.n_terms) {
-      const int a = plan.ta[t];
-      const double* Ap = plan.A[a] + al * SLAB;
-      const int t_begin = t;
-      int t_end = t;
-      while (t_end < plan.n_terms && plan.ta[t_end] == a) ++t_end;
+    f64x4 w[MT];
+    auto zero = [&]() {
 #pragma unroll
-      for (int np = 0; np < NT; ++np) {
-        // stage A for the p' tile np: w[m] = V^T[16m.., :] A_a^T[:, 16np..]
-        f64x4 w[MT];
+      for (int m = 0; m < MT; ++m) w[m] = (f64x4){0.0, 0.0, 0.0, 0.0};
+    };
+    // the lane's element of W[s P4 + 4u + lane/16][p']
+    auto wat = [&](int s, int u) { const int idx = s * P4 + 4 * u; return w[idx / 16][(idx % 16) / 4]; };
+    if (plan.n_hub > 0) {
+      zero();
+      for (int t = 0; t < plan.n_hub; ++t)
+        fused_stage_a<P, DP>(plan.A[plan.ha[t]] + al * SLAB, lds + plan.hv[t] * NVT, np, lane, w);
+      fused_product<P, DP>(plan.B[plan.hub_b] + al * SLAB, lane, y, wat);
+    }
+    for (int t = 0; t < plan.n_direct;) {
+      const int a = plan.da[t];
+      zero();
+      fused_stage_a<P, DP>(plan.A[a] + al * SLAB, lds, np, lane, w);
+      for (; t < plan.n_direct && plan.da[t] == a; ++t) {
+        const int o = plan.dop[t];
+        double oc[DP][DP];
 #pragma unroll
-        for (int m = 0; m < MT; ++m) w[m] = (f64x4){0.0, 0.0, 0.0, 0.0};
-        // the V^T operands are read from LDS at each use (the empty asm hides that the address is the
-        // same every time): keeping all of them in registers would leave too few for operand loads
-        int vo = lane;
-        __asm__ volatile("" : "+v"(vo));
+        for (int i = 0; i < DP; ++i)
 #pragma unroll
-        for (int u = 0; u < KS; ++u) {
-          double bop = Ap[(u * NT + np) * 64 + lane];
+          for (int j = 0; j < DP; ++j) oc[i][j] = (o < 0) ? (i == j ? 1.0 : 0.0) : plan.ops[o < 0 ? 0 : o][i * DP + j];
+        fused_product<P, DP>(plan.B[plan.db[t]] + al * SLAB, lane, y, [&](int sp, int u) {
+          double acc = 0.0;
 #pragma unroll
-          for (int m = 0; m < MT; ++m)
-            w[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(lds[(m * KS + u) * 64 + vo], bop, w[m], 0, 0, 0);
-        }
-        // stage B for every term of channel a, p' tile np
-        for (int tt = t_begin; tt < t_end; ++tt) {
-          const double* Bp = plan.B[plan.tb[tt]] + al * SLAB;
-          const int o = plan.to[tt];
-          double oc[DP][DP];
-#pragma unroll
-          for (int i = 0; i < DP; ++i)
-#pragma unroll
-            for (int j = 0; j < DP; ++j) oc[i][j] = (o < 0) ? (i == j ? 1.0 : 0.0) : plan.ops[o < 0 ? 0 : o][i * DP + j];
-#pragma unroll
-          for (int u = 0; u < KS; ++u) {
-            double xs[DP];
-#pragma unroll
-            for (int s = 0; s < DP; ++s) {
-              const int idx = s * P4 + 4 * u;  // the lane's row within the group is idx + lane/16
-              xs[s] = w[idx / 16][(idx % 16) / 4];
-            }
-            double x[DP];
-#pragma unroll
-            for (int sp = 0; sp < DP; ++sp) {
-              double acc = 0.0;
-#pragma unroll
-              for (int s = 0; s < DP; ++s) acc += oc[sp][s] * xs[s];
-              x[sp] = acc;
-            }
-#pragma unroll
-            for (int nq = 0; nq < NT; ++nq) {
-              double bop = Bp[(u * NT + nq) * 64 + lane];
-#pragma unroll
-              for (int sp = 0; sp < DP; ++sp)
-                y[np][nq][sp] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[sp], bop, y[np][nq][sp], 0, 0, 0);
-            }
-          }
-        }
+          for (int s = 0; s < DP; ++s) acc += oc[sp][s] * wat(s, u);
+          return acc;
+        });
       }
-      t = t_end;
     }
   }
 
-  // workgroup reduction in a fixed order: wave w writes slot w, then every thread sums slots 0..3
+  // workgroup reduction in a fixed order: team k writes slot k, then every thread sums the slots in order
   __syncthreads();
-  double* red0 = lds;
 #pragma unroll
-  for (int np = 0; np < NT; ++np)
+  for (int nq = 0; nq < NT; ++nq)
 #pragma unroll
-    for (int nq = 0; nq < NT; ++nq)
+    for (int s = 0; s < DP; ++s)
 #pragma unroll
-      for (int s = 0; s < DP; ++s)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          int pp = 16 * np + (lane >> 4) + 4 * r, qq = 16 * nq + (lane & 15);
-          if (pp < P && qq < P) red0[wave * NY + (pp * P + qq) * DP + s] = y[np][nq][s][r];
-        }
+      for (int r = 0; r < 4; ++r) {
+        int pp = 16 * np + (lane >> 4) + 4 * r, qq = 16 * nq + (lane & 15);
+        if (pp < P && qq < P) lds[team * NY + (pp * P + qq) * DP + s] = y[nq][s][r];
+      }
   __syncthreads();
-  for (int i = threadIdx.x; i < NY; i += 256)
-    partial[(int64_t)blockIdx.x * NY + i] = ((red0[i] + red0[NY + i]) + red0[2 * NY + i]) + red0[3 * NY + i];
+  for (int i = threadIdx.x; i < NY; i += NTH) {
+    double t = lds[i];
+#pragma unroll
+    for (int k = 1; k < TEAMS; ++k) t += lds[k * NY + i];
+    partial[(int64_t)blockIdx.x * NY + i] = t;
+  }
 }
 
 // y[i] = sum_g partial[g][i] in a fixed order: block = 16 consecutive outputs x 16 group slices;
@@ -352,6 +387,16 @@ __global__ void __launch_bounds__(256) fused_f32_kernel(const FusedPlan plan, co
     partial[(int64_t)blockIdx.x * NY + i] = ((lds[i] + lds[NY + i]) + lds[2 * NY + i]) + lds[3 * NY + i];
 }
 
+// alpha per team of the FP64 kernel: as many teams as fit the chip at three waves per SIMD (256 CUs x 12 waves).
+inline int64_t fused_f64_per(int64_t n_alpha, int64_t P) {
+  const int64_t teams = 3072 / ((P + 15) / 16);
+  return (n_alpha + teams - 1) / teams;
+}
+inline int64_t fused_f64_groups(int64_t n_alpha, int64_t P) {
+  const int64_t nt = (P + 15) / 16, per = fused_f64_per(n_alpha, P), teams = nt == 2 ? 6 : 4;   // Shape::TEAMS
+  return (n_alpha + teams * per - 1) / (teams * per);
+}
+
 template <int P>
 int launch_fused_f32(hipStream_t st, const FusedPlan& plan, const double* v, double* y, double* work, int groups) {
   fused_f32_kernel<P><<<groups, 256, 0, st>>>(plan, v, work);
@@ -363,12 +408,13 @@ int launch_fused_f32(hipStream_t st, const FusedPlan& plan, const double* v, dou
 }
 
 template <int P, int DP>
-int launch_fused(hipStream_t st, const FusedPlan& plan, const double* v, double* y, double* work, int groups,
-                 bool profile = true) {
+int launch_fused(hipStream_t st, const FusedPlan& plan, const double* v, double* y, double* work, bool profile = true) {
   hipEvent_t e0 = nullptr;
   int rc = profile ? cc_prof_start(st, CC_PROF_FUSED_F64, &e0) : CC_OK;
   if (rc != CC_OK) return rc;
-  fused_f64_kernel<P, DP><<<groups, 256, 0, st>>>(plan, v, work);
+  const int64_t per = fused_f64_per(plan.n_alpha, P), groups = fused_f64_groups(plan.n_alpha, P);
+  if (per > 2147483647LL) { cc_set_last_error("fused stage-3: too many slabs"); return CC_ERR_UNSUPPORTED; }
+  fused_f64_kernel<P, DP><<<(unsigned)groups, Shape<P, DP>::THREADS, 0, st>>>(plan, (int)per, v, work);
   CC_LAUNCH_CHECK();
   rc = profile ? cc_prof_stop(st, CC_PROF_FUSED_F64, e0) : CC_OK;
   if (rc != CC_OK) return rc;
@@ -378,6 +424,7 @@ int launch_fused(hipStream_t st, const FusedPlan& plan, const double* v, double*
   return CC_OK;
 }
 
+// Workgroups of the FP32 kernel.
 int fused_groups(int64_t n_alpha) {
   // four alpha per wave at the largest shapes; never more workgroups than waves of work
   int64_t g = (n_alpha + 15) / 16;
@@ -410,11 +457,11 @@ int apply_plan(hipStream_t st, const Stage3PlanHandle* h, const double* v, doubl
     return CC_ERR_UNSUPPORTED;
   }
   switch (h->P) {
-    case 4: return launch_fused<4, 2>(st, h->plan, v, y, h->work, h->groups);
-    case 9: return launch_fused<9, 2>(st, h->plan, v, y, h->work, h->groups);
-    case 16: return launch_fused<16, 2>(st, h->plan, v, y, h->work, h->groups);
-    case 25: return launch_fused<25, 2>(st, h->plan, v, y, h->work, h->groups);
-    case 36: return launch_fused<36, 2>(st, h->plan, v, y, h->work, h->groups);
+    case 4: return launch_fused<4, 2>(st, h->plan, v, y, h->work);
+    case 9: return launch_fused<9, 2>(st, h->plan, v, y, h->work);
+    case 16: return launch_fused<16, 2>(st, h->plan, v, y, h->work);
+    case 25: return launch_fused<25, 2>(st, h->plan, v, y, h->work);
+    case 36: return launch_fused<36, 2>(st, h->plan, v, y, h->work);
   }
   cc_set_last_error("fused stage-3: shape not instantiated");
   return CC_ERR_UNSUPPORTED;
@@ -445,6 +492,30 @@ int fill_plan(FusedPlan& plan, int n_a, const double* const* A_packed, int n_b, 
   for (int o = 0; o < n_ops; ++o)
     for (int e = 0; e < d * d; ++e) plan.ops[o][e] = host_ops[o * d * d + e];
   plan.n_alpha = n_alpha;
+  // the hub: the B channel with the most terms, where two of them or more save a product
+  int count[MAX_CH] = {}, hub = -1;
+  for (int t = 0; t < n_terms; ++t) ++count[term_b[t]];
+  for (int b = 0; b < n_b; ++b)
+    if (count[b] > 1 && (hub < 0 || count[b] > count[hub])) hub = b;
+  plan.hub_b = hub < 0 ? 0 : hub;
+  plan.n_vec = 1;
+  plan.vec_op[0] = -1;
+  for (int t = 0; t < n_terms; ++t) {
+    int vec = -1;
+    if (term_b[t] == hub) {
+      for (int k = 0; k < plan.n_vec; ++k)
+        if (plan.vec_op[k] == term_o[t]) vec = k;
+      if (vec < 0 && plan.n_vec < MAX_VEC) plan.vec_op[vec = plan.n_vec++] = term_o[t];
+    }
+    if (vec >= 0) {
+      plan.ha[plan.n_hub] = term_a[t];
+      plan.hv[plan.n_hub++] = vec;
+    } else {
+      plan.da[plan.n_direct] = term_a[t];
+      plan.db[plan.n_direct] = term_b[t];
+      plan.dop[plan.n_direct++] = term_o[t];
+    }
+  }
   return CC_OK;
 }
 }  // namespace
@@ -468,35 +539,45 @@ extern "C" int cc_stage3_packed_size(int64_t n_alpha, int64_t P, int64_t* out) {
 }
 
 extern "C" int cc_stage3_fused_work_size(int64_t n_alpha, int64_t P, int64_t d, int64_t* out) {
-  *out = (int64_t)fused_groups(n_alpha) * P * P * d;
+  const int64_t g32 = fused_groups(n_alpha), g64 = fused_f64_groups(n_alpha < 1 ? 1 : n_alpha, P < 1 ? 1 : P);
+  *out = (g32 > g64 ? g32 : g64) * P * P * d;   // of either kernel
   return CC_OK;
 }
 
-extern "C" int cc_stage3_pack_strided_f64(void* stream, int64_t na0, int64_t na1, int64_t d0, int64_t d1,
-                                          const int64_t* strides, const double* src, double* packed) {
+extern "C" int cc_stage3_pack_sum_f64(void* stream, int n_src, const double* const* src, const double* host_coef,
+                                      int64_t na0, int64_t na1, int64_t d0, int64_t d1, const int64_t* strides,
+                                      double* packed) {
   CCSlabMap map;
   int rc = cc_slab_map(na0, na1, d0, d1, strides, &map);
   if (rc) return rc;
+  if (n_src < 1 || n_src > CC_SLAB_SOURCES) { cc_set_last_error("pack: 1 to 8 sources"); return CC_ERR_ARG; }
   const int64_t n_alpha = na0 * na1, P = d0 * d1;
   if (P > PACK_MAX_P) { cc_set_last_error("pack: slab extent above 64"); return CC_ERR_UNSUPPORTED; }
   int NT = (int)((P + 15) / 16), KS = (int)((P + 3) / 4);
   const unsigned grid = (unsigned)(n_alpha < 16384 ? n_alpha : 16384);
   const size_t lds = (size_t)P * (P + 1) * sizeof(double);
   const CCSlabGather g = cc_slab_gather(map, d0);
+  const CCSlabSum sum = cc_slab_sum(n_src, src, host_coef);
   hipStream_t st = cc_stream(stream);
   if (d0 == map.d1 && d0 >= 2 && d0 <= 6) {
     switch (d0) {
-      case 2: pack_kernel_d<2><<<grid, 256, 0, st>>>(n_alpha, g, src, packed); break;
-      case 3: pack_kernel_d<3><<<grid, 256, 0, st>>>(n_alpha, g, src, packed); break;
-      case 4: pack_kernel_d<4><<<grid, 256, 0, st>>>(n_alpha, g, src, packed); break;
-      case 5: pack_kernel_d<5><<<grid, 256, 0, st>>>(n_alpha, g, src, packed); break;
-      default: pack_kernel_d<6><<<grid, 256, 0, st>>>(n_alpha, g, src, packed); break;
+      case 2: pack_kernel_d<2><<<grid, 256, 0, st>>>(n_alpha, g, sum, packed); break;
+      case 3: pack_kernel_d<3><<<grid, 256, 0, st>>>(n_alpha, g, sum, packed); break;
+      case 4: pack_kernel_d<4><<<grid, 256, 0, st>>>(n_alpha, g, sum, packed); break;
+      case 5: pack_kernel_d<5><<<grid, 256, 0, st>>>(n_alpha, g, sum, packed); break;
+      default: pack_kernel_d<6><<<grid, 256, 0, st>>>(n_alpha, g, sum, packed); break;
     }
   } else {
-    pack_kernel<<<grid, 256, lds, st>>>(n_alpha, NT, KS, g, src, packed);
+    pack_kernel<<<grid, 256, lds, st>>>(n_alpha, NT, KS, g, sum, packed);
   }
   CC_LAUNCH_CHECK();
   return CC_OK;
+}
+
+extern "C" int cc_stage3_pack_strided_f64(void* stream, int64_t na0, int64_t na1, int64_t d0, int64_t d1,
+                                          const int64_t* strides, const double* src, double* packed) {
+  const double one = 1.0;
+  return cc_stage3_pack_sum_f64(stream, 1, &src, &one, na0, na1, d0, d1, strides, packed);
 }
 
 extern "C" int cc_stage3_pack_f64(void* stream, int64_t n_alpha, int64_t P, const double* slabs, double* packed) {
@@ -516,13 +597,12 @@ extern "C" int cc_stage3_matvec_fused_f64(void* stream, int n_a, const double* c
   int rc = fill_plan(plan, n_a, A_packed, n_b, B_packed, n_terms, term_a, term_b, term_o, n_ops, host_ops, n_alpha, d);
   if (rc) return rc;
   hipStream_t st = cc_stream(stream);
-  int groups = fused_groups(n_alpha);
   switch (P) {
-    case 4: return launch_fused<4, 2>(st, plan, v, y, work, groups);
-    case 9: return launch_fused<9, 2>(st, plan, v, y, work, groups);
-    case 16: return launch_fused<16, 2>(st, plan, v, y, work, groups);
-    case 25: return launch_fused<25, 2>(st, plan, v, y, work, groups);
-    case 36: return launch_fused<36, 2>(st, plan, v, y, work, groups);
+    case 4: return launch_fused<4, 2>(st, plan, v, y, work);
+    case 9: return launch_fused<9, 2>(st, plan, v, y, work);
+    case 16: return launch_fused<16, 2>(st, plan, v, y, work);
+    case 25: return launch_fused<25, 2>(st, plan, v, y, work);
+    case 36: return launch_fused<36, 2>(st, plan, v, y, work);
   }
   return CC_ERR_UNSUPPORTED;
 }
@@ -568,7 +648,7 @@ extern "C" int cc_stage3_matvec_fused_f64_noalloc(void* stream, int n_a, const d
   FusedPlan plan;
   int rc = fill_plan(plan, n_a, A_packed, n_b, B_packed, n_terms, term_a, term_b, term_o, n_ops, host_ops, n_alpha, d);
   if (rc) return rc;
-  const int groups = fused_groups(n_alpha);
+  const int groups = fused_groups(n_alpha);   // the documented limit; the FP64 kernel's own partial sums always fit
   if ((int64_t)groups * P * P * d > (int64_t)CC_NOALLOC_SCRATCH_DOUBLES) {
     cc_set_last_error("noalloc stage-3: the partial sums need more than the 1048576-double (8 MiB) scratch; "
                       "use cc_stage3_matvec_fused_f64 with a workspace");
@@ -579,11 +659,11 @@ extern "C" int cc_stage3_matvec_fused_f64_noalloc(void* stream, int n_a, const d
   if (rc) return rc;
   hipStream_t st = cc_stream(stream);
   switch (P) {
-    case 4: return launch_fused<4, 2>(st, plan, v, y, scratch, groups, false);
-    case 9: return launch_fused<9, 2>(st, plan, v, y, scratch, groups, false);
-    case 16: return launch_fused<16, 2>(st, plan, v, y, scratch, groups, false);
-    case 25: return launch_fused<25, 2>(st, plan, v, y, scratch, groups, false);
-    case 36: return launch_fused<36, 2>(st, plan, v, y, scratch, groups, false);
+    case 4: return launch_fused<4, 2>(st, plan, v, y, scratch, false);
+    case 9: return launch_fused<9, 2>(st, plan, v, y, scratch, false);
+    case 16: return launch_fused<16, 2>(st, plan, v, y, scratch, false);
+    case 25: return launch_fused<25, 2>(st, plan, v, y, scratch, false);
+    case 36: return launch_fused<36, 2>(st, plan, v, y, scratch, false);
   }
   return CC_ERR_UNSUPPORTED;
 }

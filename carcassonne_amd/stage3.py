@@ -37,6 +37,56 @@ def cost_of_matrix(s2_0_shape, s2_1_shape, d):
     return int(m * x * y + m * d * d)
 
 
+MAX_SUM = 8   # channels of one sum (cc_slab_join_f64, cc_stage3_pack_sum_f64)
+
+
+def operator_groups(values):
+    """values: key -> matrix as a tuple of numbers.  Returns [(key, [(key', c)...])]: every matrix in the one group
+    whose first matrix it is an exact multiple of, values[key'] == c * values[key]."""
+    groups = []
+    for key, m in values.items():
+        for first, members in groups:
+            o = values[first]
+            k = max(range(len(o)), key=lambda i: abs(o[i]))
+            c = m[k] / o[k] if o[k] != 0 else 0.0
+            if c != 0 and all(c * x == y for x, y in zip(o, m)):
+                members.append((key, c))
+                break
+        else:
+            groups.append((key, [(key, 1.0)]))
+    return groups
+
+
+def products_of(terms):
+    """The terms (a, b, c) of one site operator as products ([(a, c)...], [(b, c)...]), a sum of A channels times a sum
+    of B channels: the channel with the most terms left takes them all as one product."""
+    left, out = list(terms), []
+    while left:
+        count = {}
+        for a, b, _ in left:
+            count[(0, a)] = count.get((0, a), 0) + 1
+            count[(1, b)] = count.get((1, b), 0) + 1
+        side, hub = max(count, key=lambda k: count[k])
+        mine = [t for t in left if t[side] == hub][:MAX_SUM]
+        left = [t for t in left if t not in mine]
+        if side == 0:
+            out.append(([(hub, 1.0)], [(b, c) for _, b, c in mine]))
+        else:
+            out.append(([(a, c) for a, _, c in mine], [(hub, 1.0)]))
+    return out
+
+
+def join_slabs(channels, coefs):
+    """sum coefs[i] * channels[i] as a contiguous (alpha, P, P) array; the channels share their leg sizes and strides."""
+    _, (na0, na1, d0, d1), st = channels[0].source()
+    out = empty((na0 * na1, d0 * d1, d0 * d1))
+    if out.numel() == 0:
+        return out
+    _lib.call("cc_slab_join_f64", stream(), len(channels), _lib.ptr_array([c.source()[0].data_ptr() for c in channels]),
+              _lib.f64_array(coefs), na0, na1, d0, d1, _lib.i64_array(st), ptr(out))
+    return out
+
+
 class _Slab:
     """One slab channel of a stage-3 operator: the stage-2 tensor t read as slab[alpha][p'][p] with
     which 0: alpha = (t0, t1) (stage2_0.join((0,1),4,5,2,3)), which 1: alpha = (t1, t0)
@@ -78,17 +128,13 @@ class _Slab:
         """(base tensor, (na0, na1, d0, d1), six strides) of the slab map."""
         st = self._st
         a0, a1 = (0, 1) if self.which == 0 else (1, 0)
-        return self._base, (self.na0, self.na1, self.shape[4], self.shape[5]), [st[a0], st[a1], st[4], st[5], st[2], st[3]]
+        return self._base, (self.na0, self.na1, self.shape[4], self.shape[5]), (st[a0], st[a1], st[4], st[5], st[2], st[3])
 
     @property
     def joined(self):
         if self._joined is None:
             if self.strided:
-                base, (na0, na1, d0, d1), st = self.source()
-                out = empty((self.n_alpha, d0 * d1, self.P))
-                _lib.call("cc_permute", stream(), _lib.CC_F64, ptr(base), ptr(out), 6,
-                          _lib.i64_array([na0, na1, d0, d1, d0, d1]), _lib.i64_array(st))
-                self._joined = HipData(out)
+                self._joined = HipData(join_slabs([self], [1.0]))
             else:
                 t = self.t
                 self._joined = t.join((0, 1), 4, 5, 2, 3) if self.which == 0 else t.join((1, 0), 4, 5, 2, 3)
@@ -149,6 +195,8 @@ class Stage3Operator:
         self.cost_of_formMatrix = sum(cost_of_matrix(a.shape, b.shape, self.d) for (a, b, _) in self.terms)
         self._work = None
         self._fused = None
+        self._formed = None     # formed.FormedOperator, once a solver has formed this operator
+        self._merge, self._joined, self._refreshed = None, {}, 0
         self.use_fused = (self.P == self.Q and all(x.strided for x in self._A + self._B) and
                           bool(_lib.load().cc_stage3_fused_supported(self.P, self.d)) and
                           self._plan_fits())
@@ -182,30 +230,102 @@ class Stage3Operator:
         rows.sort()
         return a_list, b_list, ops, rows
 
+    def _merged(self):
+        """The operator as products of summed channels: terms whose site operators are multiples of one another and
+        that share a channel are one term, c_1 A_1 (x) B (x) O + c_2 A_2 (x) B (x) O = (c_1 A_1 + c_2 A_2) (x) B (x) O.
+        The transverse-field Ising operator's seven terms become five (eight channels six), Heisenberg's fourteen
+        eight.  Returns (channels, specs, ops, rows): the distinct channels per half as _channels lists them, per half
+        the sums as tuples of (channel, coefficient), the distinct site operators, and the term table (A sum, B sum,
+        operator or -1) sorted by A sum."""
+        if self._merge is None:
+            a_list, b_list, ops, rows = self._channels()
+            legs = [[ch.source()[1:] for ch in chans] for chans in (a_list, b_list)]
+            values = {-1: tuple(float(i == j) for i in range(self.d) for j in range(self.d))}
+            values.update({o: tuple(float(x) for x in op.toArray().reshape(-1)) for o, op in enumerate(ops)})
+            groups = operator_groups(values)
+            products = []
+            for o, members in groups:
+                factor = dict(members)
+                edges = [(ia, ib, factor[oo]) for ia, _, ib, oo in rows if oo in factor]
+                for left, right in products_of(edges) if edges else ():
+                    if any(len({legs[side][i] for i, _ in part}) > 1 for side, part in ((0, left), (1, right))):
+                        products += [(((i, ci),), ((j, cj),), o) for i, ci in left for j, cj in right]
+                    else:
+                        products.append((tuple(left), tuple(right), o))
+            specs = [list(dict.fromkeys(p[side] for p in products)) for side in (0, 1)]
+            if max(map(len, specs)) > 16 or len(products) > 48:
+                specs = [[((i, 1.0),) for i in range(len(chans))] for chans in (a_list, b_list)]
+                products = [(specs[0][ia], specs[1][ib], o) for ia, _, ib, o in rows]
+            table = sorted((specs[0].index(left), specs[1].index(right), o) for left, right, o in products)
+            self._merge = (a_list, b_list), specs, ops, table
+        return self._merge
+
+    def joined(self, side, k):
+        """Sum k of half `side` as a contiguous (alpha, P, P) array, kept: it stays what it was when first asked for."""
+        t = self._joined.get((side, k))
+        if t is None:
+            channels, specs, _, _ = self._merged()
+            spec = specs[side][k]
+            parts = [channels[side][i] for i, _ in spec]
+            t = parts[0]._t if len(spec) == 1 and spec[0][1] == 1.0 else join_slabs(parts, [c for _, c in spec])
+            self._joined[(side, k)] = t
+        return t
+
+    def snapshot(self):
+        """Takes every sum of channels now (joined), so that later calls do not read the stage-2 tensors."""
+        _, specs, _, _ = self._merged()
+        for side in (0, 1):
+            for k in range(len(specs[side])):
+                self.joined(side, k)
+
+    def _pack(self, side, k, channels, out=None):
+        """Sum k of half `side` over `channels` in the fused kernel's MFMA-operand order."""
+        _, specs, _, _ = self._merged()
+        spec = specs[side][k]
+        first = channels[spec[0][0]]
+        kept = self._joined.get((side, k)) if out is None else None
+        if kept is None and out is None and len(spec) == 1 and spec[0][1] == 1.0:
+            return first.packed()
+        if out is None:
+            out = empty((_lib.query("cc_stage3_packed_size", self.n_alpha, self.P),))
+        _, (na0, na1, d0, d1), st = first.source()
+        if kept is not None:
+            P = self.P
+            _lib.call("cc_stage3_pack_strided_f64", stream(), self.n_alpha, 1, d0, d1,
+                      _lib.i64_array([P * P, 0, d1 * P, P, d1, 1]), ptr(kept), ptr(out))
+        else:
+            _lib.call("cc_stage3_pack_sum_f64", stream(), len(spec),
+                      _lib.ptr_array([channels[i].source()[0].data_ptr() for i, _ in spec]),
+                      _lib.f64_array([c for _, c in spec]), na0, na1, d0, d1, _lib.i64_array(st), ptr(out))
+        return out
+
     def refresh_fused_from(self, other):
         """Packs the channels of `other` -- an operator of the same structure (the same terms, channel
         sharing and shapes) built from new stage-2 tensors -- into this operator's packed buffers, so that
         its fused kernel and native plan apply `other` (kernels only; capturable in a HIP graph)."""
         self._ensure_fused()
+        self._formed, self._joined = None, {}     # of the environment before
+        self._refreshed += 1
         a_list, b_list, _, rows = self._channels()
         oa, ob, _, orows = other._channels()
         if ([(r[0], r[2], r[3]) for r in rows] != [(r[0], r[2], r[3]) for r in orows] or
                 [(c.n_alpha, c.P) for c in a_list + b_list] != [(c.n_alpha, c.P) for c in oa + ob]):
             raise ValueError("refresh_fused_from needs an operator of the same structure")
-        for ch, buf in zip(oa + ob, self._fused["A"] + self._fused["B"]):
-            base, (na0, na1, d0, d1), st = ch.source()
-            _lib.call("cc_stage3_pack_strided_f64", stream(), na0, na1, d0, d1, _lib.i64_array(st), ptr(base), ptr(buf))
+        _, specs, _, _ = self._merged()
+        for side, chans, bufs in ((0, oa, self._fused["A"]), (1, ob, self._fused["B"])):
+            for k, spec in enumerate(specs[side]):
+                if len({chans[i].source()[1:] for i, _ in spec}) > 1:
+                    raise ValueError("refresh_fused_from needs an operator of the same structure")
+                self._pack(side, k, chans, bufs[k])
 
     def _build_fused(self):
-        """Pack every distinct slab channel once and build the term table (sorted by A channel)."""
-        a_list, b_list, ops, rows = self._channels()
-        packs = [ch.packed() for ch in a_list + b_list]
+        """Pack every sum of slab channels once and build the term table (sorted by A channel)."""
+        channels, specs, ops, rows = self._merged()
+        A, B = ([self._pack(side, k, channels[side]) for k in range(len(specs[side]))] for side in (0, 1))
         self._fused = dict(
-            A=packs[:len(a_list)], B=packs[len(a_list):],
-            A_ptrs=_lib.ptr_array([t.data_ptr() for t in packs[:len(a_list)]]),
-            B_ptrs=_lib.ptr_array([t.data_ptr() for t in packs[len(a_list):]]),
-            ta=_lib.i32_array([r[0] for r in rows]), tb=_lib.i32_array([r[2] for r in rows]),
-            to=_lib.i32_array([r[3] for r in rows]), n_terms=len(rows), n_a=len(a_list), n_b=len(b_list),
+            A=A, B=B, A_ptrs=_lib.ptr_array([t.data_ptr() for t in A]), B_ptrs=_lib.ptr_array([t.data_ptr() for t in B]),
+            ta=_lib.i32_array([r[0] for r in rows]), tb=_lib.i32_array([r[1] for r in rows]),
+            to=_lib.i32_array([r[2] for r in rows]), n_terms=len(rows), n_a=len(A), n_b=len(B),
             n_ops=len(ops), ops=_lib.f64_array([x for o in ops for x in o.toArray().reshape(-1)]),
             work=empty((max(1, _lib.query("cc_stage3_fused_work_size", self.n_alpha, self.P, self.d)),)))
 
@@ -223,14 +343,15 @@ class Stage3Operator:
         f = self._fused
         if precision == "f32":
             if f.get("plan_f32") is None:
-                a_list, b_list, _, _ = self._channels()
+                a_list, b_list, _, rows = self._channels()
                 pa = [ch.packed_f32(0) for ch in a_list]
                 pb = [ch.packed_f32(1) for ch in b_list]
                 f["f32_slabs"] = pa + pb
                 h = ctypes.c_void_p()
-                _lib.call("cc_stage3_plan_create_f32", ctypes.byref(h), f["n_a"], _lib.ptr_array([t.data_ptr() for t in pa]),
-                          f["n_b"], _lib.ptr_array([t.data_ptr() for t in pb]), f["n_terms"], f["ta"], f["tb"], f["to"],
-                          f["n_ops"], f["ops"], self.n_alpha, self.P, self.d, ptr(f["work"]))
+                _lib.call("cc_stage3_plan_create_f32", ctypes.byref(h), len(pa), _lib.ptr_array([t.data_ptr() for t in pa]),
+                          len(pb), _lib.ptr_array([t.data_ptr() for t in pb]), len(rows), _lib.i32_array([r[0] for r in rows]),
+                          _lib.i32_array([r[2] for r in rows]), _lib.i32_array([r[3] for r in rows]), f["n_ops"], f["ops"],
+                          self.n_alpha, self.P, self.d, ptr(f["work"]))
                 f["plan_f32"] = h
             return f["plan_f32"]
         if precision != "f64":
@@ -254,6 +375,9 @@ class Stage3Operator:
 
     def apply_flat(self, x, y):
         """y = H x for flat device tensors of length n (torch float64)."""
+        if self._formed is not None and self._formed.valid():
+            self._formed.apply_flat(x, y)
+            return
         if self.use_fused:
             self._ensure_fused()
             f = self._fused

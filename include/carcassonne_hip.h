@@ -151,6 +151,10 @@ int cc_stage3_pack_f64(void* stream, int64_t n_alpha, int64_t P, const double* s
  * tensors/_2d/dense.py:115-173) and the packing in one pass (P <= 64). */
 int cc_stage3_pack_strided_f64(void* stream, int64_t na0, int64_t na1, int64_t d0, int64_t d1, const int64_t* strides,
                                const double* src, double* packed);
+/* cc_stage3_pack_strided_f64 of a weighted sum of channels, sum_i coef[i] src_i, 1 <= n_src <= 8, read through one slab
+ * map: a term (c_1 A_1 + c_2 A_2) (x) B (x) O costs what one of its two terms costs. */
+int cc_stage3_pack_sum_f64(void* stream, int n_src, const double* const* src, const double* host_coef, int64_t na0,
+                           int64_t na1, int64_t d0, int64_t d1, const int64_t* strides, double* packed);
 int cc_stage3_matvec_fused_f64(void* stream, int n_a, const double* const* A_packed, int n_b,
                                const double* const* B_packed, int n_terms, const int* term_a,
                                const int* term_b, const int* term_o, int n_ops, const double* host_ops,
@@ -196,6 +200,30 @@ int cc_stage3_plan_create(void** out, int n_a, const double* const* A_packed, in
                           int64_t n_alpha, int64_t P, int64_t d, double* work);
 int cc_stage3_plan_apply(void* stream, const void* plan, const double* x, double* y);
 int cc_stage3_plan_destroy(void* plan);
+
+/* ---- the stage-3 operator formed once as dense matrices -----------------------------
+ * H = sum_g O_g (x) G_g over the environment legs, for solves that apply H many times (the cost rule of
+ * Multiplier.isCheaperToFormMatrix, utils.py:203-206; the matrices of formDenseStage3_formMatrix,
+ * tensors/_2d/dense.py:176-203).
+ *
+ * out[alpha][p'][p] = sum_i coef[i] src_i read through one slab map (the sources share their leg sizes and strides,
+ * as cc_stage3_pack_strided_f64): the joined slab array of a channel, or of a sum of channels; 1 <= n_src <= 8. */
+int cc_slab_join_f64(void* stream, int n_src, const double* const* src, const double* host_coef, int64_t na0, int64_t na1,
+                     int64_t d0, int64_t d1, const int64_t* strides, double* out);
+/* out[g] (PQ x PQ, row-major over (p', q') and (p, q)) = sum over the products i in [group_begin[g], group_begin[g + 1])
+ * and alpha of A_i[alpha][p'][p] B_i[alpha][q'][q], slabs joined as above; at most 16 products, P and Q at most 4096.
+ * `work` holds cc_form_work_size doubles (max_products: the most products of one group). */
+int cc_form_work_size(int n_groups, int max_products, int64_t n_alpha, int64_t P, int64_t Q, int64_t* out);
+int cc_form_f64(void* stream, int n_groups, const int* group_begin, const double* const* A, const double* const* B,
+                int64_t n_alpha, int64_t P, int64_t Q, double* out, double* work);
+/* K[i] = W G[i] W^T for n_mats n x n matrices, W lower triangular and given as its transpose Wt; work as large as G. */
+int cc_whiten_f64(void* stream, int64_t n, int n_mats, const double* G, const double* Wt, double* K, double* work);
+/* Plan of y[e][s'] = sum_g sum_s O_g[s'][s] (M_g x)[e][s] + sum_s id[s'][s] x[e][s] (host_id null: no such term) for
+ * n_env x n_env matrices M_g, d = 2, at most 5 of them; the matrices stay caller-owned. */
+int cc_formed_plan_create(void** out, int64_t n_env, int64_t d, int n_mats, const double* const* mats,
+                          const double* host_ops, const double* host_id);
+int cc_formed_plan_apply(void* stream, const void* plan, const double* x, double* y);
+int cc_formed_plan_destroy(void* plan);
 
 /* Timing of the stage-3 kernels: between begin and end every launch of the FP64 fused kernel (kind 0)
  * and of the low-precision kernel (kind 1) is bracketed by HIP events on its stream; end fills
@@ -297,6 +325,11 @@ int cc_stage3_lp_plan_destroy(void* plan);
 int cc_lanczos_lp(void* stream, const void* lp_plan, int64_t n_env, int64_t d, const double* L, const double* Lt,
                   const double* W, const double* Wt, const double* x0, double tol_residual, double tol_energy,
                   int max_iter, int check_every, double* work, double* x_out, double* host_result);
+/* cc_lanczos_f64 with the operator given as a plan of whitened matrices (cc_whiten_f64): one product per step, no
+ * whitening products.  Same vectors, recurrence, checks and results. */
+int cc_lanczos_formed_f64(void* stream, const void* formed_plan, int64_t n_env, int64_t d, const double* Lt, const double* Wt,
+                          const double* x0, double tol_residual, double tol_energy, int max_iter, int check_every,
+                          double* work, double* x_out, double* host_result);
 
 /* Jacobi-Davidson refinement pieces (FP64):
  * out[j*stride_out] = U[j] . v for j < k;  out = sum_j c[j] U[j];  lowest eigenpair of the k x k
