@@ -1,0 +1,113 @@
+"""The stage-3 operator of one solve formed as dense matrices over the environment legs.
+
+    H = sum_t A_t (x) B_t (x) O_t = sum_g O_g (x) G_g,    G_g = sum over the terms with operator O_g of A_t (x) B_t
+
+with one group per distinct site operator (up to a factor) and the terms summed over shared channels first
+(Stage3Operator._merged).  The reference forms the matrix of an operator when enough multiplications follow
+(Multiplier.isCheaperToFormMatrix, carcassonne/utils.py:203-206; formDenseStage3_formMatrix,
+carcassonne/tensors/_2d/dense.py:176-203); here the eigensolvers do, in FP64.  The product of the identity channels is
+the normalization matrix N: it is not formed again, and in whitened form (W N W^T = 1 for N = L L^T, W = L^-1) it is
+the identity.
+"""
+import ctypes
+
+from . import _lib
+from .device import empty, ptr, stream
+
+MAX_PRODUCTS, MAX_MATRICES = 16, 4
+
+
+class FormedOperator:
+    """The formed matrices of a stage-3 operator, kept on it: apply_flat(x, y) is y = H x.  `factor`: the normalization
+    factor of the same environment, whose matrix is the identity channels' product."""
+
+    @staticmethod
+    def of(h_operator, n_operator, factor):
+        """The operator's formed matrices, made on the first call; None where it has no such form (no fused shape, or
+        more distinct site operators or products than one call takes)."""
+        f = h_operator._formed
+        if f is None or not f.valid() or f.norm_channels != (n_operator._A[0], n_operator._B[0]):
+            layout = FormedOperator._layout(h_operator, n_operator)
+            f = h_operator._formed = FormedOperator(h_operator, n_operator, factor, layout) if layout is not None else None
+        return f
+
+    @staticmethod
+    def _layout(h_operator, n_operator):
+        """([(O_g, [(A sum, B sum)...])...], identity): the matrices to form, by site operator, and the site operator
+        of the identity channels' product (None: there is no such term)."""
+        if not h_operator.use_fused or h_operator.d != 2:
+            return None
+        channels, specs, ops, rows = h_operator._merged()
+        values = [tuple(float(x) for x in o.toArray().reshape(-1)) for o in ops] + [(1.0, 0.0, 0.0, 1.0)]   # [-1]: 1
+        groups, identity = {}, None
+        for a, b, o in rows:
+            left, right = specs[0][a], specs[1][b]
+            if len(left) == len(right) == 1 and channels[0][left[0][0]] is n_operator._A[0] \
+                    and channels[1][right[0][0]] is n_operator._B[0]:
+                c = left[0][1] * right[0][1]
+                identity = [x + c * y for x, y in zip(identity or (0.0,) * 4, values[o])]
+            else:
+                groups.setdefault(o, []).append((a, b))
+        if len(groups) > MAX_MATRICES or sum(map(len, groups.values())) > MAX_PRODUCTS or (not groups and identity is None):
+            return None
+        return [(values[o], products) for o, products in groups.items()], identity
+
+    def __init__(self, h_operator, n_operator, factor, layout):
+        self.n_env, self.d = h_operator.n // h_operator.d, h_operator.d
+        groups, self.identity = layout
+        self.ops = [O for O, _ in groups]
+        self.norm_channels = (n_operator._A[0], n_operator._B[0])
+        self.factor, self._version = factor, factor.version
+        self._plan = None
+        na, P = h_operator.n_alpha, h_operator.P
+        self.G = empty((len(groups), self.n_env, self.n_env))
+        if groups:
+            A = [h_operator.joined(0, a) for _, products in groups for a, _ in products]
+            B = [h_operator.joined(1, b) for _, products in groups for _, b in products]
+            begin = [0]
+            for _, products in groups:
+                begin.append(begin[-1] + len(products))
+            work = empty((_lib.query("cc_form_work_size", len(groups), max(len(p) for _, p in groups), na, P, P),))
+            _lib.call("cc_form_f64", stream(), len(groups), _lib.i32_array(begin),
+                      _lib.ptr_array([t.data_ptr() for t in A]), _lib.ptr_array([t.data_ptr() for t in B]), na, P, P,
+                      ptr(self.G), ptr(work))
+
+    def valid(self):
+        """Whether the factor still holds the environment this operator was formed from."""
+        return self.factor.version == self._version
+
+    def apply_flat(self, x, y):
+        if self._plan is None:
+            mats, ops = [self.G[g] for g in range(len(self.ops))], list(self.ops)
+            if self.identity is not None:
+                mats, ops = mats + [self.factor.N_env], ops + [self.identity]
+            self._plan = FormedPlan(self.n_env, self.d, mats, ops, None)
+        self._plan.apply(x, y)
+
+    def whitened(self, factor):
+        """The plan of W H W^T with the factor's W = L^-1 (two triangular products per matrix)."""
+        K = empty(self.G.shape)
+        if self.ops:
+            work = empty(self.G.shape)
+            _lib.call("cc_whiten_f64", stream(), self.n_env, len(self.ops), ptr(self.G), ptr(factor.Wt), ptr(K), ptr(work))
+        return FormedPlan(self.n_env, self.d, [K[g] for g in range(len(self.ops))], self.ops, self.identity)
+
+
+class FormedPlan:
+    """A native plan (cc_formed_plan_create) of sum_g O_g (x) M_g + identity (x) 1, holding its matrices."""
+
+    def __init__(self, n_env, d, mats, ops, identity):
+        self.mats, self.handle = mats, ctypes.c_void_p()
+        _lib.call("cc_formed_plan_create", ctypes.byref(self.handle), n_env, d, len(mats),
+                  _lib.ptr_array([m.data_ptr() for m in mats]), _lib.f64_array([x for O in ops for x in O]),
+                  _lib.f64_array(identity) if identity is not None else None)
+
+    def apply(self, x, y):
+        _lib.call("cc_formed_plan_apply", stream(), self.handle, ptr(x), ptr(y))
+
+    def __del__(self):
+        if getattr(self, "handle", None):
+            try:
+                _lib.load().cc_formed_plan_destroy(self.handle)
+            except Exception:
+                pass

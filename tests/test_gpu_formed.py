@@ -1,0 +1,86 @@
+"""The formed stage-3 operator against the slab path: application, whitened application and the whole solve, over
+center bonds 2..6 and environment bonds whose squares are not multiples of the K step (16).  Tolerance: FP64 sums of
+at most 2^17 products per entry in another order, a few units of 1e-16 times their square root at most; 1e-13."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _operators(D, chi, model, seed, one_site=None):
+    from carcassonne_amd import pipeline, synthetic as syn
+    c, s, st = syn.make_environment(D, chi, model=model, seed=seed, noise=8.0)
+    op = syn.operator_center(model)
+    if one_site is not None:
+        op[("O",)] = one_site
+    H, N = pipeline.multipliers(*pipeline.device_environment(c, s, op), graph=False)
+    return H.operator, N.operator, torch.from_numpy(st.ravel()).cuda()
+
+
+def _rel(a, b):
+    return float((a - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("D,chi,model,one_site", [
+    (2, 3, "ising", None), (2, 8, "heisenberg", None), (3, 5, "ising", np.array([[0.5, 0.0], [0.0, -1.5]])),
+    (3, 13, "heisenberg", np.array([[0.0, 1.0], [1.0, 0.0]])), (4, 9, "ising", None), (5, 7, "heisenberg", None),
+    (6, 6, "ising", np.array([[0.3, 0.2], [0.2, -0.3]])), (6, 21, "heisenberg", None)])
+def test_formed_operator_matches_slab_path(gpu, D, chi, model, one_site):
+    from carcassonne_amd import _lib
+    from carcassonne_amd.device import ptr, stream
+    from carcassonne_amd.formed import FormedOperator
+    from carcassonne_amd.solver import NormalizationFactor
+    H, N, x = _operators(D, chi, model, 7, one_site)
+    want, got, norm_want, norm_got = (torch.empty_like(x) for _ in range(4))
+    H.apply_generic_flat(x, want)
+    factor = NormalizationFactor(N)
+    N.apply_generic_flat(x, norm_want)
+    factor.apply_n(x, norm_got)
+    assert _rel(norm_got, norm_want) < 1e-13
+    formed = FormedOperator.of(H, N, factor)
+    assert formed is not None
+    formed.apply_flat(x, got)
+    assert _rel(got, want) < 1e-13
+    # W H W^T x, the whitening products applied around the slab path
+    t, h, w = torch.empty_like(x), torch.empty_like(x), torch.empty_like(x)
+    _lib.call("cc_skinny_f64", stream(), factor.n_env, 2, ptr(factor.Wt), 2, ptr(x), ptr(t))
+    H.apply_generic_flat(t, h)
+    _lib.call("cc_skinny_f64", stream(), factor.n_env, 1, ptr(factor.W), 2, ptr(h), ptr(w))
+    formed.whitened(factor).apply(x, got)
+    assert _rel(got, w) < 1e-12                            # cond(N) of these environments is below 10
+
+
+@pytest.mark.parametrize("D,chi,model", [(2, 5, "ising"), (4, 11, "heisenberg"), (6, 10, "ising")])
+def test_formed_solve_matches_slab_solve(gpu, D, chi, model):
+    from carcassonne_amd.solver import GroundStateSolver, NormalizationFactor
+    H, N, x0 = _operators(D, chi, model, 3)
+    formed = GroundStateSolver(H, N)
+    before = formed.rayleigh_quotient(x0)                  # the slabs
+    x, theta, _, _ = formed.solve(x0, check_every=4)
+    energy = formed.rayleigh_quotient(x)
+    H2, N2, _ = _operators(D, chi, model, 3)
+    slabs = GroundStateSolver(H2, N2, factor=NormalizationFactor(N2))     # a factor from outside: the slab path
+    assert H._formed is not None and H2._formed is None
+    assert abs(before - formed.rayleigh_quotient(x0)) <= 1e-12 * abs(before)
+    y, theta2, _, _ = slabs.solve(x0, check_every=4)
+    assert abs(theta - theta2) <= 1e-12 * abs(theta2)
+    assert abs(energy - slabs.rayleigh_quotient(y)) <= 1e-12 * abs(energy)
+
+
+def test_formed_operator_follows_its_environment(gpu):
+    """A factor or operator refreshed from another environment drops the matrices formed before."""
+    from carcassonne_amd.solver import GroundStateSolver
+    H, N, x0 = _operators(3, 6, "ising", 1)
+    H2, N2, _ = _operators(3, 6, "ising", 2)
+    solver = GroundStateSolver(H, N)
+    solver.solve(x0)
+    solver.factor.refresh(N2)
+    H.refresh_fused_from(H2)
+    want, got = torch.empty_like(x0), torch.empty_like(x0)
+    H2.apply_generic_flat(x0, want)
+    H.apply_flat(x0, got)
+    assert _rel(got, want) < 1e-13
+    _, theta, _, _ = solver.solve(x0)
+    _, theta2, _, _ = GroundStateSolver(H2, N2).solve(x0)
+    assert abs(theta - theta2) <= 1e-11 * abs(theta2)
