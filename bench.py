@@ -9,9 +9,9 @@ eigensolve to a 1e-10 relative energy, and the FP64 Rayleigh quotient of the res
 checked against the oracle's eigh energy (tests/golden).
 
 Two forms are timed on the same inputs:
-  * mixed-f16 (the headline `value`): FP16 stage-3 matvecs with FP32 accumulation inside the Lanczos,
-    FP64 Jacobi-Davidson refinement, FP64 Rayleigh-Ritz energy;
-  * fp64: the plain FP64 Lanczos form (`plain_fp64_*` fields).
+  * mixed (the headline `value`): the operator formed in FP64, FP32 copies of its whitened matrices inside the
+    Lanczos and the correction equation, FP64 Jacobi-Davidson refinement, FP64 Rayleigh-Ritz energy;
+  * fp64: the plain FP64 Lanczos form on the same formed operator (`plain_fp64_*` fields).
 """
 import argparse
 import json
@@ -26,19 +26,7 @@ WORKLOAD = dict(D=6, chi=64, d=2, model="ising", h=3.0, seed=0)
 PEAK_FP64_TFLOPS = 78.6
 PEAK_HBM_GBS = 8000.0
 COPY_CALIBRATION_DOUBLES = 64 << 20   # 512 MiB read + 512 MiB written per launch
-TIMING_EVERY = 8   # stage-3 launches per HIP-event-timed launch inside the timed region
-
-
-def measured_traffic(kernel_key):
-    """HBM bytes per launch of a kernel from the committed rocprofv3 --pmc summaries (FETCH_SIZE and
-    WRITE_SIZE, each scaled by what the counter reads for a copy kernel of known size), or None."""
-    path = os.path.join(ROOT, "profiles", "traffic.json")
-    try:
-        with open(path) as f:
-            t = json.load(f)[kernel_key]
-    except (OSError, KeyError, ValueError):
-        return None
-    return 1024.0 * (t["fetch_kib_per_launch"] * t["fetch_factor"] + t["write_kib_per_launch"] * t["write_factor"])
+TIMING_EVERY = 8   # formed-operator products per HIP-event-timed one inside the timed region
 
 
 def golden_energy():
@@ -218,6 +206,25 @@ def isolated_matvecs(op, x0, reps=50):
             "note": "one application = the fused kernel + the fixed-order FP64 sum of its workgroup partials"}
 
 
+def isolated_formation(op, reps=5):
+    """Back-to-back formations of the operator's dense matrices (cc_form_f64: the products and the sum of their
+    parts) from its joined slabs: milliseconds, and TFLOP/s of 2 n_alpha P^4 per product."""
+    import torch
+    formed = op._formed
+    st = torch.cuda.current_stream()
+    formed._form(op.joined)
+    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    e0.record(st)
+    for _ in range(reps):
+        formed._form(op.joined)
+    e1.record(st)
+    e1.synchronize()
+    ms = e0.elapsed_time(e1) / reps
+    products = sum(len(p) for _, p in formed._groups)
+    flops = 2 * products * op.n_alpha * op.P ** 4
+    return {"ms": ms, "products": products, "flops": flops, "tflops": flops / (ms * 1e-3) / 1e12}
+
+
 def plain_gpu_d4_chi32(seed=0):
     """The plain GPU workload: TFIM with h drawn from U[2.5, 3.5] (seeded), D=4, chi=32: isolated H matvecs/s
     (FP64 and FP32 operands) and the whitened Lanczos to a 1e-10 Ritz residual in both, each from the same
@@ -331,14 +338,14 @@ def main():
         for _ in range(warmup):
             fn()
         synchronize()
-        # HIP events on every TIMING_EVERY-th stage-3 launch of each kind (launches of one kind do the same work)
+        # HIP events on every TIMING_EVERY-th launch of each kind
         _lib.call("cc_profile_begin_sampled", TIMING_EVERY)
         t0 = time.perf_counter()
         results = [fn() for _ in range(steps)]
         synchronize()
         t1 = time.perf_counter()
-        kms, launches = _lib.f64_array([0, 0]), _lib.i64_array([0, 0])
-        _lib.call("cc_profile_end", 2, kms, launches)
+        kms, launches = _lib.f64_array([0, 0, 0]), _lib.i64_array([0, 0, 0])
+        _lib.call("cc_profile_end", 3, kms, launches)
         return (t1 - t0) * 1e3 / steps, results[-1], list(kms), list(launches)
 
     out = {}
@@ -346,34 +353,29 @@ def main():
         ms, r, kms, nl = run(lambda: pipeline.solve(corners, sides, op_center, x0), args.steps, args.warmup)
         r_fp64 = r
         op = r["operator"]
-        flops = pipeline.flops_per_matvec(op)
-        kernel_ms = kms[0] / max(1, nl[0])
+        product_bytes = len(op._formed.ops) * (op.n // op.d) ** 2 * 8 + 2 * op.n * 8
+        product_ms = kms[2] / max(1, nl[2])
         out["fp64"] = dict(ms=ms, energy=r["energy"], err=abs(r["energy"] - e_ref) / abs(e_ref),
-                           iterations=r["iterations"], kernel_ms=kernel_ms, launches=nl[0], flops=flops,
-                           tflops=flops / (kernel_ms * 1e-3) / 1e12, terms=len(op._A))
+                           iterations=r["iterations"], product_ms=product_ms, launches=nl[2], bytes=product_bytes,
+                           gbs=product_bytes / max(product_ms * 1e-3, 1e-12) / 1e9, terms=len(op._A))
     if args.form in ("both", "mixed"):
         ms, r, kms, nl = run(lambda: pipeline.solve_mixed(corners, sides, op_center, x0, dtype="f16"),
                              args.steps, args.warmup)
-        lp = r["lp_operator"]
-        kernel_ms = kms[1] / max(1, nl[1])
-        lp_bytes = lp.bytes_per_matvec
         out["mixed"] = dict(ms=ms, energy=r["energy"], err=abs(r["energy"] - e_ref) / abs(e_ref),
-                            iterations=r["iterations"], info=r["info"], kernel_ms=kernel_ms, launches=nl[1],
-                            fp64_kernel_ms=kms[0] / max(1, nl[0]), fp64_launches=nl[0], bytes=lp_bytes,
-                            gbs=lp_bytes / (kernel_ms * 1e-3) / 1e9, flops=pipeline.flops_per_matvec(r["operator"]),
-                            kernel="lp_kernel<36,2,{},{}-split>".format(lp.dtype, lp.split))
+                            iterations=r["iterations"], info=r["info"], product_ms=kms[2] / max(1, nl[2]), launches=nl[2])
+    formation = isolated_formation(r["operator"])
 
     if "fp64" in out:
         out["isolated"] = isolated_matvecs(r_fp64["operator"], x0)
         out["plain_gpu_d4"] = plain_gpu_d4_chi32()
 
     head = out.get("mixed") or out["fp64"]
-    form = "mixed-f16" if "mixed" in out else "fp64-lanczos"
+    form = "mixed" if "mixed" in out else "fp64-lanczos"
     line = {
         "metric": "ground-state solves/sec at D=6,chi=64 to 1e-10 rel. energy vs plain FP64 GPU",
         "value": 1e3 / head["ms"], "unit": "solves/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": head["ms"], "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "f16+f64" if form == "mixed-f16" else "f64",
+        "dtype": "f64",
         "data": "synthetic (seeded environment, carcassonne_amd.synthetic seed 0)",
         "config": {"workload": "2D TFIM h=3.0, D=6, chi=64, d=2, w=3; one solve = stage 1/2 + normalization "
                                "factor + eigensolve to 1e-10 rel. energy + FP64 Rayleigh quotient",
@@ -388,27 +390,19 @@ def main():
         f = out["fp64"]
         line.update(plain_fp64_solves_per_s=1e3 / f["ms"], plain_fp64_ms_per_solve=f["ms"],
                     plain_fp64_energy_rel_err=f["err"], plain_fp64_lanczos_iterations=f["iterations"],
-                    plain_fp64_matvec_kernel_ms=f["kernel_ms"], plain_fp64_matvec_tflops=f["tflops"],
-                    plain_fp64_matvec_frac_of_fp64_peak=f["tflops"] / PEAK_FP64_TFLOPS)
+                    plain_fp64_product_ms=f["product_ms"], plain_fp64_product_gbs=f["gbs"])
     if "mixed" in out:
         m = out["mixed"]
-        line.update(mixed_lowprec_iterations=m["iterations"], mixed_info=m["info"],
-                    lp_matvec_kernel_ms=m["kernel_ms"], lp_matvec_launches_timed=m["launches"],
-                    lp_matvec_timed_every=TIMING_EVERY,
-                    lp_matvec_effective_tflops=m["flops"] / (m["kernel_ms"] * 1e-3) / 1e12)
+        line.update(mixed_lowprec_iterations=m["iterations"], mixed_info=m["info"], mixed_product_ms=m["product_ms"],
+                    products_timed=m["launches"], products_timed_every=TIMING_EVERY)
         if "fp64" in out:
             line["speedup_vs_plain_fp64"] = out["fp64"]["ms"] / m["ms"]
-        line["roofline"] = {"bound": "hbm", "achieved": m["gbs"], "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                            "frac": m["gbs"] / PEAK_HBM_GBS,
-                            "traffic": measured_traffic(m["kernel"] + " D=6 chi=64"),
-                            "kernel": m["kernel"] + " (stage-3 matvec, FP16 slabs)",
-                            "algorithmic_bytes_per_launch": m["bytes"]}
-    else:
-        f = out["fp64"]
-        line["roofline"] = {"bound": "mfma", "achieved": f["tflops"], "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
-                            "frac": f["tflops"] / PEAK_FP64_TFLOPS, "traffic": None,
-                            "kernel": "fused_f64_kernel<36,2> (stage-3 matvec)",
-                            "algorithmic_flops_per_launch": f["flops"]}
+    line["formation"] = formation
+    # the solve's largest kernel: the formation of the dense matrices
+    line["roofline"] = {"bound": "mfma", "achieved": formation["tflops"], "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
+                        "frac": formation["tflops"] / PEAK_FP64_TFLOPS, "traffic": None,
+                        "kernel": "form_kernel + form_reduce_kernel (formation of the dense operator, FP64)",
+                        "algorithmic_flops_per_launch": formation["flops"]}
     if "isolated" in out:
         line["isolated_matvecs_d6_chi64"] = out["isolated"]
         line["plain_gpu_d4_chi32"] = out["plain_gpu_d4"]

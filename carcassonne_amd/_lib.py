@@ -54,6 +54,10 @@ SIGNATURES = {
     "cc_form_f64": [_vp, _i32, _pi32, _pvp, _pvp, _i64, _i64, _i64, _vp, _vp],
     "cc_whiten_f64": [_vp, _i64, _i32, _vp, _vp, _vp, _vp],
     "cc_formed_plan_create": [ctypes.POINTER(ctypes.c_void_p), _i64, _i64, _i32, _pvp, _pf64, _vp],
+    "cc_formed_plan_create_f32": [ctypes.POINTER(ctypes.c_void_p), _i64, _i64, _i32, _pvp, _pf64, _vp],
+    "cc_jd_correction_formed": [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp],
+    "cc_jd_project_f64": [_vp, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
+    "cc_jd_expand_f64": [_vp, _i32, _i64, _vp, _vp, _vp],
     "cc_formed_plan_apply": [_vp, _vp, _vp, _vp],
     "cc_formed_plan_destroy": [_vp],
     "cc_lanczos_formed_f64": [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _f64, _f64, _i32, _i32, _vp, _vp, _pf64],

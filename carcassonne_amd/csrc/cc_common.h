@@ -54,7 +54,7 @@ int cc_internal_gemm_upper(hipStream_t st, int64_t batch, int64_t n, const doubl
 // Launch timing (between cc_profile_begin[_sampled] and cc_profile_end, single-threaded use): a kernel
 // launch is bracketed by cc_prof_start / cc_prof_stop, which record HIP events on its stream when timing
 // is on and the launch is one of the sampled ones of its kind (e0 stays null otherwise).
-enum { CC_PROF_FUSED_F64 = 0, CC_PROF_LP = 1, CC_PROF_KINDS = 2 };
+enum { CC_PROF_FUSED_F64 = 0, CC_PROF_LP = 1, CC_PROF_FORMED = 2, CC_PROF_KINDS = 3 };
 int cc_prof_start(hipStream_t st, int kind, hipEvent_t* e0);
 int cc_prof_stop(hipStream_t st, int kind, hipEvent_t e0);
 

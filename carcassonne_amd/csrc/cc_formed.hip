@@ -179,51 +179,33 @@ int form_split(int n_groups, int max_products, int64_t n_alpha, int64_t P, int64
 
 // ---- application ------------------------------------------------------------------------------------------------
 struct FormedPlan {
-  int n_env, n_mats, has_id;
-  const double* mat[FORM_MAX];
+  int n_env, n_mats, has_id, f32;   // f32: the matrices are FP32 (products and sums stay FP64)
+  const void* mat[FORM_MAX];
   double op[FORM_MAX][4];   // O_g[s'][s], d = 2
   double id[4];             // coefficient of the identity over the environment legs
 };
 
-// y[e][s'] = sum_g sum_s O_g[s'][s] sum_f M_g[e][f] x[f][s]  (+ sum_s id[s'][s] x[e][s]): one wave per row e, the
-// row's loads of all matrices in flight before their products.  Bound by reading the matrices.
-template <int NG>
+// y[e][s'] = sum_g sum_s O_g[s'][s] sum_f M_g[e][f] x[f][s]  (+ sum_s id[s'][s] x[e][s]): one wave per row e, U column
+// steps of 64 with all their loads in flight before the products.  Bound by reading the matrices (27 MB for two FP64
+// matrices at D = 6: 7.5 us, 3.6 TB/s; a workgroup's rows stay on one XCD from launch to launch).
+template <typename T, int NG>
 __global__ void __launch_bounds__(256) formed_apply_kernel(FormedPlan f, const double* __restrict__ x, double* __restrict__ y) {
   const int lane = threadIdx.x & 63, n = f.n_env;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= n) return;
   double acc[NG][2];
-  const double* m[NG];
+  const T* m[NG];
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     acc[g][0] = acc[g][1] = 0.0;
-    m[g] = f.mat[g] + (int64_t)row * n;
+    m[g] = static_cast<const T*>(f.mat[g]) + (int64_t)row * n;
   }
   constexpr int U = NG <= 2 ? 8 : 4;
-  int c = lane;
-  for (; c + 64 * (U - 1) < n; c += 64 * U) {
-    double v[U][NG];
+  for (int c = lane; c < n; c += 64 * U) {
+    T v[U][NG];
     double xv[U][2];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int g = 0; g < NG; ++g) v[u][g] = m[g][c + 64 * u];
-      xv[u][0] = x[2 * (c + 64 * u)];
-      xv[u][1] = x[2 * (c + 64 * u) + 1];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        acc[g][0] += v[u][g] * xv[u][0];
-        acc[g][1] += v[u][g] * xv[u][1];
-      }
-  }
-  {
-    double v[U][NG];
-    double xv[U][2];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {   // the rest of the row: clamped index, masked value
+    for (int u = 0; u < U; ++u) {   // past the row's end: clamped index, masked value
       const int cc = c + 64 * u < n ? c + 64 * u : n - 1;
 #pragma unroll
       for (int g = 0; g < NG; ++g) v[u][g] = m[g][cc];
@@ -235,8 +217,8 @@ __global__ void __launch_bounds__(256) formed_apply_kernel(FormedPlan f, const d
       if (c + 64 * u < n) {
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
-          acc[g][0] += v[u][g] * xv[u][0];
-          acc[g][1] += v[u][g] * xv[u][1];
+          acc[g][0] += (double)v[u][g] * xv[u][0];
+          acc[g][1] += (double)v[u][g] * xv[u][1];
         }
       }
   }
@@ -261,19 +243,27 @@ __global__ void formed_identity_kernel(FormedPlan f, const double* __restrict__ 
   if (i < 2 * f.n_env) y[i] = f.id[(i & 1) * 2] * x[i & ~1] + f.id[(i & 1) * 2 + 1] * x[i | 1];
 }
 
-int formed_apply(hipStream_t st, const FormedPlan& f, const double* x, double* y) {
+template <typename T>
+int formed_launch(hipStream_t st, const FormedPlan& f, const double* x, double* y) {
   const unsigned grid = (unsigned)((f.n_env + 3) / 4);
   switch (f.n_mats) {
     case 0: formed_identity_kernel<<<(unsigned)((2 * f.n_env + 255) / 256), 256, 0, st>>>(f, x, y); break;
-    case 1: formed_apply_kernel<1><<<grid, 256, 0, st>>>(f, x, y); break;
-    case 2: formed_apply_kernel<2><<<grid, 256, 0, st>>>(f, x, y); break;
-    case 3: formed_apply_kernel<3><<<grid, 256, 0, st>>>(f, x, y); break;
-    case 4: formed_apply_kernel<4><<<grid, 256, 0, st>>>(f, x, y); break;
-    case 5: formed_apply_kernel<5><<<grid, 256, 0, st>>>(f, x, y); break;
+    case 1: formed_apply_kernel<T, 1><<<grid, 256, 0, st>>>(f, x, y); break;
+    case 2: formed_apply_kernel<T, 2><<<grid, 256, 0, st>>>(f, x, y); break;
+    case 3: formed_apply_kernel<T, 3><<<grid, 256, 0, st>>>(f, x, y); break;
+    case 4: formed_apply_kernel<T, 4><<<grid, 256, 0, st>>>(f, x, y); break;
+    case 5: formed_apply_kernel<T, 5><<<grid, 256, 0, st>>>(f, x, y); break;
     default: cc_set_last_error("formed operator: at most 5 matrices"); return CC_ERR_UNSUPPORTED;
   }
   CC_LAUNCH_CHECK();
   return CC_OK;
+}
+int formed_apply(hipStream_t st, const FormedPlan& f, const double* x, double* y) {
+  hipEvent_t e0 = nullptr;
+  int rc = cc_prof_start(st, CC_PROF_FORMED, &e0);
+  if (rc) return rc;
+  rc = f.f32 ? formed_launch<float>(st, f, x, y) : formed_launch<double>(st, f, x, y);
+  return rc ? rc : cc_prof_stop(st, CC_PROF_FORMED, e0);
 }
 }  // namespace
 
@@ -361,8 +351,8 @@ extern "C" int cc_whiten_f64(void* stream, int64_t n, int n_mats, const double* 
   return cc_internal_gemm_upper(cc_stream(stream), n_mats, n, work, n * n, 1, n, Wt, n, K, n * n);
 }
 
-extern "C" int cc_formed_plan_create(void** out, int64_t n_env, int64_t d, int n_mats, const double* const* mats,
-                                     const double* host_ops, const double* host_id) {
+static int formed_plan_create(void** out, int64_t n_env, int64_t d, int n_mats, const void* const* mats, int f32,
+                              const double* host_ops, const double* host_id) {
   *out = nullptr;
   if (d != 2 || n_env < 1 || n_env > 1 << 20 || n_mats < 0 || n_mats > 5 || (n_mats == 0 && !host_id)) {
     cc_set_last_error("formed operator: d = 2 and at most 5 matrices");
@@ -372,6 +362,7 @@ extern "C" int cc_formed_plan_create(void** out, int64_t n_env, int64_t d, int n
   f->n_env = (int)n_env;
   f->n_mats = n_mats;
   f->has_id = host_id != nullptr;
+  f->f32 = f32;
   for (int g = 0; g < n_mats; ++g) {
     f->mat[g] = mats[g];
     for (int e = 0; e < 4; ++e) f->op[g][e] = host_ops[4 * g + e];
@@ -379,6 +370,16 @@ extern "C" int cc_formed_plan_create(void** out, int64_t n_env, int64_t d, int n
   for (int e = 0; e < 4; ++e) f->id[e] = host_id ? host_id[e] : 0.0;
   *out = f;
   return CC_OK;
+}
+
+extern "C" int cc_formed_plan_create(void** out, int64_t n_env, int64_t d, int n_mats, const double* const* mats,
+                                     const double* host_ops, const double* host_id) {
+  return formed_plan_create(out, n_env, d, n_mats, reinterpret_cast<const void* const*>(mats), 0, host_ops, host_id);
+}
+
+extern "C" int cc_formed_plan_create_f32(void** out, int64_t n_env, int64_t d, int n_mats, const float* const* mats,
+                                         const double* host_ops, const double* host_id) {
+  return formed_plan_create(out, n_env, d, n_mats, reinterpret_cast<const void* const*>(mats), 1, host_ops, host_id);
 }
 
 extern "C" int cc_formed_plan_apply(void* stream, const void* plan, const double* x, double* y) {

@@ -553,37 +553,52 @@ __global__ void __launch_bounds__(1024) cg_step_reg_kernel(int64_t n, const doub
   if (threadIdx.x == 0) rr[0] = rr_new;
 }
 
-__global__ void small_geneig_kernel(int k, const double* __restrict__ Hs, const double* __restrict__ Ns,
-                                    double* __restrict__ out, double* __restrict__ vec) {
-  // the four k x k work matrices live in LDS (no private scratch: concurrent launches on several
+// One wave; every element goes through the operations of the serial algorithm in its order, the lanes take different
+// rows (Cholesky, rotations), columns (the inverse factor) or entries (the projected matrix).  Bound by the chain of
+// rotations: k = 8 takes 34 us on average over a solve's passes, 104 us with one lane doing everything.
+__global__ void __launch_bounds__(64) small_geneig_kernel(int k, const double* __restrict__ Hs, const double* __restrict__ Ns,
+                                                          double* __restrict__ out, double* __restrict__ vec) {
+  // the k x k work matrices live in LDS (no private scratch: concurrent launches on several
   // streams would each need a large scratch allocation)
-  __shared__ double Lm[32][32], C[32][32], V[32][32], Li[32][32];
-  if (threadIdx.x != 0) return;
-  for (int i = 0; i < k; ++i)
-    for (int j = 0; j < k; ++j) { Lm[i][j] = 0.0; Li[i][j] = 0.0; V[i][j] = (i == j) ? 1.0 : 0.0; }
+  __shared__ double Lm[32][33], C[32][33], V[32][33], Li[32][33];
+  const int lane = threadIdx.x;
+  for (int e = lane; e < k * k; e += 64) {
+    const int i = e / k, j = e - i * k;
+    Lm[i][j] = 0.0;
+    Li[i][j] = 0.0;
+    V[i][j] = (i == j) ? 1.0 : 0.0;
+  }
+  __syncthreads();
   for (int j = 0; j < k; ++j) {
     double s = Ns[j * k + j];
     for (int c = 0; c < j; ++c) s -= Lm[j][c] * Lm[j][c];
-    Lm[j][j] = sqrt(fmax(s, 1e-300));
-    for (int i = j + 1; i < k; ++i) {
-      double t = Ns[i * k + j];
-      for (int c = 0; c < j; ++c) t -= Lm[i][c] * Lm[j][c];
-      Lm[i][j] = t / Lm[j][j];
+    const double djj = sqrt(fmax(s, 1e-300));
+    double t = 0.0;
+    if (lane > j && lane < k) {
+      t = Ns[lane * k + j];
+      for (int c = 0; c < j; ++c) t -= Lm[lane][c] * Lm[j][c];
+      t /= djj;
     }
+    __syncthreads();
+    if (lane == j) Lm[j][j] = djj;
+    if (lane > j && lane < k) Lm[lane][j] = t;
+    __syncthreads();
   }
-  for (int c = 0; c < k; ++c)
-    for (int i = c; i < k; ++i) {
-      double v = (i == c) ? 1.0 : 0.0;
-      for (int t = c; t < i; ++t) v -= Lm[i][t] * Li[t][c];
-      Li[i][c] = v / Lm[i][i];
+  if (lane < k)
+    for (int i = lane; i < k; ++i) {
+      double v = (i == lane) ? 1.0 : 0.0;
+      for (int t = lane; t < i; ++t) v -= Lm[i][t] * Li[t][lane];
+      Li[i][lane] = v / Lm[i][i];
     }
-  for (int i = 0; i < k; ++i)
-    for (int j = 0; j < k; ++j) {
-      double acc = 0.0;
-      for (int a = 0; a <= i; ++a)
-        for (int b = 0; b <= j; ++b) acc += Li[i][a] * Hs[a * k + b] * Li[j][b];
-      C[i][j] = acc;
-    }
+  __syncthreads();
+  for (int e = lane; e < k * k; e += 64) {
+    const int i = e / k, j = e - i * k;
+    double acc = 0.0;
+    for (int a = 0; a <= i; ++a)
+      for (int b = 0; b <= j; ++b) acc += Li[i][a] * Hs[a * k + b] * Li[j][b];
+    C[i][j] = acc;
+  }
+  __syncthreads();
   for (int sweep = 0; sweep < 50; ++sweep) {
     double off = 0.0;
     for (int i = 0; i < k; ++i)
@@ -591,36 +606,65 @@ __global__ void small_geneig_kernel(int k, const double* __restrict__ Hs, const 
     if (off < 1e-30) break;
     for (int p = 0; p < k; ++p)
       for (int q = p + 1; q < k; ++q) {
-        if (C[p][q] == 0.0) continue;
-        double th = (C[q][q] - C[p][p]) / (2.0 * C[p][q]);
-        double t = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
-        double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
-        for (int r = 0; r < k; ++r) {
-          double a = C[r][p], b = C[r][q];
-          C[r][p] = c * a - s * b;
-          C[r][q] = s * a + c * b;
+        const double cpq = C[p][q];
+        if (cpq == 0.0) continue;
+        const double th = (C[q][q] - C[p][p]) / (2.0 * cpq);
+        const double t = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
+        const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
+        __syncthreads();
+        if (lane < k) {
+          const double a = C[lane][p], b = C[lane][q], va = V[lane][p], vb = V[lane][q];
+          C[lane][p] = c * a - s * b;
+          C[lane][q] = s * a + c * b;
+          V[lane][p] = c * va - s * vb;
+          V[lane][q] = s * va + c * vb;
         }
-        for (int r = 0; r < k; ++r) {
-          double a = C[p][r], b = C[q][r];
-          C[p][r] = c * a - s * b;
-          C[q][r] = s * a + c * b;
+        __syncthreads();
+        if (lane < k) {
+          const double a = C[p][lane], b = C[q][lane];
+          C[p][lane] = c * a - s * b;
+          C[q][lane] = s * a + c * b;
         }
-        for (int r = 0; r < k; ++r) {
-          double a = V[r][p], b = V[r][q];
-          V[r][p] = c * a - s * b;
-          V[r][q] = s * a + c * b;
-        }
+        __syncthreads();
       }
   }
   int best = 0;
   for (int i = 1; i < k; ++i)
     if (C[i][i] < C[best][best]) best = i;
-  out[0] = C[best][best];
-  for (int i = 0; i < k; ++i) {  // coefficients = L^-T v
+  if (lane == 0) out[0] = C[best][best];
+  if (lane < k) {  // coefficients = L^-T v
     double acc = 0.0;
-    for (int j = i; j < k; ++j) acc += Li[j][i] * V[j][best];
-    vec[i] = acc;
+    for (int j = lane; j < k; ++j) acc += Li[j][lane] * V[j][best];
+    vec[lane] = acc;
   }
+}
+
+// out[m][i][j] = sum U_i V_j for V = V0 (m = 0) and V1 (m = 1): one block per entry, the sums of jd_dots_kernel.
+__global__ void __launch_bounds__(256) jd_gram_kernel(int64_t n, const double* __restrict__ U, const double* __restrict__ V0,
+                                                      const double* __restrict__ V1, double* __restrict__ out) {
+  __shared__ double red[256];
+  const double* V = blockIdx.z ? V1 : V0;
+  const double t = block_dot256(n, U + (int64_t)blockIdx.x * n, V + (int64_t)blockIdx.y * n, red);
+  if (threadIdx.x == 0) out[((int64_t)blockIdx.z * gridDim.x + blockIdx.x) * gridDim.y + blockIdx.y] = t;
+}
+
+// x = U^T c, r = HU^T c - rho NU^T c, nx = NU^T c over k basis vectors (k <= 32).
+__global__ void __launch_bounds__(256) jd_residual_kernel(int k, int64_t n, const double* __restrict__ U,
+                                                          const double* __restrict__ HU, const double* __restrict__ NU,
+                                                          const double* __restrict__ rho, const double* __restrict__ c,
+                                                          double* __restrict__ x, double* __restrict__ r, double* __restrict__ nx) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  double tx = 0.0, th = 0.0, tn = 0.0;
+  for (int j = 0; j < k; ++j) {
+    const double cj = c[j];
+    tx += cj * U[j * n + i];
+    th += cj * HU[j * n + i];
+    tn += cj * NU[j * n + i];
+  }
+  x[i] = tx;
+  r[i] = th - rho[0] * tn;
+  nx[i] = tn;
 }
 }  // namespace
 
@@ -644,6 +688,33 @@ extern "C" int cc_small_geneig_f64(void* stream, int k, const double* Hs, const 
   return CC_OK;
 }
 
+extern "C" int cc_jd_project_f64(void* stream, int k, int64_t n, const double* U, const double* HU, const double* NU,
+                                 double* gram, double* value, double* coef, double* x, double* r, double* nx) {
+  if (k < 1 || k > 32 || n < 1) { cc_set_last_error("jd project: 1 <= k <= 32"); return CC_ERR_ARG; }
+  hipStream_t st = cc_stream(stream);
+  jd_gram_kernel<<<dim3((unsigned)k, (unsigned)k, 2), 256, 0, st>>>(n, U, HU, NU, gram);
+  CC_LAUNCH_CHECK();
+  small_geneig_kernel<<<1, 64, 0, st>>>(k, gram, gram + k * k, value, coef);
+  CC_LAUNCH_CHECK();
+  jd_residual_kernel<<<cc_blocks(n, 256), 256, 0, st>>>(k, n, U, HU, NU, value, coef, x, r, nx);
+  CC_LAUNCH_CHECK();
+  return CC_OK;
+}
+
+extern "C" int cc_jd_expand_f64(void* stream, int k, int64_t n, double* U, double* t, double* coef) {
+  if (k < 1 || k > 32 || n < 1) { cc_set_last_error("jd expand: 1 <= k <= 32"); return CC_ERR_ARG; }
+  hipStream_t st = cc_stream(stream);
+  for (int pass = 0; pass < 2; ++pass) {
+    lz_coeff_kernel<<<k, 256, 0, st>>>(n, U, t, coef, -1);
+    CC_LAUNCH_CHECK();
+    lz_combine_kernel<<<(unsigned)((n + 15) / 16), 256, 0, st>>>(k, n, U, coef, t, 0);
+    CC_LAUNCH_CHECK();
+  }
+  lz_normalize_kernel<<<1, 1024, 0, st>>>(n, t, U + (int64_t)k * n, nullptr);
+  CC_LAUNCH_CHECK();
+  return CC_OK;
+}
+
 extern "C" int cc_jd_work_size(int64_t n, int64_t* out) {
   *out = 10 * n + 16;
   return CC_OK;
@@ -652,12 +723,10 @@ extern "C" int cc_jd_work_size(int64_t n, int64_t* out) {
 // Approximate solution of the projected correction equation
 //   (I - u u^T)(W Hlp W^T - rho)(I - u u^T) y = -(I - u u^T) W r,  u = L^T x / |L^T x|,  t = W^T (I - u u^T) y
 // by `iters` CG steps on the low-precision operator (all scalars on the device).
-extern "C" int cc_jd_correction_lp(void* stream, const void* lp_plan, int64_t n_env, int64_t d, const double* Lt,
-                                   const double* W, const double* Wt, const double* rho_dev, const double* x,
-                                   const double* r, int iters, double* work, double* t_out) {
-  hipStream_t st = cc_stream(stream);
+static int jd_correction(hipStream_t st, ApplyFn apply, const void* plan, int64_t n_env, int64_t d, const double* Lt,
+                         const double* W, const double* Wt, const double* rho_dev, const double* x, const double* r,
+                         int iters, double* work, double* t_out) {
   const int64_t n = n_env * d;
-  if (cc_internal_lp_n(lp_plan) != n) { cc_set_last_error("jd: operator size mismatch"); return CC_ERR_DIM; }
   double* u = work;
   double* y = u + n;
   double* res = y + n;
@@ -696,7 +765,7 @@ extern "C" int cc_jd_correction_lp(void* stream, const void* lp_plan, int64_t n_
   if (rc) return rc;
   for (int k = 0; k < iters; ++k) {
     // ap = P (W H W^T - rho) p   (p is kept in the projected space)
-    rc = op_whitened(st, cc_internal_lp_apply, lp_plan, wh, p, t1, t2, ap);
+    rc = op_whitened(st, apply, plan, wh, p, t1, t2, ap);
     if (rc) return rc;
     if (n <= 4096) cg_step_reg_kernel<4><<<1, 1024, 0, st>>>(n, rho_dev, u, ap, p, y, res, sc + 1);
     else cg_step_kernel<<<1, 1024, 0, st>>>(n, rho_dev, u, ap, p, y, res, sc + 1);
@@ -704,6 +773,20 @@ extern "C" int cc_jd_correction_lp(void* stream, const void* lp_plan, int64_t n_
   }
   if ((rc = project(y))) return rc;
   return cc_skinny_f64(st, n_env, 2, Wt, (int)d, y, t_out);                // t = W^T P y
+}
+
+extern "C" int cc_jd_correction_lp(void* stream, const void* lp_plan, int64_t n_env, int64_t d, const double* Lt,
+                                   const double* W, const double* Wt, const double* rho_dev, const double* x,
+                                   const double* r, int iters, double* work, double* t_out) {
+  if (cc_internal_lp_n(lp_plan) != n_env * d) { cc_set_last_error("jd: operator size mismatch"); return CC_ERR_DIM; }
+  return jd_correction(cc_stream(stream), cc_internal_lp_apply, lp_plan, n_env, d, Lt, W, Wt, rho_dev, x, r, iters, work, t_out);
+}
+
+extern "C" int cc_jd_correction_formed(void* stream, const void* formed_plan, int64_t n_env, int64_t d, const double* Lt,
+                                       const double* W, const double* Wt, const double* rho_dev, const double* x,
+                                       const double* r, int iters, double* work, double* t_out) {
+  if (!formed_plan || cc_internal_formed_n(formed_plan) != n_env * d) { cc_set_last_error("jd: operator size mismatch"); return CC_ERR_DIM; }
+  return jd_correction(cc_stream(stream), cc_internal_formed_apply, formed_plan, n_env, d, Lt, W, Wt, rho_dev, x, r, iters, work, t_out);
 }
 
 extern "C" int cc_normalize_f64(void* stream, int64_t n, const double* x, double* y) {

@@ -11,6 +11,8 @@ the identity.
 """
 import ctypes
 
+import torch
+
 from . import _lib
 from .device import empty, ptr, stream
 
@@ -54,23 +56,46 @@ class FormedOperator:
 
     def __init__(self, h_operator, n_operator, factor, layout):
         self.n_env, self.d = h_operator.n // h_operator.d, h_operator.d
-        groups, self.identity = layout
-        self.ops = [O for O, _ in groups]
+        self._groups, self.identity = layout
+        self.ops = [O for O, _ in self._groups]
         self.norm_channels = (n_operator._A[0], n_operator._B[0])
-        self.factor, self._version = factor, factor.version
+        self.factor = factor
+        self._shape = (h_operator.n_alpha, h_operator.P)
         self._plan = None
-        na, P = h_operator.n_alpha, h_operator.P
-        self.G = empty((len(groups), self.n_env, self.n_env))
-        if groups:
-            A = [h_operator.joined(0, a) for _, products in groups for a, _ in products]
-            B = [h_operator.joined(1, b) for _, products in groups for _, b in products]
-            begin = [0]
-            for _, products in groups:
-                begin.append(begin[-1] + len(products))
-            work = empty((_lib.query("cc_form_work_size", len(groups), max(len(p) for _, p in groups), na, P, P),))
-            _lib.call("cc_form_f64", stream(), len(groups), _lib.i32_array(begin),
-                      _lib.ptr_array([t.data_ptr() for t in A]), _lib.ptr_array([t.data_ptr() for t in B]), na, P, P,
-                      ptr(self.G), ptr(work))
+        self.G = empty((len(self._groups), self.n_env, self.n_env))
+        self._form(h_operator.joined)
+
+    def _form(self, joined):
+        """G from the joined sums of channels joined(half, k)."""
+        self._version = self.factor.version
+        if not self._groups:
+            return
+        na, P = self._shape
+        A = [joined(0, a) for _, products in self._groups for a, _ in products]
+        B = [joined(1, b) for _, products in self._groups for _, b in products]
+        begin = [0]
+        for _, products in self._groups:
+            begin.append(begin[-1] + len(products))
+        work = empty((_lib.query("cc_form_work_size", len(self._groups), max(len(p) for _, p in self._groups), na, P, P),))
+        _lib.call("cc_form_f64", stream(), len(self._groups), _lib.i32_array(begin),
+                  _lib.ptr_array([t.data_ptr() for t in A]), _lib.ptr_array([t.data_ptr() for t in B]), na, P, P,
+                  ptr(self.G), ptr(work))
+
+    def refresh(self, h_operator, other, factor):
+        """Forms `other`, an operator of h_operator's structure from a new environment that the factor holds already,
+        into these matrices; h_operator then applies it (kernels only: capturable in a HIP graph)."""
+        channels = h_operator.same_structure(other)
+        if factor is not self.factor:
+            self.factor, self._plan = factor, None
+        if h_operator._fused is not None:
+            h_operator.refresh_fused_from(other)
+        else:
+            h_operator._refreshed += 1
+        _, specs, _, _ = h_operator._merged()
+        h_operator._joined = {(side, k): h_operator.joined(side, k, channels)
+                              for side in (0, 1) for k in range(len(specs[side]))}
+        self._form(h_operator.joined)
+        h_operator._formed = self
 
     def valid(self):
         """Whether the factor still holds the environment this operator was formed from."""
@@ -84,12 +109,16 @@ class FormedOperator:
             self._plan = FormedPlan(self.n_env, self.d, mats, ops, None)
         self._plan.apply(x, y)
 
-    def whitened(self, factor):
-        """The plan of W H W^T with the factor's W = L^-1 (two triangular products per matrix)."""
+    def whitened(self, factor, f32=None):
+        """The plan of W H W^T with the factor's W = L^-1 (two triangular products per matrix).  f32: an FP32 array of
+        G's shape that the matrices are rounded into, for inner steps that need no more."""
         K = empty(self.G.shape)
         if self.ops:
             work = empty(self.G.shape)
             _lib.call("cc_whiten_f64", stream(), self.n_env, len(self.ops), ptr(self.G), ptr(factor.Wt), ptr(K), ptr(work))
+            if f32 is not None:
+                _lib.call("cc_cast", stream(), K.numel(), _lib.CC_F64, ptr(K), _lib.CC_F32, ptr(f32))
+        K = K if f32 is None else f32
         return FormedPlan(self.n_env, self.d, [K[g] for g in range(len(self.ops))], self.ops, self.identity)
 
 
@@ -98,7 +127,7 @@ class FormedPlan:
 
     def __init__(self, n_env, d, mats, ops, identity):
         self.mats, self.handle = mats, ctypes.c_void_p()
-        _lib.call("cc_formed_plan_create", ctypes.byref(self.handle), n_env, d, len(mats),
+        _lib.call("cc_formed_plan_create_f32" if mats and mats[0].dtype == torch.float32 else "cc_formed_plan_create", ctypes.byref(self.handle), n_env, d, len(mats),
                   _lib.ptr_array([m.data_ptr() for m in mats]), _lib.f64_array([x for O in ops for x in O]),
                   _lib.f64_array(identity) if identity is not None else None)
 

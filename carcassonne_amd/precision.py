@@ -8,15 +8,15 @@ LowPrecisionOperator -- the stage-3 operator of one solve with every distinct sl
     D=6, chi=64 that is as accurate as splitting both (the slab rounding dominates: first FP64
     energy 2.36e-7 vs 2.37e-7 off) at half the stage-B matrix-core work, while rounding the vector
     too leaves the refinement stuck near 1e-5.
-MixedSolver -- (1) Lanczos on the whitened low-precision operator (the FP64 whitening of the
-    exact N) until the Ritz value moves by less than 1e-6 relative between checks: the rounded
-    slabs bound the accuracy of its eigenvector (the FP64 energy of that vector is ~1e-7 off at
-    D=6, chi=64 however long it runs), so converging further buys nothing; (2) Jacobi-Davidson
-    refinement in FP64: each outer
-    step applies the FP64 H and N to one new basis vector, solves the small generalized
-    eigenproblem of the basis on the device (FP64 Rayleigh-Ritz), and computes the correction
-    from a fixed number of CG steps on the projected, shifted low-precision operator.  The
-    energy reported is the FP64 Rayleigh quotient of the final Ritz vector.
+MixedSolver -- (1) Lanczos on the whitened low-precision operator until the Ritz value moves by less than 1e-6 relative
+    between checks (its eigenvector is only as accurate as that operator); (2) Jacobi-Davidson refinement in FP64: each
+    outer step applies the FP64 H and N to one new basis vector, solves the small generalized eigenproblem of the basis
+    on the device (FP64 Rayleigh-Ritz), and computes the correction from a fixed number of CG steps on the projected,
+    shifted low-precision operator.  The energy reported is the FP64 Rayleigh quotient of the final Ritz vector.
+    The operator is formed in FP64 (formed.FormedOperator) and the low-precision one is its whitened matrices rounded
+    to FP32: a solve applies it 70 times or more, and forming costs as much as seven applications of the slabs.  Where
+    an operator has no such form, or the caller brings the normalization factor, the low-precision operator is the
+    FP16 / BF16 one (dtype, groups, split) between the FP64 whitening products.
 """
 import ctypes
 
@@ -25,6 +25,7 @@ import torch
 
 from . import _lib
 from .device import empty, join, ptr, stream
+from .formed import FormedOperator
 from .solver import NormalizationFactor
 
 DTYPES = {"f16": _lib.CC_F16, "bf16": _lib.CC_BF16}
@@ -143,28 +144,82 @@ class MixedSolver:
 
     def __init__(self, h_operator, n_operator, dtype="bf16", factor=None, groups=None, split="vector"):
         self.H, self.N = h_operator, n_operator
-        side = None
+        if not h_operator.use_fused:
+            raise NotImplementedError("the low-precision kernel needs P = Q in {4, 9, 16, 25, 36} and d = 2")
+        DTYPES[dtype], SPLIT_MODES[split]      # unknown names are refused whichever operator serves the solve
+        side, form = None, factor is None
         if factor is None:
             factor, side = NormalizationFactor.beside(n_operator)
         self.factor = factor
+        self.n = h_operator.n
+        self._lp_args = dict(dtype=dtype, groups=groups, split=split)
+        self._lp, self._lp_source = None, h_operator
+        self._formed = self._white = None
         try:
-            self.Hlp = LowPrecisionOperator(h_operator, dtype, groups=groups, split=split)
-            self.n = h_operator.n
-            h_operator._ensure_fused()
-            self._hplan = h_operator.plan_handle()     # N is applied through the formed N_env (factor.apply_n)
+            if form:
+                self._formed = FormedOperator.of(h_operator, n_operator, factor)
+            if self._formed is None:
+                self.Hlp
+                self._hplan = h_operator.plan_handle()     # N is applied through the formed N_env (factor.apply_n)
             self._lz_work, self._lz_max = None, 0
             self._jd_work = empty((_lib.query("cc_jd_work_size", self.n),))
         finally:
             if side is not None:
                 join(side)
+        if self._formed is not None:
+            self._K32 = empty(self._formed.G.shape, dtype=torch.float32)
+            self._white = self._formed.whitened(factor, self._K32)
+
+    @property
+    def Hlp(self):
+        """The FP16 / BF16 operator (made on first use where the formed one serves the solve)."""
+        if self._lp is None:
+            self._lp = LowPrecisionOperator(self._lp_source, **self._lp_args)
+        return self._lp
 
     def refresh(self, h_operator, n_operator):
         """The solve's setup for a new environment of the same structure, into this solver's buffers: the
-        normalization factor, the FP64 packed slabs of the H operator this solver was built with, and the
-        low-precision slabs and coefficients (kernels only: capturable in a HIP graph)."""
+        normalization factor and the formed operator, or the FP64 packed slabs of the H operator this solver was
+        built with and the low-precision slabs and coefficients (kernels only: capturable in a HIP graph)."""
         self.factor.refresh(n_operator)
-        self.H.refresh_fused_from(h_operator)
-        self.Hlp.refresh(h_operator)
+        if self._formed is not None:
+            self._formed.refresh(self.H, h_operator, self.factor)
+            self._white = self._formed.whitened(self.factor, self._K32)
+        else:
+            self.H.refresh_fused_from(h_operator)
+        if self._lp is not None:
+            self._lp.refresh(h_operator)
+        self._lp_source = h_operator
+
+    def _apply_h(self, x, y):
+        """y = H x in FP64."""
+        if self._formed is not None:
+            self._formed.apply_flat(x, y)
+        else:
+            _lib.call("cc_stage3_plan_apply", stream(), self._hplan, ptr(x), ptr(y))
+
+    def _lanczos(self, x0, tol_residual, tol_energy, max_iter, check_every, x, res):
+        f = self.factor
+        if self._lz_work is None or self._lz_max < max_iter:
+            self._lz_work = empty((_lib.query("cc_lanczos_work_size", self.n, max_iter),))
+            self._lz_max = max_iter
+        if self._white is not None:
+            _lib.call("cc_lanczos_formed_f64", stream(), self._white.handle, f.n_env, f.d, ptr(f.Lt), ptr(f.Wt), ptr(x0),
+                      float(tol_residual), float(tol_energy), max_iter, int(check_every), ptr(self._lz_work), ptr(x), res)
+        else:
+            _lib.call("cc_lanczos_lp", stream(), self.Hlp.plan, f.n_env, f.d, ptr(f.L), ptr(f.Lt), ptr(f.W), ptr(f.Wt),
+                      ptr(x0), float(tol_residual), float(tol_energy), max_iter, int(check_every), ptr(self._lz_work),
+                      ptr(x), res)
+
+    def _correction(self, rho, x, r, iters, t):
+        """t: `iters` CG steps of the correction equation of Ritz pair (rho, x) with residual r."""
+        f = self.factor
+        if self._white is not None:
+            _lib.call("cc_jd_correction_formed", stream(), self._white.handle, f.n_env, f.d, ptr(f.Lt), ptr(f.W), ptr(f.Wt),
+                      ptr(rho), ptr(x), ptr(r), iters, ptr(self._jd_work), ptr(t))
+        else:
+            _lib.call("cc_jd_correction_lp", stream(), self.Hlp.plan, f.n_env, f.d, ptr(f.Lt), ptr(f.W), ptr(f.Wt),
+                      ptr(rho), ptr(x), ptr(r), iters, ptr(self._jd_work), ptr(t))
 
     def solve(self, x0, max_lowprec_iter=300, check_every=4, inner_iters=20, max_outer=8, tol_energy=1e-13,
               tol_predicted=1e-11, lp_tol_residual=0.0, lp_tol_energy=1e-6):
@@ -174,22 +229,17 @@ class MixedSolver:
         from .data import HipData
         if isinstance(x0, HipData):
             x0 = x0._t.reshape(-1)
-        f, n = self.factor, self.n
+        n = self.n
         max_lowprec_iter = int(min(max_lowprec_iter, n))
-        if self._lz_work is None or self._lz_max < max_lowprec_iter:
-            self._lz_work = empty((_lib.query("cc_lanczos_work_size", n, max_lowprec_iter),))
-            self._lz_max = max_lowprec_iter
         x = empty((n,))
         res = _lib.f64_array([0, 0, 0])
         # (1) low-precision Lanczos until the Ritz value stops moving at the precision floor
-        _lib.call("cc_lanczos_lp", stream(), self.Hlp.plan, f.n_env, f.d, ptr(f.L), ptr(f.Lt), ptr(f.W), ptr(f.Wt),
-                  ptr(x0), float(lp_tol_residual), float(lp_tol_energy), max_lowprec_iter, int(check_every),
-                  ptr(self._lz_work), ptr(x), res)
+        self._lanczos(x0, lp_tol_residual, lp_tol_energy, max_lowprec_iter, check_every, x, res)
         lp_iters = int(res[2])
         # (2) Jacobi-Davidson in FP64
         kmax = max_outer + 1
         U, HU, NU = empty((kmax, n)), empty((kmax, n)), empty((kmax, n))
-        small = empty((kmax + 1,))
+        gram, small, coef = empty((2 * kmax * kmax,)), empty((1,)), empty((kmax,))
         xr, r, t = empty((n,)), empty((n,)), empty((n,))
         U[0].copy_(x)
         k, rho, prev = 0, None, None
@@ -198,22 +248,17 @@ class MixedSolver:
         stopped_by = None
         for outer in range(max_outer):
             # FP64 H and N on the newest basis vector, then the projected pencil
-            _lib.call("cc_stage3_plan_apply", stream(), self._hplan, ptr(U[k]), ptr(HU[k]))
-            f.apply_n(U[k], NU[k])
+            self._apply_h(U[k], HU[k])
+            self.factor.apply_n(U[k], NU[k])
             fp64_passes += 1
             k += 1
-            hs, ns = empty((k, k)), empty((k, k))
-            for j in range(k):
-                _lib.call("cc_basis_dots_f64", stream(), k, n, ptr(U), ptr(HU[j]), ptr(hs[:, j]), k)
-                _lib.call("cc_basis_dots_f64", stream(), k, n, ptr(U), ptr(NU[j]), ptr(ns[:, j]), k)
-            _lib.call("cc_small_geneig_f64", stream(), k, ptr(hs), ptr(ns), ptr(small[0:1]), ptr(small[1:1 + k]))
-            rho = float(small[0].item())
+            _lib.call("cc_jd_project_f64", stream(), k, n, ptr(U), ptr(HU), ptr(NU), ptr(gram), ptr(small), ptr(coef),
+                      ptr(xr), ptr(r), ptr(t))
+            rho = float(small.item())
             if not np.isfinite(rho):
                 raise FloatingPointError("mixed-precision solve: the FP64 Rayleigh-Ritz value is not finite "
                                          "(history {})".format(history))
             history.append(rho)
-            coeffs = small[1:1 + k].contiguous()
-            _lib.call("cc_basis_combine_f64", stream(), k, n, ptr(U), ptr(coeffs), ptr(xr))
             if prev is not None:
                 delta = abs(prev - rho)
                 if delta <= tol_energy * abs(rho):
@@ -227,20 +272,9 @@ class MixedSolver:
             prev = rho
             if outer == max_outer - 1:
                 break
-            # residual r = H xr - rho N xr from the basis products
-            _lib.call("cc_basis_combine_f64", stream(), k, n, ptr(HU), ptr(coeffs), ptr(r))
-            _lib.call("cc_basis_combine_f64", stream(), k, n, ptr(NU), ptr(coeffs), ptr(t))
-            _lib.call("cc_axpby_f64", stream(), n, -rho, ptr(t), 1.0, ptr(r))
-            _lib.call("cc_jd_correction_lp", stream(), self.Hlp.plan, f.n_env, f.d, ptr(f.Lt), ptr(f.W), ptr(f.Wt),
-                      ptr(small[0:1]), ptr(xr), ptr(r), _schedule(inner_iters, outer), ptr(self._jd_work), ptr(t))
-            # orthogonalise the correction against the basis (twice, Euclidean) and normalise
-            for _ in range(2):
-                c = empty((k,))
-                _lib.call("cc_basis_dots_f64", stream(), k, n, ptr(U), ptr(t), ptr(c), 1)
-                tmp = empty((n,))
-                _lib.call("cc_basis_combine_f64", stream(), k, n, ptr(U), ptr(c), ptr(tmp))
-                _lib.call("cc_axpby_f64", stream(), n, -1.0, ptr(tmp), 1.0, ptr(t))
-            _lib.call("cc_normalize_f64", stream(), n, ptr(t), ptr(U[k]))
+            self._correction(small, xr, r, _schedule(inner_iters, outer), t)
+            _lib.call("cc_jd_expand_f64", stream(), k, n, ptr(U), ptr(t), ptr(coef))
+        f = self.factor
         f.check()
         converged = stopped_by is not None
         return xr, rho, dict(lowprec_iterations=lp_iters, outer_steps=k, fp64_passes=fp64_passes, converged=converged,
@@ -257,44 +291,25 @@ class MixedSolver:
         from .data import HipData
         if isinstance(x0, HipData):
             x0 = x0._t.reshape(-1)
-        f, n = self.factor, self.n
+        n = self.n
         lp_iters = int(min(lp_iters, n))
-        if self._lz_work is None or self._lz_max < lp_iters:
-            self._lz_work = empty((_lib.query("cc_lanczos_work_size", n, lp_iters),))
-            self._lz_max = lp_iters
         x = empty((n,))
-        _lib.call("cc_lanczos_lp", stream(), self.Hlp.plan, f.n_env, f.d, ptr(f.L), ptr(f.Lt), ptr(f.W), ptr(f.Wt),
-                  ptr(x0), 0.0, 0.0, lp_iters, 0, ptr(self._lz_work), ptr(x), None)
-        kmax = outer
-        U, HU, NU = empty((kmax, n)), empty((kmax, n)), empty((kmax, n))
-        small = empty((kmax + 1,))
-        xr, r, t, tmp = empty((n,)), empty((n,)), empty((n,)), empty((n,))
+        self._lanczos(x0, 0.0, 0.0, lp_iters, 0, x, None)
+        U, HU, NU = empty((outer, n)), empty((outer, n)), empty((outer, n))
+        gram, small, coef = empty((2 * outer * outer,)), empty((1,)), empty((outer,))
+        xr, r, t = empty((n,)), empty((n,)), empty((n,))
         hist = empty((outer + 2,))
         U[0].copy_(x)
         for k in range(1, outer + 1):
-            _lib.call("cc_stage3_plan_apply", stream(), self._hplan, ptr(U[k - 1]), ptr(HU[k - 1]))
-            f.apply_n(U[k - 1], NU[k - 1])
-            hs, ns = empty((k, k)), empty((k, k))
-            for j in range(k):
-                _lib.call("cc_basis_dots_f64", stream(), k, n, ptr(U), ptr(HU[j]), ptr(hs[:, j]), k)
-                _lib.call("cc_basis_dots_f64", stream(), k, n, ptr(U), ptr(NU[j]), ptr(ns[:, j]), k)
-            _lib.call("cc_small_geneig_f64", stream(), k, ptr(hs), ptr(ns), ptr(small[0:1]), ptr(small[1:1 + k]))
-            coeffs = small[1:1 + k]
-            _lib.call("cc_basis_combine_f64", stream(), k, n, ptr(U), ptr(coeffs), ptr(xr))
-            _lib.call("cc_axpby_f64", stream(), 1, 1.0, ptr(small[0:1]), 0.0, ptr(hist[k - 1:k]))
-            _lib.call("cc_basis_combine_f64", stream(), k, n, ptr(HU), ptr(coeffs), ptr(r))
-            _lib.call("cc_basis_combine_f64", stream(), k, n, ptr(NU), ptr(coeffs), ptr(tmp))
-            _lib.call("cc_axpby_dev_f64", stream(), n, ptr(small[0:1]), -1.0, ptr(tmp), 1.0, ptr(r))
+            self._apply_h(U[k - 1], HU[k - 1])
+            self.factor.apply_n(U[k - 1], NU[k - 1])
+            _lib.call("cc_jd_project_f64", stream(), k, n, ptr(U), ptr(HU), ptr(NU), ptr(gram), ptr(hist[k - 1:k]), ptr(coef),
+                      ptr(xr), ptr(r), ptr(t))
             if k == outer:     # the final residual H x - rho N x and N x, for the convergence record
+                _lib.call("cc_axpby_f64", stream(), 1, 1.0, ptr(hist[k - 1:k]), 0.0, ptr(small))
                 _lib.call("cc_dot_f64", stream(), n, ptr(r), ptr(r), ptr(hist[outer:outer + 1]))
-                _lib.call("cc_dot_f64", stream(), n, ptr(tmp), ptr(tmp), ptr(hist[outer + 1:outer + 2]))
+                _lib.call("cc_dot_f64", stream(), n, ptr(t), ptr(t), ptr(hist[outer + 1:outer + 2]))
                 break
-            _lib.call("cc_jd_correction_lp", stream(), self.Hlp.plan, f.n_env, f.d, ptr(f.Lt), ptr(f.W), ptr(f.Wt),
-                      ptr(small[0:1]), ptr(xr), ptr(r), _schedule(inner_iters, k - 1), ptr(self._jd_work), ptr(t))
-            for _ in range(2):
-                c = empty((k,))
-                _lib.call("cc_basis_dots_f64", stream(), k, n, ptr(U), ptr(t), ptr(c), 1)
-                _lib.call("cc_basis_combine_f64", stream(), k, n, ptr(U), ptr(c), ptr(tmp))
-                _lib.call("cc_axpby_f64", stream(), n, -1.0, ptr(tmp), 1.0, ptr(t))
-            _lib.call("cc_normalize_f64", stream(), n, ptr(t), ptr(U[k]))
-        return xr, small[0:1], hist
+            self._correction(hist[k - 1:k], xr, r, _schedule(inner_iters, k - 1), t)
+            _lib.call("cc_jd_expand_f64", stream(), k, n, ptr(U), ptr(t), ptr(coef))
+        return xr, small, hist

@@ -260,16 +260,30 @@ class Stage3Operator:
             self._merge = (a_list, b_list), specs, ops, table
         return self._merge
 
-    def joined(self, side, k):
-        """Sum k of half `side` as a contiguous (alpha, P, P) array, kept: it stays what it was when first asked for."""
-        t = self._joined.get((side, k))
+    def joined(self, side, k, channels=None):
+        """Sum k of half `side` as a contiguous (alpha, P, P) array, kept: it stays what it was when first asked for.
+        channels: of another operator of this structure (the sum over them, not kept)."""
+        t = self._joined.get((side, k)) if channels is None else None
         if t is None:
-            channels, specs, _, _ = self._merged()
+            own, specs, _, _ = self._merged()
             spec = specs[side][k]
-            parts = [channels[side][i] for i, _ in spec]
+            parts = [(own if channels is None else channels)[side][i] for i, _ in spec]
             t = parts[0]._t if len(spec) == 1 and spec[0][1] == 1.0 else join_slabs(parts, [c for _, c in spec])
-            self._joined[(side, k)] = t
+            if channels is None:
+                self._joined[(side, k)] = t
         return t
+
+    def same_structure(self, other):
+        """The channels of `other` (per half) if it has this operator's terms, channel sharing and shapes; else
+        ValueError."""
+        a_list, b_list, _, rows = self._channels()
+        oa, ob, _, orows = other._channels()
+        if ([(r[0], r[2], r[3]) for r in rows] != [(r[0], r[2], r[3]) for r in orows] or
+                [(c.n_alpha, c.P) for c in a_list + b_list] != [(c.n_alpha, c.P) for c in oa + ob] or
+                any(len({ch[i].source()[1:] for i, _ in spec}) > 1
+                    for ch, specs in zip((oa, ob), self._merged()[1]) for spec in specs)):
+            raise ValueError("refresh needs an operator of the same structure")
+        return oa, ob
 
     def snapshot(self):
         """Takes every sum of channels now (joined), so that later calls do not read the stage-2 tensors."""
@@ -304,19 +318,13 @@ class Stage3Operator:
         sharing and shapes) built from new stage-2 tensors -- into this operator's packed buffers, so that
         its fused kernel and native plan apply `other` (kernels only; capturable in a HIP graph)."""
         self._ensure_fused()
+        channels = self.same_structure(other)
         self._formed, self._joined = None, {}     # of the environment before
         self._refreshed += 1
-        a_list, b_list, _, rows = self._channels()
-        oa, ob, _, orows = other._channels()
-        if ([(r[0], r[2], r[3]) for r in rows] != [(r[0], r[2], r[3]) for r in orows] or
-                [(c.n_alpha, c.P) for c in a_list + b_list] != [(c.n_alpha, c.P) for c in oa + ob]):
-            raise ValueError("refresh_fused_from needs an operator of the same structure")
         _, specs, _, _ = self._merged()
-        for side, chans, bufs in ((0, oa, self._fused["A"]), (1, ob, self._fused["B"])):
-            for k, spec in enumerate(specs[side]):
-                if len({chans[i].source()[1:] for i, _ in spec}) > 1:
-                    raise ValueError("refresh_fused_from needs an operator of the same structure")
-                self._pack(side, k, chans, bufs[k])
+        for side, bufs in ((0, self._fused["A"]), (1, self._fused["B"])):
+            for k in range(len(specs[side])):
+                self._pack(side, k, channels[side], bufs[k])
 
     def _build_fused(self):
         """Pack every sum of slab channels once and build the term table (sorted by A channel)."""

@@ -222,11 +222,14 @@ int cc_whiten_f64(void* stream, int64_t n, int n_mats, const double* G, const do
  * n_env x n_env matrices M_g, d = 2, at most 5 of them; the matrices stay caller-owned. */
 int cc_formed_plan_create(void** out, int64_t n_env, int64_t d, int n_mats, const double* const* mats,
                           const double* host_ops, const double* host_id);
+/* the same over FP32 matrices (products and sums in FP64): half the bytes, for the inner steps of a refined solve */
+int cc_formed_plan_create_f32(void** out, int64_t n_env, int64_t d, int n_mats, const float* const* mats,
+                              const double* host_ops, const double* host_id);
 int cc_formed_plan_apply(void* stream, const void* plan, const double* x, double* y);
 int cc_formed_plan_destroy(void* plan);
 
 /* Timing of the stage-3 kernels: between begin and end every launch of the FP64 fused kernel (kind 0)
- * and of the low-precision kernel (kind 1) is bracketed by HIP events on its stream; end fills
+ * and of the low-precision kernel (kind 1) and of a formed operator's product (kind 2) is bracketed by HIP events on its stream; end fills
  * total_ms[k] and launches[k] (the launches timed) for k < n_kinds.  begin_sampled(every) times only
  * launches 0, every, 2 every, ... of each kind, so that the event records (each idles the GPU for a few
  * microseconds) cost a fraction of the timed work.  Single-threaded use only.  (Measurement support;
@@ -343,6 +346,17 @@ int cc_jd_work_size(int64_t n, int64_t* out);
 int cc_jd_correction_lp(void* stream, const void* lp_plan, int64_t n_env, int64_t d, const double* Lt,
                         const double* W, const double* Wt, const double* rho_dev, const double* x, const double* r,
                         int iters, double* work, double* t_out);
+/* The same with a plan of formed, whitened matrices. */
+int cc_jd_correction_formed(void* stream, const void* formed_plan, int64_t n_env, int64_t d, const double* Lt,
+                            const double* W, const double* Wt, const double* rho_dev, const double* x, const double* r,
+                            int iters, double* work, double* t_out);
+/* One Rayleigh-Ritz pass over the k rows of U (k <= 32) with HU = H U, NU = N U: gram (2 k^2) receives U HU^T and U NU^T,
+ * value the lowest eigenvalue of that pencil, coef (k) its N-normalised vector, and x = U^T coef, nx = NU^T coef,
+ * r = HU^T coef - value nx. */
+int cc_jd_project_f64(void* stream, int k, int64_t n, const double* U, const double* HU, const double* NU, double* gram,
+                      double* value, double* coef, double* x, double* r, double* nx);
+/* Row k of U = t orthogonalised against rows 0..k-1 (twice, Euclidean) and normalised; t and coef (k) are overwritten. */
+int cc_jd_expand_f64(void* stream, int k, int64_t n, double* U, double* t, double* coef);
 /* y = x / |x| (one workgroup, fixed-order sum; the Lanczos normalisation). */
 int cc_normalize_f64(void* stream, int64_t n, const double* x, double* y);
 
