@@ -39,6 +39,29 @@ static inline unsigned cc_blocks(int64_t n, int threads, unsigned cap = 65535u *
   return (unsigned)b;
 }
 
+// Sum of v over the 64 lanes of a wave, the same value in every lane: four shifted adds inside each row of 16 lanes,
+// two adds of a row's total to the next rows (data-parallel moves, a few cycles each against an LDS round trip per
+// step of a shuffle), lane 63 read out.  The order depends on nothing but the lane.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double cc_dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double cc_wave_sum(double v) {
+  v = cc_dpp_add<0x111, 0xf>(v);   // row_shr:1
+  v = cc_dpp_add<0x112, 0xf>(v);   // row_shr:2
+  v = cc_dpp_add<0x114, 0xf>(v);   // row_shr:4
+  v = cc_dpp_add<0x118, 0xf>(v);   // row_shr:8: lane 15 of each row holds the row's sum
+  v = cc_dpp_add<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+  v = cc_dpp_add<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3: lane 63 holds the sum
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, 63);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
+
 // Internal (not exported through the C ABI header): operator plans used by the solvers.
 int cc_internal_stage3_apply(hipStream_t st, const void* plan, const double* x, double* y);
 int64_t cc_internal_stage3_n(const void* plan);

@@ -7,7 +7,7 @@
 //
 // with one group per distinct site operator.  A matvec through the slabs costs 8 n_alpha P^3 FLOP per product and
 // re-reads every slab; a formed matrix costs 2 n_alpha P^4 once, P / 4 matvecs' worth, and is then P^4 doubles.
-#include "cc_common.h"
+#include "cc_formed.h"
 
 namespace {
 constexpr int FORM_MAX = 16;      // products (and distinct matrices) per call
@@ -178,56 +178,41 @@ int form_split(int n_groups, int max_products, int64_t n_alpha, int64_t P, int64
 }
 
 // ---- application ------------------------------------------------------------------------------------------------
-struct FormedPlan {
-  int n_env, n_mats, has_id, f32;   // f32: the matrices are FP32 (products and sums stay FP64)
-  const void* mat[FORM_MAX];
-  double op[FORM_MAX][4];   // O_g[s'][s], d = 2
-  double id[4];             // coefficient of the identity over the environment legs
-};
+// y[e][s'] = sum_g sum_s O_g[s'][s] sum_f M_g[e][f] x[f][s]  (+ sum_s id[s'][s] x[e][s]): four rows per workgroup, two
+// waves per row, every load of a row in flight at once.  Bound by that one round of loads
+// and by the launch at these sizes: 7.0 us for two FP64 matrices at D = 6 (27 MB, 3.9 TB/s; one wave per row with the
+// columns in three rounds 8.0 us, four rows' columns split over four waves 8.2 us), 3.9 us at D = 4 (1 MB).
+template <typename T, int NG, int U>
+__global__ void __launch_bounds__(FORMED_THREADS) formed_apply_kernel(FormedPlan f, const double* __restrict__ x,
+                                                                     double* __restrict__ y) {
+  __shared__ double red[16];
+  const int row0 = blockIdx.x * FORMED_ROWS;
+  FormedRows<T, NG, U> rows;
+  rows.load(f, row0);
+  rows.apply(f, row0, [&](int c, int s) { return x[2 * c + s]; }, red, y);
+}
 
-// y[e][s'] = sum_g sum_s O_g[s'][s] sum_f M_g[e][f] x[f][s]  (+ sum_s id[s'][s] x[e][s]): one wave per row e, U column
-// steps of 64 with all their loads in flight before the products.  Bound by reading the matrices (27 MB for two FP64
-// matrices at D = 6: 7.5 us, 3.6 TB/s; a workgroup's rows stay on one XCD from launch to launch).
+// The same for matrices of more than 11 x 128 columns: one wave per row.
 template <typename T, int NG>
-__global__ void __launch_bounds__(256) formed_apply_kernel(FormedPlan f, const double* __restrict__ x, double* __restrict__ y) {
-  const int lane = threadIdx.x & 63, n = f.n_env;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+__global__ void __launch_bounds__(256) formed_apply_any_kernel(FormedPlan f, const double* __restrict__ x, double* __restrict__ y) {
+  const int lane = threadIdx.x & 63, n = f.n_env, row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= n) return;
   double acc[NG][2];
-  const T* m[NG];
 #pragma unroll
-  for (int g = 0; g < NG; ++g) {
-    acc[g][0] = acc[g][1] = 0.0;
-    m[g] = static_cast<const T*>(f.mat[g]) + (int64_t)row * n;
-  }
-  constexpr int U = NG <= 2 ? 8 : 4;
-  for (int c = lane; c < n; c += 64 * U) {
-    T v[U][NG];
-    double xv[U][2];
+  for (int g = 0; g < NG; ++g) acc[g][0] = acc[g][1] = 0.0;
+  for (int c = lane; c < n; c += 64) {
+    const double x0 = x[2 * c], x1 = x[2 * c + 1];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {   // past the row's end: clamped index, masked value
-      const int cc = c + 64 * u < n ? c + 64 * u : n - 1;
-#pragma unroll
-      for (int g = 0; g < NG; ++g) v[u][g] = m[g][cc];
-      xv[u][0] = x[2 * cc];
-      xv[u][1] = x[2 * cc + 1];
+    for (int g = 0; g < NG; ++g) {
+      const double m = (double)static_cast<const T*>(f.mat[g])[(int64_t)row * n + c];
+      acc[g][0] += m * x0;
+      acc[g][1] += m * x1;
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (c + 64 * u < n) {
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          acc[g][0] += (double)v[u][g] * xv[u][0];
-          acc[g][1] += (double)v[u][g] * xv[u][1];
-        }
-      }
   }
 #pragma unroll
   for (int g = 0; g < NG; ++g)
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) acc[g][s] += __shfl_xor(acc[g][s], o, 64);
+    for (int s = 0; s < 2; ++s) acc[g][s] = cc_wave_sum(acc[g][s]);
   if (lane < 2) {
     double t = 0.0;
 #pragma unroll
@@ -243,17 +228,23 @@ __global__ void formed_identity_kernel(FormedPlan f, const double* __restrict__ 
   if (i < 2 * f.n_env) y[i] = f.id[(i & 1) * 2] * x[i & ~1] + f.id[(i & 1) * 2 + 1] * x[i | 1];
 }
 
+template <typename T, int NG>
+void formed_launch_mats(hipStream_t st, const FormedPlan& f, const double* x, double* y) {
+  const unsigned grid = (unsigned)((f.n_env + FORMED_ROWS - 1) / FORMED_ROWS);
+  if (f.n_env <= 256) formed_apply_kernel<T, NG, 2><<<grid, FORMED_THREADS, 0, st>>>(f, x, y);
+  else if (f.n_env <= 640) formed_apply_kernel<T, NG, 5><<<grid, FORMED_THREADS, 0, st>>>(f, x, y);
+  else if (f.n_env <= 1408) formed_apply_kernel<T, NG, 11><<<grid, FORMED_THREADS, 0, st>>>(f, x, y);
+  else formed_apply_any_kernel<T, NG><<<(unsigned)((f.n_env + 3) / 4), 256, 0, st>>>(f, x, y);
+}
 template <typename T>
 int formed_launch(hipStream_t st, const FormedPlan& f, const double* x, double* y) {
-  const unsigned grid = (unsigned)((f.n_env + 3) / 4);
   switch (f.n_mats) {
     case 0: formed_identity_kernel<<<(unsigned)((2 * f.n_env + 255) / 256), 256, 0, st>>>(f, x, y); break;
-    case 1: formed_apply_kernel<T, 1><<<grid, 256, 0, st>>>(f, x, y); break;
-    case 2: formed_apply_kernel<T, 2><<<grid, 256, 0, st>>>(f, x, y); break;
-    case 3: formed_apply_kernel<T, 3><<<grid, 256, 0, st>>>(f, x, y); break;
-    case 4: formed_apply_kernel<T, 4><<<grid, 256, 0, st>>>(f, x, y); break;
-    case 5: formed_apply_kernel<T, 5><<<grid, 256, 0, st>>>(f, x, y); break;
-    default: cc_set_last_error("formed operator: at most 5 matrices"); return CC_ERR_UNSUPPORTED;
+    case 1: formed_launch_mats<T, 1>(st, f, x, y); break;
+    case 2: formed_launch_mats<T, 2>(st, f, x, y); break;
+    case 3: formed_launch_mats<T, 3>(st, f, x, y); break;
+    case 4: formed_launch_mats<T, 4>(st, f, x, y); break;
+    default: formed_launch_mats<T, 5>(st, f, x, y); break;
   }
   CC_LAUNCH_CHECK();
   return CC_OK;
@@ -354,7 +345,7 @@ extern "C" int cc_whiten_f64(void* stream, int64_t n, int n_mats, const double* 
 static int formed_plan_create(void** out, int64_t n_env, int64_t d, int n_mats, const void* const* mats, int f32,
                               const double* host_ops, const double* host_id) {
   *out = nullptr;
-  if (d != 2 || n_env < 1 || n_env > 1 << 20 || n_mats < 0 || n_mats > 5 || (n_mats == 0 && !host_id)) {
+  if (d != 2 || n_env < 1 || n_env > 1 << 20 || n_mats < 0 || n_mats > FORMED_MATS || (n_mats == 0 && !host_id)) {
     cc_set_last_error("formed operator: d = 2 and at most 5 matrices");
     return CC_ERR_UNSUPPORTED;
   }

@@ -2,7 +2,7 @@
 // operator W H W^T (W = L^-1 (x) I_d), with full (twice-applied) reorthogonalisation.  All
 // vectors and recurrence scalars stay in device memory; the host loop only reads two doubles
 // (Ritz value and residual estimate) every `check_every` steps.
-#include "cc_common.h"
+#include "cc_formed.h"
 
 #include <cmath>
 #include <vector>
@@ -10,7 +10,7 @@
 namespace {
 
 // sum_i a[i] b[i] over the 256 threads of a workgroup in a fixed order: each thread loads its DOT_U
-// pairs at once (clamped index, masked product), then a tree over the threads.
+// pairs at once (clamped index, masked product), then wave sums, added in wave order.
 constexpr int DOT_U = 12;
 __device__ inline double block_dot256(int64_t n, const double* __restrict__ a, const double* __restrict__ b, double* red) {
   double acc = 0.0;
@@ -26,19 +26,16 @@ __device__ inline double block_dot256(int64_t n, const double* __restrict__ a, c
     for (int u = 0; u < DOT_U; ++u)
       if (base + 256 * u < n) acc += x[u] * y[u];
   }
-  red[threadIdx.x] = acc;
+  acc = cc_wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
-  }
-  return red[0];
+  return ((red[0] + red[1]) + red[2]) + red[3];
 }
 
 // c[b] = Q_b . w for b < nq; a block b == nq (when launched) gives c[nq] = w . w
 __global__ void __launch_bounds__(256) lz_coeff_kernel(int64_t n, const double* __restrict__ Q, const double* __restrict__ w,
                                                        double* __restrict__ c, int nq) {
-  __shared__ double red[256];
+  __shared__ double red[4];
   const double* q = (int)blockIdx.x == nq ? w : Q + (int64_t)blockIdx.x * n;
   const double t = block_dot256(n, q, w, red);
   if (threadIdx.x == 0) c[blockIdx.x] = t;
@@ -46,6 +43,26 @@ __global__ void __launch_bounds__(256) lz_coeff_kernel(int64_t n, const double* 
 
 // w[i] -= sum_j c[j] Q[j][i]   (or z[i] = sum_j c[j] Q[j][i] when `assign`): block = 16 outputs x
 // 16 basis slices, slice sums combined in a fixed order.
+// sum_j c[j] Q[j][i] over the slice's vectors j = slice, slice + 16, ...: LZ_U loads in flight at a time
+constexpr int LZ_U = 5;
+__device__ inline double slice_combine(int m, int64_t n, const double* __restrict__ Q, const double* __restrict__ c, int slice,
+                                       int64_t i) {
+  double acc = 0.0;
+  for (int j0 = slice; j0 < m; j0 += 16 * LZ_U) {
+    double q[LZ_U], cj[LZ_U];
+#pragma unroll
+    for (int u = 0; u < LZ_U; ++u) {   // clamped index, masked product
+      const int j = j0 + 16 * u < m ? j0 + 16 * u : j0;
+      q[u] = Q[(int64_t)j * n + i];
+      cj[u] = c[j];
+    }
+#pragma unroll
+    for (int u = 0; u < LZ_U; ++u)
+      if (j0 + 16 * u < m) acc += cj[u] * q[u];
+  }
+  return acc;
+}
+
 // w -= Q^T c (assign: w = Q^T c) over the first m basis vectors; record (when given) receives c[m - 1]
 __global__ void __launch_bounds__(256) lz_combine_kernel(int m, int64_t n, const double* __restrict__ Q,
                                                          const double* __restrict__ c, double* __restrict__ w, int assign,
@@ -54,10 +71,7 @@ __global__ void __launch_bounds__(256) lz_combine_kernel(int m, int64_t n, const
   if (record != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *record = c[m - 1];
   const int e = threadIdx.x & 15, slice = threadIdx.x >> 4;
   const int64_t i = (int64_t)blockIdx.x * 16 + e;
-  double acc = 0.0;
-  if (i < n)
-    for (int j = slice; j < m; j += 16) acc += c[j] * Q[(int64_t)j * n + i];
-  red[slice][e] = acc;
+  red[slice][e] = i < n ? slice_combine(m, n, Q, c, slice, i) : 0.0;
   __syncthreads();
   if (slice == 0 && i < n) {
     double t = 0.0;
@@ -76,14 +90,14 @@ __global__ void __launch_bounds__(256) lz_combine_normalize_kernel(int m, int64_
   __shared__ double red[16][16];
   const int e = threadIdx.x & 15, slice = threadIdx.x >> 4;
   const int64_t i = (int64_t)blockIdx.x * 16 + e;
-  double acc = 0.0;
-  if (i < n)
-    for (int j = slice; j < m; j += 16) acc += c[j] * Q[(int64_t)j * n + i];
-  red[slice][e] = acc;
-  double cc = 0.0;
-  for (int j = 0; j < m; ++j) cc += c[j] * c[j];
-  const double b2 = c[m] - cc, b = b2 > 0.0 ? sqrt(b2) : 0.0, inv = b > 0.0 ? 1.0 / b : 0.0;
+  __shared__ double sq[4];
+  double cc = 0.0;   // c . c over the block
+  for (int j = threadIdx.x; j < m; j += 256) cc += c[j] * c[j];
+  red[slice][e] = i < n ? slice_combine(m, n, Q, c, slice, i) : 0.0;
+  cc = cc_wave_sum(cc);
+  if ((threadIdx.x & 63) == 0) sq[threadIdx.x >> 6] = cc;
   __syncthreads();
+  const double b2 = c[m] - (((sq[0] + sq[1]) + sq[2]) + sq[3]), b = b2 > 0.0 ? sqrt(b2) : 0.0, inv = b > 0.0 ? 1.0 / b : 0.0;
   if (slice == 0 && i < n) {
     double t = 0.0;
 #pragma unroll
@@ -427,7 +441,7 @@ namespace {
 // out[j] = sum_i U[j][i] v[i] for j < k  (one block per basis vector, fixed-order tree)
 __global__ void __launch_bounds__(256) jd_dots_kernel(int64_t n, const double* __restrict__ U, const double* __restrict__ v,
                                                       double* __restrict__ out, int stride_out) {
-  __shared__ double red[256];
+  __shared__ double red[4];
   const double t = block_dot256(n, U + (int64_t)blockIdx.x * n, v, red);
   if (threadIdx.x == 0) out[(int64_t)blockIdx.x * stride_out] = t;
 }
@@ -444,11 +458,10 @@ __global__ void cg_axpby_kernel(int64_t n, const double* __restrict__ sa, double
 
 // lowest eigenpair of the k x k pencil (Hs, Ns), k <= 32, single thread: Cholesky of Ns, cyclic Jacobi
 // on L^-1 Hs L^-T, back-transform.  out[0] = value, vec[0..k) N-normalised coefficients.
-// Sum of v over the 1024 threads of the workgroup in a fixed order (wave shuffles, then the 16 wave
-// sums in wave order); every thread gets the result.
+// Sum of v over the 1024 threads of the workgroup in a fixed order (wave sums, added in wave order);
+// every thread gets the result.
 __device__ inline double cg_block_sum(double v, double* red) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = cc_wave_sum(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __syncthreads();
   if (lane == 0) red[wave] = v;
@@ -553,6 +566,108 @@ __global__ void __launch_bounds__(1024) cg_step_reg_kernel(int64_t n, const doub
   if (threadIdx.x == 0) rr[0] = rr_new;
 }
 
+// A CG step and the next product of a formed operator in one launch (n <= 512 V): every workgroup takes the whole
+// step in registers -- the vectors come from the cache, and the loads of its matrix rows are in flight meanwhile --
+// keeps the new direction in LDS and multiplies its four rows by it.  Workgroup 0 alone writes the vectors, into the
+// other set of buffers, because the others may still be reading these.  The same step as cg_step_reg_kernel.  Bound by
+// its three sums in a row: 7.8 us at D = 6, against 7.5 us for the step and 6.3 us for the product as two launches.
+template <typename T, int NG, int U, int V>
+__global__ void __launch_bounds__(FORMED_THREADS) cg_formed_kernel(FormedPlan f, const double* __restrict__ rho_dev,
+                                                           const double* __restrict__ u, const double* __restrict__ ap,
+                                                           const double* __restrict__ p, const double* __restrict__ res,
+                                                           const double* __restrict__ rr, double* __restrict__ y,
+                                                           double* __restrict__ ap_out, double* __restrict__ p_out,
+                                                           double* __restrict__ res_out, double* __restrict__ rr_out) {
+  __shared__ double pn[V * 512];
+  __shared__ double red[16];
+  const int n = 2 * f.n_env, row0 = blockIdx.x * FORMED_ROWS, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  FormedRows<T, NG, U> rows;
+  rows.load(f, row0);
+  const double rho = rho_dev[0], rr0 = rr[0];
+  double a[V], pv[V], uv[V], rv[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) {   // past the end: clamped index, zeroed value (adds nothing to any sum)
+    const int i = threadIdx.x + 512 * k, ic = i < n ? i : 0;
+    const bool in = i < n;
+    a[k] = in ? ap[ic] : 0.0;
+    pv[k] = in ? p[ic] : 0.0;
+    uv[k] = in ? u[ic] : 0.0;
+    rv[k] = in ? res[ic] : 0.0;
+  }
+  auto block_sum = [&](double v) {   // fixed order: lanes, then waves; every thread gets it
+    v = cc_wave_sum(v);
+    __syncthreads();
+    if (lane == 0) red[wave] = v;
+    __syncthreads();
+    double t = red[0];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) t += red[w];
+    return t;
+  };
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    a[k] -= rho * pv[k];
+    s += uv[k] * a[k];
+  }
+  const double c = block_sum(s);
+  s = 0.0;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    a[k] -= c * uv[k];
+    s += pv[k] * a[k];
+  }
+  const double pap = block_sum(s);
+  // a converged (zero) residual or search direction ends the iteration with y unchanged, not a NaN
+  const double alpha = (pap != 0.0 && rr0 != 0.0) ? rr0 / pap : 0.0;
+  s = 0.0;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    rv[k] -= alpha * a[k];
+    s += rv[k] * rv[k];
+  }
+  const double rr1 = block_sum(s), beta = rr0 != 0.0 ? rr1 / rr0 : 0.0;
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    const int i = threadIdx.x + 512 * k;
+    const double q = rv[k] + beta * pv[k];
+    pn[i] = q;
+    if (blockIdx.x == 0 && i < n) {
+      y[i] += alpha * pv[k];
+      res_out[i] = rv[k];
+      p_out[i] = q;
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) rr_out[0] = rr1;
+  __syncthreads();
+  rows.apply(f, row0, [&](int col, int sp) { return pn[2 * col + sp]; }, red, ap_out);
+}
+
+template <typename T, int NG>
+void cg_formed_launch(hipStream_t st, const FormedPlan& f, const double* rho, const double* u, const double* ap, const double* p,
+                      const double* res, const double* rr, double* y, double* ap_out, double* p_out, double* res_out,
+                      double* rr_out) {
+  const unsigned grid = (unsigned)((f.n_env + FORMED_ROWS - 1) / FORMED_ROWS);
+  if (f.n_env <= 256) cg_formed_kernel<T, NG, 2, 1><<<grid, FORMED_THREADS, 0, st>>>(f, rho, u, ap, p, res, rr, y, ap_out, p_out, res_out, rr_out);
+  else if (f.n_env <= 640) cg_formed_kernel<T, NG, 5, 3><<<grid, FORMED_THREADS, 0, st>>>(f, rho, u, ap, p, res, rr, y, ap_out, p_out, res_out, rr_out);
+  else cg_formed_kernel<T, NG, 11, 6><<<grid, FORMED_THREADS, 0, st>>>(f, rho, u, ap, p, res, rr, y, ap_out, p_out, res_out, rr_out);
+}
+
+// Whether cg_formed_step serves the plan (FP32 matrices, one to four of them, at most 1408 rows).
+bool cg_formed_serves(const FormedPlan& f) { return f.f32 && f.n_mats >= 1 && f.n_mats <= 4 && f.n_env <= 1408; }
+int cg_formed_step(hipStream_t st, const FormedPlan& f, const double* rho, const double* u, const double* ap, const double* p,
+                   const double* res, const double* rr, double* y, double* ap_out, double* p_out, double* res_out,
+                   double* rr_out) {
+  switch (f.n_mats) {
+    case 1: cg_formed_launch<float, 1>(st, f, rho, u, ap, p, res, rr, y, ap_out, p_out, res_out, rr_out); break;
+    case 2: cg_formed_launch<float, 2>(st, f, rho, u, ap, p, res, rr, y, ap_out, p_out, res_out, rr_out); break;
+    case 3: cg_formed_launch<float, 3>(st, f, rho, u, ap, p, res, rr, y, ap_out, p_out, res_out, rr_out); break;
+    default: cg_formed_launch<float, 4>(st, f, rho, u, ap, p, res, rr, y, ap_out, p_out, res_out, rr_out); break;
+  }
+  CC_LAUNCH_CHECK();
+  return CC_OK;
+}
+
 // One wave; every element goes through the operations of the serial algorithm in its order, the lanes take different
 // rows (Cholesky, rotations), columns (the inverse factor) or entries (the projected matrix).  Bound by the chain of
 // rotations: k = 8 takes 34 us on average over a solve's passes, 104 us with one lane doing everything.
@@ -642,7 +757,7 @@ __global__ void __launch_bounds__(64) small_geneig_kernel(int k, const double* _
 // out[m][i][j] = sum U_i V_j for V = V0 (m = 0) and V1 (m = 1): one block per entry, the sums of jd_dots_kernel.
 __global__ void __launch_bounds__(256) jd_gram_kernel(int64_t n, const double* __restrict__ U, const double* __restrict__ V0,
                                                       const double* __restrict__ V1, double* __restrict__ out) {
-  __shared__ double red[256];
+  __shared__ double red[4];
   const double* V = blockIdx.z ? V1 : V0;
   const double t = block_dot256(n, U + (int64_t)blockIdx.x * n, V + (int64_t)blockIdx.y * n, red);
   if (threadIdx.x == 0) out[((int64_t)blockIdx.z * gridDim.x + blockIdx.x) * gridDim.y + blockIdx.y] = t;
@@ -763,6 +878,24 @@ static int jd_correction(hipStream_t st, ApplyFn apply, const void* plan, int64_
   CC_LAUNCH_CHECK();
   rc = cc_dot_f64(st, n, res, res, sc + 1);
   if (rc) return rc;
+  const FormedPlan* formed = apply == cc_internal_formed_apply ? static_cast<const FormedPlan*>(plan) : nullptr;
+  if (formed && cg_formed_serves(*formed) && iters > 0) {
+    // t1, t2 and tmp are free here: the second set of ap, res and p
+    double *ap2 = t1, *res2 = t2, *p2 = tmp, *rr = sc + 1, *rr2 = sc + 2;
+    if ((rc = apply(st, plan, p, ap))) return rc;
+    for (int k = 0; k + 1 < iters; ++k) {
+      if ((rc = cg_formed_step(st, *formed, rho_dev, u, ap, p, res, rr, y, ap2, p2, res2, rr2))) return rc;
+      double* s;
+      s = ap, ap = ap2, ap2 = s;
+      s = res, res = res2, res2 = s;
+      s = p, p = p2, p2 = s;
+      s = rr, rr = rr2, rr2 = s;
+    }
+    if (n <= 4096) cg_step_reg_kernel<4><<<1, 1024, 0, st>>>(n, rho_dev, u, ap, p, y, res, rr);
+    else cg_step_kernel<<<1, 1024, 0, st>>>(n, rho_dev, u, ap, p, y, res, rr);
+    CC_LAUNCH_CHECK();
+    iters = 0;
+  }
   for (int k = 0; k < iters; ++k) {
     // ap = P (W H W^T - rho) p   (p is kept in the projected space)
     rc = op_whitened(st, apply, plan, wh, p, t1, t2, ap);
