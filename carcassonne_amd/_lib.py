@@ -106,6 +106,8 @@ SIGNATURES = {
     "cc_stage3_pack_sum_f64": [_vp, _i32, _pvp, _pf64, _i64, _i64, _i64, _i64, _vp, _vp],
     "cc_stage3_matvec_fused_f64": [_vp, _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32, _i32, _pf64, _i64, _i64,
                                    _i64, _vp, _vp, _vp],
+    "cc_stage3_matvec_slabs_f64": [_vp, _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32, _i32, _pf64, _i64, _i64,
+                                   _i64, _vp, _vp, _vp],
     "cc_stage3_matvec_fused_f64_noalloc": [_vp, _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32, _i32, _pf64, _i64,
                                            _i64, _i64, _vp, _vp],
 }

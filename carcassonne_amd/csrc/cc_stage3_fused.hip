@@ -36,11 +36,13 @@ struct FusedPlan {
 };
 
 
-template <int P, int DP>
+// The FP64 kernel's tiling of slabs of extent P, 4 KS - 3 <= P <= 4 KS (the kernel takes P itself at run time: it only
+// enters where the vector is read and the partial sums are written).
+template <int KS_, int DP>
 struct Shape {
-  static constexpr int P4 = (P + 3) / 4 * 4;      // padded p / q extent (multiple of 4)
-  static constexpr int NT = (P + 15) / 16;         // 16-wide tiles over p' and q'
-  static constexpr int KS = P4 / 4;                // 4-deep k steps over p (stage A) and q (stage B)
+  static constexpr int KS = KS_;                   // 4-deep k steps over p (stage A) and q (stage B)
+  static constexpr int P4 = 4 * KS;                // padded p / q extent
+  static constexpr int NT = (P4 + 15) / 16;        // 16-wide tiles over p' and q'
   static constexpr int IDX = DP * P4;              // stage-A rows idx = s*P4 + q
   static constexpr int MT = (IDX + 15) / 16;       // stage-A row tiles
   static constexpr int SLAB = KS * NT * 64;        // packed doubles per alpha
@@ -88,9 +90,9 @@ __global__ void __launch_bounds__(256) pack_kernel_d(int64_t n_alpha, CCSlabGath
 }
 
 // Y += X B_b for one B channel at one alpha: X[s'](p' tile, q) against all q' tiles.
-template <int P, int DP, typename F>
-__device__ __forceinline__ void fused_product(const double* __restrict__ Bp, int lane, f64x4 (&y)[Shape<P, DP>::NT][DP], F x) {
-  constexpr int NT = Shape<P, DP>::NT, KS = Shape<P, DP>::KS;
+template <int KS, int DP, typename F>
+__device__ __forceinline__ void fused_product(const double* __restrict__ Bp, int lane, f64x4 (&y)[Shape<KS, DP>::NT][DP], F x) {
+  constexpr int NT = Shape<KS, DP>::NT;
   // B operands one K step ahead; the barrier keeps the scheduler from starting every step's loads at once, which
   // would take more registers than three waves per SIMD leave
   double bop[2][NT];
@@ -113,10 +115,10 @@ __device__ __forceinline__ void fused_product(const double* __restrict__ Bp, int
 }
 
 // Stage A: w[m] += V^T[16m.., :] A_a^T[:, 16np..] for one A channel at one alpha (V^T operands in LDS).
-template <int P, int DP>
+template <int KS, int DP>
 __device__ __forceinline__ void fused_stage_a(const double* __restrict__ Ap, const double* vt, int np, int lane,
-                                              f64x4 (&w)[Shape<P, DP>::MT]) {
-  constexpr int NT = Shape<P, DP>::NT, KS = Shape<P, DP>::KS, MT = Shape<P, DP>::MT;
+                                              f64x4 (&w)[Shape<KS, DP>::MT]) {
+  constexpr int NT = Shape<KS, DP>::NT, MT = Shape<KS, DP>::MT;
   double aop[KS];
 #pragma unroll
   for (int u = 0; u < KS; ++u) aop[u] = Ap[(u * NT + np) * 64 + lane];
@@ -137,20 +139,20 @@ __device__ __forceinline__ void fused_stage_a(const double* __restrict__ Ap, con
 // costs neither vector work nor registers.  D = 6, chi = 64, transverse-field Ising: 1026 MFMAs per alpha (1674 with a
 // stage B per term of the unsummed channels), 282 -> 146 us per application (109 us at the matrix rate); Heisenberg at
 // D = 5, chi = 37: 230 -> 44 us (there the earlier fixed sixteen alpha per workgroup left two thirds of the CUs idle).
-template <int P, int DP>
-__global__ void __launch_bounds__((Shape<P, DP>::THREADS), 3) fused_f64_kernel(const FusedPlan plan, int per,
+template <int KS, int DP>
+__global__ void __launch_bounds__((Shape<KS, DP>::THREADS), 3) fused_f64_kernel(const FusedPlan plan, int P, int per,
                                                                                        const double* __restrict__ v,
                                                                                        double* __restrict__ partial) {
-  using S = Shape<P, DP>;
-  constexpr int P4 = S::P4, NT = S::NT, KS = S::KS, MT = S::MT, SLAB = S::SLAB, TEAMS = S::TEAMS, NTH = S::THREADS;
+  using S = Shape<KS, DP>;
+  constexpr int P4 = S::P4, NT = S::NT, MT = S::MT, SLAB = S::SLAB, TEAMS = S::TEAMS, NTH = S::THREADS;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), np = wave % NT, team = wave / NT;
   const int64_t a0 = ((int64_t)blockIdx.x * TEAMS + team) * per, a1 = a0 + per < plan.n_alpha ? a0 + per : plan.n_alpha;
 
   // stage-A A operands (V O^T)^T[idx][p] (idx = 16m + lane%16, p = 4u + lane/16) of every vector, stored in LDS in
   // lane order so each read is conflict-free; the same LDS is reused for the final reduction.
-  constexpr int NY = P * P * DP;
-  constexpr int NVT = MT * KS * 64;
-  constexpr int NLDS = (MAX_VEC * NVT > TEAMS * NY) ? MAX_VEC * NVT : TEAMS * NY;
+  constexpr int NVT = MT * KS * 64, NYMAX = P4 * P4 * DP;
+  constexpr int NLDS = (MAX_VEC * NVT > TEAMS * NYMAX) ? MAX_VEC * NVT : TEAMS * NYMAX;
+  const int NY = P * P * DP;
   __shared__ double lds[NLDS];
   for (int e = threadIdx.x; e < NVT; e += NTH) {
     const int l = e & 63, mu = e >> 6, u = mu % KS, m = mu / KS;
@@ -186,13 +188,13 @@ __global__ void __launch_bounds__((Shape<P, DP>::THREADS), 3) fused_f64_kernel(c
     if (plan.n_hub > 0) {
       zero();
       for (int t = 0; t < plan.n_hub; ++t)
-        fused_stage_a<P, DP>(plan.A[plan.ha[t]] + al * SLAB, lds + plan.hv[t] * NVT, np, lane, w);
-      fused_product<P, DP>(plan.B[plan.hub_b] + al * SLAB, lane, y, wat);
+        fused_stage_a<KS, DP>(plan.A[plan.ha[t]] + al * SLAB, lds + plan.hv[t] * NVT, np, lane, w);
+      fused_product<KS, DP>(plan.B[plan.hub_b] + al * SLAB, lane, y, wat);
     }
     for (int t = 0; t < plan.n_direct;) {
       const int a = plan.da[t];
       zero();
-      fused_stage_a<P, DP>(plan.A[a] + al * SLAB, lds, np, lane, w);
+      fused_stage_a<KS, DP>(plan.A[a] + al * SLAB, lds, np, lane, w);
       for (; t < plan.n_direct && plan.da[t] == a; ++t) {
         const int o = plan.dop[t];
         double oc[DP][DP];
@@ -200,7 +202,7 @@ __global__ void __launch_bounds__((Shape<P, DP>::THREADS), 3) fused_f64_kernel(c
         for (int i = 0; i < DP; ++i)
 #pragma unroll
           for (int j = 0; j < DP; ++j) oc[i][j] = (o < 0) ? (i == j ? 1.0 : 0.0) : plan.ops[o < 0 ? 0 : o][i * DP + j];
-        fused_product<P, DP>(plan.B[plan.db[t]] + al * SLAB, lane, y, [&](int sp, int u) {
+        fused_product<KS, DP>(plan.B[plan.db[t]] + al * SLAB, lane, y, [&](int sp, int u) {
           double acc = 0.0;
 #pragma unroll
           for (int s = 0; s < DP; ++s) acc += oc[sp][s] * wat(s, u);
@@ -407,21 +409,38 @@ int launch_fused_f32(hipStream_t st, const FusedPlan& plan, const double* v, dou
   return CC_OK;
 }
 
-template <int P, int DP>
-int launch_fused(hipStream_t st, const FusedPlan& plan, const double* v, double* y, double* work, bool profile = true) {
+template <int KS>
+int launch_fused(hipStream_t st, const FusedPlan& plan, int P, const double* v, double* y, double* work, bool profile) {
   hipEvent_t e0 = nullptr;
   int rc = profile ? cc_prof_start(st, CC_PROF_FUSED_F64, &e0) : CC_OK;
   if (rc != CC_OK) return rc;
   const int64_t per = fused_f64_per(plan.n_alpha, P), groups = fused_f64_groups(plan.n_alpha, P);
   if (per > 2147483647LL) { cc_set_last_error("fused stage-3: too many slabs"); return CC_ERR_UNSUPPORTED; }
-  fused_f64_kernel<P, DP><<<(unsigned)groups, Shape<P, DP>::THREADS, 0, st>>>(plan, (int)per, v, work);
+  fused_f64_kernel<KS, 2><<<(unsigned)groups, Shape<KS, 2>::THREADS, 0, st>>>(plan, P, (int)per, v, work);
   CC_LAUNCH_CHECK();
   rc = profile ? cc_prof_stop(st, CC_PROF_FUSED_F64, e0) : CC_OK;
   if (rc != CC_OK) return rc;
-  const int64_t n = (int64_t)P * P * DP;
+  const int64_t n = (int64_t)P * P * 2;
   reduce_partials_kernel<<<(unsigned)((n + 15) / 16), 256, 0, st>>>(groups, n, work, y);
   CC_LAUNCH_CHECK();
   return CC_OK;
+}
+
+// The FP64 matvec for any slab extent 1 <= P <= 36 (d = 2).
+int fused_f64(hipStream_t st, const FusedPlan& plan, int64_t P, const double* v, double* y, double* work, bool profile = true) {
+  switch ((P + 3) / 4) {
+    case 1: return launch_fused<1>(st, plan, (int)P, v, y, work, profile);
+    case 2: return launch_fused<2>(st, plan, (int)P, v, y, work, profile);
+    case 3: return launch_fused<3>(st, plan, (int)P, v, y, work, profile);
+    case 4: return launch_fused<4>(st, plan, (int)P, v, y, work, profile);
+    case 5: return launch_fused<5>(st, plan, (int)P, v, y, work, profile);
+    case 6: return launch_fused<6>(st, plan, (int)P, v, y, work, profile);
+    case 7: return launch_fused<7>(st, plan, (int)P, v, y, work, profile);
+    case 8: return launch_fused<8>(st, plan, (int)P, v, y, work, profile);
+    case 9: return launch_fused<9>(st, plan, (int)P, v, y, work, profile);
+  }
+  cc_set_last_error("fused stage-3: slab extent above 36");
+  return CC_ERR_UNSUPPORTED;
 }
 
 // Workgroups of the FP32 kernel.
@@ -456,15 +475,7 @@ int apply_plan(hipStream_t st, const Stage3PlanHandle* h, const double* v, doubl
     cc_set_last_error("fused stage-3: shape not instantiated");
     return CC_ERR_UNSUPPORTED;
   }
-  switch (h->P) {
-    case 4: return launch_fused<4, 2>(st, h->plan, v, y, h->work);
-    case 9: return launch_fused<9, 2>(st, h->plan, v, y, h->work);
-    case 16: return launch_fused<16, 2>(st, h->plan, v, y, h->work);
-    case 25: return launch_fused<25, 2>(st, h->plan, v, y, h->work);
-    case 36: return launch_fused<36, 2>(st, h->plan, v, y, h->work);
-  }
-  cc_set_last_error("fused stage-3: shape not instantiated");
-  return CC_ERR_UNSUPPORTED;
+  return fused_f64(st, h->plan, h->P, v, y, h->work);
 }
 
 int fill_plan(FusedPlan& plan, int n_a, const double* const* A_packed, int n_b, const double* const* B_packed,
@@ -596,15 +607,19 @@ extern "C" int cc_stage3_matvec_fused_f64(void* stream, int n_a, const double* c
   FusedPlan plan;
   int rc = fill_plan(plan, n_a, A_packed, n_b, B_packed, n_terms, term_a, term_b, term_o, n_ops, host_ops, n_alpha, d);
   if (rc) return rc;
-  hipStream_t st = cc_stream(stream);
-  switch (P) {
-    case 4: return launch_fused<4, 2>(st, plan, v, y, work);
-    case 9: return launch_fused<9, 2>(st, plan, v, y, work);
-    case 16: return launch_fused<16, 2>(st, plan, v, y, work);
-    case 25: return launch_fused<25, 2>(st, plan, v, y, work);
-    case 36: return launch_fused<36, 2>(st, plan, v, y, work);
-  }
-  return CC_ERR_UNSUPPORTED;
+  return fused_f64(cc_stream(stream), plan, P, v, y, work);
+}
+
+extern "C" int cc_stage3_matvec_slabs_f64(void* stream, int n_a, const double* const* A_packed, int n_b,
+                                          const double* const* B_packed, int n_terms, const int* term_a,
+                                          const int* term_b, const int* term_o, int n_ops, const double* host_ops,
+                                          int64_t n_alpha, int64_t P, int64_t d, const double* v, double* y,
+                                          double* work) {
+  if (d != 2 || P < 1 || P > 36) { cc_set_last_error("slab stage-3: needs d = 2 and P <= 36"); return CC_ERR_UNSUPPORTED; }
+  FusedPlan plan;
+  int rc = fill_plan(plan, n_a, A_packed, n_b, B_packed, n_terms, term_a, term_b, term_o, n_ops, host_ops, n_alpha, d);
+  if (rc) return rc;
+  return fused_f64(cc_stream(stream), plan, P, v, y, work);
 }
 
 // ---- the allocation-free entry point -----------------------------------------------------------
@@ -657,15 +672,7 @@ extern "C" int cc_stage3_matvec_fused_f64_noalloc(void* stream, int n_a, const d
   double* scratch = nullptr;
   rc = noalloc_scratch(&scratch);
   if (rc) return rc;
-  hipStream_t st = cc_stream(stream);
-  switch (P) {
-    case 4: return launch_fused<4, 2>(st, plan, v, y, scratch, false);
-    case 9: return launch_fused<9, 2>(st, plan, v, y, scratch, false);
-    case 16: return launch_fused<16, 2>(st, plan, v, y, scratch, false);
-    case 25: return launch_fused<25, 2>(st, plan, v, y, scratch, false);
-    case 36: return launch_fused<36, 2>(st, plan, v, y, scratch, false);
-  }
-  return CC_ERR_UNSUPPORTED;
+  return fused_f64(cc_stream(stream), plan, P, v, y, scratch, false);
 }
 
 extern "C" int cc_stage3_plan_create(void** out, int n_a, const double* const* A_packed, int n_b,

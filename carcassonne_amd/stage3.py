@@ -15,6 +15,7 @@ import ctypes
 import weakref
 
 import numpy as np
+import torch
 
 from . import _lib
 from .data import HipData
@@ -158,7 +159,6 @@ class _Slab:
         """The channel in the FP32 kernel's operand order (cc_stage3_pack_strided_f32): role 0 as an A
         channel, role 1 as a B channel."""
         if role not in self._packed_f32:
-            import torch
             buf = torch.empty(_lib.query("cc_stage3_packed_size_f32", self.n_alpha, self.P, role), dtype=torch.float32,
                               device=self._base.device)
             base, (na0, na1, d0, d1), st = self.source()
@@ -197,9 +197,11 @@ class Stage3Operator:
         self._fused = None
         self._formed = None     # formed.FormedOperator, once a solver has formed this operator
         self._merge, self._joined, self._refreshed = None, {}, 0
-        self.use_fused = (self.P == self.Q and all(x.strided for x in self._A + self._B) and
-                          bool(_lib.load().cc_stage3_fused_supported(self.P, self.d)) and
-                          self._plan_fits())
+        # the slab kernels read P = Q <= 36, d = 2; the solvers, plans and low-precision forms (use_fused) serve the
+        # extents D * D of equal center bonds
+        self._use_slabs = (self.P == self.Q and self.P <= 36 and self.d == 2 and self.n_alpha > 0 and
+                           all(x.strided for x in self._A + self._B) and self._plan_fits())
+        self.use_fused = self._use_slabs and bool(_lib.load().cc_stage3_fused_supported(self.P, self.d))
 
     def _plan_fits(self):
         na = len({id(a) for a in self._A})
@@ -386,10 +388,11 @@ class Stage3Operator:
         if self._formed is not None and self._formed.valid():
             self._formed.apply_flat(x, y)
             return
-        if self.use_fused:
+        if self._use_slabs and (self.use_fused or self._fused is not None or not torch.cuda.is_current_stream_capturing()):
+            # also for unequal center bonds (packing may read site operators back, so not first under capture)
             self._ensure_fused()
             f = self._fused
-            _lib.call("cc_stage3_matvec_fused_f64", stream(), f["n_a"], f["A_ptrs"], f["n_b"], f["B_ptrs"],
+            _lib.call("cc_stage3_matvec_slabs_f64", stream(), f["n_a"], f["A_ptrs"], f["n_b"], f["B_ptrs"],
                       f["n_terms"], f["ta"], f["tb"], f["to"], f["n_ops"], f["ops"], self.n_alpha, self.P, self.d,
                       ptr(x), ptr(y), ptr(f["work"]))
             return
