@@ -5,8 +5,8 @@
 // Parameters live in one FP32 master buffer laid out [W1 (H x K0), b1 (H), W2 (H x H), b2 (H), W3 (NO x H),
 // b3 (NO)] (weights row-major out x in) with an FP16 mirror.  The forward pass multiplies FP16 activations
 // by FP16 weights on matrix cores (v_mfma_f32_16x16x16f16, FP32 accumulation) and keeps each hidden layer
-// in FP32 and as the FP16 copy the next layer reads.  The backward pass is FP32 (tiled FMA GEMMs over the
-// same FP16 values the forward used), the loss is the sign-free misalignment 1 - (y.v)^2 / (|y|^2 |v|^2)
+// in FP32 and as the FP16 copy the next layer reads.  The backward pass is FP32 (FP32 matrix-core products
+// over the same FP16 values the forward used), the loss is the sign-free misalignment 1 - (y.v)^2 / (|y|^2 |v|^2)
 // with the converged state v, and Adam updates the FP32 master and refreshes the FP16 mirror.  All sums
 // run in a fixed order.
 #include "cc_common.h"
@@ -33,115 +33,175 @@ MlpDims mlp_dims(int64_t K0, int64_t H, int64_t NO) {
   return d;
 }
 
-// Y[i][j] = act(sum_k X[i][k] W[j][k] + b[j]) for a 64 x 64 output tile per 256-thread workgroup; each wave
-// owns a 32 x 32 quarter as 2 x 2 MFMA tiles.  X (M x K) and W (N x K) are FP16 row-major, K % 16 == 0,
-// N % 64 == 0; rows past M are read as zero and not written.  Writes Y (FP32) and, if Yh, its FP16 copy.
+// Y[i][j] = act(sum_k X[i][k] W[j][k] + b[j]): one 16 x 16 MFMA tile per wave, 32 x 32 outputs per workgroup, the
+// operands loaded straight from memory in fragment order, MLP_AHEAD K steps at a time.  X (M x K) and W (N x K) are FP16
+// row-major, K % 16 == 0, N % 32 == 0; rows past M read the last row and are not written.  Writes Y (FP32) and, if Yh,
+// its FP16 copy.  Bound by load latency (a layer's weights are 0.5 MB): at 256 rows, 512 x 512, 12.7 us with 64 x 64
+// tiles through LDS (32 workgroups), 9.3 us here.  The sums run over K in order, so results do not depend on the tiling.
 // Operand fragments: A[i][k] in lane i + 16(k/4), element k%4; B[k][j] in lane j + 16(k/4), element k%4;
 // D[i][j] in lane j + 16(i/4), register i%4.
+constexpr int MLP_AHEAD = 8;
 __global__ void __launch_bounds__(256) mlp_linear_kernel(int64_t M, int64_t N, int64_t K, const _Float16* __restrict__ X,
                                                          const _Float16* __restrict__ W, const float* __restrict__ b,
                                                          int relu, float* __restrict__ Y, _Float16* __restrict__ Yh) {
-  __shared__ h4 As[64][4 + 1];
-  __shared__ h4 Bs[64][4 + 1];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wy = wave >> 1, wx = wave & 1;
-  const int64_t i0 = (int64_t)blockIdx.y * 64, j0 = (int64_t)blockIdx.x * 64;
-  f32x4 acc[2][2];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t j = (int64_t)blockIdx.x * 32 + 16 * (wave & 1) + (lane & 15);
+  const h4* wp = reinterpret_cast<const h4*>(W + j * K) + (lane >> 4);
+  const int steps = (int)(K / 16);
+  for (int64_t i0 = (int64_t)blockIdx.y * 32 + 16 * (wave >> 1); i0 < M; i0 += (int64_t)gridDim.y * 32) {
+    const int64_t xi = i0 + (lane & 15) < M ? i0 + (lane & 15) : M - 1;
+    const h4* xp = reinterpret_cast<const h4*>(X + xi * K) + (lane >> 4);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < steps; s0 += MLP_AHEAD) {
+      h4 xa[MLP_AHEAD], wb[MLP_AHEAD];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+      for (int u = 0; u < MLP_AHEAD; ++u) {
+        const int s = s0 + u < steps ? s0 + u : steps - 1;   // clamped; skipped below
+        xa[u] = xp[4 * s];
+        wb[u] = wp[4 * s];
+      }
 #pragma unroll
-    for (int c = 0; c < 2; ++c) acc[a][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const int lr = t >> 2, lq = t & 3;  // loader: row lr of the tile, 4-element quad lq of the 16-wide K step
-  for (int64_t k0 = 0; k0 < K; k0 += 16) {
-    const int64_t xi = i0 + lr;
-    h4 xa = {};
-    if (xi < M) xa = *reinterpret_cast<const h4*>(X + xi * K + k0 + 4 * lq);
-    As[lr][lq] = xa;
-    Bs[lr][lq] = *reinterpret_cast<const h4*>(W + (j0 + lr) * K + k0 + 4 * lq);
-    __syncthreads();
+      for (int u = 0; u < MLP_AHEAD; ++u)
+        if (s0 + u < steps) acc = __builtin_amdgcn_mfma_f32_16x16x16f16(xa[u], wb[u], acc, 0, 0, 0);
+    }
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const h4 af = As[32 * wy + 16 * a + (lane & 15)][lane >> 4];
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const h4 bf = Bs[32 * wx + 16 * c + (lane & 15)][lane >> 4];
-        acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x16f16(af, bf, acc[a][c], 0, 0, 0);
+    for (int r = 0; r < 4; ++r) {
+      const int64_t i = i0 + 4 * (lane >> 4) + r;
+      if (i < M) {
+        float v = acc[r] + b[j];
+        if (relu) v = v > 0.f ? v : 0.f;
+        Y[i * N + j] = v;
+        if (Yh) Yh[i * N + j] = (_Float16)v;
       }
     }
-    __syncthreads();
   }
+}
+
+// One product of the backward pass: C[i][j] = sum_k A(i, k) B[k][j], A FP32, B FP16 row-major with N columns, C
+// row-major.  A is stored M x K (`rows`: the gradient passed on, K % 64 == 0, any M) or K x M (a weight gradient,
+// M % 64 == 0, any K).  `mask`: C is zeroed where mask[i][j] <= 0 (the activation the ReLU left).  `rowsum`: also
+// receives sum_k A(i, k).
+struct MlpJob {
+  int64_t M, N, K;
+  const float* A;
+  bool rows;
+  const _Float16* B;
+  float* C;
+  const float* mask;
+  float* rowsum;
+};
+struct MlpJobs {
+  MlpJob job[2];
+  int64_t tiles0, tiles;   // tiles of the first product, of all
+};
+
+// element-aligned vectors: the pointers are a caller's
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef _Float16 h2u __attribute__((ext_vector_type(2), aligned(2)));
+
+// One wave's part of a tile, K chunks c0 .. c1 of 16 each.  Chunk c is summed in the order k = 16 c + 4 g + u for lane
+// group g at step u, so that a lane's four steps are neighbours in memory; rows and columns alternate between the two
+// 16-wide tiles of a pair (2 (lane % 16) + t), so that one load feeds both.  MLP_CHUNKS chunks are loaded together.
+// Rows past M and columns past N read the last ones and are not written; steps past K count as zero.
+constexpr int MLP_CHUNKS = 4;
+template <bool ROWS>
+__device__ inline void mlp_grad_wave(const MlpJob& jb, int64_t i0, int64_t j0, int64_t c0, int64_t c1, int l, int g,
+                                     f32x4 (&acc)[2][2], float (&rs)[2]) {
+  const int64_t M = jb.M, N = jb.N, K = jb.K;
+  const float* __restrict__ A = jb.A;
+  const _Float16* __restrict__ B = jb.B + (j0 + 2 * l < N ? j0 + 2 * l : N - 2);   // N is even
+  const int64_t r0 = i0 + 2 * l < M ? i0 + 2 * l : M - 1, r1 = i0 + 2 * l + 1 < M ? i0 + 2 * l + 1 : M - 1;
+  for (int64_t c = c0; c < c1; c += MLP_CHUNKS) {
+    float av[MLP_CHUNKS][2][4];
+    h2u bv[MLP_CHUNKS][4];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+    for (int q = 0; q < MLP_CHUNKS; ++q) {
+      const int64_t k0 = 16 * (c + q < c1 ? c + q : c1 - 1) + 4 * g;
+      if (ROWS) {
+        const f4u x0 = *reinterpret_cast<const f4u*>(A + r0 * K + k0), x1 = *reinterpret_cast<const f4u*>(A + r1 * K + k0);
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+        for (int u = 0; u < 4; ++u) { av[q][0][u] = x0[u]; av[q][1][u] = x1[u]; }
+      }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t i = i0 + 32 * wy + 16 * a + 4 * (lane >> 4) + r, j = j0 + 32 * wx + 16 * c + (lane & 15);
-        if (i < M) {
-          float v = acc[a][c][r] + b[j];
-          if (relu) v = v > 0.f ? v : 0.f;
-          Y[i * N + j] = v;
-          if (Yh) Yh[i * N + j] = (_Float16)v;
+      for (int u = 0; u < 4; ++u) {
+        const int64_t k = ROWS || k0 + u < K ? k0 + u : K - 1;
+        bv[q][u] = *reinterpret_cast<const h2u*>(B + k * N);
+        if (!ROWS) {
+          const f2u x = *reinterpret_cast<const f2u*>(A + k * M + r0);
+          av[q][0][u] = x[0];
+          av[q][1][u] = x[1];
+          if (k0 + u >= K) {
+            av[q][0][u] = av[q][1][u] = 0.f;
+            bv[q][u] = (h2u){0, 0};
+          }
         }
       }
-}
-
-// FP32 GEMM C[i][j] = sum_k A(i, k) B(k, j) (+ C[i][j] when accumulate), A(i, k) = A[i*sai + k*sak] and
-// B(k, j) = B[k*sbk + j*sbj] in element strides, either operand FP32 or FP16 (converted on load).  64 x 64
-// tile per 256-thread workgroup, 4 x 4 outputs per thread, K in steps of 16 through LDS.
-template <typename TA, typename TB>
-__global__ void __launch_bounds__(256) mlp_sgemm_kernel(int64_t M, int64_t N, int64_t K, const TA* __restrict__ A,
-                                                        int64_t sai, int64_t sak, const TB* __restrict__ B, int64_t sbk,
-                                                        int64_t sbj, float* __restrict__ C, int accumulate) {
-  __shared__ float As[16][64 + 1];
-  __shared__ float Bs[16][64 + 1];
-  const int t = threadIdx.x, ty = t >> 4, tx = t & 15;
-  const int64_t i0 = (int64_t)blockIdx.y * 64, j0 = (int64_t)blockIdx.x * 64;
-  float acc[4][4] = {};
-  for (int64_t k0 = 0; k0 < K; k0 += 16) {
-    for (int e = t; e < 16 * 64; e += 256) {
-      const int kk = e >> 6, ii = e & 63;
-      const int64_t i = i0 + ii, j = j0 + ii, k = k0 + kk;
-      As[kk][ii] = (i < M && k < K) ? (float)A[i * sai + k * sak] : 0.f;
-      Bs[kk][ii] = (j < N && k < K) ? (float)B[k * sbk + j * sbj] : 0.f;
     }
-    __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float av[4], bv[4];
+    for (int q = 0; q < MLP_CHUNKS; ++q) {
+      if (c + q >= c1) break;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        av[r] = As[kk][ty + 16 * r];
-        bv[r] = Bs[kk][tx + 16 * r];
-      }
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
+        for (int a = 0; a < 2; ++a) {
+          rs[a] += av[q][a][u];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[r][c] += av[r] * bv[c];
+          for (int b = 0; b < 2; ++b)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[q][a][u], (float)bv[q][u][b], acc[a][b], 0, 0, 0);
+        }
     }
-    __syncthreads();
   }
+}
+
+// Up to two products in one launch (a layer's weight gradient and the gradient passed on share their operand).  32 x 32
+// outputs per workgroup on v_mfma_f32_16x16x4f32; the four waves take a quarter of K each, straight from memory, and
+// are added in order through LDS, so that a product of 256 x 512 x 512 fills the chip and a wave's K loop is short.
+// FP32 throughout; bound by load latency.  At 256 samples, widths 272-512-512-512, a whole backward pass takes 39 us (each
+// launch 11.7 us); as FMA tiles on 64 to 128 workgroups (64 us a product), with the bias sums as one thread per column
+// (36 us) and the masks as kernels of their own, it took 443 us; at 8192 samples a whole training step 1.01 ms for 10.8.
+__global__ void __launch_bounds__(256) mlp_grad_kernel(const MlpJobs jobs) {
+  __shared__ float part[4][32][33];
+  __shared__ float rows[4][32];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l = lane & 15, g = lane >> 4;
+  for (int64_t t = blockIdx.x; t < jobs.tiles; t += gridDim.x) {
+    const MlpJob& jb = jobs.job[t >= jobs.tiles0];
+    const int64_t tile = t >= jobs.tiles0 ? t - jobs.tiles0 : t, tiles_n = (jb.N + 31) / 32, tn = tile % tiles_n;
+    const int64_t i0 = tile / tiles_n * 32, j0 = tn * 32;
+    const int64_t chunks = (jb.K + 15) / 16, c0 = chunks * wave / 4, c1 = chunks * (wave + 1) / 4;
+    f32x4 acc[2][2];
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int64_t i = i0 + ty + 16 * r, j = j0 + tx + 16 * c;
-      if (i < M && j < N) C[i * N + j] = acc[r][c] + (accumulate ? C[i * N + j] : 0.f);
+      for (int b = 0; b < 2; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    float rs[2] = {0.f, 0.f};
+    if (jb.rows) mlp_grad_wave<true>(jb, i0, j0, c0, c1, l, g, acc, rs);
+    else mlp_grad_wave<false>(jb, i0, j0, c0, c1, l, g, acc, rs);
+    __syncthreads();   // the previous tile's sums are read
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[wave][2 * (4 * g + r) + a][2 * l + b] = acc[a][b][r];
+      rs[a] += __shfl_xor(rs[a], 16, 64);
+      rs[a] += __shfl_xor(rs[a], 32, 64);
+      if (g == 0) rows[wave][2 * l + a] = rs[a];
     }
-}
-
-// g[j] = sum_i D[i][j] (rows in order), one thread per column
-__global__ void mlp_colsum_kernel(int64_t M, int64_t N, const float* __restrict__ D, float* __restrict__ g) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= N) return;
-  float s = 0.f;
-  for (int64_t i = 0; i < M; ++i) s += D[i * N + j];
-  g[j] = s;
-}
-
-// D *= (Hact > 0) elementwise (ReLU backward through the stored activation)
-__global__ void mlp_relu_bwd_kernel(int64_t n, const float* __restrict__ Hact, float* __restrict__ D) {
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x)
-    if (!(Hact[e] > 0.f)) D[e] = 0.f;
+    __syncthreads();
+    for (int e = threadIdx.x; e < 32 * 32; e += 256) {
+      const int i = e >> 5, j = e & 31;
+      const int64_t gi = i0 + i, gj = j0 + j;
+      if (gi < jb.M && gj < jb.N) {
+        float v = ((part[0][i][j] + part[1][i][j]) + part[2][i][j]) + part[3][i][j];
+        if (jb.mask && !(jb.mask[gi * jb.N + gj] > 0.f)) v = 0.f;
+        jb.C[gi * jb.N + gj] = v;
+      }
+    }
+    if (jb.rowsum && tn == 0 && threadIdx.x < 32)   // M % 64 == 0 where it is asked for
+      jb.rowsum[i0 + threadIdx.x] =
+          ((rows[0][threadIdx.x] + rows[1][threadIdx.x]) + rows[2][threadIdx.x]) + rows[3][threadIdx.x];
+  }
 }
 
 // Per sample b (one 256-thread workgroup): loss[b] = 1 - (y.v)^2 / (|y|^2 |v|^2) and
@@ -212,11 +272,15 @@ __global__ void mlp_features_kernel(int n_spec, int k, const double* __restrict_
   }
 }
 
-template <typename TA, typename TB>
-int sgemm(hipStream_t st, int64_t M, int64_t N, int64_t K, const TA* A, int64_t sai, int64_t sak, const TB* B, int64_t sbk,
-          int64_t sbj, float* C, int accumulate) {
-  const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
-  mlp_sgemm_kernel<TA, TB><<<grid, 256, 0, st>>>(M, N, K, A, sai, sak, B, sbk, sbj, C, accumulate);
+int mlp_grad(hipStream_t st, const MlpJob& first, const MlpJob* second) {
+  MlpJobs jobs = {};
+  jobs.job[0] = first;
+  jobs.tiles0 = jobs.tiles = (first.M + 31) / 32 * ((first.N + 31) / 32);
+  if (second) {
+    jobs.job[1] = *second;
+    jobs.tiles += (second->M + 31) / 32 * ((second->N + 31) / 32);
+  }
+  mlp_grad_kernel<<<(unsigned)(jobs.tiles < 65536 ? jobs.tiles : 65536), 256, 0, st>>>(jobs);
   CC_LAUNCH_CHECK();
   return CC_OK;
 }
@@ -256,13 +320,13 @@ extern "C" int cc_mlp_forward(void* stream, int64_t B, int64_t K0, int64_t H, in
   _Float16* h2h = h1h + B * H;
   float* h1 = A32;
   float* h2 = A32 + B * H;
-  const unsigned gy = (unsigned)((B + 63) / 64);
-  mlp_linear_kernel<<<dim3((unsigned)(H / 64), gy), 256, 0, st>>>(B, H, K0, static_cast<const _Float16*>(X16), p + d.w1,
+  const unsigned gy = (unsigned)(B < 32 * 65535LL ? (B + 31) / 32 : 65535);
+  mlp_linear_kernel<<<dim3((unsigned)(H / 32), gy), 256, 0, st>>>(B, H, K0, static_cast<const _Float16*>(X16), p + d.w1,
                                                                   P32 + d.b1, 1, h1, h1h);
   CC_LAUNCH_CHECK();
-  mlp_linear_kernel<<<dim3((unsigned)(H / 64), gy), 256, 0, st>>>(B, H, H, h1h, p + d.w2, P32 + d.b2, 1, h2, h2h);
+  mlp_linear_kernel<<<dim3((unsigned)(H / 32), gy), 256, 0, st>>>(B, H, H, h1h, p + d.w2, P32 + d.b2, 1, h2, h2h);
   CC_LAUNCH_CHECK();
-  mlp_linear_kernel<<<dim3((unsigned)(NO / 64), gy), 256, 0, st>>>(B, NO, H, h2h, p + d.w3, P32 + d.b3, 0, Y, nullptr);
+  mlp_linear_kernel<<<dim3((unsigned)(NO / 32), gy), 256, 0, st>>>(B, NO, H, h2h, p + d.w3, P32 + d.b3, 0, Y, nullptr);
   CC_LAUNCH_CHECK();
   return CC_OK;
 }
@@ -290,25 +354,15 @@ extern "C" int cc_mlp_backward(void* stream, int64_t B, int64_t K0, int64_t H, i
   float* dZ1 = dZ2 + B * H;
   mlp_loss_kernel<<<(unsigned)B, 256, 0, st>>>(NO, Y, target, 1.f / (float)B, loss, dY);
   CC_LAUNCH_CHECK();
-  // layer 3: dW3 = dY^T h2h, db3 = colsum dY, dZ2 = (dY W3) * [h2 > 0]
-  if ((rc = sgemm<float, _Float16>(st, NO, H, B, dY, 1, NO, h2h, H, 1, G + d.w3, 0))) return rc;
-  mlp_colsum_kernel<<<(unsigned)((NO + 255) / 256), 256, 0, st>>>(B, NO, dY, G + d.b3);
-  CC_LAUNCH_CHECK();
-  if ((rc = sgemm<float, _Float16>(st, B, H, NO, dY, NO, 1, p + d.w3, H, 1, dZ2, 0))) return rc;
-  mlp_relu_bwd_kernel<<<cc_blocks(B * H, 256), 256, 0, st>>>(B * H, h2, dZ2);
-  CC_LAUNCH_CHECK();
-  // layer 2
-  if ((rc = sgemm<float, _Float16>(st, H, H, B, dZ2, 1, H, h1h, H, 1, G + d.w2, 0))) return rc;
-  mlp_colsum_kernel<<<(unsigned)((H + 255) / 256), 256, 0, st>>>(B, H, dZ2, G + d.b2);
-  CC_LAUNCH_CHECK();
-  if ((rc = sgemm<float, _Float16>(st, B, H, H, dZ2, H, 1, p + d.w2, H, 1, dZ1, 0))) return rc;
-  mlp_relu_bwd_kernel<<<cc_blocks(B * H, 256), 256, 0, st>>>(B * H, h1, dZ1);
-  CC_LAUNCH_CHECK();
-  // layer 1
-  if ((rc = sgemm<float, _Float16>(st, H, K0, B, dZ1, 1, H, x, K0, 1, G + d.w1, 0))) return rc;
-  mlp_colsum_kernel<<<(unsigned)((H + 255) / 256), 256, 0, st>>>(B, H, dZ1, G + d.b1);
-  CC_LAUNCH_CHECK();
-  return CC_OK;
+  // per layer: dW = dZ^T h with its bias sums, and the gradient passed on, dZ W where the activation is positive
+  const MlpJob w3 = {NO, H, B, dY, false, h2h, G + d.w3, nullptr, G + d.b3};
+  const MlpJob z2 = {B, H, NO, dY, true, p + d.w3, dZ2, h2, nullptr};
+  if ((rc = mlp_grad(st, w3, &z2))) return rc;
+  const MlpJob w2 = {H, H, B, dZ2, false, h1h, G + d.w2, nullptr, G + d.b2};
+  const MlpJob z1 = {B, H, H, dZ2, true, p + d.w2, dZ1, h1, nullptr};
+  if ((rc = mlp_grad(st, w2, &z1))) return rc;
+  const MlpJob w1 = {H, K0, B, dZ1, false, x, G + d.w1, nullptr, G + d.b1};
+  return mlp_grad(st, w1, nullptr);
 }
 
 extern "C" int cc_mlp_adam(void* stream, int64_t n, float* P32, const float* G, float* M, float* V, void* P16, double lr,

@@ -68,6 +68,32 @@ def test_gradients_match_oracle(gpu):
         assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b) + 1e-10, name
 
 
+# (batch, spectra width, output, hidden): one sample, batches that leave a partial K chunk, a partial row tile or waves
+# without work, input widths of one and a half column tiles, the smallest widths and unequal ones
+@pytest.mark.parametrize("B,k,NO,H", [(1, 1, 64, 64), (5, 4, 64, 128), (17, 1, 192, 64), (33, 5, 128, 64), (100, 2, 64, 192),
+                                      (250, 16, 128, 128)])
+def test_gradients_at_ragged_sizes(gpu, B, k, NO, H):
+    """As above; FP32 sums of at most 250 terms: 1e-4 is ten times 250 x 2^-24, for some cancellation."""
+    net = _net(k=k, NO=NO, H=H)
+    X, V = _batch(net, B, 4)
+    Xd, Vd = torch.from_numpy(X).cuda(), torch.from_numpy(V).cuda()
+    loss, _ = net.loss_and_grad(Xd, Vd)
+    Yf, (A16, A32) = net.forward(Xd)
+    h = A32.cpu().numpy().reshape(2, B, H)
+    hr = A16.float().cpu().numpy().reshape(2, B, H)
+    p = net.P32.cpu().numpy().astype(np.float64)
+    want, _ = OM.forward(p, X.astype(np.float64), net.K0, H, NO)
+    assert np.linalg.norm(Yf.cpu().numpy() - want) <= 1e-4 * np.linalg.norm(want)
+    saved = dict(h1=h[0], h2=h[1], h1r=hr[0], h2r=hr[1], y=Yf.cpu().numpy())
+    g_want, l_want = OM.backward(p, X.astype(np.float64), V.astype(np.float64), net.K0, H, NO, saved=saved)
+    np.testing.assert_allclose(loss.cpu().numpy(), l_want, rtol=1e-4, atol=1e-6)
+    g = net.G.cpu().numpy()
+    parts = OM.split_params(np.arange(g.size), net.K0, H, NO)
+    for name, idx in zip(("W1", "b1", "W2", "b2", "W3", "b3"), parts):
+        a, b = g[idx.ravel()], g_want[idx.ravel()]
+        assert np.linalg.norm(a - b) <= 1e-4 * np.linalg.norm(b) + 1e-10, name
+
+
 def test_adam_step(gpu):
     net = _net()
     X, V = _batch(net, 64, 2)
