@@ -206,124 +206,250 @@ __global__ void __launch_bounds__(SVD_THREADS) svd_jacobi_kernel(int64_t m, int 
     __syncthreads();
   }
 }
-// Eigen-decomposition of a symmetric n x n matrix (n <= 64) by the parallel cyclic Jacobi method, matrix and
-// eigenvectors in LDS: each round of the round-robin ordering rotates n/2 disjoint (p, q) pairs, G -> J^T G J
-// and V -> V J, in one phase over the 2 x 2 blocks that pairs of pairs cut out of G.  A pair is rotated while
-// |g_pq| > 1e-15 sqrt(|g_pp g_qq|) and |g_pq| > 1e-15 tr|G| (off-diagonal entries below the second bound move
-// the eigenvalues by less than the rounding of G itself, and rotating them would not terminate for
-// rank-deficient G).  Outputs: lam descending (stable by index) and Vt[r][i] = component i of eigenvector r.
-constexpr int SYM_THREADS = 1024;
+// Eigen-decomposition of a symmetric n x n matrix (n <= 64) by the parallel cyclic Jacobi method on one workgroup.  The
+// odd-even ordering: rounds alternate between the position pairs (2k, 2k + 1) and (2k + 1, 2k + 2), and a pair swaps
+// places as it rotates (G -> J^T G J, V -> V J), so that after np rounds every two columns have met once and the order is
+// reversed.  A pair is rotated while |g_pq| > 1e-15 sqrt(|g_pp g_qq|) and |g_pq| > 1e-15 tr|G| (off-diagonal entries
+// below the second bound move the eigenvalues by less than the rounding of G itself, and rotating them would not
+// terminate for rank-deficient G), otherwise it only swaps.  Outputs: lam descending and Vt[r][i] = component i of
+// eigenvector r.
+//
+// Bound by the chain of a round (read, angle, rotate, write, barrier), 64 of them per sweep, so everything in it is
+// short: one barrier per round; the angle from two reciprocal square roots; the matrix in position coordinates, where
+// addresses are fixed per thread and parity and free of bank conflicts, its upper half only.  Waves 0 to 3 (one per
+// SIMD) hold G: each computes all angles itself and rotates the 2 x 2 blocks between pair k and pairs k + d; what a
+// round reads and what it writes of the diagonal and of the pairs' own entries are different cells.  Waves 4 to 7
+// keep V in registers, a row's columns 2k, 2k + 1 in lane k, one round behind.  n = 64, ten sweeps: 309 us (0.48 us a round,
+// half of it the LDS reads, the rotation and the barrier), against 733 us for the round-robin order with two barriers,
+// three divides and two square roots per round and V in LDS; n = 21: 75 us for 150.
+constexpr int SYM_THREADS = 512;
 constexpr int SYM_MAX_N = 64;
-constexpr int SYM_TASKS = SYM_MAX_N * (SYM_MAX_N / 2) / SYM_THREADS;  // (entry pair) tasks per thread and phase
-static_assert(SYM_TASKS * SYM_THREADS == SYM_MAX_N * (SYM_MAX_N / 2), "tasks must cover n * n/2 exactly");
+constexpr int SYM_HALF = SYM_MAX_N / 2;
+// LDS cells (doubles): G, then the pairs' entries as the next round of their parity reads them (GP) and as the last one
+// left them (GA), then cells for lanes without a block
+constexpr int SYM_G = (SYM_HALF + 1) * SYM_MAX_N, SYM_GP = SYM_G, SYM_GA = SYM_GP + 2 * SYM_HALF,
+              SYM_IDLE = SYM_GA + 2 * SYM_HALF, SYM_CELLS = SYM_IDLE + 64;
 
-template <int NC>  // NC = n known at compile time (index arithmetic by shifts and constant divisors), 0 = any n
-__global__ void __launch_bounds__(SYM_THREADS) sym_jacobi_kernel(int n_rt, const double* __restrict__ A,
-                                                                 double* __restrict__ lam, double* __restrict__ Vt) {
-  const int n = NC ? NC : n_rt;
-  __shared__ double G[SYM_MAX_N * SYM_MAX_N];
-  __shared__ double V[SYM_MAX_N * SYM_MAX_N];
-  __shared__ double rot_c[SYM_MAX_N / 2], rot_s[SYM_MAX_N / 2];
-  __shared__ int rot_p[SYM_MAX_N / 2], rot_q[SYM_MAX_N / 2], rot_on[SYM_MAX_N / 2];
-  __shared__ int perm[SYM_MAX_N];
-  __shared__ double trace_abs;
-  __shared__ int rotated;
-  const int tid = threadIdx.x;
-  for (int e = tid; e < n * n; e += SYM_THREADS) {
-    G[e] = A[e];
-    V[e] = (e / n == e % n) ? 1.0 : 0.0;
+// cell of entry (i, j), i != j mod np: by circular distance and row, rows of one parity next to each other
+__device__ inline int sym_cell(int i, int j, int np) {
+  const int h = np / 2;
+  i %= np;
+  j %= np;
+  int d = j - i + (j < i ? np : 0);
+  if (d > h || (d == h && i >= h)) {
+    i = j;
+    d = np - d;
   }
-  __syncthreads();
-  if (tid == 0) {
-    double t = 0.0;
-    for (int i = 0; i < n; ++i) t += fabs(G[i * n + i]);
-    trace_abs = t;
-  }
-  __syncthreads();
-  const double floor_abs = 1e-15 * trace_abs;
-  const int np = (n + 1) & ~1, half = np / 2;
-  for (int sweep = 0; sweep < 60; ++sweep) {
-    if (tid == 0) rotated = 0;
-    __syncthreads();
-    for (int round = 0; round < np - 1; ++round) {
-      if (tid < half) {
-        int p = tournament_player(tid, round, np), q = tournament_player(np - 1 - tid, round, np);
-        if (p > q) { const int t = p; p = q; q = t; }
-        int on = 0;
-        if (q < n) {
-          const double a = G[p * n + p], b = G[q * n + q], g = G[p * n + q];
-          if (fabs(g) > 1e-15 * sqrt(fabs(a * b)) && fabs(g) > floor_abs) {
-            const double theta = (b - a) / (2.0 * g);
-            const double t = (theta >= 0.0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-            const double c = 1.0 / sqrt(t * t + 1.0);
-            rot_c[tid] = c;
-            rot_s[tid] = t * c;
-            on = 1;
-            rotated = 1;
-          }
-        }
-        rot_p[tid] = p;
-        rot_q[tid] = q;
-        rot_on[tid] = on;
-      }
-      __syncthreads();
-      // One phase: thread t < half^2 takes the 2 x 2 block of G on the rows of pair t / half and the columns
-      // of pair t % half and forms J1^T (B J2) in that order (the column rotation, then the row rotation,
-      // each entry through the same operations as a columns-then-rows sweep of the whole matrix); the V
-      // columns of every pair (V J) are spread over all threads.  Blocks and V entries are disjoint, so
-      // one barrier ends the round.  A pair that does not rotate acts as the identity.
-      if (tid < half * half) {
-        const int k1 = tid / half, k2 = tid - (tid / half) * half;
-        const int a0 = rot_p[k1], a1 = rot_q[k1], b0 = rot_p[k2], b1 = rot_q[k2];
-        const bool on1 = rot_on[k1], on2 = rot_on[k2];
-        if (on1 || on2) {
-          const double c1 = on1 ? rot_c[k1] : 1.0, s1 = on1 ? rot_s[k1] : 0.0;
-          const double c2 = on2 ? rot_c[k2] : 1.0, s2 = on2 ? rot_s[k2] : 0.0;
-          const bool r0 = a0 < n, r1 = a1 < n, q0 = b0 < n, q1 = b1 < n;   // indices past n are padding
-          const double x00 = (r0 && q0) ? G[a0 * n + b0] : 0.0, x01 = (r0 && q1) ? G[a0 * n + b1] : 0.0;
-          const double x10 = (r1 && q0) ? G[a1 * n + b0] : 0.0, x11 = (r1 && q1) ? G[a1 * n + b1] : 0.0;
-          // columns (B J2)
-          const double y00 = c2 * x00 - s2 * x01, y01 = s2 * x00 + c2 * x01;
-          const double y10 = c2 * x10 - s2 * x11, y11 = s2 * x10 + c2 * x11;
-          // rows (J1^T (B J2))
-          if (r0 && q0) G[a0 * n + b0] = c1 * y00 - s1 * y10;
-          if (r0 && q1) G[a0 * n + b1] = c1 * y01 - s1 * y11;
-          if (r1 && q0) G[a1 * n + b0] = s1 * y00 + c1 * y10;
-          if (r1 && q1) G[a1 * n + b1] = s1 * y01 + c1 * y11;
-        }
-      }
-      {  // columns p, q of V
+  return (2 * d + (i & 1)) * SYM_HALF + (i >> 1);
+}
+
+// 1 / sqrt(x), x > 0 normal: the hardware's estimate (24 bits) and one step of third order
+__device__ inline double sym_rsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x), e = __builtin_fma(-(x * y), y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+
+// lane l takes `v` of lane l + 1; the last lane zero
+__device__ inline double sym_from_next(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x130, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x130, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// lane l takes `v` of lane l - 1; lane 0 keeps `old`
+__device__ inline double sym_from_previous(double old, double v) {
+  const long long b = __double_as_longlong(v), o = __double_as_longlong(old);
+  const int lo = __builtin_amdgcn_update_dpp((int)o, (int)b, 0x138, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(b >> 32), 0x138, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+struct SymLds {
+  double g[SYM_CELLS];
+  double dg[2][SYM_MAX_N];                     // diagonal, read by rounds of one parity, written by the other's
+  double rc[2][SYM_HALF], rs[2][SYM_HALF];     // rotations of the last two rounds
+  int rank[SYM_MAX_N];
+  int again;
+};
+
+// one thread's part of G
+struct SymBlocks {
+  int k, h, np;
+  double floor_abs;
+  int partner[2];
+  int cell[2][2][4];      // [parity][block][entry]
+  int next_pair[2];       // where entry 2 of block 0 goes when it is a pair's entry of the next round, else its cell
+};
+
+// Pair k of a round of parity O: positions 2k + O and 2k + 1 + O mod np.  New values (x the first's, y the second's):
+// s x + c y and c x - s y.  In odd rounds the last pair (position np - 1 and 0) stays as it is: c = 0, s = 1, + s y.
+template <int O>
+__device__ inline bool sym_round(SymLds& L, const SymBlocks& B, bool writer) {
+  const int k = B.k, P = 2 * k + O, Q = (O && k == B.h - 1) ? 0 : P + 1;
+  const bool still = k >= B.h || (O && k == B.h - 1);
+  const int Pc = k < B.h ? P : 0, Qc = k < B.h ? Q : 0;
+  const double a = L.dg[O][Pc], bb = L.dg[O][Qc], g = L.g[SYM_GP + O * SYM_HALF + k];
+  __builtin_amdgcn_sched_barrier(0);   // the angle's operands first
+  double x[2][4];
 #pragma unroll
-        for (int it = 0; it < SYM_TASKS; ++it) {
-          const int e = tid + it * SYM_THREADS, k = e % half, i = e / half;
-          if (e < n * half && rot_on[k]) {
-            const int ip = i * n + rot_p[k], iq = i * n + rot_q[k];
-            const double c = rot_c[k], sn = rot_s[k], vx = V[ip], vy = V[iq];
-            V[ip] = c * vx - sn * vy;
-            V[iq] = sn * vx + c * vy;
-          }
-        }
-      }
-      __syncthreads();
-    }
-    const int any = rotated;
-    __syncthreads();
-    if (!any) break;
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[b][e] = L.g[B.cell[O][b][e]];
+  __builtin_amdgcn_sched_barrier(0);
+  const double gg = g * g;
+  const bool on = !still & (fabs(g) > B.floor_abs) & (gg > 1e-30 * fabs(a * bb));
+  const double d = bb - a;
+  const double r = sym_rsqrt(__builtin_fma(4.0, gg, d * d));
+  const double c2 = __builtin_fma(0.5 * fabs(d), r, 0.5), q = sym_rsqrt(c2);
+  const double sr = (d >= 0.0 ? g : -g) * r * q;
+  const double c = on ? c2 * q : (still ? 0.0 : 1.0), s = on ? sr : (still ? 1.0 : 0.0);
+  double c1[2], s1[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    c1[b] = __shfl(c, B.partner[b], 64);
+    s1[b] = __shfl(s, B.partner[b], 64);
   }
-  for (int j = tid; j < n; j += SYM_THREADS) {
-    const double dj = G[j * n + j];
-    int r = 0;
-    for (int k = 0; k < n; ++k) {
-      const double dk = G[k * n + k];
-      r += (dk > dj) || (dk == dj && k < j);
+  const double sq = (O && k == B.h - 1) ? s : -s;
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const double q1 = (O && B.partner[b] == B.h - 1) ? s1[b] : -s1[b];
+    const double y00 = s * x[b][0] + c * x[b][2], y01 = s * x[b][1] + c * x[b][3];
+    const double y10 = c * x[b][0] + sq * x[b][2], y11 = c * x[b][1] + sq * x[b][3];
+    L.g[B.cell[O][b][0]] = s1[b] * y00 + c1[b] * y01;
+    L.g[B.cell[O][b][1]] = c1[b] * y00 + q1 * y01;
+    L.g[b ? B.cell[O][b][2] : B.next_pair[O]] = s1[b] * y10 + c1[b] * y11;
+    L.g[B.cell[O][b][3]] = c1[b] * y10 + q1 * y11;
+  }
+  if (writer) {
+    const double tg = on ? sr * q * g : 0.0;
+    L.rc[O][k] = c;
+    L.rs[O][k] = s;
+    if (k < B.h) {
+      L.dg[1 - O][P] = still ? a : bb + tg;
+      L.dg[1 - O][Q] = still ? bb : a - tg;
+      L.g[SYM_GA + O * SYM_HALF + k] = on ? 0.0 : g;
     }
-    perm[r] = j;
+  }
+  return on;
+}
+
+// V through the rotations of a round of parity O: x0, x1 = columns 2k, 2k + 1 of eight rows, two rows per wave step in
+// the half waves.  In odd rounds a lane borrows column 2k + 2 from the next lane and hands it back; where the next lane
+// is not the next pair (the last pair, idle lanes) it goes back as it came (c = 0, s = 1, + s y).
+template <int O>
+__device__ inline void sym_vectors(const SymLds& L, int k, int h, double (&x0)[8], double (&x1)[8]) {
+  const double c = L.rc[O][k], s = L.rs[O][k], sq = (O && k >= h - 1) ? s : -s;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    if (O == 0) {
+      const double a = s * x0[u] + c * x1[u], b = c * x0[u] + sq * x1[u];
+      x0[u] = a;
+      x1[u] = b;
+    } else {
+      const double y = sym_from_next(x0[u]);   // column 2k + 2
+      const double a = s * x1[u] + c * y, b = c * x1[u] + sq * y;
+      x1[u] = a;
+      x0[u] = sym_from_previous(x0[u], b);
+    }
+  }
+}
+
+__global__ void __launch_bounds__(SYM_THREADS) sym_jacobi_kernel(int n, const double* __restrict__ A,
+                                                                 double* __restrict__ lam, double* __restrict__ Vt) {
+  __shared__ SymLds L;
+  const int np = n > 5 ? (n + 1) & ~1 : 6, h = np / 2;   // positions past n hold zeros; at least three pairs
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, k = lane & 31;
+  const double tr = cc_wave_sum(lane < n ? fabs(A[lane * n + lane]) : 0.0);
+  const int ex = tr > 0.0 && tr < INFINITY ? ilogb(tr) : 0;   // scaled by 2^-ex: the trace is in [1, 2)
+  for (int e = tid; e < np * np; e += SYM_THREADS) {
+    const int i = e / np, j = e % np;
+    const double v = i < n && j < n ? ldexp(A[i * n + j], -ex) : 0.0;
+    if (i == j) L.dg[0][i] = v;
+    else if (i < j) L.g[sym_cell(i, j, np)] = v;
+    if (j == i + 1) L.g[(i & 1 ? SYM_GA : SYM_GP) + (i & 1) * SYM_HALF + (i >> 1)] = v;
+    if (i == 0 && j == np - 1) L.g[SYM_GA + SYM_HALF + h - 1] = v;
+  }
+  if (tid < 64) L.g[SYM_IDLE + tid] = 0.0;
+  SymBlocks B;
+  double x0[8], x1[8];
+  const bool vectors = wave >= 4;
+  if (!vectors) {
+    __builtin_amdgcn_s_setprio(2);   // the chain; V has time to spare
+    B.k = k;
+    B.h = h;
+    B.np = np;
+    B.floor_abs = 1e-15 * ldexp(tr, -ex);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int d = 2 * wave + (lane >> 5) + 1 + 8 * b;
+      const bool active = k < h && (2 * d < h || (2 * d == h && k < h / 2));
+      B.partner[b] = active ? (k + d) % h : 0;
+#pragma unroll
+      for (int O = 0; O < 2; ++O)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          B.cell[O][b][e] = active ? sym_cell(2 * k + O + (e >> 1), 2 * (k + d) + O + (e & 1), np) : SYM_IDLE + lane;
+    }
+    // between a pair's second and the next pair's first position lies a pair of the other parity
+#pragma unroll
+    for (int O = 0; O < 2; ++O) {
+      B.next_pair[O] = B.cell[O][0][2];
+      if (wave == 0 && lane < 32 && k < h) {
+        const int pair = O ? (k + 1) % h : k;
+        B.next_pair[O] = SYM_GP + (1 - O) * SYM_HALF + pair;
+        B.cell[O][0][2] = SYM_GA + (1 - O) * SYM_HALF + pair;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = 2 * (wave - 4) + (lane >> 5) + 8 * u;
+      x0[u] = 2 * k == i && i < np ? 1.0 : 0.0;
+      x1[u] = 2 * k + 1 == i && i < np ? 1.0 : 0.0;
+    }
   }
   __syncthreads();
-  for (int r = tid; r < n; r += SYM_THREADS) lam[r] = G[perm[r] * n + perm[r]];
-  for (int e = tid; e < n * n; e += SYM_THREADS) {
-    const int r = e / n, i = e % n;
-    Vt[e] = V[i * n + perm[r]];
+  int sweeps = 0;
+  for (;;) {
+    bool on = false;
+    for (int t = 0; t < np; t += 2) {
+      if (!vectors) on |= sym_round<0>(L, B, wave == 0 && lane < 32);
+      else if (sweeps + t > 0) sym_vectors<1>(L, k, h, x0, x1);
+      __syncthreads();
+      if (!vectors) on |= sym_round<1>(L, B, wave == 0 && lane < 32);
+      else sym_vectors<0>(L, k, h, x0, x1);
+      __syncthreads();
+    }
+    ++sweeps;
+    const bool any = __any(on);
+    if (tid == 0) L.again = any;
+    __syncthreads();
+    if (!L.again || sweeps == 60) break;
+  }
+  if (vectors) sym_vectors<1>(L, k, h, x0, x1);
+  if (tid < np) {
+    const bool back = sweeps & 1;
+    const double dj = L.dg[0][tid];
+    int r = 0;
+    for (int i = 0; i < np; ++i) {
+      const double di = L.dg[0][i];
+      if ((back ? np - 1 - i : i) < n) r += (di > dj) || (di == dj && i < tid);
+    }
+    const bool real = (back ? np - 1 - tid : tid) < n;
+    L.rank[tid] = real ? r : -1;
+    if (real && r < n) lam[r] = ldexp(dj, ex);
+  }
+  __syncthreads();
+  if (vectors && k < h) {
+    const int r0 = L.rank[2 * k], r1 = L.rank[2 * k + 1];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = 2 * (wave - 4) + (lane >> 5) + 8 * u;
+      if (i < n) {
+        if (r0 >= 0) Vt[(int64_t)r0 * n + i] = x0[u];
+        if (r1 >= 0) Vt[(int64_t)r1 * n + i] = x1[u];
+      }
+    }
   }
 }
 
@@ -477,10 +603,8 @@ extern "C" int cc_fused_truncation_f64(void* stream, int64_t nx, int64_t na, int
     rc = cc_gemm_f64(stream, 1, far, far, m, 1.0, Cs, 0, 1, far, Cs, 0, far, 1, 0.0, G, 0, far, 1);
   }
   if (rc) return rc;
-  if (far == SYM_MAX_N)
-    sym_jacobi_kernel<SYM_MAX_N><<<1, SYM_THREADS, 0, st>>>((int)far, G, lam, Vt);
-  else if (far < SYM_MAX_N)
-    sym_jacobi_kernel<0><<<1, SYM_THREADS, 0, st>>>((int)far, G, lam, Vt);
+  if (far <= SYM_MAX_N)
+    sym_jacobi_kernel<<<1, SYM_THREADS, 0, st>>>((int)far, G, lam, Vt);
   else
     launch_svd(st, 1, far, (int)far, G, Ug, lam, Vt, work);
   CC_LAUNCH_CHECK();

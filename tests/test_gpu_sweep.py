@@ -124,3 +124,39 @@ def test_fused_truncation_basis_matches_oracle(gpu, nx, D, far, k, rank):
     G = U[:, kept].T @ U[:, kept]
     assert np.abs(G - np.eye(G.shape[0])).max() < 1e-6, np.abs(G - np.eye(G.shape[0])).max()
     assert not np.any(U[:, ~kept])
+
+
+# far bond n <= 64: one and two columns (padded to three pairs), odd ones, every pair occupied, and rank deficient
+@pytest.mark.parametrize("n,rank", [(1, 1), (2, 2), (3, 3), (5, 5), (6, 6), (7, 7), (8, 8), (21, 21), (33, 33), (62, 62),
+                                    (63, 63), (64, 64), (24, 9), (64, 40), (5, 0)])
+def test_fused_truncation_diagonalizes_the_gram_matrix(gpu, n, rank):
+    """cc_fused_truncation_f64 on a symmetrized C (D = 2) of condition at most 10 on its range: singular values and
+    the products C^T U against NumPy's.  The Gram matrix is diagonalized to about n 1e-15 of its trace, so values and
+    directions of the range are good to 100 x n x 1e-15 x n; 1e-10 leaves a factor of 2."""
+    import torch
+    from carcassonne_amd import _lib
+    from carcassonne_amd.device import empty, ptr, stream
+    rng = np.random.default_rng(100 * n + rank)
+    nx = n + 2
+    left = np.linalg.qr(rng.standard_normal((nx * 3, max(rank, 1))))[0]
+    right = np.linalg.qr(rng.standard_normal((n, max(rank, 1))))[0]
+    sym = (left * np.linspace(1.0, 0.1, max(rank, 1)) * (rank > 0)) @ right.T        # (x, [00, 11, 01 + 10]) x n
+    C = np.zeros((nx, 2, 2, n))
+    sym = sym.reshape(nx, 3, n)
+    C[:, 0, 0], C[:, 1, 1] = sym[:, 0], sym[:, 1]
+    odd = rng.standard_normal((nx, n))
+    C[:, 0, 1], C[:, 1, 0] = sym[:, 2] / np.sqrt(2) + odd, sym[:, 2] / np.sqrt(2) - odd   # the odd part drops out
+    Cs = 0.5 * (C + C.transpose(0, 2, 1, 3)).reshape(nx * 4, n)
+    U, S = empty((nx * 4, n)), empty((n,))
+    work = empty((_lib.query("cc_fused_truncation_work_size", nx, 2, n),))
+    _lib.call("cc_fused_truncation_f64", stream(), nx, 2, n, n, ptr(torch.from_numpy(C).cuda()), ptr(U), ptr(S), ptr(work))
+    U, S = U.cpu().numpy(), S.cpu().numpy()
+    want = np.linalg.svd(Cs, compute_uv=False)
+    assert np.all(np.diff(S) <= 0)
+    assert np.abs(S[:rank] - want[:rank]).max(initial=0) <= 1e-10
+    Ur = U[:, :rank]
+    assert np.abs(Ur.T @ Ur - np.eye(rank)).max(initial=0) <= 1e-10
+    T = Cs.T @ Ur
+    assert np.abs(T.T @ T - np.diag(want[:rank] ** 2)).max(initial=0) <= 1e-10
+    if rank == 0:
+        assert not U.any()
