@@ -33,40 +33,75 @@ MlpDims mlp_dims(int64_t K0, int64_t H, int64_t NO) {
   return d;
 }
 
-// Y[i][j] = act(sum_k X[i][k] W[j][k] + b[j]): one 16 x 16 MFMA tile per wave, 32 x 32 outputs per workgroup, the
-// operands loaded straight from memory in fragment order, MLP_AHEAD K steps at a time.  X (M x K) and W (N x K) are FP16
-// row-major, K % 16 == 0, N % 32 == 0; rows past M read the last row and are not written.  Writes Y (FP32) and, if Yh,
-// its FP16 copy.  Bound by load latency (a layer's weights are 0.5 MB): at 256 rows, 512 x 512, 12.7 us with 64 x 64
-// tiles through LDS (32 workgroups), 9.3 us here.  The sums run over K in order, so results do not depend on the tiling.
+// element-aligned vectors: the pointers are a caller's
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef _Float16 h8u __attribute__((ext_vector_type(8), aligned(2)));
+
+// Both products of this file: 32 x 32 outputs per workgroup, one 16 x 16 MFMA tile per wave, K in chunks through LDS.
+// Their operands are small (half a megabyte per layer), so what counts is the wait for the first loads and the chain of
+// a tile's matrix instructions: tiles small enough to reach every CU, MLP_AHEAD chunks of loads in flight.  Every sum
+// runs over k in order (v_mfma_f32_16x16x4f32 rounds once per term, like an FMA chain), so results do not depend on
+// the tiling.
+constexpr int MLP_AHEAD = 4;
+
+// Y[i][j] = act(sum_k X[i][k] W[j][k] + b[j]), X (M x K) and W (N x K) FP16 row-major, K % 16 == 0, N % 32 == 0; writes Y
+// (FP32) and, if Yh, its FP16 copy.  At 256 rows, 512 x 512: 6.5 us; with 64 x 64 tiles (32 workgroups) and 16 k per
+// step 12.7 us.  LDS rows of 136: a fragment read touches every bank once.
 // Operand fragments: A[i][k] in lane i + 16(k/4), element k%4; B[k][j] in lane j + 16(k/4), element k%4;
 // D[i][j] in lane j + 16(i/4), register i%4.
-constexpr int MLP_AHEAD = 8;
+constexpr int MLP_FC = 128, MLP_FLD = MLP_FC + 8;
 __global__ void __launch_bounds__(256) mlp_linear_kernel(int64_t M, int64_t N, int64_t K, const _Float16* __restrict__ X,
                                                          const _Float16* __restrict__ W, const float* __restrict__ b,
                                                          int relu, float* __restrict__ Y, _Float16* __restrict__ Yh) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t j = (int64_t)blockIdx.x * 32 + 16 * (wave & 1) + (lane & 15);
-  const h4* wp = reinterpret_cast<const h4*>(W + j * K) + (lane >> 4);
-  const int steps = (int)(K / 16);
-  for (int64_t i0 = (int64_t)blockIdx.y * 32 + 16 * (wave >> 1); i0 < M; i0 += (int64_t)gridDim.y * 32) {
-    const int64_t xi = i0 + (lane & 15) < M ? i0 + (lane & 15) : M - 1;
-    const h4* xp = reinterpret_cast<const h4*>(X + xi * K) + (lane >> 4);
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < steps; s0 += MLP_AHEAD) {
-      h4 xa[MLP_AHEAD], wb[MLP_AHEAD];
-#pragma unroll
-      for (int u = 0; u < MLP_AHEAD; ++u) {
-        const int s = s0 + u < steps ? s0 + u : steps - 1;   // clamped; skipped below
-        xa[u] = xp[4 * s];
-        wb[u] = wp[4 * s];
+  __shared__ __attribute__((aligned(16))) _Float16 Xs[2][32 * MLP_FLD];
+  __shared__ __attribute__((aligned(16))) _Float16 Ws[2][32 * MLP_FLD];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, l = lane & 15, g = lane >> 4;
+  const int row = t >> 3, kt = 16 * (t & 7), at = row * MLP_FLD + kt;
+  const int x_from = (16 * (wave >> 1) + l) * MLP_FLD + 4 * g, w_from = (16 * (wave & 1) + l) * MLP_FLD + 4 * g;
+  const int64_t chunks = (K + MLP_FC - 1) / MLP_FC, j = (int64_t)blockIdx.x * 32 + 16 * (wave & 1) + l;
+  const _Float16* wp = W + ((int64_t)blockIdx.x * 32 + row) * K + kt;
+  for (int64_t i0 = (int64_t)blockIdx.y * 32; i0 < M; i0 += (int64_t)gridDim.y * 32) {
+    const _Float16* xp = X + (i0 + row) * K + kt;
+    const bool in = i0 + row < M;
+    h8u xr[MLP_AHEAD][2], wr[MLP_AHEAD][2];
+    auto load = [&](h8u (&x)[2], h8u (&w)[2], int64_t c) {
+      x[0] = x[1] = w[0] = w[1] = (h8u){0, 0, 0, 0, 0, 0, 0, 0};
+      if (c * MLP_FC + kt < K) {
+        w[0] = *reinterpret_cast<const h8u*>(wp + c * MLP_FC);
+        w[1] = *reinterpret_cast<const h8u*>(wp + c * MLP_FC + 8);
+        if (in) {
+          x[0] = *reinterpret_cast<const h8u*>(xp + c * MLP_FC);
+          x[1] = *reinterpret_cast<const h8u*>(xp + c * MLP_FC + 8);
+        }
       }
+    };
 #pragma unroll
-      for (int u = 0; u < MLP_AHEAD; ++u)
-        if (s0 + u < steps) acc = __builtin_amdgcn_mfma_f32_16x16x16f16(xa[u], wb[u], acc, 0, 0, 0);
+    for (int q = 0; q < MLP_AHEAD; ++q) load(xr[q], wr[q], q);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int64_t c0 = 0; c0 < chunks; c0 += MLP_AHEAD) {
+#pragma unroll
+      for (int q = 0; q < MLP_AHEAD; ++q) {
+        const int64_t c = c0 + q;
+        if (c >= chunks) break;
+        _Float16* xs = Xs[q & 1];
+        _Float16* ws = Ws[q & 1];
+        *reinterpret_cast<h8u*>(xs + at) = xr[q][0];
+        *reinterpret_cast<h8u*>(xs + at + 8) = xr[q][1];
+        *reinterpret_cast<h8u*>(ws + at) = wr[q][0];
+        *reinterpret_cast<h8u*>(ws + at + 8) = wr[q][1];
+        __syncthreads();
+        load(xr[q], wr[q], c + MLP_AHEAD);
+#pragma unroll
+        for (int s = 0; s < MLP_FC / 16; ++s)
+          if (c * MLP_FC + 16 * s < K)
+            acc = __builtin_amdgcn_mfma_f32_16x16x16f16(*reinterpret_cast<const h4*>(xs + x_from + 16 * s),
+                                                        *reinterpret_cast<const h4*>(ws + w_from + 16 * s), acc, 0, 0, 0);
+      }
     }
+    __syncthreads();   // the next rows are written where these were read
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int64_t i = i0 + 4 * (lane >> 4) + r;
+      const int64_t i = i0 + 16 * (wave >> 1) + 4 * g + r;
       if (i < M) {
         float v = acc[r] + b[j];
         if (relu) v = v > 0.f ? v : 0.f;
@@ -78,9 +113,8 @@ __global__ void __launch_bounds__(256) mlp_linear_kernel(int64_t M, int64_t N, i
 }
 
 // One product of the backward pass: C[i][j] = sum_k A(i, k) B[k][j], A FP32, B FP16 row-major with N columns, C
-// row-major.  A is stored M x K (`rows`: the gradient passed on, K % 64 == 0, any M) or K x M (a weight gradient,
-// M % 64 == 0, any K).  `mask`: C is zeroed where mask[i][j] <= 0 (the activation the ReLU left).  `rowsum`: also
-// receives sum_k A(i, k).
+// row-major.  A is stored M x K (`rows`: the gradient passed on, K % 64 == 0, any M; C is zeroed where mask[i][j] <= 0,
+// the activation the ReLU left) or K x M (a weight gradient, M % 64 == 0, any K; `rowsum` also receives sum_k A(i, k)).
 struct MlpJob {
   int64_t M, N, K;
   const float* A;
@@ -95,112 +129,94 @@ struct MlpJobs {
   int64_t tiles0, tiles;   // tiles of the first product, of all
 };
 
-// element-aligned vectors: the pointers are a caller's
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
-typedef _Float16 h2u __attribute__((ext_vector_type(2), aligned(2)));
+// Up to two products in one launch (a layer's weight gradient and the gradient passed on share their operand), FP32 on
+// v_mfma_f32_16x16x4f32; bias sums are a product with ones.  LDS rows: A stored M x K keeps k contiguous (stride 68), A
+// stored K x M and B keep i and j contiguous (stride 48); both reads then touch every bank once.  At 256 samples, widths
+// 272-512-512-512, a whole backward pass takes 29 us (6 to 14 us per launch); as FMA tiles on 64 to 128 workgroups (64 us a
+// product), with the bias sums as one thread per column (36 us) and the masks as kernels of their own, 443 us; 8192 samples, a whole training step: 0.47 ms for 10.8.
+constexpr int MLP_KC = 64, MLP_LDR = MLP_KC + 4, MLP_LDK = 48;
 
-// One wave's part of a tile, K chunks c0 .. c1 of 16 each.  Chunk c is summed in the order k = 16 c + 4 g + u for lane
-// group g at step u, so that a lane's four steps are neighbours in memory; rows and columns alternate between the two
-// 16-wide tiles of a pair (2 (lane % 16) + t), so that one load feeds both.  MLP_CHUNKS chunks are loaded together.
-// Rows past M and columns past N read the last ones and are not written; steps past K count as zero.
-constexpr int MLP_CHUNKS = 4;
-template <bool ROWS>
-__device__ inline void mlp_grad_wave(const MlpJob& jb, int64_t i0, int64_t j0, int64_t c0, int64_t c1, int l, int g,
-                                     f32x4 (&acc)[2][2], float (&rs)[2]) {
-  const int64_t M = jb.M, N = jb.N, K = jb.K;
-  const float* __restrict__ A = jb.A;
-  const _Float16* __restrict__ B = jb.B + (j0 + 2 * l < N ? j0 + 2 * l : N - 2);   // N is even
-  const int64_t r0 = i0 + 2 * l < M ? i0 + 2 * l : M - 1, r1 = i0 + 2 * l + 1 < M ? i0 + 2 * l + 1 : M - 1;
-  for (int64_t c = c0; c < c1; c += MLP_CHUNKS) {
-    float av[MLP_CHUNKS][2][4];
-    h2u bv[MLP_CHUNKS][4];
+// One tile.  SUMS: also the row sums of A (the waves of the first columns, where they are asked for).
+template <bool ROWS, bool SUMS>
+__device__ inline void mlp_grad_tile(const MlpJob& jb, int64_t i0, int64_t j0, float (&As)[2][MLP_KC * MLP_LDK],
+                                     float (&Bs)[2][MLP_KC * MLP_LDK]) {
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, l = lane & 15, g = lane >> 4;
+  const int wi = 16 * (wave >> 1), wj = 16 * (wave & 1);
+  const int a_at = ROWS ? (t >> 3) * MLP_LDR + 8 * (t & 7) : (t >> 2) * MLP_LDK + 8 * (t & 3);
+  const int b_at = (t >> 2) * MLP_LDK + 8 * (t & 3);
+  const int a_from = ROWS ? (wi + l) * MLP_LDR + g : g * MLP_LDK + wi + l;
+  constexpr int a_step = ROWS ? 4 : 4 * MLP_LDK;
+  const int b_from = g * MLP_LDK + wj + l;
+  // this thread's share of a chunk: eight values of A, eight columns of B's row t / 4; out of range: zero
+  const int64_t K = jb.K, kb = t >> 2, N = jb.N, j8 = j0 + 8 * (t & 3), ia = ROWS ? i0 + (t >> 3) : i0 + 8 * (t & 3);
+  const float* pa = ROWS ? jb.A + ia * K + 8 * (t & 7) : jb.A + kb * jb.M + ia;
+  const int64_t a_next = ROWS ? MLP_KC : MLP_KC * jb.M, b_next = MLP_KC * N;
+  const _Float16* pb = jb.B + kb * N + j8;
+  const int64_t ka = ROWS ? (ia < jb.M ? 0 : K) : kb, kj = j8 < N ? kb : K;   // the first k this thread loads
+  f4u a[MLP_AHEAD][2];
+  h8u b[MLP_AHEAD];
+  int64_t k0 = 0;   // of the next chunk to load
+  auto load = [&](f4u (&x)[2], h8u& y) {
+    x[0] = x[1] = (f4u){0.f, 0.f, 0.f, 0.f};
+    y = (h8u){0, 0, 0, 0, 0, 0, 0, 0};
+    if (k0 + ka < K) {
+      x[0] = *reinterpret_cast<const f4u*>(pa);
+      x[1] = *reinterpret_cast<const f4u*>(pa + 4);
+    }
+    if (k0 + kj < K) y = *reinterpret_cast<const h8u*>(pb);
+    pa += a_next;
+    pb += b_next;
+    k0 += MLP_KC;
+  };
 #pragma unroll
-    for (int q = 0; q < MLP_CHUNKS; ++q) {
-      const int64_t k0 = 16 * (c + q < c1 ? c + q : c1 - 1) + 4 * g;
-      if (ROWS) {
-        const f4u x0 = *reinterpret_cast<const f4u*>(A + r0 * K + k0), x1 = *reinterpret_cast<const f4u*>(A + r1 * K + k0);
+  for (int q = 0; q < MLP_AHEAD; ++q) load(a[q], b[q]);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f}, sum = {0.f, 0.f, 0.f, 0.f};
+  const int chunks = (int)((K + MLP_KC - 1) / MLP_KC);
+  for (int c = 0; c < chunks; c += MLP_AHEAD) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) { av[q][0][u] = x0[u]; av[q][1][u] = x1[u]; }
-      }
+    for (int q = 0; q < MLP_AHEAD; ++q) {
+      if (c + q >= chunks) break;
+      float* as = As[q & 1];
+      float* bs = Bs[q & 1];
+      *reinterpret_cast<f32x4*>(as + a_at) = a[q][0];
+      *reinterpret_cast<f32x4*>(as + a_at + 4) = a[q][1];
+      *reinterpret_cast<f32x4*>(bs + b_at) = (f32x4){(float)b[q][0], (float)b[q][1], (float)b[q][2], (float)b[q][3]};
+      *reinterpret_cast<f32x4*>(bs + b_at + 4) = (f32x4){(float)b[q][4], (float)b[q][5], (float)b[q][6], (float)b[q][7]};
+      __syncthreads();
+      load(a[q], b[q]);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t k = ROWS || k0 + u < K ? k0 + u : K - 1;
-        bv[q][u] = *reinterpret_cast<const h2u*>(B + k * N);
-        if (!ROWS) {
-          const f2u x = *reinterpret_cast<const f2u*>(A + k * M + r0);
-          av[q][0][u] = x[0];
-          av[q][1][u] = x[1];
-          if (k0 + u >= K) {
-            av[q][0][u] = av[q][1][u] = 0.f;
-            bv[q][u] = (h2u){0, 0};
-          }
-        }
+      for (int s = 0; s < MLP_KC / 4; ++s) {
+        const float x = as[a_from + s * a_step], y = bs[b_from + s * 4 * MLP_LDK];
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, acc, 0, 0, 0);
+        if (SUMS) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(x, 1.f, sum, 0, 0, 0);
       }
     }
+  }
+  const int64_t j = j0 + wj + l;
 #pragma unroll
-    for (int q = 0; q < MLP_CHUNKS; ++q) {
-      if (c + q >= c1) break;
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          rs[a] += av[q][a][u];
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[q][a][u], (float)bv[q][u][b], acc[a][b], 0, 0, 0);
-        }
+  for (int r = 0; r < 4; ++r) {
+    const int64_t i = i0 + wi + 4 * g + r;
+    if (i < jb.M && j < N) {
+      float v = acc[r];
+      if (ROWS && !(jb.mask[i * N + j] > 0.f)) v = 0.f;
+      jb.C[i * N + j] = v;
     }
+    if (SUMS && wj == 0 && l == 0) jb.rowsum[i] = sum[r];   // M % 64 == 0
   }
 }
 
-// Up to two products in one launch (a layer's weight gradient and the gradient passed on share their operand).  32 x 32
-// outputs per workgroup on v_mfma_f32_16x16x4f32; the four waves take a quarter of K each, straight from memory, and
-// are added in order through LDS, so that a product of 256 x 512 x 512 fills the chip and a wave's K loop is short.
-// FP32 throughout; bound by load latency.  At 256 samples, widths 272-512-512-512, a whole backward pass takes 39 us (each
-// launch 11.7 us); as FMA tiles on 64 to 128 workgroups (64 us a product), with the bias sums as one thread per column
-// (36 us) and the masks as kernels of their own, it took 443 us; at 8192 samples a whole training step 1.01 ms for 10.8.
 __global__ void __launch_bounds__(256) mlp_grad_kernel(const MlpJobs jobs) {
-  __shared__ float part[4][32][33];
-  __shared__ float rows[4][32];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l = lane & 15, g = lane >> 4;
-  for (int64_t t = blockIdx.x; t < jobs.tiles; t += gridDim.x) {
-    const MlpJob& jb = jobs.job[t >= jobs.tiles0];
-    const int64_t tile = t >= jobs.tiles0 ? t - jobs.tiles0 : t, tiles_n = (jb.N + 31) / 32, tn = tile % tiles_n;
-    const int64_t i0 = tile / tiles_n * 32, j0 = tn * 32;
-    const int64_t chunks = (jb.K + 15) / 16, c0 = chunks * wave / 4, c1 = chunks * (wave + 1) / 4;
-    f32x4 acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    float rs[2] = {0.f, 0.f};
-    if (jb.rows) mlp_grad_wave<true>(jb, i0, j0, c0, c1, l, g, acc, rs);
-    else mlp_grad_wave<false>(jb, i0, j0, c0, c1, l, g, acc, rs);
-    __syncthreads();   // the previous tile's sums are read
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) part[wave][2 * (4 * g + r) + a][2 * l + b] = acc[a][b][r];
-      rs[a] += __shfl_xor(rs[a], 16, 64);
-      rs[a] += __shfl_xor(rs[a], 32, 64);
-      if (g == 0) rows[wave][2 * l + a] = rs[a];
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < 32 * 32; e += 256) {
-      const int i = e >> 5, j = e & 31;
-      const int64_t gi = i0 + i, gj = j0 + j;
-      if (gi < jb.M && gj < jb.N) {
-        float v = ((part[0][i][j] + part[1][i][j]) + part[2][i][j]) + part[3][i][j];
-        if (jb.mask && !(jb.mask[gi * jb.N + gj] > 0.f)) v = 0.f;
-        jb.C[gi * jb.N + gj] = v;
-      }
-    }
-    if (jb.rowsum && tn == 0 && threadIdx.x < 32)   // M % 64 == 0 where it is asked for
-      jb.rowsum[i0 + threadIdx.x] =
-          ((rows[0][threadIdx.x] + rows[1][threadIdx.x]) + rows[2][threadIdx.x]) + rows[3][threadIdx.x];
+  __shared__ __attribute__((aligned(16))) float As[2][MLP_KC * MLP_LDK];
+  __shared__ __attribute__((aligned(16))) float Bs[2][MLP_KC * MLP_LDK];
+  static_assert(32 * MLP_LDR <= MLP_KC * MLP_LDK, "both layouts of A fit");
+  for (int64_t u = blockIdx.x; u < jobs.tiles; u += gridDim.x) {
+    const MlpJob jb = u >= jobs.tiles0 ? jobs.job[1] : jobs.job[0];
+    const int64_t tile = u >= jobs.tiles0 ? u - jobs.tiles0 : u, tiles_n = (jb.N + 31) / 32;
+    const int64_t i0 = tile / tiles_n * 32, j0 = tile % tiles_n * 32;
+    if (jb.rows) mlp_grad_tile<true, false>(jb, i0, j0, As, Bs);
+    else if (j0 == 0) mlp_grad_tile<false, true>(jb, i0, j0, As, Bs);
+    else mlp_grad_tile<false, false>(jb, i0, j0, As, Bs);
+    __syncthreads();   // the next tile writes where this one's last chunks were read
   }
 }
 
