@@ -24,6 +24,8 @@ SIGNATURES = {
     "cc_permute": [_vp, _i32, _vp, _vp, _i32, _pi64, _pi64],
     "cc_gemm_f64": [_vp, _i64, _i64, _i64, _i64, _f64, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _f64,
                     _vp, _i64, _i64, _i64],
+    "cc_contract_work_size": [_i32, _i32, _i32, _pi64, _i32, _pi32, _pi64],
+    "cc_contract_f64": [_vp, _i32, _i32, _i32, _pi64, _i32, _pi32, _pvp, _pvp, _pvp, _vp],
     "cc_axpby_f64": [_vp, _i64, _f64, _vp, _f64, _vp],
     "cc_fill_f64": [_vp, _i64, _f64, _vp],
     "cc_set_identity_f64": [_vp, _i64, _vp],

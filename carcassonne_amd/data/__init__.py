@@ -13,6 +13,7 @@ import numpy as np
 import torch
 
 from .. import _lib
+from ..contraction import contract
 from ..device import ONES_LEN, device, empty, ones, ptr, stream
 
 __all__ = ["Data", "HipData", "NDArrayData"]

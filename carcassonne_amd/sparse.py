@@ -211,6 +211,19 @@ def contractSparseTensors(dense_contractors, tensor_1, tensor_2):
     return result
 
 
+def matchSparseTensors(dense_contractors, tensor_1, tensor_2):
+    """The products contractSparseTensors would form: result tag -> [(data_1, data_2, dense fn)], tags and products in
+    its order."""
+    matched = {}
+    for tag_1, data_1 in tensor_1.items():
+        for tag_2, data_2 in tensor_2.items():
+            rule = dense_contractors.get((type(tag_1), type(tag_2)))
+            handler = rule(tag_1, tag_2) if rule is not None else None
+            if handler is not None and handler[0] is not None:
+                matched.setdefault(handler[0], []).append((data_1, data_2, handler[1]))
+    return matched
+
+
 def formSparseContractor(dense_contractors):
     return lambda t1, t2: contractSparseTensors(dense_contractors, t1, t2)
 

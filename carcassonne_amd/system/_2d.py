@@ -13,6 +13,7 @@ import numpy as np
 
 from .base import BaseSystem
 from ..compression import computeProductCompressor
+from ..contraction import contract
 from ..data import HipData
 from ..errors import InvariantViolatedError
 from ..sparse import (Identity, OneSiteOperator, TwoSiteOperator, TwoSiteOperatorCompressed, makeSimpleSparseOperator,
@@ -59,6 +60,22 @@ def _project_corner(t, bond_legs, basis):
         return out.split(sh[0], sh[1], sh[2], k, 1, 1)
     out = basis.contractWith(t.join((0, 1, 2), (3, 4, 5)), (0,), (0,), split_long_sums=True)
     return out.split(k, 1, 1, sh[3], sh[4], sh[5])
+
+
+def _project_corners(corner, bond_legs, basis):
+    """Every channel of a corner through _project_corner, in one launch where they all have one layout."""
+    sh, k = corner[Identity()].shape, basis.shape[1]
+    right = tuple(bond_legs) == (3, 4, 5)
+    bond = sh[3:] if right else sh[:3]
+    out = None
+    if basis.shape[0] == bond[0] * bond[1] * bond[2] and all(t.shape == sh for t in corner.values()):
+        split = basis.split(*bond, k)
+        out = contract("abcdef", "defk" if right else "abck", "abck" if right else "kdef",
+                       [[(t, split)] for t in corner.values()])
+    if out is None:
+        return mapOverSparseData(lambda t: _project_corner(t, bond_legs, basis), corner)
+    shape = tuple(sh[:3]) + (k, 1, 1) if right else (k, 1, 1) + tuple(sh[3:])
+    return {tag: HipData(t.reshape(shape)) for tag, t in zip(corner, out)}
 
 
 class System(BaseSystem):
@@ -420,8 +437,8 @@ class System(BaseSystem):
             join(side, produced)
         self.sides[i] = absorbSparseCenterSOSIntoSideProjected(i, self.sides[i], iso, self.operator_center_tensor,
                                                                left, right, iso.conj())
-        self.corners[i] = mapOverSparseData(lambda t: _project_corner(t, (3, 4, 5), left), corner_l)
-        self.corners[R(i)] = mapOverSparseData(lambda t: _project_corner(t, (0, 1, 2), right), corner_r)
+        self.corners[i] = _project_corners(corner_l, (3, 4, 5), left)
+        self.corners[R(i)] = _project_corners(corner_r, (0, 1, 2), right)
         self.setStateCenter(self.state_center_data.normalizeAxis(i)[0].absorbMatrixAt(i, den))
 
     # -- multipliers (_2d.py:455-488) --------------------------------------------------------

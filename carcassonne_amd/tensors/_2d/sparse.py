@@ -10,9 +10,25 @@ from .dense import *  # noqa: F401,F403
 from .dense import (absorbDenseCenterSOSIntoSide, absorbDenseCenterSOSIntoSideProjected, absorbDenseCenterSSIntoSide,
                     absorbDenseSideIntoCornerFromLeft,
                     absorbDenseSideIntoCornerFromRight, formNormalizationStage1, formNormalizationStage2)
+from ...contraction import contract
+from ...data import HipData
 from ...sparse import (Complete, Identity, OneSiteOperator, TwoSiteOperator, TwoSiteOperatorCompressed,
-                       addStandardCompleteAndIdentityTerms, contractSparseTensors, getInformationFromOperatorCenter)
+                       addStandardCompleteAndIdentityTerms, contractSparseTensors, getInformationFromOperatorCenter,
+                       matchSparseTensors)
+from ...utils import L, O, R
 from ... import stage3
+
+
+def _contract_channels(a, b, out, join, rules, tensor_1, tensor_2):
+    """contractSparseTensors for rules that all stand for one dense contraction (`a`, `b`, `out`: its legs): every result
+    channel in one launch.  None where the channels do not all have one layout."""
+    matched = matchSparseTensors(rules, tensor_1, tensor_2)
+    if not matched or not all(isinstance(x, HipData) for t in (tensor_1, tensor_2) for x in t.values()):
+        return None
+    results = contract(a, b, out, [[(x, y) for x, y, _ in pairs] for pairs in matched.values()])
+    if results is None:
+        return None
+    return {tag: HipData(t.reshape(join(t.shape))) for tag, t in zip(matched, results)}
 
 
 def absorbSparseSideIntoCornerFromLeft(corner, side):
@@ -26,7 +42,9 @@ def absorbSparseSideIntoCornerFromLeft(corner, side):
         (TwoSiteOperator, TwoSiteOperator): lambda c, s: (s.matches(c), f),
         (TwoSiteOperatorCompressed, TwoSiteOperatorCompressed): lambda c, s: (s.matches(c), f),
     })
-    return contractSparseTensors(terms, corner, side)
+    result = _contract_channels("abcdef", "ghiabcjk", "ghidjekf",
+                                lambda n: (n[0], n[1], n[2], n[3] * n[4], n[5] * n[6], n[7]), terms, corner, side)
+    return contractSparseTensors(terms, corner, side) if result is None else result
 
 
 def absorbSparseSideIntoCornerFromRight(corner, side):
@@ -40,7 +58,9 @@ def absorbSparseSideIntoCornerFromRight(corner, side):
         (TwoSiteOperator, TwoSiteOperator): lambda c, s: (c.matches(s), f),
         (TwoSiteOperatorCompressed, TwoSiteOperatorCompressed): lambda c, s: (s.matches(c), f),
     })
-    return contractSparseTensors(terms, corner, side)
+    result = _contract_channels("abcdef", "defghijk", "ajbkcghi",
+                                lambda n: (n[0] * n[1], n[2] * n[3], n[4], n[5], n[6], n[7]), terms, corner, side)
+    return contractSparseTensors(terms, corner, side) if result is None else result
 
 
 def _center_into_side_terms(direction, ss, sos):
@@ -85,7 +105,54 @@ def absorbSparseCenterSOSIntoSideProjected(direction, side, state_center_data, o
     def sos(side_data, op_data):
         return absorbDenseCenterSOSIntoSideProjected(direction, side_data, state_center_data, op_data, left, right,
                                                      state_center_data_conj)
-    return contractSparseTensors(_center_into_side_terms(direction, ss, sos), side, operator_center_data)
+    rules = _center_into_side_terms(direction, ss, sos)
+    result = _project_channels(direction, matchSparseTensors(rules, side, operator_center_data), sos, state_center_data,
+                               state_center_data_conj, left, right)
+    return contractSparseTensors(rules, side, operator_center_data) if result is None else result
+
+
+def _project_channels(direction, matched, sos, state, state_conj, left, right):
+    """The result channels `matched` (matchSparseTensors) of the projected absorption, four launches for all of them: a
+    side channel meets the left basis and the center once, whatever number of operators it meets after that, and the
+    products that add to one channel meet the right basis once.  The operators act on the conjugate center, O[s', s]
+    from its s' side.  None where the channels do not all have one layout."""
+    pairs = [p for products in matched.values() for p in products]
+    if not pairs or not all(isinstance(t, HipData) for p in pairs for t in p[:2] if t is not None):
+        return None
+    sh = pairs[0][0].shape
+    if len(sh) != 8 or sh[1] * sh[2] * sh[4] * sh[5] != 1 or any(p[0].shape != sh for p in pairs):
+        return None
+    x, y, i = sh[0], sh[3], direction
+    legs = [None] * 5
+    conj = [None] * 5
+    for at, ket, bra in ((i, "i", "j"), (L(i), "a", "b"), (R(i), "c", "e"), (O(i), "o", "p"), (4, "s", "s")):
+        legs[at], conj[at] = ket, bra
+    legs, conj = "".join(legs), "".join(conj)
+    D_a, D_c = state.shape[L(i)], state.shape[R(i)]
+    if left.shape[0] != x * D_a * D_a or right.shape[0] != y * D_c * D_c:
+        return None
+    lt, rt = left.split(x, D_a, D_a, left.shape[1]), right.split(y, D_c, D_c, right.shape[1])
+    sides = {id(p[0]): p[0] for p in pairs}
+    operators = {id(p[1]): p[1] for p in pairs if p[2] is sos}
+    grown = contract("xabk", "xyij", "abkyij", [[(lt, t.split(x, y, sh[6], sh[7]))] for t in sides.values()])
+    if grown is None:
+        return None
+    met = contract("abkyij", legs, "bkyjcos", [[(HipData(t), state)] for t in grown])
+    acted = contract("ts", conj.replace("s", "t"), conj, [[(op, state_conj)] for op in operators.values()]) if operators else []
+    if met is None or acted is None:
+        return None
+    met = {key: HipData(t) for key, t in zip(sides, met)}
+    acted = {key: HipData(t) for key, t in zip(operators, acted)}
+    summed = contract("bkyjcos", conj, "kycoep",
+                      [[(met[id(t)], acted[id(op)] if f is sos else state_conj) for t, op, f in products]
+                       for products in matched.values()])
+    if summed is None:
+        return None
+    out = contract("kycoep", "yceq", "kqop", [[(HipData(t), rt)] for t in summed])
+    if out is None:
+        return None
+    return {tag: HipData(t.reshape(t.shape[0], 1, 1, t.shape[1], 1, 1, t.shape[2], t.shape[3]))
+            for tag, t in zip(matched, out)}
 
 
 def formExpectationStage1(corner, side):

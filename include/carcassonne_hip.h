@@ -55,6 +55,16 @@ int cc_gemm_f64(void* stream, int64_t batch, int64_t M, int64_t N, int64_t K, do
                 const double* B, int64_t sBb, int64_t sBk, int64_t sBn, double beta,
                 double* C, int64_t sCb, int64_t sCm, int64_t sCn);
 
+/* FP64 contractions with strided legs, several outputs and several products per output:
+ *   C_o[m, n] = sum over o's terms t and over k of A_t[m, k] B_t[k, n]
+ * `legs` holds {extent, stride, stride} of the rm legs m (strides in A and C), then the rn legs n (in B and C), then the
+ * rk legs k (in A and B), in elements; all A are laid out alike, all B and all C.  `terms`: products of each output (1 to
+ * 32), whose operands follow each other in A and B.  Extents are at least 1, up to 12 legs per group, offsets within 31
+ * bits.  `work`: cc_contract_work_size doubles (null: long sums are not split). */
+int cc_contract_work_size(int rm, int rn, int rk, const int64_t* legs, int n_out, const int* terms, int64_t* out);
+int cc_contract_f64(void* stream, int rm, int rn, int rk, const int64_t* legs, int n_out, const int* terms,
+                    const double* const* A, const double* const* B, double* const* C, double* work);
+
 /* y = alpha * x + beta * y.   NDArrayData.__add__/__iadd__/__mul__  data/__init__.py:93-139 */
 int cc_axpby_f64(void* stream, int64_t n, double alpha, const double* x, double beta, double* y);
 /* y = (alpha_scale * alpha_dev[0]) * x + beta * y with the coefficient read from device memory (solver steps
