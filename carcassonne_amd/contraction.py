@@ -1,5 +1,5 @@
 """Contractions of whole sets of channels in one launch (cc_contract_f64): operands and results keep their legs where
-they lie, the outputs of a call share a launch, and the products that add to one output are one long sum.
+they lie, the outputs of a call share a launch, and the products that add to one output are added in it.
 
 Shapes, strides and the resulting leg lists are memoised; nothing is kept about the tensors themselves.
 """
@@ -74,10 +74,11 @@ def _pointers(tensors):
     return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
 
 
-def contract(a, b, out, outputs):
+def contract(a, b, out, outputs, split_long_sums=False):
     """One device tensor per entry of `outputs`, each the sum of A B over its pairs (A, B): `a`, `b` and `out` name the
     legs of the first operands, the second ones and the results (a leg in both operands is summed, every other is in
-    `out`).  None where the kernel does not take the contraction."""
+    `out`).  split_long_sums: long sums with small results are summed in slices (their rounding then differs from one
+    sum's, so only callers that ask for it get it).  None where the kernel does not take the contraction."""
     if any(len(pairs) > MAX_TERMS for pairs in outputs):
         return None
     A = [_layout(x) for pairs in outputs for x, _ in pairs]
@@ -89,7 +90,7 @@ def contract(a, b, out, outputs):
     if not plan.ok:
         return None
     results = [empty(plan.shape) for _ in outputs]
-    work = empty((plan.work,)) if plan.work else None
+    work = empty((plan.work,)) if plan.work and split_long_sums else None
     _lib.call("cc_contract_f64", stream(), *plan.counts, plan.legs, len(outputs), plan.terms,
               _pointers([t for t, _ in A]), _pointers([t for t, _ in B]), _pointers(results),
               ptr(work) if work is not None else None)

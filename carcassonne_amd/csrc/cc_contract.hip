@@ -140,11 +140,17 @@ __global__ void __launch_bounds__(256) contract_kernel(const ContractArgs g) {
       ++term;
     }
   };
-  f64x4 acc[TM][TN];
+  f64x4 acc[TM][TN], sum[TM][TN];   // of the term at hand, of the finished ones
+  auto clear = [&](f64x4 (&v)[TM][TN]) {
 #pragma unroll
-  for (int a = 0; a < TM; ++a)
+    for (int a = 0; a < TM; ++a)
 #pragma unroll
-    for (int b = 0; b < TN; ++b) acc[a][b] = (f64x4){0.0, 0.0, 0.0, 0.0};
+      for (int b = 0; b < TN; ++b) v[a][b] = (f64x4){0.0, 0.0, 0.0, 0.0};
+  };
+  clear(acc);
+  clear(sum);
+  int left = per_term - s0 % per_term;   // steps of the term at hand
+  bool single = true;
   if (s0 < s1) load();
   for (int s = s0; s < s1; ++s) {
     double* as = As[(s - s0) & 1];
@@ -177,6 +183,21 @@ __global__ void __launch_bounds__(256) contract_kernel(const ContractArgs g) {
 #pragma unroll
         for (int b = 0; b < TN; ++b) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[a], bf[b], acc[a][b], 0, 0, 0);
     }
+    if (--left == 0 && s + 1 < s1) {   // the next term
+#pragma unroll
+      for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) sum[a][b] = single ? acc[a][b] : sum[a][b] + acc[a][b];
+      clear(acc);
+      left = per_term;
+      single = false;
+    }
+  }
+  if (!single) {
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+      for (int b = 0; b < TN; ++b) acc[a][b] = sum[a][b] + acc[a][b];
   }
 
   double* C = g.splits > 1 ? g.work + (int64_t)blockIdx.z * g.M * g.N : g.C[o];

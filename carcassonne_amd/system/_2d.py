@@ -71,7 +71,7 @@ def _project_corners(corner, bond_legs, basis):
     if basis.shape[0] == bond[0] * bond[1] * bond[2] and all(t.shape == sh for t in corner.values()):
         split = basis.split(*bond, k)
         out = contract("abcdef", "defk" if right else "abck", "abck" if right else "kdef",
-                       [[(t, split)] for t in corner.values()])
+                       [[(t, split)] for t in corner.values()], split_long_sums=True)
     if out is None:
         return mapOverSparseData(lambda t: _project_corner(t, bond_legs, basis), corner)
     shape = tuple(sh[:3]) + (k, 1, 1) if right else (k, 1, 1) + tuple(sh[3:])

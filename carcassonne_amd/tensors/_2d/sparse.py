@@ -5,13 +5,14 @@ carcassonne_amd.sparse.contractSparseTensors.  Stage 3 gathers every compatible
 matvec of the whole expectation multiplier is a single HIP call.
 """
 import itertools
+import math
 
 from .dense import *  # noqa: F401,F403
 from .dense import (absorbDenseCenterSOSIntoSide, absorbDenseCenterSOSIntoSideProjected, absorbDenseCenterSSIntoSide,
                     absorbDenseSideIntoCornerFromLeft,
                     absorbDenseSideIntoCornerFromRight, formNormalizationStage1, formNormalizationStage2)
 from ...contraction import contract
-from ...data import HipData
+from ...data import HipData, PermutedView
 from ...sparse import (Complete, Identity, OneSiteOperator, TwoSiteOperator, TwoSiteOperatorCompressed,
                        addStandardCompleteAndIdentityTerms, contractSparseTensors, getInformationFromOperatorCenter,
                        matchSparseTensors)
@@ -19,16 +20,28 @@ from ...utils import L, O, R
 from ... import stage3
 
 
-def _contract_channels(a, b, out, join, rules, tensor_1, tensor_2):
-    """contractSparseTensors for rules that all stand for one dense contraction (`a`, `b`, `out`: its legs): every result
-    channel in one launch.  None where the channels do not all have one layout."""
+def _contract_channels(a, b, out, finish, rules, tensor_1, tensor_2):
+    """contractSparseTensors for rules that all stand for one dense contraction (`a`, `b`, `out`: its legs, `finish`: what
+    makes a channel of its result): every result channel in one launch; the pairwise loop where the channels do not
+    all have one layout."""
     matched = matchSparseTensors(rules, tensor_1, tensor_2)
-    if not matched or not all(isinstance(x, HipData) for t in (tensor_1, tensor_2) for x in t.values()):
-        return None
-    results = contract(a, b, out, [[(x, y) for x, y, _ in pairs] for pairs in matched.values()])
+    results = None
+    if matched and all(isinstance(x, HipData) for t in (tensor_1, tensor_2) for x in t.values()):
+        results = contract(a, b, out, [[(x, y) for x, y, _ in pairs] for pairs in matched.values()])
     if results is None:
-        return None
-    return {tag: HipData(t.reshape(join(t.shape))) for tag, t in zip(matched, results)}
+        return contractSparseTensors(rules, tensor_1, tensor_2)
+    return {tag: finish(t) for tag, t in zip(matched, results)}
+
+
+def _joined(*groups):
+    """A result with its legs joined in groups of the given sizes."""
+    def finish(t):
+        shape, at = [], 0
+        for n in groups:
+            shape.append(math.prod(t.shape[at:at + n]))
+            at += n
+        return HipData(t.reshape(shape))
+    return finish
 
 
 def absorbSparseSideIntoCornerFromLeft(corner, side):
@@ -42,9 +55,7 @@ def absorbSparseSideIntoCornerFromLeft(corner, side):
         (TwoSiteOperator, TwoSiteOperator): lambda c, s: (s.matches(c), f),
         (TwoSiteOperatorCompressed, TwoSiteOperatorCompressed): lambda c, s: (s.matches(c), f),
     })
-    result = _contract_channels("abcdef", "ghiabcjk", "ghidjekf",
-                                lambda n: (n[0], n[1], n[2], n[3] * n[4], n[5] * n[6], n[7]), terms, corner, side)
-    return contractSparseTensors(terms, corner, side) if result is None else result
+    return _contract_channels("abcdef", "ghiabcjk", "ghidjekf", _joined(1, 1, 1, 2, 2, 1), terms, corner, side)
 
 
 def absorbSparseSideIntoCornerFromRight(corner, side):
@@ -58,9 +69,7 @@ def absorbSparseSideIntoCornerFromRight(corner, side):
         (TwoSiteOperator, TwoSiteOperator): lambda c, s: (c.matches(s), f),
         (TwoSiteOperatorCompressed, TwoSiteOperatorCompressed): lambda c, s: (s.matches(c), f),
     })
-    result = _contract_channels("abcdef", "defghijk", "ajbkcghi",
-                                lambda n: (n[0] * n[1], n[2] * n[3], n[4], n[5], n[6], n[7]), terms, corner, side)
-    return contractSparseTensors(terms, corner, side) if result is None else result
+    return _contract_channels("abcdef", "defghijk", "ajbkcghi", _joined(2, 2, 1, 1, 1, 1), terms, corner, side)
 
 
 def _center_into_side_terms(direction, ss, sos):
@@ -148,7 +157,7 @@ def _project_channels(direction, matched, sos, state, state_conj, left, right):
                        for products in matched.values()])
     if summed is None:
         return None
-    out = contract("kycoep", "yceq", "kqop", [[(HipData(t), rt)] for t in summed])
+    out = contract("kycoep", "yceq", "kqop", [[(HipData(t), rt)] for t in summed], split_long_sums=True)
     if out is None:
         return None
     return {tag: HipData(t.reshape(t.shape[0], 1, 1, t.shape[1], 1, 1, t.shape[2], t.shape[3]))
@@ -168,7 +177,7 @@ def formExpectationStage1(corner, side):
         (Identity, TwoSiteOperatorCompressed): lambda c, s: (s.matchesCornerIdentityOnLeftForStage1(), f),
         (TwoSiteOperatorCompressed, TwoSiteOperatorCompressed): lambda c, s: (c.matches(s), f),
     })
-    return contractSparseTensors(terms, corner, side)
+    return _contract_channels("abcdef", "defghijk", "abcghijk", _joined(3, 3, 1, 1), terms, corner, side)
 
 
 def formExpectationStage2(right, left):
@@ -184,7 +193,8 @@ def formExpectationStage2(right, left):
         (Identity, TwoSiteOperatorCompressed): lambda r, l: (l.matchesStage1IdentityOnRight(), f),
         (TwoSiteOperatorCompressed, TwoSiteOperatorCompressed): lambda r, l: (l.matches(r), f),
     })
-    return contractSparseTensors(terms, right, left)
+    # in the product's own leg order; the packers read the slabs through strides
+    return _contract_channels("abcd", "eafg", "bcdefg", lambda t: PermutedView(t, [3, 0, 1, 4, 2, 5]), terms, right, left)
 
 
 STAGE3_RULES = {

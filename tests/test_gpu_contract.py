@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 EPS = 2.0 ** -53
 
 
-def _check(a, b, out, dims, terms, seed, permute=False):
+def _check(a, b, out, dims, terms, seed, permute=False, split=True):
     import torch
     from carcassonne_amd.contraction import contract
     from carcassonne_amd.data import HipData
@@ -24,7 +24,7 @@ def _check(a, b, out, dims, terms, seed, permute=False):
         return HipData.fromArray(np.ascontiguousarray(x.transpose())).permuted_lazily(list(back))
     pairs = [(up(x), up(y)) for x, y in zip(A, B)]
     at = np.cumsum([0] + list(terms))
-    got = contract(a, b, out, [pairs[at[o]:at[o + 1]] for o in range(len(terms))])
+    got = contract(a, b, out, [pairs[at[o]:at[o + 1]] for o in range(len(terms))], split_long_sums=split)
     assert got is not None
     K = int(np.prod([dims[x] for x in a if x in b], dtype=np.int64))
     spec = "{},{}->{}".format(a, b, out)
@@ -54,7 +54,8 @@ def _check(a, b, out, dims, terms, seed, permute=False):
      ((4, 4), (5, 5), (6, 6), (7, 8), (9, 8), (9, 9))])                         # 16 to 80 columns and one past
 @pytest.mark.parametrize("permute", [False, True])
 def test_contract_matches_numpy(gpu, a, b, out, dims, terms, permute):
-    _check(a, b, out, dims, terms, len(a) + 10 * len(b) + sum(dims.values()), permute)
+    for split in (False, True):
+        _check(a, b, out, dims, terms, len(a) + 10 * len(b) + sum(dims.values()), permute, split)
 
 
 @pytest.mark.parametrize("outputs", [15, 16, 17, 40])
