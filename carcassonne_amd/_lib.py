@@ -71,6 +71,7 @@ SIGNATURES = {
     "cc_trtri_lower_f64": [_vp, _i64, _vp, _vp, _vp],
     "cc_cholesky_inverse_f64": [_vp, _i64, _vp, _vp, _vp, _vp],
     "cc_transpose_f64": [_vp, _i64, _vp, _vp],
+    "cc_relax_krylov_f64": [_vp, _i64, _i32, _vp, _vp, _vp, _i32, _pf64, _i32, _vp, _vp, _vp, _vp],
     "cc_skinny_f64": [_vp, _i64, _i32, _vp, _i32, _vp, _vp],
     "cc_lanczos_work_size": [_i64, _i32, _pi64],
     "cc_lanczos_f64": [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _f64, _f64, _i32, _i32, _vp, _vp, _pf64],

@@ -226,9 +226,10 @@ __global__ void __launch_bounds__(256) contract_reduce_kernel(const ContractArgs
   g.C[blockIdx.y][(int64_t)rc + cc] = v;
 }
 
-// Legs in the order given by stride `by` (largest first), unit legs dropped, neighbours merged where both tensors allow.
+// Legs in the order given by stride `by` (largest first; by < 0: as they are), unit legs dropped, neighbours merged where
+// both tensors allow.
 int arrange(Legs& v, int by, LegGroup& g, int64_t& total) {
-  for (int i = 1; i < v.count; ++i)
+  for (int i = 1; i < v.count && by >= 0; ++i)
     for (int j = i; j > 0 && v.l[j - 1].s[by] < v.l[j].s[by]; --j) std::swap(v.l[j - 1], v.l[j]);
   int n = 0;
   total = 1;
@@ -294,11 +295,15 @@ int plan(int rm, int rn, int rk, const int64_t* legs, int n_out, const int* term
     std::swap(v[0], v[1]);
     for (int i = 0; i < rk; ++i) std::swap(v[2].l[i].s[0], v[2].l[i].s[1]);
   }
-  sh.a_k_fast = least(v[2], 0) < least(v[0], 0);
+  // sums run over k in the caller's order of its legs
+  int64_t fastest = INT64_MAX;
+  for (int i = 0; i < rk; ++i)
+    if (v[2].l[i].n > 1) fastest = v[2].l[i].s[0];
+  sh.a_k_fast = fastest < least(v[0], 0);
   int64_t M, N, K;
   int rc = arrange(v[0], 0, g.m, M);
   if (!rc) rc = arrange(v[1], 1, g.n, N);
-  if (!rc) rc = arrange(v[2], sh.a_k_fast ? 0 : 1, g.k, K);
+  if (!rc) rc = arrange(v[2], -1, g.k, K);
   if (rc || reach(g.m, 0) + reach(g.k, 0) > 2147483647LL || reach(g.n, 0) + reach(g.k, 1) > 2147483647LL ||
       reach(g.m, 1) + reach(g.n, 1) > 2147483647LL || K > 2147483647LL - 64) {
     cc_set_last_error("contract: legs beyond 32-bit offsets");

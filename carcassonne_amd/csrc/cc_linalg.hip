@@ -472,3 +472,110 @@ extern "C" int cc_skinny_f64(void* stream, int64_t n, int tri, const double* M, 
   CC_LAUNCH_CHECK();
   return CC_OK;
 }
+
+// ---- relaxOver's restart (one native call; the scalars stay on the device) ---------------------------------------
+namespace {
+constexpr int RELAX_MAX_K = 16;
+struct RelaxCoef {
+  double c[RELAX_MAX_K];
+};
+// x . y on the whole workgroup, summed as cc_dot_f64 sums it
+__device__ double block_dot(int64_t n, const double* x, const double* y, double* red) {
+  double acc = 0.0;
+  for (int64_t i = threadIdx.x; i < n; i += 1024) acc += x[i] * y[i];
+  __syncthreads();
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  for (int s = 512; s > 0; s >>= 1) {
+    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+    __syncthreads();
+  }
+  return red[0];
+}
+// v = sum_j c[j] basis[j], scaled to unit norm, into basis[0]
+__global__ void __launch_bounds__(1024) relax_combine_kernel(int64_t n, int count, const RelaxCoef coef, double* basis,
+                                                             double* tmp, double* out) {
+  __shared__ double red[1024];
+  for (int64_t i = threadIdx.x; i < n; i += 1024) {
+    double v = 0.0;
+    for (int j = 0; j < count; ++j) v += coef.c[j] * basis[j * n + i];
+    tmp[i] = v;
+  }
+  __syncthreads();
+  const double s = 1.0 / sqrt(block_dot(n, tmp, tmp, red));
+  for (int64_t i = threadIdx.x; i < n; i += 1024) basis[i] = s * tmp[i];
+  if (threadIdx.x == 0) out[0] = 0.0;   // vectors of the basis, once it has ended
+}
+// basis[m] = mbasis[m - 1] orthogonalized against basis[0..m-1] (the coefficients first, then the subtractions), scaled;
+// zero, and out[0] = m, where nothing is left of it
+__global__ void __launch_bounds__(1024) relax_extend_kernel(int64_t n, int m, double* basis, const double* mbasis,
+                                                            double* out) {
+  __shared__ double red[1024];
+  double* w = basis + m * n;
+  const double* y = mbasis + (m - 1) * n;
+  double c[RELAX_MAX_K];
+#pragma unroll
+  for (int j = 0; j < RELAX_MAX_K; ++j)
+    if (j < m) c[j] = block_dot(n, basis + j * n, y, red);
+  for (int64_t i = threadIdx.x; i < n; i += 1024) {
+    double v = y[i];
+#pragma unroll
+    for (int j = 0; j < RELAX_MAX_K; ++j)
+      if (j < m) v += -c[j] * basis[j * n + i];
+    w[i] = v;
+  }
+  __syncthreads();
+  const double nn = block_dot(n, w, w, red), norm = sqrt(nn > 0.0 ? nn : 0.0);
+  const bool ended = norm <= 1e-14 || out[0] > 0.0;   // a vector after the basis has ended stays zero
+  const double s = 1.0 / norm;
+  __syncthreads();
+  for (int64_t i = threadIdx.x; i < n; i += 1024) w[i] = ended ? 0.0 : s * w[i];
+  if (threadIdx.x == 0 && ended && !(out[0] > 0.0)) out[0] = m;
+}
+// out[1 + i k + j] = basis[i] . mbasis[j]; the number of vectors where the basis did not end before
+__global__ void __launch_bounds__(1024) relax_products_kernel(int64_t n, int k, const double* basis, const double* mbasis,
+                                                              double* out) {
+  __shared__ double red[1024];
+  const int i = blockIdx.x / k, j = blockIdx.x % k;
+  const double v = block_dot(n, basis + i * n, mbasis + j * n, red);
+  if (threadIdx.x == 0) {
+    out[1 + blockIdx.x] = v;
+    if (blockIdx.x == 0 && !(out[0] > 0.0)) out[0] = k;
+  }
+}
+}  // namespace
+
+// A restart is a chain of small matrix-vector products and reductions; what it costs is launches and, with a host that
+// reads every scalar, a synchronization per scalar: at n = 32, k = 3 (9 products, 21 dots) 0.50 ms from Python and
+// 0.06 ms here.
+extern "C" int cc_relax_krylov_f64(void* stream, int64_t n, int k, const double* H, const double* W, const double* Wt,
+                                   int count, const double* coef, int last, double* basis, double* mbasis, double* tmp,
+                                   double* out) {
+  if (n < 1 || k < 1 || k > RELAX_MAX_K || count < 1 || count > k) { cc_set_last_error("relax: bad sizes"); return CC_ERR_ARG; }
+  hipStream_t st = cc_stream(stream);
+  RelaxCoef c = {};
+  for (int j = 0; j < count; ++j) c.c[j] = coef[j];
+  relax_combine_kernel<<<1, 1024, 0, st>>>(n, count, c, basis, tmp, out);
+  CC_LAUNCH_CHECK();
+  for (int i = 0; i < (last ? 1 : k); ++i) {
+    const double* x = basis + i * n;
+    double* y = mbasis + i * n;
+    int rc;
+    if (!W) {
+      rc = cc_skinny_f64(stream, n, 0, H, 1, x, y);
+    } else {
+      rc = cc_skinny_f64(stream, n, 0, H, 1, x, tmp);
+      if (!rc && Wt) rc = cc_skinny_f64(stream, n, 1, W, 1, tmp, tmp + n);
+      if (!rc) rc = Wt ? cc_skinny_f64(stream, n, 2, Wt, 1, tmp + n, y) : cc_skinny_f64(stream, n, 0, W, 1, tmp, y);
+    }
+    if (rc) return rc;
+    if (!last && i + 1 < k) {
+      relax_extend_kernel<<<1, 1024, 0, st>>>(n, i + 1, basis, mbasis, out);
+      CC_LAUNCH_CHECK();
+    }
+  }
+  const int rows = last ? 1 : k;
+  relax_products_kernel<<<(unsigned)(rows * rows), 1024, 0, st>>>(n, rows, basis, mbasis, out);
+  CC_LAUNCH_CHECK();
+  return CC_OK;
+}

@@ -197,14 +197,13 @@ class _DenseInverse:
     def __init__(self, matrix):
         n = matrix.shape[0]
         base = matrix.tensor()
-        trace = float(torch.diagonal(base).sum().item())
         work = empty((_lib.query("cc_linalg_work_size", n),))
         info = torch.zeros(1, dtype=torch.int32, device=base.device)
         self.W, self.Ninv, self.n = empty((n, n)), None, n
         for shift in (0.0, 1e-14, 1e-12, 1e-10):
             L = base.clone()
             if shift:
-                L.view(-1)[:: n + 1] += shift * abs(trace) / n
+                L.view(-1)[:: n + 1] += shift * abs(float(torch.diagonal(base).sum().item())) / n
             _lib.call("cc_cholesky_inverse_f64", stream(), n, ptr(L), ptr(self.W), ptr(info), ptr(work))
             if int(info.item()) == 0:
                 break
@@ -276,27 +275,93 @@ def dense_lowest_eigenpair(H, N):
     return x, value
 
 
+class _FormedKrylov:
+    """relaxOver's restarts for a formed expectation matrix, one native call each (cc_relax_krylov_f64): only the k x k
+    projected matrix comes to the host."""
+    MAX_K = 16
+
+    def __init__(self, v, k, Hm, inv):
+        self.n, self.k, self.Hm = v.numel(), k, Hm
+        self.W, self.Wt = (None, None) if inv is None else (inv.Ninv, None) if inv.Ninv is not None else (inv.W, inv.Wt)
+        self.basis, self.mbasis = empty((k, self.n)), empty((k, self.n))
+        self.basis[0].copy_(v)
+        self.tmp, self.out = empty((2 * self.n,)), empty((1 + k * k,))
+
+    def _restart(self, coefficients, last):
+        opt = lambda t: ptr(t) if t is not None else None
+        _lib.call("cc_relax_krylov_f64", stream(), self.n, self.k, ptr(self.Hm), opt(self.W), opt(self.Wt), len(coefficients),
+                  _lib.f64_array(coefficients), int(last), ptr(self.basis), ptr(self.mbasis), ptr(self.tmp), ptr(self.out))
+        return self.out.cpu().numpy()
+
+    def restart(self, coefficients):
+        """The projected matrix of the Krylov basis that starts from the combination of the last one."""
+        r = self._restart(coefficients, False)
+        m = int(r[0])
+        return r[1:].reshape(self.k, self.k)[:m, :m]
+
+    def finish(self, coefficients):
+        """(the normalized combination, its value)"""
+        r = self._restart(coefficients, True)
+        return self.basis[0].clone(), float(r[1])
+
+
+class _Krylov:
+    """relaxOver's restarts for any multiplier (vectors on the device, scalars on the host)."""
+
+    def __init__(self, v, k, multiply):
+        self.k, self.multiply, self.basis = k, multiply, [v]
+
+    def _combine(self, coefficients):
+        combo = torch.zeros_like(self.basis[0])
+        for cf, b in zip(coefficients, self.basis):
+            _axpby(float(cf), b, 1.0, combo)
+        cn = np.sqrt(_dot(combo, combo))
+        _axpby(0.0, combo, 1.0 / cn, combo)
+        return combo
+
+    def restart(self, coefficients):
+        basis, mbasis = [self._combine(coefficients)], []
+        for i in range(self.k):
+            mbasis.append(self.multiply(basis[i]))
+            if i < self.k - 1:
+                w = mbasis[i].clone()
+                coeffs = [_dot(b, mbasis[i]) for b in basis]     # classical Gram-Schmidt, one pass
+                for cf, b in zip(coeffs, basis):
+                    _axpby(-cf, b, 1.0, w)
+                nrm = np.sqrt(max(_dot(w, w), 0.0))
+                if nrm <= 1e-14:
+                    break
+                _axpby(0.0, w, 1.0 / nrm, w)
+                basis.append(w)
+        self.basis = basis
+        return np.array([[_dot(b, mb) for mb in mbasis] for b in basis])
+
+    def finish(self, coefficients):
+        combo = self._combine(coefficients)
+        return combo, _dot(combo, self.multiply(combo))
+
+
 def relax_over(initial, expectation_multiplier, normalization_multiplier=None, maximum_number_of_multiplications=None,
                tolerance=1e-7, dimension_of_krylov_space=None, stats=None):
     """relaxOver (utils.py:805-878) with the vectors in device memory."""
     shape = initial.shape
-    v = initial._t.reshape(-1).clone()
-    nv = np.sqrt(_dot(v, v))
-    _axpby(0.0, v, 1.0 / nv, v)
+    v = initial._t.reshape(-1)
     N = v.numel()
     k = 3 if dimension_of_krylov_space is None else dimension_of_krylov_space
 
-    if normalization_multiplier is None:
-        inv_N = lambda x: x
-    else:
+    inv_N = None
+    if normalization_multiplier is not None:
         inv_N = _DenseInverse(normalization_multiplier.formMatrix())
     if expectation_multiplier.isCheaperToFormMatrix(2 * k):
         Hm = expectation_multiplier.formMatrix().tensor()
-
-        def mul_H(x):
-            y = torch.empty_like(x)
-            _lib.call("cc_skinny_f64", stream(), N, 0, ptr(Hm), 1, ptr(x), ptr(y))
-            return y
+        if 1 <= k <= _FormedKrylov.MAX_K and tuple(Hm.shape) == (N, N) and (inv_N is None or inv_N.n == N):
+            krylov = _FormedKrylov(v, k, Hm.contiguous(), inv_N)
+        else:
+            def mul_H(x):
+                y = torch.empty_like(x)
+                _lib.call("cc_skinny_f64", stream(), N, 0, ptr(Hm), 1, ptr(x), ptr(y))
+                return y
+            krylov = None
     else:
         op = getattr(expectation_multiplier, "operator", None)
 
@@ -306,46 +371,28 @@ def relax_over(initial, expectation_multiplier, normalization_multiplier=None, m
                 op.apply_flat(x, y)
                 return y
             return expectation_multiplier(HipData(x.reshape(shape))).tensor().reshape(-1)
-    multiply = lambda x: inv_N(mul_H(x))
-    initial_value = _dot(v, multiply(v))
-    mults, last, complete, restarts = 0, None, (k == N), 0
+        krylov = None
+    if krylov is None:
+        krylov = _Krylov(v, k, mul_H if inv_N is None else lambda x: inv_N(mul_H(x)))
+    mults, last, complete, restarts, vec, initial_value = 0, None, (k == N), 0, [1.0], None
     while True:
-        basis = [v]
-        mbasis = []
-        for i in range(k):
-            mbasis.append(multiply(basis[i]))
-            if i < k - 1:
-                w = mbasis[i].clone()
-                coeffs = [_dot(b, mbasis[i]) for b in basis]     # classical Gram-Schmidt, one pass
-                for cf, b in zip(coeffs, basis):
-                    _axpby(-cf, b, 1.0, w)
-                nrm = np.sqrt(max(_dot(w, w), 0.0))
-                if nrm <= 1e-14:
-                    complete = True
-                    break
-                _axpby(0.0, w, 1.0 / nrm, w)
-                basis.append(w)
-        basis = basis[:len(mbasis)]
+        M = krylov.restart(vec)
+        if initial_value is None:
+            initial_value = float(M[0, 0])
+        complete = complete or len(M) < k
         mults += k
         restarts += 1
-        M = np.array([[_dot(b, mb) for mb in mbasis] for b in basis])
         evals, evecs = eig(M)
         j = int(np.argmin(evals.real))
-        lam, vec = evals[j], evecs[:, j]
+        lam, vec = evals[j], evecs[:, j].real
         stop = complete or (last is not None and abs(last - lam) <= tolerance) or \
             (maximum_number_of_multiplications is not None and mults >= maximum_number_of_multiplications)
-        combo = torch.zeros_like(v)
-        for cf, b in zip(vec.real, basis):
-            _axpby(float(cf), b, 1.0, combo)
-        cn = np.sqrt(_dot(combo, combo))
-        _axpby(0.0, combo, 1.0 / cn, combo)
         if stop:
-            final_value = _dot(combo, multiply(combo))
+            combo, final_value = krylov.finish(vec)
             if stats is not None:
                 stats.update(restarts=restarts, mults=mults + 2, value=final_value)
             denom = abs(final_value) + abs(initial_value)
             if denom > 0 and (final_value - initial_value) / denom > 1 + 1e-7:
                 raise RelaxFailed(initial_value, final_value)
             return HipData(combo.reshape(shape))
-        v = combo
         last = lam

@@ -18,6 +18,7 @@ import numpy as np
 import torch
 
 from . import _lib
+from .contraction import contract
 from .data import HipData
 from .device import empty, ptr, stream
 
@@ -418,11 +419,18 @@ class Stage3Operator:
         return HipData(out)
 
     def form_matrix(self):
+        """The dense matrix: the environment matrices of all terms in one contraction, their products with the site
+        operators, added term by term, in another."""
         from .tensors._2d.dense import _form_matrix
         eye = HipData.newIdentity(self.d)
+        ops = [op if op is not None else eye for (_, _, op) in self.terms]
+        G = contract("xyabcd", "yxefgh", "cdghabef", [[(a, b)] for (a, b, _) in self.terms])
+        m = G and contract("cdghabef", "st", "cdghsabeft", [[(HipData(g), op) for g, op in zip(G, ops)]])
+        if m:
+            return HipData(m[0].reshape(self.n, self.n))
         m = None
-        for (a, b, op) in self.terms:
-            t = _form_matrix(a, b, op if op is not None else eye)
+        for (a, b, _), op in zip(self.terms, ops):
+            t = _form_matrix(a, b, op)
             m = t if m is None else m + t
         return m
 

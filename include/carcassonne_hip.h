@@ -59,7 +59,7 @@ int cc_gemm_f64(void* stream, int64_t batch, int64_t M, int64_t N, int64_t K, do
  *   C_o[m, n] = sum over o's terms t and over k of A_t[m, k] B_t[k, n]
  * `legs` holds {extent, stride, stride} of the rm legs m (strides in A and C), then the rn legs n (in B and C), then the
  * rk legs k (in A and B), in elements; all A are laid out alike, all B and all C.  `terms`: products of each output (1 to
- * 32), whose operands follow each other in A and B.  Extents are at least 1, up to 12 legs per group, offsets within 31
+ * 32), whose operands follow each other in A and B.  Sums run over k in the order of its legs.  Extents are at least 1, up to 12 legs per group, offsets within 31
  * bits.  `work`: cc_contract_work_size doubles (null: long sums are not split). */
 int cc_contract_work_size(int rm, int rn, int rk, const int64_t* legs, int n_out, const int* terms, int64_t* out);
 int cc_contract_f64(void* stream, int rm, int rn, int rk, const int64_t* legs, int n_out, const int* terms,
@@ -281,6 +281,15 @@ int cc_cholesky_inverse_f64(void* stream, int64_t n, double* A, double* X, int* 
 int cc_transpose_f64(void* stream, int64_t n, const double* A, double* B);
 /* Y (n x nrhs) = M (n x n) X restricted to tri = 0 full, 1 lower, 2 upper; nrhs <= 4. */
 int cc_skinny_f64(void* stream, int64_t n, int tri, const double* M, int nrhs, const double* X, double* Y);
+
+/* One restart of relaxOver (utils.py:805-878) for formed matrices: v = sum_j coef[j] basis[j] over `count` vectors, scaled
+ * to unit norm, into basis[0]; then, unless `last`, the Krylov basis basis[0..k-1] of N^-1 H by one pass of classical
+ * Gram-Schmidt and mbasis[i] = N^-1 H basis[i], up to the first residual of norm at most 1e-14.  N^-1: W^T W
+ * (W lower triangular and its transpose), or one full matrix (W its inverse, Wt null), or none (both null).
+ * out: [0] the number of basis vectors, [1 + i k + j] = basis[i] . mbasis[j]; with `last` out[1] = v . N^-1 H v alone.
+ * basis, mbasis: k x n; tmp: 2 n doubles. */
+int cc_relax_krylov_f64(void* stream, int64_t n, int k, const double* H, const double* W, const double* Wt, int count,
+                        const double* coef, int last, double* basis, double* mbasis, double* tmp, double* out);
 
 /* Lanczos with full reorthogonalisation for the lowest eigenpair of the pencil (H, N),
  * N = (L L^T) (x) I_d, on the whitened operator W H W^T (W = L^-1).  H is a stage-3 plan.
