@@ -51,6 +51,7 @@ SIGNATURES = {
                               _i32, _pf64, _i64, _i64, _i64, _vp],
     "cc_stage3_plan_apply": [_vp, _vp, _vp, _vp],
     "cc_stage3_plan_destroy": [_vp],
+    "cc_slab_take_f64": [_vp, _i32, _pi32, _pvp, _pf64, _i64, _i64, _i64, _i64, _pi64, _pvp, _pvp],
     "cc_slab_join_f64": [_vp, _i32, _pvp, _pf64, _i64, _i64, _i64, _i64, _vp, _vp],
     "cc_form_work_size": [_i32, _i32, _i64, _i64, _i64, _pi64],
     "cc_form_f64": [_vp, _i32, _pi32, _pvp, _pvp, _i64, _i64, _i64, _vp, _vp],

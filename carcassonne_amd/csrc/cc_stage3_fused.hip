@@ -585,6 +585,78 @@ extern "C" int cc_stage3_pack_sum_f64(void* stream, int n_src, const double* con
   return CC_OK;
 }
 
+namespace {
+// Sums of channels taken at once: joined into a (alpha, P, P) array, packed, or both from one read.
+constexpr int TAKE_JOBS = 8;
+struct TakeJobs {
+  CCSlabGather g[TAKE_JOBS];
+  CCSlabSum src[TAKE_JOBS];
+  double *joined[TAKE_JOBS], *packed[TAKE_JOBS];
+};
+// One job per blockIdx.y.  HBM-bound: a pass over the sources and one over each result; in one launch because the ten
+// sums of a Heisenberg operator are 10 MB each at D = 5, chi = 45 and an operator of small bonds is all launches.
+// D: legs of one extent known at compile time, 0: any.
+template <int D>
+__global__ void __launch_bounds__(256) slab_take_kernel(int64_t n_alpha, int P_rt, const TakeJobs jobs) {
+  extern __shared__ double s[];
+  const int P = D ? D * D : P_rt, NT = (P + 15) / 16, KS = (P + 3) / 4, per = KS * NT * 64, ld = P + 1, j = blockIdx.y;
+  for (int64_t al = blockIdx.x; al < n_alpha; al += gridDim.x) {
+    if (D) cc_slab_load_sum_d<D ? D : 1, 256>(jobs.g[j], jobs.src[j], al, s, ld);
+    else cc_slab_load_sum(jobs.g[j], jobs.src[j], al, s, ld);
+    __syncthreads();
+    if (jobs.joined[j]) {
+      double* out = jobs.joined[j] + al * P * P;
+      for (int e = threadIdx.x; e < P * P; e += 256) out[e] = s[e / P * ld + e % P];
+    }
+    if (jobs.packed[j]) {
+      double* out = jobs.packed[j] + al * per;
+      for (int r = threadIdx.x; r < per; r += 256) {
+        const int lane = r & 63, t = r >> 6, n = t % NT, u = t / NT;
+        const int row = 16 * n + (lane & 15), col = 4 * u + (lane >> 4);
+        out[r] = (row < P && col < P) ? s[row * ld + col] : 0.0;
+      }
+    }
+    __syncthreads();
+  }
+}
+}  // namespace
+
+extern "C" int cc_slab_take_f64(void* stream, int n_jobs, const int* n_src, const double* const* src,
+                                const double* host_coef, int64_t na0, int64_t na1, int64_t d0, int64_t d1,
+                                const int64_t* strides, double* const* joined, double* const* packed) {
+  const int64_t n_alpha = na0 * na1, P = d0 * d1;
+  if (P > PACK_MAX_P) { cc_set_last_error("slab take: slab extent above 64"); return CC_ERR_UNSUPPORTED; }
+  const size_t lds = (size_t)P * (P + 1) * sizeof(double);
+  hipStream_t st = cc_stream(stream);
+  TakeJobs jobs = {};
+  for (int j = 0, at = 0; j < n_jobs;) {
+    const int n = n_jobs - j < TAKE_JOBS ? n_jobs - j : TAKE_JOBS;
+    for (int i = 0; i < n; ++i) {
+      CCSlabMap map;
+      const int rc = cc_slab_map(na0, na1, d0, d1, strides + 6 * (j + i), &map);
+      if (rc) return rc;
+      if (n_src[j + i] < 1 || n_src[j + i] > CC_SLAB_SOURCES) { cc_set_last_error("slab take: 1 to 8 sources"); return CC_ERR_ARG; }
+      jobs.g[i] = cc_slab_gather(map, d0);
+      jobs.src[i] = cc_slab_sum(n_src[j + i], src + at, host_coef + at);
+      jobs.joined[i] = joined[j + i];
+      jobs.packed[i] = packed[j + i];
+      at += n_src[j + i];
+    }
+    const dim3 grid((unsigned)(n_alpha < 16384 ? n_alpha : 16384), (unsigned)n);
+    switch (d0 == d1 ? d0 : 0) {
+      case 2: slab_take_kernel<2><<<grid, 256, lds, st>>>(n_alpha, (int)P, jobs); break;
+      case 3: slab_take_kernel<3><<<grid, 256, lds, st>>>(n_alpha, (int)P, jobs); break;
+      case 4: slab_take_kernel<4><<<grid, 256, lds, st>>>(n_alpha, (int)P, jobs); break;
+      case 5: slab_take_kernel<5><<<grid, 256, lds, st>>>(n_alpha, (int)P, jobs); break;
+      case 6: slab_take_kernel<6><<<grid, 256, lds, st>>>(n_alpha, (int)P, jobs); break;
+      default: slab_take_kernel<0><<<grid, 256, lds, st>>>(n_alpha, (int)P, jobs);
+    }
+    CC_LAUNCH_CHECK();
+    j += n;
+  }
+  return CC_OK;
+}
+
 extern "C" int cc_stage3_pack_strided_f64(void* stream, int64_t na0, int64_t na1, int64_t d0, int64_t d1,
                                           const int64_t* strides, const double* src, double* packed) {
   const double one = 1.0;

@@ -78,6 +78,30 @@ def products_of(terms):
     return out
 
 
+_MERGES = {}   # merged_terms by what it depends on
+
+
+def merged_terms(d, rows, values, legs):
+    """(specs, table) of Stage3Operator._merged from the term table, the numbers of the site operators and the legs and
+    strides of the channels."""
+    values = dict(enumerate(values))
+    values[-1] = tuple(float(i == j) for i in range(d) for j in range(d))
+    products = []
+    for o, members in operator_groups({o: values[o] for o in (-1, *range(len(values) - 1))}):
+        factor = dict(members)
+        edges = [(ia, ib, factor[oo]) for ia, _, ib, oo in rows if oo in factor]
+        for left, right in products_of(edges) if edges else ():
+            if any(len({legs[side][i] for i, _ in part}) > 1 for side, part in ((0, left), (1, right))):
+                products += [(((i, ci),), ((j, cj),), o) for i, ci in left for j, cj in right]
+            else:
+                products.append((tuple(left), tuple(right), o))
+    specs = [list(dict.fromkeys(p[side] for p in products)) for side in (0, 1)]
+    if max(map(len, specs)) > 16 or len(products) > 48:
+        specs = [[((i, 1.0),) for i in range(len(legs[side]))] for side in (0, 1)]
+        products = [(specs[0][ia], specs[1][ib], o) for ia, _, ib, o in rows]
+    return specs, sorted((specs[0].index(left), specs[1].index(right), o) for left, right, o in products)
+
+
 def join_slabs(channels, coefs):
     """sum coefs[i] * channels[i] as a contiguous (alpha, P, P) array; the channels share their leg sizes and strides."""
     _, (na0, na1, d0, d1), st = channels[0].source()
@@ -87,6 +111,18 @@ def join_slabs(channels, coefs):
     _lib.call("cc_slab_join_f64", stream(), len(channels), _lib.ptr_array([c.source()[0].data_ptr() for c in channels]),
               _lib.f64_array(coefs), na0, na1, d0, d1, _lib.i64_array(st), ptr(out))
     return out
+
+
+_PACKED_SIZES = {}
+
+
+def _packed_size(n_alpha, P):
+    size = _PACKED_SIZES.get((n_alpha, P))
+    if size is None:
+        size = _lib.query("cc_stage3_packed_size", n_alpha, P)
+        if len(_PACKED_SIZES) < 4096:
+            _PACKED_SIZES[(n_alpha, P)] = size
+    return size
 
 
 class _Slab:
@@ -197,7 +233,7 @@ class Stage3Operator:
         self._work = None
         self._fused = None
         self._formed = None     # formed.FormedOperator, once a solver has formed this operator
-        self._merge, self._joined, self._refreshed = None, {}, 0
+        self._merge, self._joined, self._packs, self._refreshed = None, {}, {}, 0
         # the slab kernels read P = Q <= 36, d = 2; the solvers, plans and low-precision forms (use_fused) serve the
         # extents D * D of equal center bonds
         self._use_slabs = (self.P == self.Q and self.P <= 36 and self.d == 2 and self.n_alpha > 0 and
@@ -242,24 +278,15 @@ class Stage3Operator:
         operator or -1) sorted by A sum."""
         if self._merge is None:
             a_list, b_list, ops, rows = self._channels()
-            legs = [[ch.source()[1:] for ch in chans] for chans in (a_list, b_list)]
-            values = {-1: tuple(float(i == j) for i in range(self.d) for j in range(self.d))}
-            values.update({o: tuple(float(x) for x in op.toArray().reshape(-1)) for o, op in enumerate(ops)})
-            groups = operator_groups(values)
-            products = []
-            for o, members in groups:
-                factor = dict(members)
-                edges = [(ia, ib, factor[oo]) for ia, _, ib, oo in rows if oo in factor]
-                for left, right in products_of(edges) if edges else ():
-                    if any(len({legs[side][i] for i, _ in part}) > 1 for side, part in ((0, left), (1, right))):
-                        products += [(((i, ci),), ((j, cj),), o) for i, ci in left for j, cj in right]
-                    else:
-                        products.append((tuple(left), tuple(right), o))
-            specs = [list(dict.fromkeys(p[side] for p in products)) for side in (0, 1)]
-            if max(map(len, specs)) > 16 or len(products) > 48:
-                specs = [[((i, 1.0),) for i in range(len(chans))] for chans in (a_list, b_list)]
-                products = [(specs[0][ia], specs[1][ib], o) for ia, _, ib, o in rows]
-            table = sorted((specs[0].index(left), specs[1].index(right), o) for left, right, o in products)
+            legs = tuple(tuple(ch.source()[1:] for ch in chans) for chans in (a_list, b_list))
+            values = tuple(tuple(float(x) for x in op.toArray().reshape(-1)) for op in ops)
+            key = (self.d, tuple(rows), values, legs)
+            merge = _MERGES.get(key)
+            if merge is None:
+                merge = merged_terms(*key)
+                if len(_MERGES) < 256:
+                    _MERGES[key] = merge
+            specs, table = merge
             self._merge = (a_list, b_list), specs, ops, table
         return self._merge
 
@@ -289,22 +316,66 @@ class Stage3Operator:
         return oa, ob
 
     def snapshot(self):
-        """Takes every sum of channels now (joined), so that later calls do not read the stage-2 tensors."""
-        _, specs, _, _ = self._merged()
+        """Takes every sum of channels now (joined and packed), so that later calls do not read the stage-2 tensors."""
+        self._take(True)
+
+    def _take(self, joined):
+        """The sums of channels not taken yet, packed and with `joined` joined as well, one launch per half."""
+        channels, specs, _, _ = self._merged()
         for side in (0, 1):
-            for k in range(len(specs[side])):
-                self.joined(side, k)
+            jobs = []
+            for k, spec in enumerate(specs[side]):
+                # a channel by itself is kept with the channel, for every operator built from it
+                one = channels[side][spec[0][0]] if len(spec) == 1 and spec[0][1] == 1.0 else None
+                need_j = joined and (one._joined is None if one else (side, k) not in self._joined)
+                need_p = (side, k) not in self._packs and (one._packed is None if one else True)
+                if need_p and not need_j and (side, k) in self._joined:
+                    self._packs[(side, k)] = self._pack(side, k, channels[side])     # what was taken before
+                elif need_j or need_p:
+                    jobs.append((k, spec, one, need_j, need_p))
+            while jobs:     # channels of one leg size at a time (all of them, as a rule)
+                sizes = channels[side][jobs[0][1][0][0]].source()[1]
+                alike = [job for job in jobs if channels[side][job[1][0][0]].source()[1] == sizes]
+                jobs = [job for job in jobs if job not in alike]
+                self._take_alike(side, channels[side], sizes, alike)
+            for k, spec in enumerate(specs[side]):
+                if (side, k) not in self._packs:
+                    self._packs[(side, k)] = channels[side][spec[0][0]]._packed
+                if joined and (side, k) not in self._joined:
+                    self._joined[(side, k)] = channels[side][spec[0][0]]._t
+
+    def _take_alike(self, side, channels, sizes, jobs):
+        n_packed = _packed_size(self.n_alpha, self.P)
+        out, sources, coefs, strides = [], [], [], []
+        for k, spec, one, need_j, need_p in jobs:
+            j = empty((self.n_alpha, self.P, self.P)) if need_j else None
+            p = empty((n_packed,)) if need_p else None
+            out.append((j, p))
+            sources += [channels[i].source()[0].data_ptr() for i, _ in spec]
+            coefs += [c for _, c in spec]
+            strides += channels[spec[0][0]].source()[2]
+        _lib.call("cc_slab_take_f64", stream(), len(jobs), _lib.i32_array([len(spec) for _, spec, _, _, _ in jobs]),
+                  _lib.ptr_array(sources), _lib.f64_array(coefs), *sizes, _lib.i64_array(strides),
+                  _lib.ptr_array([j.data_ptr() if j is not None else 0 for j, _ in out]),
+                  _lib.ptr_array([p.data_ptr() if p is not None else 0 for _, p in out]))
+        for (k, _, one, need_j, need_p), (j, p) in zip(jobs, out):
+            if need_j and one:
+                one._joined = HipData(j)
+            elif need_j:
+                self._joined[(side, k)] = j
+            if need_p and one:
+                one._packed = p
+            elif need_p:
+                self._packs[(side, k)] = p
 
     def _pack(self, side, k, channels, out=None):
-        """Sum k of half `side` over `channels` in the fused kernel's MFMA-operand order."""
+        """Sum k of half `side` in the fused kernel's MFMA-operand order: over `channels` into `out`, or as it was joined."""
         _, specs, _, _ = self._merged()
         spec = specs[side][k]
         first = channels[spec[0][0]]
-        kept = self._joined.get((side, k)) if out is None else None
-        if kept is None and out is None and len(spec) == 1 and spec[0][1] == 1.0:
-            return first.packed()
+        kept = self._joined[(side, k)] if out is None else None
         if out is None:
-            out = empty((_lib.query("cc_stage3_packed_size", self.n_alpha, self.P),))
+            out = empty((_packed_size(self.n_alpha, self.P),))
         _, (na0, na1, d0, d1), st = first.source()
         if kept is not None:
             P = self.P
@@ -332,7 +403,9 @@ class Stage3Operator:
     def _build_fused(self):
         """Pack every sum of slab channels once and build the term table (sorted by A channel)."""
         channels, specs, ops, rows = self._merged()
-        A, B = ([self._pack(side, k, channels[side]) for k in range(len(specs[side]))] for side in (0, 1))
+        self._take(False)
+        A, B = ([self._packs[(side, k)] for k in range(len(specs[side]))] for side in (0, 1))
+        self._packs = {}
         self._fused = dict(
             A=A, B=B, A_ptrs=_lib.ptr_array([t.data_ptr() for t in A]), B_ptrs=_lib.ptr_array([t.data_ptr() for t in B]),
             ta=_lib.i32_array([r[0] for r in rows]), tb=_lib.i32_array([r[1] for r in rows]),

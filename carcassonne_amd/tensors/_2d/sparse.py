@@ -4,7 +4,6 @@ carcassonne_amd.sparse.contractSparseTensors.  Stage 3 gathers every compatible
 (stage2_0 tag, stage2_1 tag, operator tag) triple into one Stage3Operator, so a
 matvec of the whole expectation multiplier is a single HIP call.
 """
-import itertools
 import math
 
 from .dense import *  # noqa: F401,F403
@@ -208,16 +207,24 @@ STAGE3_RULES = {
 }
 
 
+_STAGE3_BY_PAIR = {}   # (type, type) of the stage-2 tags -> type of the operator's tag -> rule
+for (_x, _y, _z), _rule in STAGE3_RULES.items():
+    _STAGE3_BY_PAIR.setdefault((_x, _y), {})[_z] = _rule
+
+
 def stage3_terms(stage2_0, stage2_1, operator_center):
     """The compatible tag triples in the reference's enumeration order (sparse.py:116-127),
     as (stage2_0 data, stage2_1 data, operator data or None for an identity operator)."""
     terms = []
-    for tags in itertools.product(stage2_0, stage2_1, operator_center):
-        rule = STAGE3_RULES.get(tuple(type(t) for t in tags))
-        if rule is None or not rule(*tags):
-            continue
-        x, y, z = tags
-        terms.append((stage2_0[x], stage2_1[y], None if z == Identity() else operator_center[z]))
+    for x, data_0 in stage2_0.items():
+        for y, data_1 in stage2_1.items():
+            rules = _STAGE3_BY_PAIR.get((type(x), type(y)))
+            if rules is None:
+                continue
+            for z, op in operator_center.items():
+                rule = rules.get(type(z))
+                if rule is not None and rule(x, y, z):
+                    terms.append((data_0, data_1, None if type(z) is Identity else op))
     return terms
 
 

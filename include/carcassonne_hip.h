@@ -165,6 +165,12 @@ int cc_stage3_pack_strided_f64(void* stream, int64_t na0, int64_t na1, int64_t d
  * map: a term (c_1 A_1 + c_2 A_2) (x) B (x) O costs what one of its two terms costs. */
 int cc_stage3_pack_sum_f64(void* stream, int n_src, const double* const* src, const double* host_coef, int64_t na0,
                            int64_t na1, int64_t d0, int64_t d1, const int64_t* strides, double* packed);
+/* Several sums of channels at once, each joined into a contiguous (alpha, P, P) array (cc_slab_join_f64), packed
+ * (cc_stage3_pack_sum_f64), or both (null: not wanted): n_src[j] sources and coefficients follow each other, six strides
+ * per sum; the leg sizes are common. */
+int cc_slab_take_f64(void* stream, int n_jobs, const int* n_src, const double* const* src, const double* host_coef,
+                     int64_t na0, int64_t na1, int64_t d0, int64_t d1, const int64_t* strides, double* const* joined,
+                     double* const* packed);
 int cc_stage3_matvec_fused_f64(void* stream, int n_a, const double* const* A_packed, int n_b,
                                const double* const* B_packed, int n_terms, const int* term_a,
                                const int* term_b, const int* term_o, int n_ops, const double* host_ops,
