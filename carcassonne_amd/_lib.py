@@ -49,6 +49,8 @@ SIGNATURES = {
     "cc_stage3_pack_strided_f64": [_vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp],
     "cc_stage3_plan_create": [ctypes.POINTER(ctypes.c_void_p), _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32,
                               _i32, _pf64, _i64, _i64, _i64, _vp],
+    "cc_stage3_slab_plan_create": [ctypes.POINTER(ctypes.c_void_p), _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32,
+                                   _i32, _pf64, _i64, _i64, _i64, _vp],
     "cc_stage3_plan_apply": [_vp, _vp, _vp, _vp],
     "cc_stage3_plan_destroy": [_vp],
     "cc_slab_take_f64": [_vp, _i32, _pi32, _pvp, _pf64, _i64, _i64, _i64, _i64, _pi64, _pvp, _pvp],
@@ -110,8 +112,6 @@ SIGNATURES = {
     "cc_stage3_pack_sum_f64": [_vp, _i32, _pvp, _pf64, _i64, _i64, _i64, _i64, _vp, _vp],
     "cc_stage3_matvec_fused_f64": [_vp, _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32, _i32, _pf64, _i64, _i64,
                                    _i64, _vp, _vp, _vp],
-    "cc_stage3_matvec_slabs_f64": [_vp, _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32, _i32, _pf64, _i64, _i64,
-                                   _i64, _vp, _vp, _vp],
     "cc_stage3_matvec_fused_f64_noalloc": [_vp, _i32, _pvp, _i32, _pvp, _i32, _pi32, _pi32, _pi32, _i32, _pf64, _i64,
                                            _i64, _i64, _vp, _vp],
 }
@@ -163,8 +163,9 @@ def check(rc, what=""):
 
 
 def call(name, *args):
-    lib = load()
-    check(getattr(lib, name)(*args), name)
+    rc = getattr(_lib or load(), name)(*args)
+    if rc != CC_OK:
+        check(rc, name)
 
 
 def i64_array(values):

@@ -16,6 +16,7 @@
 #include "cc_common.h"
 
 #include <mutex>
+#include <new>
 #include <vector>
 
 namespace {
@@ -682,18 +683,6 @@ extern "C" int cc_stage3_matvec_fused_f64(void* stream, int n_a, const double* c
   return fused_f64(cc_stream(stream), plan, P, v, y, work);
 }
 
-extern "C" int cc_stage3_matvec_slabs_f64(void* stream, int n_a, const double* const* A_packed, int n_b,
-                                          const double* const* B_packed, int n_terms, const int* term_a,
-                                          const int* term_b, const int* term_o, int n_ops, const double* host_ops,
-                                          int64_t n_alpha, int64_t P, int64_t d, const double* v, double* y,
-                                          double* work) {
-  if (d != 2 || P < 1 || P > 36) { cc_set_last_error("slab stage-3: needs d = 2 and P <= 36"); return CC_ERR_UNSUPPORTED; }
-  FusedPlan plan;
-  int rc = fill_plan(plan, n_a, A_packed, n_b, B_packed, n_terms, term_a, term_b, term_o, n_ops, host_ops, n_alpha, d);
-  if (rc) return rc;
-  return fused_f64(cc_stream(stream), plan, P, v, y, work);
-}
-
 // ---- the allocation-free entry point -----------------------------------------------------------
 // Scratch of cc_stage3_matvec_fused_f64_noalloc: the workgroup partial sums (groups x P^2 d doubles).
 // Every GPU the library runs on holds its own copy until the process ends.
@@ -747,13 +736,14 @@ extern "C" int cc_stage3_matvec_fused_f64_noalloc(void* stream, int n_a, const d
   return fused_f64(cc_stream(stream), plan, P, v, y, scratch, false);
 }
 
-extern "C" int cc_stage3_plan_create(void** out, int n_a, const double* const* A_packed, int n_b,
-                                     const double* const* B_packed, int n_terms, const int* term_a, const int* term_b,
-                                     const int* term_o, int n_ops, const double* host_ops, int64_t n_alpha, int64_t P,
-                                     int64_t d, double* work) {
+extern "C" int cc_stage3_slab_plan_create(void** out, int n_a, const double* const* A_packed, int n_b,
+                                          const double* const* B_packed, int n_terms, const int* term_a,
+                                          const int* term_b, const int* term_o, int n_ops, const double* host_ops,
+                                          int64_t n_alpha, int64_t P, int64_t d, double* work) {
   *out = nullptr;
-  if (!cc_stage3_fused_supported(P, d)) { cc_set_last_error("fused stage-3: shape not instantiated"); return CC_ERR_UNSUPPORTED; }
-  Stage3PlanHandle* h = new Stage3PlanHandle();
+  if (d != 2 || P < 1 || P > 36) { cc_set_last_error("slab stage-3: needs d = 2 and P <= 36"); return CC_ERR_UNSUPPORTED; }
+  Stage3PlanHandle* h = new (std::nothrow) Stage3PlanHandle();
+  if (!h) { cc_set_last_error("slab stage-3: out of host memory"); return CC_ERR_OOM; }
   int rc = fill_plan(h->plan, n_a, A_packed, n_b, B_packed, n_terms, term_a, term_b, term_o, n_ops, host_ops, n_alpha, d);
   if (rc) { delete h; return rc; }
   h->P = P;
@@ -763,6 +753,16 @@ extern "C" int cc_stage3_plan_create(void** out, int n_a, const double* const* A
   h->work = work;
   *out = h;
   return CC_OK;
+}
+
+extern "C" int cc_stage3_plan_create(void** out, int n_a, const double* const* A_packed, int n_b,
+                                     const double* const* B_packed, int n_terms, const int* term_a, const int* term_b,
+                                     const int* term_o, int n_ops, const double* host_ops, int64_t n_alpha, int64_t P,
+                                     int64_t d, double* work) {
+  *out = nullptr;
+  if (!cc_stage3_fused_supported(P, d)) { cc_set_last_error("fused stage-3: shape not instantiated"); return CC_ERR_UNSUPPORTED; }
+  return cc_stage3_slab_plan_create(out, n_a, A_packed, n_b, B_packed, n_terms, term_a, term_b, term_o, n_ops, host_ops,
+                                    n_alpha, P, d, work);
 }
 
 extern "C" int cc_stage3_packed_size_f32(int64_t n_alpha, int64_t P, int role, int64_t* out) {

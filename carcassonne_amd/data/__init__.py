@@ -7,7 +7,6 @@ cc_gemm_f64, cc_svd_f64, elementwise and reduction kernels).  Complex data is
 rejected: the accelerated path is real (Hermitian = symmetric), which covers the
 transverse-field Ising model and the Heisenberg model written with iY.
 """
-import ctypes
 
 import numpy as np
 import torch
@@ -87,6 +86,9 @@ class HipData(Data):
         return d
 
     def __init__(self, t):
+        if type(t) is torch.Tensor and t.dtype == torch.float64 and t.is_cuda:
+            self._t = t.contiguous()
+            return
         if isinstance(t, np.ndarray) or np.isscalar(t):
             t = HipData._upload(np.asarray(t))
         if not isinstance(t, torch.Tensor):
@@ -552,10 +554,10 @@ def _gemm(M, N, K, A, sAm, sAk, B, sBk, sBn, out):
     _lib.call("cc_gemm_f64", stream(), S, M, N, kc, 1.0, ptr(A), kc * sAk, sAm, sAk, ptr(B), kc * sBk, sBk, sBn,
               0.0, ptr(parts), M * N, N, 1)
     if rest:
-        a_rest = ptr(A).value + S * kc * sAk * 8
-        b_rest = ptr(B).value + S * kc * sBk * 8
-        _lib.call("cc_gemm_f64", stream(), 1, M, N, rest, 1.0, ctypes.c_void_p(a_rest), 0, sAm, sAk,
-                  ctypes.c_void_p(b_rest), 0, sBk, sBn, 0.0, ptr(parts[S]), 0, N, 1)
+        a_rest = ptr(A) + S * kc * sAk * 8
+        b_rest = ptr(B) + S * kc * sBk * 8
+        _lib.call("cc_gemm_f64", stream(), 1, M, N, rest, 1.0, a_rest, 0, sAm, sAk,
+                  b_rest, 0, sBk, sBn, 0.0, ptr(parts[S]), 0, N, 1)
     n_parts = parts.shape[0]
     assert n_parts <= ONES_LEN
     _lib.call("cc_gemm_f64", stream(), 1, 1, M * N, n_parts, 1.0, ptr(ones()), 0, n_parts, 1, ptr(parts), 0, M * N, 1,

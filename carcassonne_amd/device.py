@@ -1,6 +1,4 @@
 """Device memory and stream plumbing (PyTorch-ROCm tensors as buffers; no torch compute)."""
-import ctypes
-
 import torch
 
 _DEVICE = None
@@ -33,20 +31,21 @@ _DEVICE_INDEX = None
 
 
 def stream():
-    """The caller's current HIP stream as a void* for the C ABI (the raw handle: this is called before
-    every kernel launch, and building a torch Stream object each time costs microseconds)."""
+    """The caller's current HIP stream for the C ABI (the raw handle as a number: this is called before
+    every kernel launch, and building a torch Stream or a ctypes object each time costs microseconds)."""
     global _DEVICE_INDEX
     if _DEVICE_INDEX is None:
         _DEVICE_INDEX = device().index
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(_DEVICE_INDEX))
+    return torch._C._cuda_getCurrentRawStream(_DEVICE_INDEX)
 
 
 def empty(shape, dtype=torch.float64):
-    return torch.empty([int(s) for s in shape], dtype=dtype, device=_DEVICE if _DEVICE is not None else device())
+    return torch.empty(shape if type(shape) is torch.Size else [int(s) for s in shape], dtype=dtype,
+                       device=_DEVICE if _DEVICE is not None else device())
 
 
 def ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t.numel() else ctypes.c_void_p(0)
+    return t.data_ptr()   # 0 for an empty tensor
 
 
 def synchronize():

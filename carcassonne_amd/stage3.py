@@ -215,7 +215,7 @@ class Stage3Operator:
         s0, s1, o = self.terms[0]
         self.d = int(physical_dimension if physical_dimension is not None else
                      next((op.shape[0] for (_, _, op) in self.terms if op is not None), None))
-        self.state_shape = (s0.shape[2], s0.shape[3], s1.shape[2], s1.shape[3], self.d)
+        self.state_shape = torch.Size((s0.shape[2], s0.shape[3], s1.shape[2], s1.shape[3], self.d))
         self.n = int(np.prod(self.state_shape))
         self.P, self.Q = s0.shape[2] * s0.shape[3], s1.shape[2] * s1.shape[3]
         self.n_alpha = s0.shape[0] * s0.shape[1]
@@ -411,7 +411,10 @@ class Stage3Operator:
             ta=_lib.i32_array([r[0] for r in rows]), tb=_lib.i32_array([r[1] for r in rows]),
             to=_lib.i32_array([r[2] for r in rows]), n_terms=len(rows), n_a=len(A), n_b=len(B),
             n_ops=len(ops), ops=_lib.f64_array([x for o in ops for x in o.toArray().reshape(-1)]),
-            work=empty((max(1, _lib.query("cc_stage3_fused_work_size", self.n_alpha, self.P, self.d)),)))
+            work=empty((max(1, _lib.query("cc_stage3_fused_work_size", self.n_alpha, self.P, self.d)),)), plan=ctypes.c_void_p())
+        f = self._fused
+        _lib.call("cc_stage3_slab_plan_create", ctypes.byref(f["plan"]), f["n_a"], f["A_ptrs"], f["n_b"], f["B_ptrs"],
+                  f["n_terms"], f["ta"], f["tb"], f["to"], f["n_ops"], f["ops"], self.n_alpha, self.P, self.d, ptr(f["work"]))
 
     def _join(self, t, which):
         return _Slab.of(t, which)
@@ -440,12 +443,8 @@ class Stage3Operator:
             return f["plan_f32"]
         if precision != "f64":
             raise ValueError("precision must be 'f64' or 'f32', not {!r}".format(precision))
-        if f.get("plan") is None:
-            h = ctypes.c_void_p()
-            _lib.call("cc_stage3_plan_create", ctypes.byref(h), f["n_a"], f["A_ptrs"], f["n_b"], f["B_ptrs"],
-                      f["n_terms"], f["ta"], f["tb"], f["to"], f["n_ops"], f["ops"], self.n_alpha, self.P, self.d,
-                      ptr(f["work"]))
-            f["plan"] = h
+        if not self.use_fused:
+            raise NotImplementedError("the operator has no instantiated fused shape")
         return f["plan"]
 
     def __del__(self):
@@ -462,13 +461,11 @@ class Stage3Operator:
         if self._formed is not None and self._formed.valid():
             self._formed.apply_flat(x, y)
             return
-        if self._use_slabs and (self.use_fused or self._fused is not None or not torch.cuda.is_current_stream_capturing()):
-            # also for unequal center bonds (packing may read site operators back, so not first under capture)
-            self._ensure_fused()
-            f = self._fused
-            _lib.call("cc_stage3_matvec_slabs_f64", stream(), f["n_a"], f["A_ptrs"], f["n_b"], f["B_ptrs"],
-                      f["n_terms"], f["ta"], f["tb"], f["to"], f["n_ops"], f["ops"], self.n_alpha, self.P, self.d,
-                      ptr(x), ptr(y), ptr(f["work"]))
+        # also for unequal center bonds (packing may read site operators back, so not first under capture)
+        if self._fused is None and self._use_slabs and (self.use_fused or not torch.cuda.is_current_stream_capturing()):
+            self._build_fused()
+        if self._fused is not None:
+            _lib.call("cc_stage3_plan_apply", stream(), self._fused["plan"], ptr(x), ptr(y))
             return
         self.apply_generic_flat(x, y)
 
@@ -485,11 +482,11 @@ class Stage3Operator:
                   self.n_alpha, self.P, self.Q, self.d, ptr(x), ptr(y), ptr(self._work))
 
     def apply(self, v):
-        if tuple(v.shape) != self.state_shape and v.size() != self.n:
+        if v.shape != self.state_shape and v.size() != self.n:
             raise ValueError("state shape {} does not match the operator's {}".format(v.shape, self.state_shape))
         out = empty(self.state_shape)
-        self.apply_flat(v._t.reshape(-1), out.view(-1))
-        return HipData(out)
+        self.apply_flat(v._t, out)
+        return HipData._wrap(out)
 
     def form_matrix(self):
         """The dense matrix: the environment matrices of all terms in one contraction, their products with the site

@@ -176,12 +176,6 @@ int cc_stage3_matvec_fused_f64(void* stream, int n_a, const double* const* A_pac
                                const int* term_b, const int* term_o, int n_ops, const double* host_ops,
                                int64_t n_alpha, int64_t P, int64_t d, const double* v, double* y,
                                double* work);
-/* The same kernel for slabs of any extent P = Q <= 36 (center bonds that differ by direction), d = 2: packing, workspace
- * and arguments as above. */
-int cc_stage3_matvec_slabs_f64(void* stream, int n_a, const double* const* A_packed, int n_b, const double* const* B_packed,
-                               int n_terms, const int* term_a, const int* term_b, const int* term_o, int n_ops,
-                               const double* host_ops, int64_t n_alpha, int64_t P, int64_t d, const double* v, double* y,
-                               double* work);
 
 /* cc_stage3_matvec_fused_f64 without any allocation and without a workspace argument: no counterpart in the
  * reference; for callers that cannot allocate device memory (code under HIP graph capture, serving loops,
@@ -220,6 +214,11 @@ int cc_stage3_plan_create(void** out, int n_a, const double* const* A_packed, in
                           const double* const* B_packed, int n_terms, const int* term_a,
                           const int* term_b, const int* term_o, int n_ops, const double* host_ops,
                           int64_t n_alpha, int64_t P, int64_t d, double* work);
+/* The same for slabs of any extent P = Q <= 36 (center bonds that differ by direction), d = 2. */
+int cc_stage3_slab_plan_create(void** out, int n_a, const double* const* A_packed, int n_b,
+                               const double* const* B_packed, int n_terms, const int* term_a,
+                               const int* term_b, const int* term_o, int n_ops, const double* host_ops,
+                               int64_t n_alpha, int64_t P, int64_t d, double* work);
 int cc_stage3_plan_apply(void* stream, const void* plan, const double* x, double* y);
 int cc_stage3_plan_destroy(void* plan);
 
