@@ -319,14 +319,16 @@ int plan(int rm, int rn, int rk, const int64_t* legs, int n_out, const int* term
   const int64_t tall = (M + 127) / 128 * n_out, square = (M + 63) / 64 * ((N + 63) / 64) * n_out;
   sh.tall = N <= 80 && tall >= 160 ? (int)((N + 15) / 16) : 0;
   sh.T = square >= 160 ? 64 : 32;
+  // long sums: three workgroups per CU where that leaves each at least eight steps of 16 (64 x 64 tiles: five outputs of
+  // 64 x 2304 with K = 2304 take 144 us whole and 94 us split), one per CU and four steps of 32 for the small tiles
   sh.splits = 1;
-  if (!sh.tall && sh.T == 32) {
-    const int64_t tiles = (M + 31) / 32 * ((N + 31) / 32) * n_out;
+  if (!sh.tall) {
+    const int T = sh.T;
+    const int64_t tiles = (M + T - 1) / T * ((N + T - 1) / T) * n_out;
     int most = 0;
     for (int o = 0; o < n_out; ++o) most = std::max(most, terms[o]);
-    const int64_t steps = (K + 31) / 32 * most;
-    // at least four steps per workgroup; no more workgroups than CUs
-    sh.splits = (int)std::max<int64_t>(1, std::min(steps / 4, 256 / tiles));
+    const int64_t steps = T == 64 ? (K + 15) / 16 * most : (K + 31) / 32 * most;
+    sh.splits = (int)std::max<int64_t>(1, T == 64 ? std::min(steps / 8, 768 / tiles) : std::min(steps / 4, 256 / tiles));
   }
   return CC_OK;
 }

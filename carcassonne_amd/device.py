@@ -55,19 +55,19 @@ def synchronize():
 _SIDE = {}
 
 
-def side_stream():
-    """A second stream (default priority) on the current device, for setup work that runs beside the
+def side_stream(k=0):
+    """Another stream (default priority) on the current device, number k of those, for setup work that runs beside the
     caller's stream: fork() starts it after everything the caller's stream has queued, join() makes the
     caller's stream wait for it."""
     d = device()
-    s = _SIDE.get(d.index)
+    s = _SIDE.get((d.index, k))
     if s is None:
-        s = _SIDE[d.index] = torch.cuda.Stream(d)
+        s = _SIDE[(d.index, k)] = torch.cuda.Stream(d)
     return s
 
 
-def fork():
-    side = side_stream()
+def fork(k=0):
+    side = side_stream(k)
     side.wait_stream(torch.cuda.current_stream())
     return side
 

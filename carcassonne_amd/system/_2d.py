@@ -422,10 +422,9 @@ class System(BaseSystem):
         import torch
         from ..device import fork, join
         i = direction
-        iso, _, den = self.state_center_data.normalizeAxis(O(i))
-        # the two corners and their truncation bases are independent: the right one on a side stream
-        # (the bases' 64 x 64 eigen-decompositions run on one workgroup each)
-        side, produced = fork(), []
+        # the two corners and their truncation bases and the gauge of the center are independent: the right corner and
+        # the gauge on streams of their own (the eigen-decompositions run on one workgroup each)
+        side, gauge, produced, gauged = fork(), fork(1), [], []
         try:
             with torch.cuda.stream(side):
                 corner_r = absorbSparseSideIntoCornerFromRight(self.corners[R(i)], self.sides[R(i)])
@@ -433,13 +432,18 @@ class System(BaseSystem):
                 produced = list(corner_r.values()) + [right]
             corner_l = absorbSparseSideIntoCornerFromLeft(self.corners[i], self.sides[L(i)])
             left = fusedTruncationBasis(corner_l[Identity()], (3, 4, 5), (0, 1, 2), new_dimension)
+            with torch.cuda.stream(gauge):
+                iso, _, den = self.state_center_data.normalizeAxis(O(i))
+                center = self.state_center_data.normalizeAxis(i)[0].absorbMatrixAt(i, den)
+                gauged = [iso, den, center]
         finally:
             join(side, produced)
+            join(gauge, gauged)
         self.sides[i] = absorbSparseCenterSOSIntoSideProjected(i, self.sides[i], iso, self.operator_center_tensor,
                                                                left, right, iso.conj())
         self.corners[i] = _project_corners(corner_l, (3, 4, 5), left)
         self.corners[R(i)] = _project_corners(corner_r, (0, 1, 2), right)
-        self.setStateCenter(self.state_center_data.normalizeAxis(i)[0].absorbMatrixAt(i, den))
+        self.setStateCenter(center)
 
     # -- multipliers (_2d.py:455-488) --------------------------------------------------------
     def formExpectationAndNormalizationMultipliers(self, operator_center_tensor=None):
