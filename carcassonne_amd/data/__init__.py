@@ -8,6 +8,8 @@ rejected: the accelerated path is real (Hermitian = symmetric), which covers the
 transverse-field Ising model and the Heisenberg model written with iY.
 """
 
+import functools
+
 import numpy as np
 import torch
 
@@ -78,6 +80,11 @@ def _contract_plan(ssh, osh, self_axes, other_axes):
     legs = tuple(range(sn)), tuple(self_axes[other_axes.index(j)] if j in other_axes else sn + j for j in range(on)), \
         tuple(fa) + tuple(sn + j for j in fb)
     return M, N, K, out_shape, a_mode, fa + self_axes, b_mode, other_axes + fb, legs
+
+
+@functools.lru_cache(maxsize=4096)
+def _svd_work_size(m, n):
+    return _lib.query("cc_svd_work_size", 1, m, n)
 
 
 class HipData(Data):
@@ -470,9 +477,7 @@ class HipData(Data):
             Ut, S, Vtt = HipData(self._t.t().contiguous()).svd(False)
             return Vtt.join(1, 0), S, Ut.join(1, 0)
         U, S, Vt = empty((m, n)), empty((n,)), empty((n, n))
-        ws = _lib.i64_array([0])
-        _lib.call("cc_svd_work_size", 1, m, n, ws)
-        work = empty((max(1, ws[0]),))
+        work = empty((max(1, _svd_work_size(m, n)),))
         _lib.call("cc_svd_f64", stream(), 1, m, n, ptr(self._t), ptr(U), ptr(S), ptr(Vt), ptr(work))
         return HipData(U), HipData(S), HipData(Vt)
 
@@ -489,6 +494,14 @@ class HipData(Data):
 
     def normalizeAxis(self, axis, sqrt_svals=False, dont_recip_under=1e-14):
         """data/__init__.py:263-301."""
+        return self._normalized(axis, sqrt_svals, dont_recip_under)
+
+    def isometryAt(self, axis, normalizer=False):
+        """normalizeAxis without the matrices that are not wanted: (normalized data, normalizer or None)."""
+        iso, _, den = self._normalized(axis, inverse=False, normalizer=normalizer)
+        return iso, den
+
+    def _normalized(self, axis, sqrt_svals=False, dont_recip_under=1e-14, inverse=True, normalizer=True):
         if self.shape[axis] == 1:
             n = self.norm()
             if sqrt_svals:
@@ -501,21 +514,28 @@ class HipData(Data):
             raise ValueError("the total number of degrees of freedom in all other axes ({}) are not enough to "
                              "normalize axis ({}) with dimension ({})".format(M.shape[0], axis, M.shape[1]))
         U, S, V = M.svd(full_matrices=False)
-        U = U.contractWith(V, (1,), (0,))
         S = S.split(S.shape[0], 1)
-        SI = HipData(empty(S.shape))
-        if dont_recip_under:
-            _lib.call("cc_unary_f64", stream(), 1, S.size(), ptr(S._t), float(dont_recip_under), ptr(SI._t))
-        else:
-            _lib.call("cc_unary_f64", stream(), 4, S.size(), ptr(S._t), 0.0, ptr(SI._t))
+        if inverse or sqrt_svals:
+            SI = HipData(empty(S.shape))
+            if dont_recip_under:
+                _lib.call("cc_unary_f64", stream(), 1, S.size(), ptr(S._t), float(dont_recip_under), ptr(SI._t))
+            else:
+                _lib.call("cc_unary_f64", stream(), 4, S.size(), ptr(S._t), 0.0, ptr(SI._t))
         if sqrt_svals:
             S, SI = S.sqrt(), SI.sqrt()
             return (V * SI), V * S
-        U_split = [self.shape[i] for i in others] + [U.shape[1]]
-        U_join = list(range(self.ndim - 1))
-        U_join.insert(axis, self.ndim - 1)
-        return (U.split(*U_split).join(*U_join), V.transpose().contractWith(V * SI, (1,), (0,)),
-                V.transpose().contractWith(V * S, (1,), (0,)))
+        # U V with its legs back in place: (others..., k) x (k, axis)
+        legs = tuple(range(self.ndim))
+        U = U.split(*([self.shape[i] for i in others] + [U.shape[1]]))
+        iso = contract(tuple(others) + (-1,), (-1, axis % self.ndim), legs, [[(U, V)]])
+        if iso is not None:
+            iso = HipData._wrap(iso[0])
+        else:
+            order = list(range(self.ndim - 1))
+            order.insert(axis, self.ndim - 1)
+            iso = U.contractWith(V, (self.ndim - 1,), (0,)).transpose(order)
+        return (iso, V.contractWith(V * SI, (0,), (0,)) if inverse else None,
+                V.contractWith(V * S, (0,), (0,)) if normalizer else None)
 
     def normalizeAxisAndDenormalize(self, axis_to_norm, axis_to_denorm, data_to_denormalize=None, sqrt_svals=False,
                                     dont_recip_under=1e-14):

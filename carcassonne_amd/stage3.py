@@ -12,6 +12,7 @@ HIP library: the fused MFMA kernel for the instantiated slab shapes, the generic
 GEMM path for any other shape.
 """
 import ctypes
+import functools
 import weakref
 
 import numpy as np
@@ -113,16 +114,9 @@ def join_slabs(channels, coefs):
     return out
 
 
-_PACKED_SIZES = {}
-
-
+@functools.lru_cache(maxsize=4096)
 def _packed_size(n_alpha, P):
-    size = _PACKED_SIZES.get((n_alpha, P))
-    if size is None:
-        size = _lib.query("cc_stage3_packed_size", n_alpha, P)
-        if len(_PACKED_SIZES) < 4096:
-            _PACKED_SIZES[(n_alpha, P)] = size
-    return size
+    return _lib.query("cc_stage3_packed_size", n_alpha, P)
 
 
 class _Slab:

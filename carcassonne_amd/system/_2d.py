@@ -8,6 +8,7 @@ residual-controlled FP64 Lanczos and solver="mixed" the FP16/BF16 precision form
 an instantiated fused shape, P = D0*D1 in {4, 9, 16, 25, 36}, d = 2).
 """
 import copy as _copy
+import functools
 
 import numpy as np
 
@@ -29,6 +30,12 @@ def sideFromCorner(corner_id, direction):
     return (corner_id + 1 - direction) % 4
 
 
+@functools.lru_cache(maxsize=4096)
+def _truncation_work_size(nx, D, far):
+    from .. import _lib
+    return _lib.query("cc_fused_truncation_work_size", nx, D, far)
+
+
 def fusedTruncationBasis(corner, bond_legs, far_legs, new_dimension):
     """The (x D D) x k truncation basis of a grown fused corner bond, bond legs (x D, D, 1) with the old bond
     x and the absorbed side's center ket / bra legs D, from the corner's Identity channel matricized bond x
@@ -46,7 +53,7 @@ def fusedTruncationBasis(corner, bond_legs, far_legs, new_dimension):
     C = corner.join(tuple(bond_legs), tuple(far_legs)).tensor().contiguous()
     m = nx * D * D
     U, S = empty((m, k)), empty((far,))
-    work = empty((_lib.query("cc_fused_truncation_work_size", nx, D, far),))
+    work = empty((_truncation_work_size(nx, D, far),))
     _lib.call("cc_fused_truncation_f64", stream(), nx, D, far, k, ptr(C), ptr(U), ptr(S), ptr(work))
     return HipData(U)
 
@@ -433,8 +440,8 @@ class System(BaseSystem):
             corner_l = absorbSparseSideIntoCornerFromLeft(self.corners[i], self.sides[L(i)])
             left = fusedTruncationBasis(corner_l[Identity()], (3, 4, 5), (0, 1, 2), new_dimension)
             with torch.cuda.stream(gauge):
-                iso, _, den = self.state_center_data.normalizeAxis(O(i))
-                center = self.state_center_data.normalizeAxis(i)[0].absorbMatrixAt(i, den)
+                iso, den = self.state_center_data.isometryAt(O(i), normalizer=True)
+                center = self.state_center_data.isometryAt(i)[0].absorbMatrixAt(i, den)
                 gauged = [iso, den, center]
         finally:
             join(side, produced)
