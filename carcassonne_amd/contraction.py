@@ -74,11 +74,12 @@ def _pointers(tensors):
     return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
 
 
-def contract(a, b, out, outputs, split_long_sums=False):
+def contract(a, b, out, outputs, split_long_sums=False, together=False):
     """One device tensor per entry of `outputs`, each the sum of A B over its pairs (A, B): `a`, `b` and `out` name the
     legs of the first operands, the second ones and the results (a leg in both operands is summed, every other is in
     `out`).  split_long_sums: long sums with small results are summed in slices (their rounding then differs from one
-    sum's, so only callers that ask for it get it).  None where the kernel does not take the contraction."""
+    sum's, so only callers that ask for it get it).  together: the results are parts of one allocation (for intermediate
+    tensors).  None where the kernel does not take the contraction."""
     if any(len(pairs) > MAX_TERMS for pairs in outputs):
         return None
     A = [_layout(x) for pairs in outputs for x, _ in pairs]
@@ -89,7 +90,7 @@ def contract(a, b, out, outputs, split_long_sums=False):
     plan = _plan(a, b, out, la, lb, tuple(len(pairs) for pairs in outputs))
     if not plan.ok:
         return None
-    results = [empty(plan.shape) for _ in outputs]
+    results = empty([len(outputs)] + plan.shape).unbind(0) if together else [empty(plan.shape) for _ in outputs]
     work = empty((plan.work,)) if plan.work and split_long_sums else None
     _lib.call("cc_contract_f64", stream(), *plan.counts, plan.legs, len(outputs), plan.terms,
               _pointers([t for t, _ in A]), _pointers([t for t, _ in B]), _pointers(results),

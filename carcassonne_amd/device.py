@@ -72,6 +72,15 @@ def fork(k=0):
     return side
 
 
+def fork_both():
+    """fork() of the first two side streams at one point of the caller's stream."""
+    at = torch.cuda.current_stream().record_event()
+    sides = side_stream(0), side_stream(1)
+    for side in sides:
+        side.wait_event(at)
+    return sides
+
+
 def join(side, produced=()):
     """The caller's stream waits for `side`; the device tensors of the objects in `produced` (made on
     `side`, used on the caller's stream from here on) are recorded as in use on the caller's stream, so

@@ -427,11 +427,11 @@ class System(BaseSystem):
             raise InvariantViolatedError("Contracting the current center would blow up the condition number of the "
                                          "normalization matrix;  optimize it or replace it first.")
         import torch
-        from ..device import fork, join
+        from ..device import fork_both, join
         i = direction
         # the two corners and their truncation bases and the gauge of the center are independent: the right corner and
         # the gauge on streams of their own (the eigen-decompositions run on one workgroup each)
-        side, gauge, produced, gauged = fork(), fork(1), [], []
+        (side, gauge), produced, gauged = fork_both(), [], []
         try:
             with torch.cuda.stream(side):
                 corner_r = absorbSparseSideIntoCornerFromRight(self.corners[R(i)], self.sides[R(i)])

@@ -142,21 +142,23 @@ def _project_channels(direction, matched, sos, state, state_conj, left, right):
     lt, rt = left.split(x, D_a, D_a, left.shape[1]), right.split(y, D_c, D_c, right.shape[1])
     sides = {id(p[0]): p[0] for p in pairs}
     operators = {id(p[1]): p[1] for p in pairs if p[2] is sos}
-    grown = contract("xabk", "xyij", "abkyij", [[(lt, t.split(x, y, sh[6], sh[7]))] for t in sides.values()])
+    grown = contract("xabk", "xyij", "abkyij", [[(lt, t.split(x, y, sh[6], sh[7]))] for t in sides.values()],
+                     together=True)
     if grown is None:
         return None
-    met = contract("abkyij", legs, "bkyjcos", [[(HipData(t), state)] for t in grown])
-    acted = contract("ts", conj.replace("s", "t"), conj, [[(op, state_conj)] for op in operators.values()]) if operators else []
+    met = contract("abkyij", legs, "bkyjcos", [[(HipData._wrap(t), state)] for t in grown], together=True)
+    acted = contract("ts", conj.replace("s", "t"), conj, [[(op, state_conj)] for op in operators.values()],
+                     together=True) if operators else []
     if met is None or acted is None:
         return None
-    met = {key: HipData(t) for key, t in zip(sides, met)}
-    acted = {key: HipData(t) for key, t in zip(operators, acted)}
+    met = {key: HipData._wrap(t) for key, t in zip(sides, met)}
+    acted = {key: HipData._wrap(t) for key, t in zip(operators, acted)}
     summed = contract("bkyjcos", conj, "kycoep",
                       [[(met[id(t)], acted[id(op)] if f is sos else state_conj) for t, op, f in products]
-                       for products in matched.values()])
+                       for products in matched.values()], together=True)
     if summed is None:
         return None
-    out = contract("kycoep", "yceq", "kqop", [[(HipData(t), rt)] for t in summed], split_long_sums=True)
+    out = contract("kycoep", "yceq", "kqop", [[(HipData._wrap(t), rt)] for t in summed], split_long_sums=True)
     if out is None:
         return None
     return {tag: HipData(t.reshape(t.shape[0], 1, 1, t.shape[1], 1, 1, t.shape[2], t.shape[3]))
