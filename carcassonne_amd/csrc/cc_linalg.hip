@@ -57,153 +57,355 @@ __device__ __forceinline__ void tri_sweep(double (&r)[CB], double s, F src) {
 // c[j] = -d_i X[j][i] (j > i).  The symmetric updates keep c_i[j] == c_j[i] bit for bit (the same two
 // factors meet in each FMA).  A non-positive pivot of a real row records its 1-based index in bad and is
 // replaced by 1e-300.
-// Blocks of 64R x 64R on 4R waves: wave w holds columns 16w .. 16w + 15, lane i rows i + 64r (r < R).
-// The sweep goes in panels of PB = 4 columns.  The wave owning a panel factors it alone: per step the
-// pivot, the multipliers (published in LDS) and the step's update of the panel's later columns, with the
-// row multipliers it needs taken by readlane.  After one barrier every wave with columns past the panel
-// applies the panel's four updates, in step order, so each element sees the same FMAs in the same order
-// as in a column-by-column sweep.  The owner of the next panel first brings that panel's columns up to
-// date and factors it into the other LDS buffer (look-ahead), so the pivot chain overlaps the other
-// columns' updates.  Panels at or past the block's kb real rows only meet the identity padding and change
-// nothing, so the sweep ends there (steps past kb inside the last panel leave the real rows unchanged).
-constexpr int CW = 16, PB = 4;
-// Steps K .. KE - 1 of one panel in its owner wave (wave K / CW); multipliers of step K into sp[K % PB].
-template <int K, int KE, int R>
-__device__ __forceinline__ void chol_panel_steps(double (&c)[R][CW], double (*sp)[64 * R], int i, int kb, int& bad) {
-  if constexpr (K < KE) {
-    constexpr int k = K % CW;
-    double d = readlane_f64(c[K / 64][k], K % 64);
-    if (!(d > 0.0)) {
-      if (K < kb && bad == 0) bad = K + 1;
-      d = 1e-300;
-    }
-    // 1/sqrt(d): the hardware estimate and two Newton steps y += (y/2)(1 - d y^2) (each squares the
-    // relative error; within an ulp or so of the rounded quotient), sqrt(d) = d / sqrt(d); far shorter
-    // than a correctly rounded square root followed by a division on this step's critical path
-    double inv = __builtin_amdgcn_rsq(d);
-#pragma unroll
-    for (int it = 0; it < 2; ++it) inv = fma(0.5 * inv, fma(-d * inv, inv, 1.0), inv);
-    const double sd = d * inv;
-    double sv[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int row = i + 64 * r;
-      sv[r] = (row == K) ? 0.0 : c[r][k] * inv;
-      c[r][k] = (row == K) ? sd : sv[r];
-      sp[K % PB][row] = sv[r];
-    }
+// The block lies in the matrix-core accumulators of four waves, and the sweep goes in panels of 4 columns, the K of one
+// MFMA (chol_panels): a panel passes through LDS, every wave factors it for itself, row i in its lane i, and each
+// takes the panel's four updates of its accumulators as one product S S^T of the multipliers per 16 columns, the
+// next panel's columns first.  One barrier per panel; no update is on the vector units but those inside a panel.
+constexpr int PB = 4;
+// Steps K .. of the panel at column `first`; the multipliers of step K are left in s[K].
+template <int K>
+__device__ __forceinline__ void chol_panel_steps(double (&c)[PB], double (&s)[PB], int first, int i, int kb, int& bad) {
+  if constexpr (K < PB) {
+    const int at = first + K;
+    const double pivot = readlane_f64(c[K], at);
+    const double d = fmax(pivot, 4.9406564584124654e-324);   // finite whatever the pivot; `bad` says so below
+    // 1/sqrt(d): the hardware estimate y (relative error below 2^-22) and one step of third order in e = 1 - d y^2,
+    // y + y e (1/2 + 3 e / 8), which leaves e^3 and rounding (within an ulp or so of the rounded quotient);
+    // sqrt(d) = d / sqrt(d); far shorter than a correctly rounded square root followed by a division on this step's
+    // critical path
+    const double y = __builtin_amdgcn_rsq(d);
+    const double e = fma(-d * y, y, 1.0);
+    const double inv = fma(y * e, fma(0.375, e, 0.5), y);
+    const double u = c[K] * inv;
+    s[K] = (i == at) ? 0.0 : u;
+    c[K] = (i == at) ? d * inv : s[K];
     // this step on the panel's later columns j (row j's multiplier from its lane)
 #pragma unroll
-    for (int j = K + 1; j < KE; ++j) {
-      const double sj = readlane_f64(sv[j / 64], j % 64);
-#pragma unroll
-      for (int r = 0; r < R; ++r) c[r][j % CW] -= sv[r] * sj;
-    }
-    chol_panel_steps<K + 1, KE, R>(c, sp, i, kb, bad);
+    for (int j = K + 1; j < PB; ++j) c[j] -= s[K] * readlane_f64(u, first + j);
+    chol_panel_steps<K + 1>(c, s, first, i, kb, bad);
+    if (!(pivot > 0.0) && at < kb) bad = at + 1;     // the first of a panel last
   }
 }
 
-// Panel K0 .. K0 + PB - 1 (its multipliers already in sbuf[(K0 / PB) & 1]) applied past the panel.
-template <int K0, int R>
-__device__ __forceinline__ void chol_inv_panels(double (&c)[R][CW], double (*sbuf)[PB][64 * R], int w, int i, int kb, int& bad) {
-  if constexpr (K0 < 64 * R) {
-    if (K0 >= kb) return;
-    constexpr int o = K0 / CW, k0 = K0 % CW;
-    constexpr bool ahead = K0 + PB < 64 * R;
-    constexpr int K1 = ahead ? K0 + PB : 0, o1 = K1 / CW, k1 = K1 % CW;
+constexpr int CLD = CB + 2;   // LDS row of a 64 x 64 tile: 16 rows x 2 k of a half wave's MFMA operand hit all 64 banks
+typedef double CholTile[CB * CLD];
+typedef double CholPanel[CB * PB];
+constexpr int CHOL_PANELS = 6;      // in LDS: two in turn that the waves share, one of each wave
+
+// Panel P (columns PB P ..) to LDS
+template <int P>
+__device__ __forceinline__ void panel_publish(CholPanel* pan, const f64x4 (&acc)[4], int w, int lane) {
+  if (((lane & 15) / PB) == P % 4)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) pan[P & 1][(16 * w + 4 * r + (lane >> 4)) * PB + lane % PB] = acc[P / 4][r];
+}
+
+// Panel P, published, and the ones after it; row i's results to s.
+template <int P>
+__device__ __forceinline__ void chol_panels(f64x4 (&acc)[4], CholTile& s, CholPanel* pan, int w, int lane, int kb, int& bad) {
+  if constexpr (P < CB / PB) {
+    if (P * PB >= kb) return;
     __syncthreads();
-    double (*sp)[64 * R] = sbuf[(K0 / PB) & 1];
-    if (w >= o) {
-      double si[PB][R];
+    double c[PB], m[PB];
 #pragma unroll
-      for (int kk = 0; kk < PB; ++kk)
+    for (int j = 0; j < PB; ++j) c[j] = pan[P & 1][lane * PB + j];
+    int failed = 0;
+    chol_panel_steps<0>(c, m, P * PB, lane, kb, failed);
+    bad = bad ? bad : failed;
+    double* own = pan[2 + w];     // read back by this wave alone
 #pragma unroll
-        for (int r = 0; r < R; ++r) si[kk][r] = sp[kk][i + 64 * r];
-      if (ahead && w == o1) {
+    for (int j = 0; j < PB; ++j) own[lane * PB + j] = m[j];
+    if (w == P % 4)
 #pragma unroll
-        for (int jj = k1; jj < k1 + PB; ++jj)
+      for (int j = 0; j < PB; ++j) s[lane * CLD + P * PB + j] = c[j];
+    if constexpr (P + 1 < CB / PB) {
+      const double a = -own[(16 * w + (lane & 15)) * PB + (lane >> 4)];
 #pragma unroll
-          for (int kk = 0; kk < PB; ++kk) {
-            const double sj = sp[kk][CW * o1 + jj];
-#pragma unroll
-            for (int r = 0; r < R; ++r) c[r][jj] -= si[kk][r] * sj;
-          }
-        if constexpr (ahead) chol_panel_steps<K1, K1 + PB, R>(c, sbuf[(K1 / PB) & 1], i, kb, bad);
+      for (int t = (P + 1) / 4; t < 4; ++t) {
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, own[(16 * t + (lane & 15)) * PB + (lane >> 4)], acc[t], 0, 0, 0);
+        if (t == (P + 1) / 4) panel_publish<P + 1>(pan, acc, w, lane);
       }
-      // this wave's columns past the panel, less the next panel's when the look-ahead took them
-      const double* sw = &sp[0][0] + CW * w;
-      const int j0 = (w == o) ? k0 + PB : 0;
-#pragma unroll
-      for (int jj = 0; jj < CW; ++jj)
-        if (jj >= j0 && !(ahead && w == o1 && jj >= k1 && jj < k1 + PB)) {
-#pragma unroll
-          for (int kk = 0; kk < PB; ++kk) {
-            const double sj = sw[kk * 64 * R + jj];
-#pragma unroll
-            for (int r = 0; r < R; ++r) c[r][jj] -= si[kk][r] * sj;
-          }
-        }
     }
-    chol_inv_panels<K0 + PB, R>(c, sbuf, w, i, kb, bad);
+    chol_panels<P + 1>(acc, s, pan, w, lane, kb, bad);
   }
 }
 
-// Cholesky and inverse of one diagonal block of at most 64R x 64R (see chol_inv_panels): A's block at
-// (k0, k0) (lower triangle read; rows >= kb padded with the identity) is replaced by L with its upper
-// triangle zeroed, X's block at (x0, x0) receives L^-1, info the first non-positive pivot (1-based,
-// global index).
-template <int R>
-__global__ void __launch_bounds__(256 * R) chol_leaf_kernel(int64_t lda, int64_t k0, int kb, double* __restrict__ A,
-                                                         double* __restrict__ X, int64_t ldx, int64_t x0,
-                                                         int* __restrict__ info) {
-  constexpr int BN = 64 * R, NW = BN / CW;
-  __shared__ double Ls[BN][BN + 1];
-  __shared__ double sbuf[2][PB][BN];
-  __shared__ int badw[NW];
+// Factors and inverts a diagonal block of kb rows held in the accumulators of four waves (wave w: row 16 w + 4 r +
+// lane / 16, column 16 t + lane % 16 of acc[t][r]; symmetric, anything past kb): L (upper triangle zero) to A, L^-1
+// to X, each with its leading dimension; returns the block's first failing pivot in every thread (1-based, 0: none).
+// s and pan are scratch.  A dependent chain of 64 pivots.
+__device__ __forceinline__ int chol_block(f64x4 (&acc)[4], CholTile& s, CholPanel* pan, int kb, double* __restrict__ A,
+                                          int64_t lda, double* __restrict__ X, int64_t ldx) {
   const int i = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  double c[R][CW];
-  // row i + 64r of the lower triangle, then its column mirrored into j > row (identity past kb); every
-  // load index clamped into the block
+  if (kb < CB) {      // the identity past kb
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int row = i + 64 * r, rc = row < kb ? row : 0;
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int jj = 0; jj < CW; ++jj) {
-      const int j = CW * w + jj, jc = j < kb ? j : 0;
-      const double v = A[(k0 + (j <= row ? rc : jc)) * lda + k0 + (j <= row ? jc : rc)];
-      c[r][jj] = (row < kb && j < kb) ? v : (row == j ? 1.0 : 0.0);
-    }
-  }
-  int bad = 0;  // first failing pivot among this wave's columns
-  if (w == 0) chol_panel_steps<0, PB, R>(c, sbuf[0], i, kb, bad);
-  chol_inv_panels<0, R>(c, sbuf, w, i, kb, bad);
-  if (i == 0) badw[w] = bad;
-#pragma unroll
-  for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int jj = 0; jj < CW; ++jj) Ls[i + 64 * r][CW * w + jj] = c[r][jj];
-  __syncthreads();
-  if (threadIdx.x == 0 && *info == 0)
-    for (int v = 0; v < NW; ++v)
-      if (badw[v]) {
-        *info = (int)(k0 + badw[v]);
-        break;
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * w + 4 * r + (i >> 4), col = 16 * t + (i & 15);
+        if (row >= kb || col >= kb) acc[t][r] = row == col ? 1.0 : 0.0;
       }
-  for (int rr = w; rr < kb; rr += NW)
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int col = i + 64 * r;
-      if (col < kb) A[(k0 + rr) * lda + k0 + col] = (col <= rr) ? Ls[rr][col] : 0.0;
-    }
+  }
+  int bad = 0;  // first failing pivot, the same in every wave
+  panel_publish<0>(pan, acc, w, i);
+  chol_panels<0>(acc, s, pan, w, i, kb, bad);
+  __syncthreads();
   // X[m][row] = -c_row[m] / d_row below the diagonal, 1 / L[row][row] on it
+  const double xd = 1.0 / s[i * CLD + i], rd = -xd * xd;
+  double l[16], x[16];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int row = i + 64 * r;
-    if (row < kb) {
-      const double xd = 1.0 / Ls[row][row], rd = -xd * xd;
-      for (int m = w; m < kb; m += NW) X[(x0 + m) * ldx + x0 + row] = (m > row) ? Ls[row][m] * rd : (m == row ? xd : 0.0);
+  for (int r = 0; r < 16; ++r) {
+    l[r] = s[(w + 4 * r) * CLD + i];
+    x[r] = s[i * CLD + w + 4 * r];
+  }
+  A += (int64_t)w * lda + i;
+  X += (int64_t)w * ldx + i;
+#pragma unroll
+  for (int r = 0; r < 16; ++r, A += 4 * lda, X += 4 * ldx) {
+    const int m = w + 4 * r;
+    if (m < kb && i < kb) {
+      *A = (i <= m) ? l[r] : 0.0;
+      *X = (m > i) ? x[r] * rd : (m == i ? xd : 0.0);
     }
   }
+  return bad;
+}
+
+// Tiles in the accumulators of four waves: row 16 w + lane / 16 + 4 r, column 16 t + lane % 16 of acc[t][r].  Every
+// access of a thread is one address that advances by four rows, clamped at the edge rather than skipped: loads under a
+// condition wait for one another, and a 64-bit product per element costs more than the load.
+// The 64 x 64 tile at p, rows x cols of it, zero past them.
+__device__ __forceinline__ void tile_to_acc(f64x4 (&acc)[4], const double* p, int64_t ld, int rows, int cols, int w, int lane) {
+  const int i0 = 16 * w + (lane >> 4), j0 = lane & 15;
+  p += (int64_t)(i0 < rows ? i0 : rows - 1) * ld;
+  int j[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) j[t] = j0 + 16 * t < cols ? j0 + 16 * t : cols - 1;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t][r] = p[j[t]];
+    p += i0 + 4 * (r + 1) < rows ? 4 * ld : 0;
+  }
+  if (rows < CB || cols < CB) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[t][r] = (i0 + 4 * r < rows && j0 + 16 * t < cols) ? acc[t][r] : 0.0;
+  }
+}
+// The same for a symmetric tile of kb rows whose lower triangle is read.
+__device__ __forceinline__ void tile_to_acc_lower(f64x4 (&acc)[4], const double* p, int64_t ld, int kb, int w, int lane) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 16 * w + 4 * r + (lane >> 4), j = 16 * t + (lane & 15);
+      const int row = i > j ? i : j, col = i > j ? j : i;
+      acc[t][r] = p[(int64_t)(row < kb ? row : kb - 1) * ld + (col < kb ? col : kb - 1)];
+    }
+}
+__device__ __forceinline__ void tile_write_acc(const f64x4 (&acc)[4], double* p, int64_t ld, int rows, int cols, int w, int lane) {
+  const int i0 = 16 * w + (lane >> 4), j0 = lane & 15;
+  p += (int64_t)i0 * ld + j0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r, p += 4 * ld)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (i0 + 4 * r < rows && j0 + 16 * t < cols) p[16 * t] = acc[t][r];
+}
+
+// Cholesky and inverse of one diagonal block of at most 64 x 64 rows (lower triangle read): A's block at (k0, k0) is
+// replaced by L with its upper triangle zeroed, X receives L^-1, info the first non-positive pivot (1-based, global
+// index; `begin`: info is set, else only where no earlier block failed).
+__global__ void __launch_bounds__(256) chol_leaf_kernel(int64_t lda, int64_t k0, int kb, double* __restrict__ A,
+                                                        double* __restrict__ X, int64_t ldx, int* __restrict__ info, int begin) {
+  __shared__ CholTile s;
+  __shared__ __attribute__((aligned(16))) CholPanel pan[CHOL_PANELS];
+  double* Ak = A + k0 * lda + k0;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  f64x4 acc[4];
+  tile_to_acc_lower(acc, Ak, lda, kb, w, lane);
+  const int bad = chol_block(acc, s, pan, kb, Ak, lda, X, ldx);
+  if (threadIdx.x == 0 && (begin || (*info == 0 && bad))) *info = bad ? (int)(k0 + bad) : 0;
+}
+
+// A 64 x 64 tile at p in registers (element r of a thread: row tid / 64 + 4 r, column tid % 64; `trans`: the tile's
+// transpose), zero past `rows` and `cols` of the tile as stored; then to LDS.
+__device__ __forceinline__ void tile_load(double (&v)[16], const double* __restrict__ p, int64_t ld, int rows, int cols, int tid) {
+  const int c = tid & 63, r0 = tid >> 6;
+  p += (int64_t)(r0 < rows ? r0 : rows - 1) * ld + (c < cols ? c : cols - 1);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    v[r] = *p;
+    p += r0 + 4 * (r + 1) < rows ? 4 * ld : 0;
+  }
+  if (rows < CB || cols < CB) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = (r0 + 4 * r < rows && c < cols) ? v[r] : 0.0;
+  }
+}
+template <bool TRANS>
+__device__ __forceinline__ void tile_store(CholTile& s, const double (&v)[16], int tid) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int row = (tid >> 6) + 4 * r, c = tid & 63;
+    s[TRANS ? c * CLD + row : row * CLD + c] = v[r];
+  }
+}
+
+// acc = S T^T of two tiles in LDS; wave w takes rows 16 w .. 16 w + 15.  LOWER: T is lower triangular, so column tile t
+// sums over its first 16 (t + 1) indices only.
+template <bool LOWER>
+__device__ __forceinline__ void tile_product(f64x4 (&acc)[4], const CholTile& S, const CholTile& T, int w, int lane) {
+  const int row = lane & 15, k4 = lane >> 4;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) acc[t] = (f64x4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int kk = 0; kk < CB; kk += 4) {
+    const double a = S[(16 * w + row) * CLD + kk + k4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      if (!LOWER || kk < 16 * (t + 1))
+        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, T[(16 * t + row) * CLD + kk + k4], acc[t], 0, 0, 0);
+  }
+}
+__device__ __forceinline__ void tile_from_acc(CholTile& s, const f64x4 (&acc)[4], int w, int lane) {
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s[(16 * w + 4 * r + (lane >> 4)) * CLD + 16 * t + (lane & 15)] = acc[t][r];
+}
+// s transposed to the 64 x 64 tile at p (rows x cols of it exist)
+__device__ __forceinline__ void tile_write_transposed(const CholTile& s, double* __restrict__ p, int64_t ld, int rows, int cols, int tid) {
+  const int c = tid & 63;
+  double v[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) v[r] = s[c * CLD + (tid >> 6) + 4 * r];
+  p += (int64_t)(tid >> 6) * ld + c;
+#pragma unroll
+  for (int r = 0; r < 16; ++r, p += 4 * ld)
+    if (c < cols && (tid >> 6) + 4 * r < rows) *p = v[r];
+}
+
+// Step k of A = L L^T with X = L^-1, in blocks of 64, once block k of the diagonal is factored (L_kk, X_kk stored).
+// The rows of A are extended by those of the identity, which elimination turns into L^-T:
+//   [A; 1] L^-T = [L; L^-T].
+// Row blocks M_s of the extended matrix (s > k of A, s <= k of the identity, whose parts so far are held in X's upper
+// triangle) and column blocks i > k: M(s, i) -= (M(s, k) X_kk^T) (A(i, k) X_kk^T)^T.  Each workgroup updates one such
+// tile and makes both factors itself, so a step is one launch, and the workgroup of the next diagonal block goes on to
+// factor it: the chain per step is two tile products and a 64 x 64 factorization.  Finished column blocks go where nothing
+// is read any more: L(i, k)^T to A's upper triangle, X(k, j) to X's lower one; chol_finish_kernel moves the former
+// into place.
+// Latency-bound, 17 us a step: 9 us for the 64 pivots (335 cycles each), 3.2 us for the two products on one CU, 2.5 us
+// for the loads (10 us with a 64-bit product per element's address), 1.3 us for the results.  n = 256 / 625 / 1296 /
+// 2592 / 4096: 74 / 181 / 380 / 1070 / 2920 us, against 107 / 311 / 757 / 1940 / 4160 us for a recursion with leaves of
+// 128 rows on one workgroup (39 us each), four products around each and a copy.  The three products per tile
+// instead of one cost nothing while a step's tiles fit the chip (n <= 1400), and less than the recursion's small
+// products beyond.
+__global__ void __launch_bounds__(256) chol_step_kernel(int64_t n, int k, int blocks, double* __restrict__ A, double* __restrict__ X,
+                                                        int* __restrict__ info) {
+  __shared__ __attribute__((aligned(16))) CholTile sa;
+  __shared__ CholTile sx;
+  CholPanel* pan = reinterpret_cast<CholPanel*>(sa);    // sa is free once the next diagonal block is factored
+  static_assert(CHOL_PANELS * CB * PB <= CB * CLD, "the panels in one tile");
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // tiles in order: A's lower triangle of the m blocks left (the next diagonal block first), the identity's rows
+  // (j <= k) x the m columns, then the finished blocks X(k, j), j < k
+  const int m = blocks - 1 - k, lower = m * (m + 1) / 2;
+  int b = blockIdx.x, s = 0, i = 0, kind = 0;   // 0: A's rows, 1: the identity's, 2: finished X(k, s)
+  if (b < lower) {
+    while (b > s) b -= ++s;   // row s, column b <= s
+    i = k + 1 + b;
+    s += k + 1;
+  } else if ((b -= lower) < m * (k + 1)) {
+    kind = 1;
+    s = b / m;
+    i = k + 1 + b % m;
+  } else {
+    kind = 2;
+    s = b - m * (k + 1);
+  }
+  const int64_t k0 = (int64_t)k * CB, s0 = (int64_t)s * CB, i0 = (int64_t)i * CB;
+  auto left = [&](int64_t at) { return (int)(n - at < CB ? n - at : CB); };
+  const int kb = left(k0), sb = left(s0), ib = kind == 2 ? 0 : left(i0);
+  const bool diagonal = kind == 0 && s == i;
+  const double* Xk = X + k0 * n + k0;
+  double vx[16], vi[16], vs[16];
+  tile_load(vx, Xk, n, kb, kb, tid);
+  if (kind != 2) tile_load(vi, A + i0 * n + k0, n, ib, kb, tid);
+  if (kind == 0) { if (!diagonal) tile_load(vs, A + s0 * n + k0, n, sb, kb, tid); }
+  else if (s != k) tile_load(vs, X + s0 * n + k0, n, sb, kb, tid);
+  // the tile itself, as the products leave it (row 16 w + 4 r + lane / 16, column 16 t + lane % 16)
+  double* M = (kind == 0 ? A : X) + s0 * n + i0;
+  f64x4 out[4];
+  const bool fresh = kind == 1 && s == k;      // the identity's row k: nothing there yet
+  if (diagonal && k == 0) {
+    tile_to_acc_lower(out, M, n, sb, w, lane);    // the caller's; written back with both triangles
+  } else if (kind != 2 && !fresh) {
+    tile_to_acc(out, M, n, sb, ib, w, lane);
+  } else {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) out[t] = (f64x4){0.0, 0.0, 0.0, 0.0};
+  }
+  tile_store<false>(sx, vx, tid);
+  if (kind != 2) tile_store<false>(sa, vi, tid);
+  else tile_store<false>(sa, vs, tid);
+  __syncthreads();
+  f64x4 p[4], q[4];
+  tile_product<true>(p, sa, sx, w, lane);      // L(i, k); kind 2: the finished block, X(k, s)^T
+  if (kind == 2) {
+    __syncthreads();
+    tile_from_acc(sa, p, w, lane);
+    __syncthreads();
+    tile_write_transposed(sa, X + k0 * n + s0, n, kb, sb, tid);
+    return;
+  }
+  if (!diagonal && !fresh) {
+    __syncthreads();
+    tile_store<false>(sa, vs, tid);
+    __syncthreads();
+    tile_product<true>(q, sa, sx, w, lane);
+  }
+  __syncthreads();
+  tile_from_acc(sa, p, w, lane);
+  if (fresh) tile_store<true>(sx, vx, tid);    // X_kk^T
+  else if (!diagonal) tile_from_acc(sx, q, w, lane);
+  __syncthreads();
+  f64x4 d[4];
+  tile_product<false>(d, diagonal ? sa : sx, sa, w, lane);
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[t][r] -= d[t][r];
+  if (diagonal && i == k + 1) {
+    __syncthreads();   // sa has been read
+    const int bad = chol_block(out, sx, pan, ib, M, n, X + i0 * n + i0, n);
+    if (tid == 0 && bad && *info == 0) *info = (int)(i0 + bad);
+    return;
+  }
+  tile_write_acc(out, M, n, sb, ib, w, lane);
+  if (fresh) tile_write_transposed(sa, A + k0 * n + i0, n, kb, ib, tid);   // L(i, k)^T
+}
+
+// L's blocks below the diagonal from A's upper triangle, whose blocks and X's are then zero.  32 x 32 tiles; those of
+// the diagonal 64 x 64 blocks are in place.
+__global__ void __launch_bounds__(256) chol_finish_kernel(int64_t n, double* __restrict__ A, double* __restrict__ X) {
+  __shared__ double tile[32][33];
+  if (blockIdx.x / 2 <= blockIdx.y / 2) return;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int64_t c = (int64_t)blockIdx.x * 32, r = (int64_t)blockIdx.y * 32;
+#pragma unroll
+  for (int k = 0; k < 32; k += 8)
+    if (c + tx < n) {   // rows r .. r + 31 lie above c, so they exist
+      const int64_t at = (r + ty + k) * n + c + tx;
+      tile[ty + k][tx] = A[at];
+      A[at] = X[at] = 0.0;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 32; k += 8)
+    if (c + ty + k < n) A[(c + ty + k) * n + r + tx] = tile[tx][ty + k];
 }
 
 // Column sweep of L x = e_j, steps Q..CB-1: x[Q] *= 1/L[Q][Q], then x[m] -= L[m][Q] x[Q] for m > Q.
@@ -253,8 +455,6 @@ __global__ void copy2d_kernel(int64_t rows, int64_t cols, const double* __restri
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < rows * cols; e += (int64_t)gridDim.x * blockDim.x)
     dst[(e / cols) * ldd + e % cols] = src[(e / cols) * lds + e % cols];
 }
-
-__global__ void set_int_kernel(int* p, int v) { *p = v; }
 
 // Zero the strict upper triangle.
 __global__ void zero_upper_kernel(int64_t n, double* __restrict__ A) {
@@ -331,41 +531,6 @@ __global__ void __launch_bounds__(256) transpose_kernel(int64_t n, const double*
 // Split of a diagonal range of sz > CB rows at a block boundary near its middle.
 inline int64_t split_rows(int64_t sz) { return ((sz + CB - 1) / CB / 2) * CB; }
 
-// Recursive Cholesky with inverse of the diagonal range [off, off + sz) of A (leading dimension n):
-//   (L11, X11) = chol_inv(A11); L21 = A21 X11^T; A22 -= L21 L21^T; (L22, X22) = chol_inv(A22);
-//   X21 = -X22 (L21 X11).
-// The GEMMs have the full K of each level (not the block width), so they fill the chip; leaves are
-// chol_leaf_kernel (blocks of up to 128 rows, split at multiples of 128).  tmp holds n1 x n2 <= sz^2 / 4
-// doubles.
-int chol_inv_rec(void* stream, int64_t n, int64_t off, int64_t sz, double* A, double* X, double* tmp, int* info) {
-  hipStream_t st = cc_stream(stream);
-  if (sz <= 2 * CB) {
-    if (sz <= CB) chol_leaf_kernel<1><<<1, 256, 0, st>>>(n, off, (int)sz, A, X, n, off, info);
-    else chol_leaf_kernel<2><<<1, 512, 0, st>>>(n, off, (int)sz, A, X, n, off, info);
-    CC_LAUNCH_CHECK();
-    return CC_OK;
-  }
-  const int64_t n1 = ((sz + 2 * CB - 1) / (2 * CB) / 2) * (2 * CB), n2 = sz - n1;
-  int rc = chol_inv_rec(stream, n, off, n1, A, X, tmp, info);
-  if (rc) return rc;
-  double* A21 = A + (off + n1) * n + off;
-  double* A22 = A21 + n1;
-  const double* X11 = X + off * n + off;
-  double* X21 = X + (off + n1) * n + off;
-  const double* X22 = X21 + n1;
-  rc = cc_gemm_f64(stream, 1, n2, n1, n1, 1.0, A21, 0, n, 1, X11, 0, 1, n, 0.0, tmp, 0, n1, 1);
-  if (rc) return rc;
-  copy2d_kernel<<<cc_blocks(n2 * n1, 256), 256, 0, st>>>(n2, n1, tmp, n1, A21, n);
-  CC_LAUNCH_CHECK();
-  rc = cc_gemm_f64(stream, 1, n2, n2, n1, -1.0, A21, 0, n, 1, A21, 0, 1, n, 1.0, A22, 0, n, 1);
-  if (rc) return rc;
-  rc = chol_inv_rec(stream, n, off + n1, n2, A, X, tmp, info);
-  if (rc) return rc;
-  rc = cc_gemm_f64(stream, 1, n2, n1, n1, 1.0, A21, 0, n, 1, X11, 0, n, 1, 0.0, tmp, 0, n1, 1);
-  if (rc) return rc;
-  return cc_gemm_f64(stream, 1, n2, n1, n2, -1.0, X22, 0, n, 1, tmp, 0, n1, 1, 0.0, X21, 0, n, 1);
-}
-
 // Recursive inverse of the lower-triangular range [off, off + sz) of L: X11, X22 recursively, then
 // X21 = -X22 (L21 X11); leaves are tri_leaf_kernel.
 int trtri_rec(void* stream, int64_t n, int64_t off, int64_t sz, const double* L, double* X, double* tmp) {
@@ -402,11 +567,9 @@ extern "C" int cc_cholesky_f64(void* stream, int64_t n, double* A, int* info_dev
   hipStream_t st = cc_stream(stream);
   double* dinv = work;
   double* tmp = work + CB * CB;
-  set_int_kernel<<<1, 1, 0, st>>>(info_dev, 0);
-  CC_LAUNCH_CHECK();
   for (int64_t k0 = 0; k0 < n; k0 += CB) {
     int kb = (int)((n - k0) < CB ? (n - k0) : CB);
-    chol_leaf_kernel<1><<<1, 256, 0, st>>>(n, k0, kb, A, dinv, kb, 0, info_dev);
+    chol_leaf_kernel<<<1, 256, 0, st>>>(n, k0, kb, A, dinv, kb, info_dev, k0 == 0);
     CC_LAUNCH_CHECK();
     int64_t rest = n - k0 - kb;
     if (rest > 0) {
@@ -426,17 +589,23 @@ extern "C" int cc_cholesky_f64(void* stream, int64_t n, double* A, int* info_dev
   return CC_OK;
 }
 
-// A = L L^T in place (upper zeroed) and X = L^-1 (upper zero) in one recursive pass.
+// A = L L^T in place (upper zeroed) and X = L^-1 (upper zero) in one pass over the block columns (chol_step_kernel).
 extern "C" int cc_cholesky_inverse_f64(void* stream, int64_t n, double* A, double* X, int* info_dev, double* work) {
+  (void)work;
   if (n <= 0) { cc_set_last_error("cholesky_inverse: n must be positive"); return CC_ERR_ARG; }
+  const int64_t blocks = (n + CB - 1) / CB;
+  if (blocks > 32767) { cc_set_last_error("cholesky_inverse: matrix too large"); return CC_ERR_UNSUPPORTED; }
   hipStream_t st = cc_stream(stream);
-  set_int_kernel<<<1, 1, 0, st>>>(info_dev, 0);
+  chol_leaf_kernel<<<1, 256, 0, st>>>(n, 0, (int)(n < CB ? n : CB), A, X, n, info_dev, 1);
   CC_LAUNCH_CHECK();
-  int rc = cc_fill_f64(stream, n * n, 0.0, X);
-  if (rc) return rc;
-  rc = chol_inv_rec(stream, n, 0, n, A, X, work, info_dev);
-  if (rc) return rc;
-  zero_upper_kernel<<<cc_blocks(n * n, 256), 256, 0, st>>>(n, A);
+  if (blocks == 1) return CC_OK;
+  for (int k = 0; k < (int)blocks; ++k) {
+    const int64_t m = blocks - 1 - k, tiles = m * (m + 1) / 2 + m * (k + 1) + k;
+    chol_step_kernel<<<(unsigned)tiles, 256, 0, st>>>(n, k, (int)blocks, A, X, info_dev);
+    CC_LAUNCH_CHECK();
+  }
+  const unsigned t32 = (unsigned)((n + 31) / 32);
+  chol_finish_kernel<<<dim3(t32, t32), 256, 0, st>>>(n, A, X);
   CC_LAUNCH_CHECK();
   return CC_OK;
 }

@@ -79,6 +79,34 @@ def test_cholesky_inverse_recursive(gpu):
             assert int(info.item()) == bad, (name, n, bad, int(info.item()))
 
 
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 129, 192, 321, 1345])
+def test_cholesky_inverse_blocks(gpu, n):
+    """cc_cholesky_inverse_f64 at the edges of its 64-row blocks (and past one tile per CU): only the lower triangle is
+    read (NaN above it) and the first failing pivot is reported, also with later ones.  N = g g^T / n + 1 / 2 has a
+    condition number below 10, so L and X are good to 64 n eps."""
+    from carcassonne_amd import _lib
+    from carcassonne_amd.device import ptr, stream
+    rng = np.random.default_rng(n)
+    g = rng.standard_normal((n, n))
+    a = g @ g.T / n + 0.5 * np.eye(n)
+    lower = np.tril(a) + np.triu(np.full((n, n), np.nan), 1)
+    A, X = torch.from_numpy(lower).cuda(), torch.full((n, n), np.nan, dtype=torch.float64, device="cuda")
+    info, work = torch.full((1,), 9, dtype=torch.int32, device="cuda"), torch.empty(0, dtype=torch.float64, device="cuda")
+    _lib.call("cc_cholesky_inverse_f64", stream(), n, ptr(A), ptr(X), ptr(info), ptr(work))
+    L, Xh, want = A.cpu().numpy(), X.cpu().numpy(), np.linalg.cholesky(a)
+    assert int(info.item()) == 0
+    tol = 64 * max(n, 8) * np.finfo(float).eps
+    assert np.abs(L - want).max() < tol * np.abs(want).max()
+    assert np.abs(Xh @ want - np.eye(n)).max() < tol
+    assert not np.triu(L, 1).any() and not np.triu(Xh, 1).any()
+    for bad in {1, (n + 1) // 2, n}:
+        m = lower.copy()
+        m[bad - 1, bad - 1] = m[n - 1, n - 1] = -1.0
+        A = torch.from_numpy(m).cuda()
+        _lib.call("cc_cholesky_inverse_f64", stream(), n, ptr(A), ptr(X), ptr(info), ptr(work))
+        assert int(info.item()) == bad
+
+
 @pytest.mark.parametrize("D,chi,model,seed", [(2, 8, "ising", 0), (3, 6, "heisenberg", 1), (4, 8, "ising", 2),
                                               (4, 16, "heisenberg", 3)])
 def test_lanczos_matches_generalized_eigh(gpu, D, chi, model, seed):
