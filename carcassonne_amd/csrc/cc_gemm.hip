@@ -19,7 +19,8 @@ struct GemmArgs {
   const double* B; int64_t sBb, sBk, sBn;
   double* C; int64_t sCb, sCm, sCn;
   int64_t batch0;
-  int upper;   // B is upper triangular: columns up to n0 + T - 1 of C take k < n0 + T only
+  // > 0: B is upper triangular (columns up to n0 + T - 1 of C take k < n0 + T only); tiles per dimension, one-dimensional grid
+  unsigned upper, batches;
 };
 
 // The operand tile of one K step (T rows or columns x BK) in LDS, in the order its loader writes without
@@ -48,10 +49,20 @@ __global__ void __launch_bounds__(256) gemm_f64_kernel(GemmArgs g) {
   __shared__ double Bs[2][TB::SIZE];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wr = wave >> 1, wc = wave & 1;
-  const int64_t bz = g.batch0 + blockIdx.z;
+  int64_t bz = g.batch0 + blockIdx.z, m0 = (int64_t)blockIdx.y * T, n0 = (int64_t)blockIdx.x * T;
+  if (g.upper) {
+    // Tiles of the last columns have the longest sums.  They are dealt out to 256 CUs from the longest down and back
+    // again, so that the tiles a CU holds at once add up to the same everywhere; in the order of a plain grid some CUs had
+    // two thirds more than the mean.  Both products of one / two / four matrices of 1296 rows: 178 / 274 / 515 -> 149 /
+    // 233 / 423 us.
+    const unsigned t = g.upper, per_col = t * g.batches, at = blockIdx.x % 256, round = blockIdx.x - at;
+    const unsigned width = gridDim.x - round < 256 ? gridDim.x - round : 256;
+    const unsigned rank = round + (round / 256 % 2 ? width - 1 - at : at);
+    bz = rank % per_col / t;
+    m0 = (int64_t)(rank % t) * T;
+    n0 = (int64_t)(t - 1 - rank / per_col) * T;
+  }
   double* C = g.C + bz * g.sCb;
-  // an upper-triangular B: the last columns have the longest sums and start first
-  const int64_t m0 = (int64_t)blockIdx.y * T, n0 = (int64_t)(g.upper ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * T;
   const int64_t K = g.upper && n0 + T < g.K ? n0 + T : g.K;
 
   f64x4 acc[TM][TM];
@@ -155,7 +166,7 @@ extern "C" int cc_gemm_f64(void* stream, int64_t batch, int64_t M, int64_t N, in
                            double* C, int64_t sCb, int64_t sCm, int64_t sCn) {
   if (batch < 0 || M < 0 || N < 0 || K < 0) { cc_set_last_error("cc_gemm_f64: negative size"); return CC_ERR_ARG; }
   if (batch == 0 || M == 0 || N == 0) return CC_OK;
-  GemmArgs g{M, N, K, alpha, beta, A, sAb, sAm, sAk, B, sBb, sBk, sBn, C, sCb, sCm, sCn, 0, 0};
+  GemmArgs g{M, N, K, alpha, beta, A, sAb, sAm, sAk, B, sBb, sBk, sBn, C, sCb, sCm, sCn, 0, 0, 0};
   // 64-wide tiles unless that grid would leave most of the 256 CUs idle
   const int64_t tiles64 = ((N + 63) / 64) * ((M + 63) / 64) * batch;
   const int T = tiles64 < 160 ? 32 : 64;
@@ -177,12 +188,13 @@ extern "C" int cc_gemm_f64(void* stream, int64_t batch, int64_t M, int64_t N, in
 
 int cc_internal_gemm_upper(hipStream_t st, int64_t batch, int64_t n, const double* A, int64_t sAb, int64_t sAm, int64_t sAk,
                            const double* B, int64_t ldb, double* C, int64_t sCb) {
-  GemmArgs g{n, n, n, 1.0, 0.0, A, sAb, sAm, sAk, B, 0, ldb, 1, C, sCb, n, 1, 0, 1};
+  GemmArgs g{n, n, n, 1.0, 0.0, A, sAb, sAm, sAk, B, 0, ldb, 1, C, sCb, n, 1, 0, 0, (unsigned)batch};
   const int64_t tiles64 = ((n + 63) / 64) * ((n + 63) / 64) * batch;
   const int T = tiles64 < 160 ? 32 : 64;
   const int64_t t = (n + T - 1) / T;
-  if (t > 65535 || batch > 65535) { cc_set_last_error("gemm: matrix too large for one launch"); return CC_ERR_UNSUPPORTED; }
-  const dim3 grid((unsigned)t, (unsigned)t, (unsigned)batch);
+  if (batch > 65535 || t * t > 2147483647LL / batch) { cc_set_last_error("gemm: matrix too large for one launch"); return CC_ERR_UNSUPPORTED; }
+  g.upper = (unsigned)t;
+  const dim3 grid((unsigned)(t * t * batch));
   if (T == 32) launch_gemm<32>(g, grid, sAk == 1, true, st);
   else launch_gemm<64>(g, grid, sAk == 1, true, st);
   CC_LAUNCH_CHECK();

@@ -84,3 +84,18 @@ def test_formed_operator_follows_its_environment(gpu):
     _, theta, _, _ = solver.solve(x0)
     _, theta2, _, _ = GroundStateSolver(H2, N2).solve(x0)
     assert abs(theta - theta2) <= 1e-11 * abs(theta2)
+
+
+@pytest.mark.parametrize("n,count", [(1, 1), (32, 2), (33, 1), (65, 3), (513, 2), (700, 3)])
+def test_whitening_products(gpu, n, count):
+    """W G W^T for lower-triangular W over partial rounds of the tile order, 32- and 64-wide tiles: two sums of n products,
+    each within n eps of the sum of magnitudes."""
+    from carcassonne_amd import _lib
+    from carcassonne_amd.device import empty, ptr, stream
+    rng = np.random.default_rng(n)
+    G, W = rng.standard_normal((count, n, n)), np.tril(rng.standard_normal((n, n)))
+    g, wt = torch.from_numpy(G).cuda(), torch.from_numpy(np.ascontiguousarray(W.T)).cuda()
+    K, work = empty((count, n, n)), empty((count, n, n))
+    _lib.call("cc_whiten_f64", stream(), n, count, ptr(g), ptr(wt), ptr(K), ptr(work))
+    bound = 2 * (n + 2) * np.finfo(float).eps * (abs(W) @ abs(G) @ abs(W.T))
+    assert np.all(abs(K.cpu().numpy() - W @ G @ W.T) <= bound)
