@@ -118,17 +118,17 @@ __global__ void __launch_bounds__(256) lz_combine_normalize_kernel(int m, int64_
 // 11.5 us, n = 2592 (D = 6, chi = 64) 19.7 -> 15.3 us.
 
 // c[b] = Q_b . w, d[b] = Q_b . y for b < m; block m: w . w and w . y
-__global__ void __launch_bounds__(256) lz_coeff2_kernel(int64_t n, int m, const double* __restrict__ Q,
+__global__ void __launch_bounds__(256) lz_coeff2_kernel(int n, int m, const double* __restrict__ Q,
                                                         const double* __restrict__ w, const double* __restrict__ y,
                                                         double* __restrict__ c, double* __restrict__ d) {
   __shared__ double red[2][4];
   const double* q = (int)blockIdx.x == m ? w : Q + (int64_t)blockIdx.x * n;
   double aw = 0.0, ay = 0.0;
-  for (int64_t base = threadIdx.x; base < n; base += 256 * DOT_U) {
+  for (int base = threadIdx.x; base < n; base += 256 * DOT_U) {
     double x[DOT_U], u[DOT_U], v[DOT_U];
 #pragma unroll
     for (int k = 0; k < DOT_U; ++k) {   // clamped index, masked product
-      const int64_t i = base + 256 * k < n ? base + 256 * k : base;
+      const int i = base + 256 * k < n ? base + 256 * k : base;
       x[k] = q[i];
       u[k] = w[i];
       v[k] = y[i];
@@ -153,38 +153,44 @@ __global__ void __launch_bounds__(256) lz_coeff2_kernel(int64_t n, int m, const 
   }
 }
 
+// One round of loads for 160 vectors, the last terms' operands among them: with half as many in flight and those read
+// behind the barrier a step waits for two more rounds (a solve of 160 steps at
+// D = 6, chi = 64 5.29 -> 5.07 ms, at D = 4, chi = 32 2.52 -> 2.40 ms).
+constexpr int LZ_STEP_U = 10;
 // The step's combinations from c and d (m vectors before this one); w is replaced by the next candidate.  Block = 16
 // outputs x 16 basis slices, slice sums combined in a fixed order.
-__global__ void __launch_bounds__(256) lz_step_kernel(int m, int64_t n, double* __restrict__ Q, const double* __restrict__ c,
+__global__ void __launch_bounds__(256) lz_step_kernel(int m, int n, double* __restrict__ Q, const double* __restrict__ c,
                                                       const double* __restrict__ d, double* __restrict__ w,
                                                       const double* __restrict__ y, double* __restrict__ alpha,
                                                       double* __restrict__ beta) {
   __shared__ double red[2][16][16], sq[2][4];
   const int e = threadIdx.x & 15, slice = threadIdx.x >> 4;
-  const int64_t i = (int64_t)blockIdx.x * 16 + e;
+  const int i = blockIdx.x * 16 + e, ic = i < n ? i : n - 1;
+  const double wi = w[ic], yi = y[ic], ww = c[m], wy = d[m], last = c[m > 0 ? m - 1 : 0];   // ahead of the barrier
   double cc = 0.0, cd = 0.0;   // c . c and c . d over the block
   for (int j = threadIdx.x; j < m; j += 256) {
     cc += c[j] * c[j];
     cd += c[j] * d[j];
   }
   double ac = 0.0, ad = 0.0;
-  if (i < n)
-    for (int j0 = slice; j0 < m; j0 += 16 * LZ_U) {
-      double q[LZ_U], cj[LZ_U], dj[LZ_U];
+  for (int j0 = slice; j0 < m; j0 += 16 * LZ_STEP_U) {
+    double q[LZ_STEP_U], cj[LZ_STEP_U], dj[LZ_STEP_U];
+    const double* p = Q + (int64_t)j0 * n + ic;
 #pragma unroll
-      for (int u = 0; u < LZ_U; ++u) {   // clamped index, masked product
-        const int j = j0 + 16 * u < m ? j0 + 16 * u : j0;
-        q[u] = Q[(int64_t)j * n + i];
-        cj[u] = c[j];
-        dj[u] = d[j];
-      }
-#pragma unroll
-      for (int u = 0; u < LZ_U; ++u)
-        if (j0 + 16 * u < m) {
-          ac += cj[u] * q[u];
-          ad += dj[u] * q[u];
-        }
+    for (int u = 0; u < LZ_STEP_U; ++u) {   // clamped index, masked product
+      const int j = j0 + 16 * u < m ? j0 + 16 * u : j0;
+      q[u] = *p;
+      cj[u] = c[j];
+      dj[u] = d[j];
+      if (j0 + 16 * (u + 1) < m) p += (int64_t)16 * n;
     }
+#pragma unroll
+    for (int u = 0; u < LZ_STEP_U; ++u)
+      if (j0 + 16 * u < m) {
+        ac += cj[u] * q[u];
+        ad += dj[u] * q[u];
+      }
+  }
   red[0][slice][e] = ac;
   red[1][slice][e] = ad;
   cc = cc_wave_sum(cc);
@@ -194,9 +200,9 @@ __global__ void __launch_bounds__(256) lz_step_kernel(int m, int64_t n, double* 
     sq[1][threadIdx.x >> 6] = cd;
   }
   __syncthreads();
-  const double b2 = c[m] - (((sq[0][0] + sq[0][1]) + sq[0][2]) + sq[0][3]);
+  const double b2 = ww - (((sq[0][0] + sq[0][1]) + sq[0][2]) + sq[0][3]);
   const double b = b2 > 0.0 ? sqrt(b2) : 0.0, inv = b > 0.0 ? 1.0 / b : 0.0;
-  const double on = (d[m] - (((sq[1][0] + sq[1][1]) + sq[1][2]) + sq[1][3])) * inv;   // q_j . y
+  const double on = (wy - (((sq[1][0] + sq[1][1]) + sq[1][2]) + sq[1][3])) * inv;   // q_j . y
   if (slice == 0 && i < n) {
     double tc = 0.0, td = 0.0;
 #pragma unroll
@@ -204,12 +210,12 @@ __global__ void __launch_bounds__(256) lz_step_kernel(int m, int64_t n, double* 
       tc += red[0][k][e];
       td += red[1][k][e];
     }
-    const double q = (w[i] - tc) * inv;
+    const double q = (wi - tc) * inv;
     Q[(int64_t)m * n + i] = q;
-    w[i] = ((y[i] - td) - on * q) * inv;
+    w[i] = ((yi - td) - on * q) * inv;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *alpha = on * inv - (m > 0 ? c[m - 1] : 0.0);
+    *alpha = on * inv - (m > 0 ? last : 0.0);
     if (m > 0) *beta = b;
   }
 }
@@ -513,9 +519,9 @@ static int lanczos_driver(hipStream_t st, ApplyFn apply, const void* plan, int64
     if (delayed) {
       rc = op_whitened(st, apply, plan, wh, w, t1, t2, y);
       if (rc) return rc;
-      lz_coeff2_kernel<<<j + 1, 256, 0, st>>>(n, j, Q, w, y, c, dots);
+      lz_coeff2_kernel<<<j + 1, 256, 0, st>>>((int)n, j, Q, w, y, c, dots);
       CC_LAUNCH_CHECK();
-      lz_step_kernel<<<(unsigned)((n + 15) / 16), 256, 0, st>>>(j, n, Q, c, dots, w, y, alpha + j, beta + j - 1);
+      lz_step_kernel<<<(unsigned)((n + 15) / 16), 256, 0, st>>>(j, (int)n, Q, c, dots, w, y, alpha + j, beta + j - 1);
       CC_LAUNCH_CHECK();
     } else {
       rc = op_whitened(st, apply, plan, wh, qj, t1, t2, w);
