@@ -33,6 +33,10 @@ struct FormedRows {
   template <typename F>
   __device__ __forceinline__ void apply(const FormedPlan& f, int row0, F x, double* red, double* __restrict__ y) {
     const int n = f.n_env, wave = threadIdx.x >> 6;
+    // the identity's part, loaded with the rest rather than behind the barrier (160 steps at D = 6: 5.20 -> 5.14 ms)
+    const int k = threadIdx.x, r = row0 + (k >> 1), sp1 = k & 1;
+    double own = 0.0;
+    if (f.has_id && k < 2 * FORMED_ROWS && r < n) own = f.id[2 * sp1] * x(r, 0) + f.id[2 * sp1 + 1] * x(r, 1);
     double acc[NG][2];
 #pragma unroll
     for (int g = 0; g < NG; ++g) acc[g][0] = acc[g][1] = 0.0;
@@ -55,11 +59,6 @@ struct FormedRows {
       if ((threadIdx.x & 63) == 0) red[wave * 2 + sp] = a;
     }
     __syncthreads();
-    const int k = threadIdx.x, r = row0 + (k >> 1), sp = k & 1;
-    if (k < 2 * FORMED_ROWS && r < n) {
-      double a = red[(k >> 1) * 4 + sp] + red[(k >> 1) * 4 + 2 + sp];
-      if (f.has_id) a += f.id[2 * sp] * x(r, 0) + f.id[2 * sp + 1] * x(r, 1);
-      y[2 * r + sp] = a;
-    }
+    if (k < 2 * FORMED_ROWS && r < n) y[2 * r + sp1] = red[(k >> 1) * 4 + sp1] + red[(k >> 1) * 4 + 2 + sp1] + own;
   }
 };

@@ -172,8 +172,8 @@ __device__ __forceinline__ int chol_block(f64x4 (&acc)[4], CholTile& s, CholPane
 }
 
 // Tiles in the accumulators of four waves: row 16 w + lane / 16 + 4 r, column 16 t + lane % 16 of acc[t][r].  Every
-// access of a thread is one address that advances by four rows, clamped at the edge rather than skipped: loads under a
-// condition wait for one another, and a 64-bit product per element costs more than the load.
+// access of a thread is one address that advances by four rows, clamped at the edge: a 64-bit product per element costs
+// more than the load (33000 cycles for the tiles of a step, 6000 with advancing addresses).
 // The 64 x 64 tile at p, rows x cols of it, zero past them.
 __device__ __forceinline__ void tile_to_acc(f64x4 (&acc)[4], const double* p, int64_t ld, int rows, int cols, int w, int lane) {
   const int i0 = 16 * w + (lane >> 4), j0 = lane & 15;
