@@ -815,29 +815,33 @@ int cg_formed_step(hipStream_t st, const FormedPlan& f, const double* rho, const
   return CC_OK;
 }
 
-// One wave; every element goes through the operations of the serial algorithm in its order, the lanes take different
-// rows (Cholesky, rotations), columns (the inverse factor) or entries (the projected matrix).  Bound by the chain of
-// rotations: k = 8 takes 34 us on average over a solve's passes, 104 us with one lane doing everything.
+// One wave; the lanes take different rows (Cholesky), columns (the inverse factor), entries (the projected matrix) and
+// disjoint rotations: a sweep of the Jacobi iteration is k - 1 rounds (k even; k rounds otherwise) of the circle method,
+// each of up to k / 2 rotations, instead of k (k - 1) / 2 one after the other.  Bound by the chain of rounds: 20 us on
+// average over a refined solve of eight passes, 33 us with single rotations and the matrices read from memory (k = 8, dense:
+// 43 against 99 us; 32: 1.15 against 2.27 ms; 3: 12.0 against 10.6).
 __global__ void __launch_bounds__(64) small_geneig_kernel(int k, const double* __restrict__ Hs, const double* __restrict__ Ns,
                                                           double* __restrict__ out, double* __restrict__ vec) {
   // the k x k work matrices live in LDS (no private scratch: concurrent launches on several
   // streams would each need a large scratch allocation)
-  __shared__ double Lm[32][33], C[32][33], V[32][33], Li[32][33];
+  __shared__ double Lm[32][33], C[32][33], V[32][33], Li[32][33], hs[32][33], rot[2][16];
+  __shared__ int pair[16];
   const int lane = threadIdx.x;
   for (int e = lane; e < k * k; e += 64) {
     const int i = e / k, j = e - i * k;
-    Lm[i][j] = 0.0;
+    Lm[i][j] = Ns[e];     // replaced column by column
+    hs[i][j] = Hs[e];
     Li[i][j] = 0.0;
     V[i][j] = (i == j) ? 1.0 : 0.0;
   }
   __syncthreads();
   for (int j = 0; j < k; ++j) {
-    double s = Ns[j * k + j];
+    double s = Lm[j][j];
     for (int c = 0; c < j; ++c) s -= Lm[j][c] * Lm[j][c];
     const double djj = sqrt(fmax(s, 1e-300));
     double t = 0.0;
     if (lane > j && lane < k) {
-      t = Ns[lane * k + j];
+      t = Lm[lane][j];
       for (int c = 0; c < j; ++c) t -= Lm[lane][c] * Lm[j][c];
       t /= djj;
     }
@@ -857,38 +861,58 @@ __global__ void __launch_bounds__(64) small_geneig_kernel(int k, const double* _
     const int i = e / k, j = e - i * k;
     double acc = 0.0;
     for (int a = 0; a <= i; ++a)
-      for (int b = 0; b <= j; ++b) acc += Li[i][a] * Hs[a * k + b] * Li[j][b];
+      for (int b = 0; b <= j; ++b) acc += Li[i][a] * hs[a][b] * Li[j][b];
     C[i][j] = acc;
   }
   __syncthreads();
+  const int even = k + (k & 1), rounds = even - 1, pairs = even / 2;
+  const int width = k <= 8 ? 8 : k <= 16 ? 16 : 32, l = lane & (width - 1), first = lane / width, stride = 64 / width;
   for (int sweep = 0; sweep < 50; ++sweep) {
-    double off = 0.0;
-    for (int i = 0; i < k; ++i)
-      for (int j = i + 1; j < k; ++j) off += C[i][j] * C[i][j];
-    if (off < 1e-30) break;
-    for (int p = 0; p < k; ++p)
-      for (int q = p + 1; q < k; ++q) {
-        const double cpq = C[p][q];
-        if (cpq == 0.0) continue;
-        const double th = (C[q][q] - C[p][p]) / (2.0 * cpq);
-        const double t = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
-        const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
-        __syncthreads();
-        if (lane < k) {
-          const double a = C[lane][p], b = C[lane][q], va = V[lane][p], vb = V[lane][q];
-          C[lane][p] = c * a - s * b;
-          C[lane][q] = s * a + c * b;
-          V[lane][p] = c * va - s * vb;
-          V[lane][q] = s * va + c * vb;
+    double off = 0.0;     // of the upper triangle, row by row
+    if (lane < k)
+      for (int j = lane + 1; j < k; ++j) off += C[lane][j] * C[lane][j];
+    if (cc_wave_sum(off) < 1e-30) break;
+    for (int r = 0; r < rounds; ++r) {
+      if (lane < pairs) {
+        // the last player stays, the others go round; with k odd the last is none
+        const int x = lane ? (r + lane) % rounds : r, y = lane ? (r - lane + rounds) % rounds : even - 1;
+        const int p = x < y ? x : y, q = x < y ? y : x;
+        const double cpq = q < k ? C[p][q] : 0.0;
+        double c = 1.0, sn = 0.0;
+        if (cpq != 0.0) {
+          const double th = (C[q][q] - C[p][p]) / (2.0 * cpq);
+          const double t = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
+          c = 1.0 / sqrt(t * t + 1.0);
+          sn = t * c;
         }
-        __syncthreads();
-        if (lane < k) {
-          const double a = C[p][lane], b = C[q][lane];
-          C[p][lane] = c * a - s * b;
-          C[q][lane] = s * a + c * b;
-        }
-        __syncthreads();
+        rot[0][lane] = c;
+        rot[1][lane] = sn;
+        pair[lane] = p | (q < k ? q : p) << 8;     // p alone: no rotation
       }
+      __syncthreads();
+      for (int m = first; m < pairs; m += stride) {
+        const int p = pair[m] & 255, q = pair[m] >> 8;
+        const double c = rot[0][m], sn = rot[1][m];
+        if (l < k && p != q) {
+          const double a = C[l][p], b = C[l][q], va = V[l][p], vb = V[l][q];
+          C[l][p] = c * a - sn * b;
+          C[l][q] = sn * a + c * b;
+          V[l][p] = c * va - sn * vb;
+          V[l][q] = sn * va + c * vb;
+        }
+      }
+      __syncthreads();
+      for (int m = first; m < pairs; m += stride) {
+        const int p = pair[m] & 255, q = pair[m] >> 8;
+        const double c = rot[0][m], sn = rot[1][m];
+        if (l < k && p != q) {
+          const double a = C[p][l], b = C[q][l];
+          C[p][l] = c * a - sn * b;
+          C[q][l] = sn * a + c * b;
+        }
+      }
+      __syncthreads();
+    }
   }
   int best = 0;
   for (int i = 1; i < k; ++i)

@@ -107,6 +107,27 @@ def test_cholesky_inverse_blocks(gpu, n):
         assert int(info.item()) == bad
 
 
+@pytest.mark.parametrize("k", [1, 2, 3, 7, 8, 9, 16, 17, 31, 32])
+def test_small_generalized_eigenproblem(gpu, k):
+    """cc_small_geneig_f64 against scipy over the widths of its rounds (8, 16, 32 rows), even and odd: value and residual
+    to 4 k^2 eps times the condition of N (rotations and both factor products act on k rows k times)."""
+    from scipy.linalg import eigh
+    from carcassonne_amd import _lib
+    from carcassonne_amd.device import ptr, stream
+    rng = np.random.default_rng(k)
+    g, r = rng.standard_normal((k, k)), rng.standard_normal((k, 2 * k))
+    h, n = g + g.T, r @ r.T / (2 * k) + 0.2 * np.eye(k)
+    for matrix in (h, np.diag(np.diag(h)), np.diag(np.diag(h)) + 1e-9 * h):
+        H, N = torch.from_numpy(matrix.copy()).cuda(), torch.from_numpy(n).cuda()
+        out, vec = torch.empty(1, dtype=torch.float64, device="cuda"), torch.empty(k, dtype=torch.float64, device="cuda")
+        _lib.call("cc_small_geneig_f64", stream(), k, ptr(H), ptr(N), ptr(out), ptr(vec))
+        values, v, scale = eigh(matrix, n, eigvals_only=True), vec.cpu().numpy(), np.linalg.norm(matrix, 2)
+        tol = 4 * k * k * np.finfo(float).eps * np.linalg.cond(n)
+        assert abs(out.item() - values[0]) <= tol * abs(values).max()
+        assert abs(v @ n @ v - 1.0) <= tol
+        assert np.linalg.norm(matrix @ v - out.item() * (n @ v)) <= tol * scale * np.linalg.norm(v)
+
+
 @pytest.mark.parametrize("D,chi,model,seed", [(2, 8, "ising", 0), (3, 6, "heisenberg", 1), (4, 8, "ising", 2),
                                               (4, 16, "heisenberg", 3)])
 def test_lanczos_matches_generalized_eigh(gpu, D, chi, model, seed):
