@@ -167,7 +167,8 @@ __global__ void __launch_bounds__(256) form_reduce_kernel(int split, int P, int 
 }
 
 // Parts of a group's K range: enough workgroups for several waves of the chip (256 CUs x 3), each with at least
-// FORM_MIN_STEPS K steps, a multiple of 8 parts in all so that each stays on one XCD.
+// FORM_MIN_STEPS K steps, a multiple of 8 parts in all so that each stays on one XCD.  The sums of parts are also the more
+// accurate ones: N at D = 2, chi = 50 is 1.3e-16 off sums in 80 bits, 1.3e-15 as one running sum per entry.
 constexpr int FORM_MIN_STEPS = 8;
 int form_split(int n_groups, int max_products, int64_t n_alpha, int64_t P, int64_t Q) {
   const int64_t tiles = ((P * P + FT - 1) / FT) * ((Q * Q + FT - 1) / FT);
