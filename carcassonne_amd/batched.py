@@ -85,12 +85,13 @@ class BatchedSolve:
         synchronize()
 
     def autotune(self):
-        """Workgroup count of the low-precision kernel per shape bucket (on the bucket's first system)."""
+        """Workgroup count of the low-precision kernel per shape bucket (on the bucket's first system); dtype "f32" has no
+        such kernel."""
         for (corners, sides, opc, _) in self.inputs:
             H, _ = S2.formExpectationAndNormalizationMultipliers(corners, sides, opc)
             key = (H.operator.P, H.operator.n_alpha)
             if key not in self.tuning:
-                g, timings = autotune_groups(H.operator, self.dtype)
+                g, timings = (None, {}) if self.dtype == "f32" else autotune_groups(H.operator, self.dtype)
                 self.tuning[key] = dict(groups=g, timings_us={k: v * 1e6 for k, v in timings.items()})
         synchronize()
 

@@ -147,9 +147,11 @@ def solve(corners, sides, op_center, x0, tol_residual=1e-10, tol_energy=1e-13, m
 
 
 def solve_mixed(corners, sides, op_center, x0, dtype="f16", graph=True, **kw):
-    """The precision form of the same solve: stage 1/2 and the normalization factor in FP64, FP16/BF16
-    Lanczos on the whitened operator, FP64 Jacobi-Davidson refinement.  The energy is the FP64
-    Rayleigh-Ritz value of the refined vector (its Rayleigh quotient, from FP64 H and N products)."""
+    """The precision form of the same solve: stage 1/2 and the normalization factor in FP64, Lanczos on the
+    whitened operator in FP16 or BF16 products or on its formed matrices in FP32 (dtype "f16", "bf16" or
+    "f32", see MixedSolver), FP64 Jacobi-Davidson refinement.  The energy is the FP64 Rayleigh-Ritz value of
+    the refined vector (its Rayleigh quotient, from FP64 H and N products).  lp_operator: the FP16 / BF16
+    operator, None for "f32"."""
     H, N = multipliers(corners, sides, op_center, graph=graph)
     solver = MixedSolver(H.operator, N.operator, dtype=dtype)
     x, rho, info = solver.solve(x0, **kw)

@@ -13,10 +13,11 @@ MixedSolver -- (1) Lanczos on the whitened low-precision operator until the Ritz
     outer step applies the FP64 H and N to one new basis vector, solves the small generalized eigenproblem of the basis
     on the device (FP64 Rayleigh-Ritz), and computes the correction from a fixed number of CG steps on the projected,
     shifted low-precision operator.  The energy reported is the FP64 Rayleigh quotient of the final Ritz vector.
-    The operator is formed in FP64 (formed.FormedOperator) and the low-precision one is its whitened matrices rounded
-    to FP32: a solve applies it 70 times or more, and forming costs as much as seven applications of the slabs.  Where
-    an operator has no such form, or the caller brings the normalization factor, the low-precision operator is the
-    FP16 / BF16 one (dtype, groups, split) between the FP64 whitening products.
+    The low-precision operator is the caller's choice.  dtype "f16" or "bf16": a LowPrecisionOperator (groups, split)
+    between the FP64 whitening products.  dtype "f32": the operator formed in FP64 (formed.FormedOperator), whitened
+    and rounded to FP32, whose FP64 matrices also serve the refinement.  A refinement of fixed work on an environment
+    with a small gap can end before its state has converged, and the last digits of that state are those of the operator
+    inside: none is taken in another's place.
 """
 import ctypes
 
@@ -25,7 +26,7 @@ import torch
 
 from . import _lib
 from .device import empty, join, ptr, stream
-from .formed import FormedOperator
+from .formed import MAX_MATRICES, MAX_PRODUCTS, FormedOperator
 from .solver import NormalizationFactor
 
 DTYPES = {"f16": _lib.CC_F16, "bf16": _lib.CC_BF16}
@@ -143,23 +144,29 @@ class MixedSolver:
     """Lowest eigenpair of (H, N) to FP64 accuracy with low-precision matvecs doing the bulk."""
 
     def __init__(self, h_operator, n_operator, dtype="bf16", factor=None, groups=None, split="vector"):
+        """dtype: "f16", "bf16" (with groups and split of its LowPrecisionOperator) or "f32" (formed matrices)."""
         self.H, self.N = h_operator, n_operator
         if not h_operator.use_fused:
             raise NotImplementedError("the low-precision kernel needs P = Q in {4, 9, 16, 25, 36} and d = 2")
-        DTYPES[dtype], SPLIT_MODES[split]      # unknown names are refused whichever operator serves the solve
-        side, form = None, factor is None
+        form, side = dtype == "f32", None
+        if form and (groups is not None or split != "vector"):
+            raise ValueError("groups and split belong to the FP16 / BF16 kernel, not to dtype 'f32'")
+        if not form:
+            DTYPES[dtype], SPLIT_MODES[split]      # unknown names are refused before anything is launched
         if factor is None:
             factor, side = NormalizationFactor.beside(n_operator)
         self.factor = factor
         self.n = h_operator.n
-        self._lp_args = dict(dtype=dtype, groups=groups, split=split)
-        self._lp, self._lp_source = None, h_operator
+        self.Hlp = None     # the FP16 / BF16 operator
         self._formed = self._white = None
         try:
             if form:
                 self._formed = FormedOperator.of(h_operator, n_operator, factor)
-            if self._formed is None:
-                self.Hlp
+                if self._formed is None:
+                    raise NotImplementedError("dtype 'f32' needs an operator of at most {} distinct site operators and "
+                                              "{} products".format(MAX_MATRICES, MAX_PRODUCTS))
+            else:
+                self.Hlp = LowPrecisionOperator(h_operator, dtype, groups=groups, split=split)
                 self._hplan = h_operator.plan_handle()     # N is applied through the formed N_env (factor.apply_n)
             self._lz_work, self._lz_max = None, 0
             self._jd_work = empty((_lib.query("cc_jd_work_size", self.n),))
@@ -169,13 +176,6 @@ class MixedSolver:
         if self._formed is not None:
             self._K32 = empty(self._formed.G.shape, dtype=torch.float32)
             self._white = self._formed.whitened(factor, self._K32)
-
-    @property
-    def Hlp(self):
-        """The FP16 / BF16 operator (made on first use where the formed one serves the solve)."""
-        if self._lp is None:
-            self._lp = LowPrecisionOperator(self._lp_source, **self._lp_args)
-        return self._lp
 
     def refresh(self, h_operator, n_operator):
         """The solve's setup for a new environment of the same structure, into this solver's buffers: the
@@ -187,9 +187,7 @@ class MixedSolver:
             self._white = self._formed.whitened(self.factor, self._K32)
         else:
             self.H.refresh_fused_from(h_operator)
-        if self._lp is not None:
-            self._lp.refresh(h_operator)
-        self._lp_source = h_operator
+            self.Hlp.refresh(h_operator)
 
     def _apply_h(self, x, y):
         """y = H x in FP64."""

@@ -4,8 +4,9 @@ compression entry points, observables, growth (contractTowards), gauge moves, ba
 increase and the solve.
 
 minimizeExpectation keeps the reference's relaxOver by default; solver="lanczos" runs the
-residual-controlled FP64 Lanczos and solver="mixed" the FP16/BF16 precision form (both need
-an instantiated fused shape, P = D0*D1 in {4, 9, 16, 25, 36}, d = 2).
+residual-controlled FP64 Lanczos and solver="mixed" the precision form (FP16 products, or those of
+solver_options["dtype"]; both need an instantiated fused shape, P = D0*D1 in {4, 9, 16, 25, 36},
+d = 2).
 """
 import copy as _copy
 import functools
