@@ -62,8 +62,12 @@ def operator_groups(values):
 
 def products_of(terms):
     """The terms (a, b, c) of one site operator as products ([(a, c)...], [(b, c)...]), a sum of A channels times a sum
-    of B channels: the channel with the most terms left takes them all as one product."""
-    left, out = list(terms), []
+    of B channels: the channel with the most terms left takes them all as one product, MAX_SUM at a time.  Terms of one
+    pair of channels are one term first, with their coefficients added."""
+    pairs, out = {}, []
+    for a, b, c in terms:
+        pairs[(a, b)] = pairs.get((a, b), 0.0) + c
+    left = [(a, b, c) for (a, b), c in pairs.items()]
     while left:
         count = {}
         for a, b, _ in left:

@@ -18,6 +18,20 @@ def test_products_cover_every_term_once(seed):
     assert got == {(a, b): c for a, b, c in terms}
 
 
+@pytest.mark.parametrize("same,others", [(2, 0), (8, 1), (9, 0), (17, 3)])
+def test_products_add_equal_terms(same, others):
+    """Terms of one pair of channels (one-site operators of one matrix under several tags) all count, past a sum's eight
+    channels too."""
+    from carcassonne_amd.stage3 import products_of
+    terms = [(0, 100, 1.0)] * same + [(0, 101 + i, 2.0) for i in range(others)]
+    got = {}
+    for left, right in products_of(terms):
+        for a, ca in left:
+            for b, cb in right:
+                got[(a, b)] = got.get((a, b), 0.0) + ca * cb
+    assert got == dict([((0, 100), float(same))] + [((0, 101 + i), 2.0) for i in range(others)])
+
+
 def test_star_of_terms_takes_two_products():
     from carcassonne_amd.stage3 import products_of
     # the identity channels (0 and 100) each meet several others
