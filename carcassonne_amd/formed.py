@@ -25,8 +25,9 @@ class FormedOperator:
 
     @staticmethod
     def of(h_operator, n_operator, factor):
-        """The operator's formed matrices, made on the first call; None where it has no such form (no fused shape, or
-        more distinct site operators or products than one call takes)."""
+        """The operator's formed matrices, made on the first call; None where it has no such form (no fused shape, more
+        distinct site operators or products than one call takes, or an operator refreshed from another: only its packed
+        slabs hold that environment, its own channels are those it was built from)."""
         f = h_operator._formed
         if f is None or not f.valid() or f.norm_channels != (n_operator._A[0], n_operator._B[0]):
             layout = FormedOperator._layout(h_operator, n_operator)
@@ -37,7 +38,7 @@ class FormedOperator:
     def _layout(h_operator, n_operator):
         """([(O_g, [(A sum, B sum)...])...], identity): the matrices to form, by site operator, and the site operator
         of the identity channels' product (None: there is no such term)."""
-        if not h_operator.use_fused or h_operator.d != 2:
+        if not h_operator.use_fused or h_operator.d != 2 or h_operator._refreshed:
             return None
         channels, specs, ops, rows = h_operator._merged()
         values = [tuple(float(x) for x in o.toArray().reshape(-1)) for o in ops] + [(1.0, 0.0, 0.0, 1.0)]   # [-1]: 1
@@ -87,10 +88,7 @@ class FormedOperator:
         channels = h_operator.same_structure(other)
         if factor is not self.factor:
             self.factor, self._plan = factor, None
-        if h_operator._fused is not None:
-            h_operator.refresh_fused_from(other)
-        else:
-            h_operator._refreshed += 1
+        h_operator.refresh_fused_from(other)
         _, specs, _, _ = h_operator._merged()
         h_operator._joined = {(side, k): h_operator.joined(side, k, channels)
                               for side in (0, 1) for k in range(len(specs[side]))}

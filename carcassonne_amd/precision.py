@@ -164,7 +164,7 @@ class MixedSolver:
                 self._formed = FormedOperator.of(h_operator, n_operator, factor)
                 if self._formed is None:
                     raise NotImplementedError("dtype 'f32' needs an operator of at most {} distinct site operators and "
-                                              "{} products".format(MAX_MATRICES, MAX_PRODUCTS))
+                                              "{} products, not refreshed from another".format(MAX_MATRICES, MAX_PRODUCTS))
             else:
                 self.Hlp = LowPrecisionOperator(h_operator, dtype, groups=groups, split=split)
                 self._hplan = h_operator.plan_handle()     # N is applied through the formed N_env (factor.apply_n)

@@ -107,9 +107,10 @@ class GroundStateSolver:
         self.H, self.N = h_operator, n_operator
         side = None
         # FP64: the solve applies the formed operator, whose identity part is the factor's matrix -- so only where this
-        # solver makes the factor itself.  The channels are taken here, the matrices formed by the first solve: a
-        # caller that only asks for an energy applies the slabs once (D = 6, chi = 64: 0.2 against 1.1 ms).
-        self._form = factor is None and precision == "f64"
+        # solver makes the factor itself, and from the operator's own channels (FormedOperator.of).  The channels are
+        # taken here, the matrices formed by the first solve: a caller that only asks for an energy applies the slabs
+        # once (D = 6, chi = 64: 0.2 against 1.1 ms).
+        self._form = factor is None and precision == "f64" and not h_operator._refreshed
         if factor is None:
             factor, side = NormalizationFactor.beside(n_operator)
         self.factor = self._own_factor = factor

@@ -86,6 +86,39 @@ def test_formed_operator_follows_its_environment(gpu):
     assert abs(theta - theta2) <= 1e-11 * abs(theta2)
 
 
+@pytest.mark.parametrize("through", ["operator", "f16", "f32"])
+def test_new_solver_on_a_refreshed_operator(gpu, through):
+    """A solver made for an operator that was refreshed from another (by itself or through a mixed solver) solves the
+    environment it was refreshed from, and the operator still applies it afterwards."""
+    from carcassonne_amd.precision import MixedSolver
+    from carcassonne_amd.solver import GroundStateSolver
+    H, N, x0 = _operators(3, 6, "ising", 1)
+    H2, N2, _ = _operators(3, 6, "ising", 2)
+    if through == "operator":
+        GroundStateSolver(H, N).solve(x0)
+        H.refresh_fused_from(H2)
+    else:
+        MixedSolver(H, N, dtype=through).refresh(H2, N2)
+    want, got = torch.empty_like(x0), torch.empty_like(x0)
+    H2.apply_generic_flat(x0, want)
+    _, theta2, _, _ = GroundStateSolver(H2, N2).solve(x0)
+    solver = GroundStateSolver(H, N2)
+    x, theta, _, _ = solver.solve(x0)
+    assert abs(theta - theta2) <= 1e-11 * abs(theta2)
+    assert abs(solver.rayleigh_quotient(x) - theta2) <= 1e-11 * abs(theta2)
+    H.apply_flat(x0, got)
+    assert _rel(got, want) < 1e-13
+    # the FP16 slabs are converted from the operator's own channels, so this solve need not converge; its value is that
+    # of its state in the new environment
+    y, rho, _ = MixedSolver(H, N2, dtype="f16").solve(x0)
+    hy, ny = torch.empty_like(x0), torch.empty_like(x0)
+    H2.apply_generic_flat(y, hy)
+    N2.apply_generic_flat(y, ny)
+    assert abs(rho - float(y @ hy) / float(y @ ny)) <= 1e-11 * abs(rho)
+    with pytest.raises(NotImplementedError):
+        MixedSolver(H, N2, dtype="f32")
+
+
 @pytest.mark.parametrize("n,count", [(1, 1), (32, 2), (33, 1), (65, 3), (513, 2), (700, 3)])
 def test_whitening_products(gpu, n, count):
     """W G W^T for lower-triangular W over partial rounds of the tile order, 32- and 64-wide tiles: two sums of n products,
