@@ -20,19 +20,17 @@ MAX_PRODUCTS, MAX_MATRICES = 16, 4
 
 
 class FormedOperator:
-    """The formed matrices of a stage-3 operator, kept on it: apply_flat(x, y) is y = H x.  `factor`: the normalization
-    factor of the same environment, whose matrix is the identity channels' product."""
+    """The formed matrices of a stage-3 operator, one set per solver: apply_flat(x, y) is y = H x.  `factor`: the
+    normalization factor of the same environment, whose matrix is the identity channels' product."""
 
     @staticmethod
     def of(h_operator, n_operator, factor):
-        """The operator's formed matrices, made on the first call; None where it has no such form (no fused shape, more
+        """Formed matrices of the operator; None where it has no such form (no fused shape, more
         distinct site operators or products than one call takes, or an operator refreshed from another: only its packed
         slabs hold that environment, its own channels are those it was built from)."""
-        f = h_operator._formed
-        if f is None or not f.valid() or f.norm_channels != (n_operator._A[0], n_operator._B[0]):
-            layout = FormedOperator._layout(h_operator, n_operator)
-            f = h_operator._formed = FormedOperator(h_operator, n_operator, factor, layout) if layout is not None else None
-        return f
+        layout = FormedOperator._layout(h_operator, n_operator)
+        h_operator._formed = FormedOperator(h_operator, factor, layout) if layout is not None else None
+        return h_operator._formed
 
     @staticmethod
     def _layout(h_operator, n_operator):
@@ -55,11 +53,10 @@ class FormedOperator:
             return None
         return [(values[o], products) for o, products in groups.items()], identity
 
-    def __init__(self, h_operator, n_operator, factor, layout):
+    def __init__(self, h_operator, factor, layout):
         self.n_env, self.d = h_operator.n // h_operator.d, h_operator.d
         self._groups, self.identity = layout
         self.ops = [O for O, _ in self._groups]
-        self.norm_channels = (n_operator._A[0], n_operator._B[0])
         self.factor = factor
         self._shape = (h_operator.n_alpha, h_operator.P)
         self._plan = None
@@ -68,7 +65,7 @@ class FormedOperator:
 
     def _form(self, joined):
         """G from the joined sums of channels joined(half, k)."""
-        self._version = self.factor.version
+        self._version = self.factor.version     # counted on the host, at capture in a graph: with the refresh of all three
         if not self._groups:
             return
         na, P = self._shape
@@ -84,7 +81,7 @@ class FormedOperator:
 
     def refresh(self, h_operator, other, factor):
         """Forms `other`, an operator of h_operator's structure from a new environment that the factor holds already,
-        into these matrices; h_operator then applies it (kernels only: capturable in a HIP graph)."""
+        into these matrices; h_operator then applies it too (kernels only: capturable in a HIP graph)."""
         channels = h_operator.same_structure(other)
         if factor is not self.factor:
             self.factor, self._plan = factor, None
@@ -93,11 +90,10 @@ class FormedOperator:
         h_operator._joined = {(side, k): h_operator.joined(side, k, channels)
                               for side in (0, 1) for k in range(len(specs[side]))}
         self._form(h_operator.joined)
-        h_operator._formed = self
 
-    def valid(self):
-        """Whether the factor still holds the environment this operator was formed from."""
-        return self.factor.version == self._version
+    def valid(self, factor):
+        """Whether `factor` is the factor formed beside and still holds that environment."""
+        return factor is self.factor and factor.version == self._version
 
     def apply_flat(self, x, y):
         if self._plan is None:

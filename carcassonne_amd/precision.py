@@ -174,6 +174,7 @@ class MixedSolver:
             if side is not None:
                 join(side)
         if self._formed is not None:
+            self._refreshed = h_operator._refreshed
             self._K32 = empty(self._formed.G.shape, dtype=torch.float32)
             self._white = self._formed.whitened(factor, self._K32)
 
@@ -184,6 +185,7 @@ class MixedSolver:
         self.factor.refresh(n_operator)
         if self._formed is not None:
             self._formed.refresh(self.H, h_operator, self.factor)
+            self._refreshed = self.H._refreshed
             self._white = self._formed.whitened(self.factor, self._K32)
         else:
             self.H.refresh_fused_from(h_operator)
@@ -195,6 +197,12 @@ class MixedSolver:
             self._formed.apply_flat(x, y)
         else:
             _lib.call("cc_stage3_plan_apply", stream(), self._hplan, ptr(x), ptr(y))
+
+    def _check_environment(self):
+        """A formed solver's operator and factor are refreshed together, by refresh()."""
+        if self._formed is not None and not (self._formed.valid(self.factor) and self.H._refreshed == self._refreshed):
+            raise RuntimeError("the operator or the normalization factor was given another environment than the formed "
+                               "matrices of this solver; MixedSolver.refresh takes all three there")
 
     def _lanczos(self, x0, tol_residual, tol_energy, max_iter, check_every, x, res):
         f = self.factor
@@ -225,6 +233,7 @@ class MixedSolver:
         when the remaining error predicted from the last two changes (geometric convergence,
         d_k * q / (1 - q) with q = d_k / d_{k-1}) is at most tol_predicted |rho_k|."""
         from .data import HipData
+        self._check_environment()
         if isinstance(x0, HipData):
             x0 = x0._t.reshape(-1)
         n = self.n
@@ -287,6 +296,7 @@ class MixedSolver:
         record[outer], record[outer + 1] are |H x - rho N x|^2 and |N x|^2 of the final vector (the
         convergence record that lets a caller check, after a replay, that the fixed work converged)."""
         from .data import HipData
+        self._check_environment()
         if isinstance(x0, HipData):
             x0 = x0._t.reshape(-1)
         n = self.n

@@ -117,7 +117,7 @@ class GroundStateSolver:
         self._version, self._refreshed = factor.version, h_operator._refreshed   # of the environment taken here
         self.n = h_operator.n
         self.precision = precision
-        self._white = None
+        self._formed = self._white = None
         try:
             if self._form:
                 h_operator.snapshot()
@@ -151,23 +151,27 @@ class GroundStateSolver:
         f.check()
         return x, float(res[0]), float(res[1]), int(res[2])
 
+    def _unchanged(self):
+        """Whether the operator and the factor still hold the environment taken when this solver was made."""
+        return self.factor is self._own_factor and self.factor.version == self._version \
+            and self.H._refreshed == self._refreshed
+
     def _whitened(self):
         """The formed, whitened operator's plan, made on the first solve; None where the solve applies the slabs (no
-        formed matrices, or the operator or the factor has been given another environment since)."""
-        if not self._form or self.factor is not self._own_factor or self.factor.version != self._version \
-                or self.H._refreshed != self._refreshed:
+        formed matrices, or another environment since)."""
+        if not self._form or not self._unchanged():
             return None
         if self._white is None:
-            formed = FormedOperator.of(self.H, self.N, self.factor)
-            if formed is None:
+            self._formed = FormedOperator.of(self.H, self.N, self.factor)
+            if self._formed is None:
                 return None
-            self._white = formed.whitened(self.factor)
+            self._white = self._formed.whitened(self.factor)
         return self._white
 
     def rayleigh_quotient(self, x):
         """(x^T H x) / (x^T N x) in FP64 on the device."""
         hx, nx = torch.empty_like(x), torch.empty_like(x)
-        self.H.apply_flat(x, hx)
+        (self._formed if self._formed is not None and self._unchanged() else self.H).apply_flat(x, hx)
         self.factor.apply_n(x, nx)
         out = empty((2,))
         _lib.call("cc_dot_f64", stream(), self.n, ptr(x), ptr(hx), ptr(out[0:1]))

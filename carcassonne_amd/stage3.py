@@ -230,7 +230,7 @@ class Stage3Operator:
         self.cost_of_formMatrix = sum(cost_of_matrix(a.shape, b.shape, self.d) for (a, b, _) in self.terms)
         self._work = None
         self._fused = None
-        self._formed = None     # formed.FormedOperator, once a solver has formed this operator
+        self._formed = None     # formed.FormedOperator of the last solver that formed this operator
         self._merge, self._joined, self._packs, self._refreshed = None, {}, {}, 0
         # the slab kernels read P = Q <= 36, d = 2; the solvers, plans and low-precision forms (use_fused) serve the
         # extents D * D of equal center bonds
@@ -391,7 +391,7 @@ class Stage3Operator:
         its fused kernel and native plan apply `other` (kernels only; capturable in a HIP graph)."""
         self._ensure_fused()
         channels = self.same_structure(other)
-        self._formed, self._joined = None, {}     # of the environment before
+        self._joined = {}       # of the environment before
         self._refreshed += 1
         _, specs, _, _ = self._merged()
         for side, bufs in ((0, self._fused["A"]), (1, self._fused["B"])):
@@ -455,10 +455,7 @@ class Stage3Operator:
                     pass
 
     def apply_flat(self, x, y):
-        """y = H x for flat device tensors of length n (torch float64)."""
-        if self._formed is not None and self._formed.valid():
-            self._formed.apply_flat(x, y)
-            return
+        """y = H x for flat device tensors of length n (torch float64), through the slabs whatever solves came before."""
         # also for unequal center bonds (packing may read site operators back, so not first under capture)
         if self._fused is None and self._use_slabs and (self.use_fused or not torch.cuda.is_current_stream_capturing()):
             self._build_fused()

@@ -86,6 +86,54 @@ def test_formed_operator_follows_its_environment(gpu):
     assert abs(theta - theta2) <= 1e-11 * abs(theta2)
 
 
+def test_application_does_not_depend_on_solves(gpu):
+    """H(x) is the same bits before and after a solve of H, and a graph that captured it after a solve still replays
+    the operator once the solver is gone and the operator has been refreshed."""
+    from carcassonne_amd.solver import GroundStateSolver
+    H, N, x0 = _operators(3, 6, "ising", 1)
+    H2, _, _ = _operators(3, 6, "ising", 2)
+    before, after, y = (torch.empty_like(x0) for _ in range(3))
+    H.apply_flat(x0, before)
+    solver = GroundStateSolver(H, N)
+    solver.solve(x0)
+    H.apply_flat(x0, after)
+    assert torch.equal(before, after)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        H.apply_flat(x0, y)
+    del solver
+    for other in (None, H2):
+        if other is not None:
+            H.refresh_fused_from(other)
+            other.apply_flat(x0, after)
+        for _ in range(2):
+            graph.replay()
+            assert _rel(y, after) < 1e-13
+
+
+def test_formed_solvers_of_one_operator_share_nothing(gpu):
+    """Two formed solvers of one operator: another environment in the factor of the first leaves the second as it was
+    and is refused by the first until it is refreshed as a whole."""
+    from carcassonne_amd.precision import MixedSolver
+    H, N, x0 = _operators(3, 6, "ising", 1)
+    H2, N2, _ = _operators(3, 6, "ising", 2)
+    first, second = MixedSolver(H, N, dtype="f32"), MixedSolver(H, N, dtype="f32")
+    _, want, _ = second.solve(x0)
+    first.factor.refresh(N2)
+    _, rho, _ = second.solve(x0)
+    assert rho == want
+    with pytest.raises(RuntimeError):
+        first.solve(x0)
+    with pytest.raises(RuntimeError):
+        first.solve_fixed(x0)
+    first.refresh(H2, N2)
+    _, rho, _ = first.solve(x0)
+    _, want, _ = MixedSolver(H2, N2, dtype="f32").solve(x0)
+    assert abs(rho - want) <= 1e-11 * abs(want)
+    with pytest.raises(RuntimeError):
+        second.solve(x0)
+
+
 @pytest.mark.parametrize("through", ["operator", "f16", "f32"])
 def test_new_solver_on_a_refreshed_operator(gpu, through):
     """A solver made for an operator that was refreshed from another (by itself or through a mixed solver) solves the
