@@ -107,8 +107,18 @@ def merged_terms(d, rows, values, legs):
     return specs, sorted((specs[0].index(left), specs[1].index(right), o) for left, right, o in products)
 
 
+def _alike(channels):
+    return len(channels) == 1 or len({ch.source()[1:] for ch in channels}) == 1
+
+
 def join_slabs(channels, coefs):
-    """sum coefs[i] * channels[i] as a contiguous (alpha, P, P) array; the channels share their leg sizes and strides."""
+    """sum coefs[i] * channels[i] as a contiguous (alpha, P, P) array, in one pass where the channels share their leg sizes
+    and strides."""
+    if not _alike(channels):
+        out = join_slabs(channels[:1], coefs[:1])
+        for ch, c in zip(channels[1:], coefs[1:]):
+            _lib.call("cc_axpby_f64", stream(), out.numel(), 1.0, ptr(join_slabs([ch], [c])), 1.0, ptr(out))
+        return out
     _, (na0, na1, d0, d1), st = channels[0].source()
     out = empty((na0 * na1, d0 * d1, d0 * d1))
     if out.numel() == 0:
@@ -307,9 +317,7 @@ class Stage3Operator:
         a_list, b_list, _, rows = self._channels()
         oa, ob, _, orows = other._channels()
         if ([(r[0], r[2], r[3]) for r in rows] != [(r[0], r[2], r[3]) for r in orows] or
-                [(c.n_alpha, c.P) for c in a_list + b_list] != [(c.n_alpha, c.P) for c in oa + ob] or
-                any(len({ch[i].source()[1:] for i, _ in spec}) > 1
-                    for ch, specs in zip((oa, ob), self._merged()[1]) for spec in specs)):
+                [(c.n_alpha, c.P) for c in a_list + b_list] != [(c.n_alpha, c.P) for c in oa + ob]):
             raise ValueError("refresh needs an operator of the same structure")
         return oa, ob
 
@@ -370,19 +378,18 @@ class Stage3Operator:
         """Sum k of half `side` in the fused kernel's MFMA-operand order: over `channels` into `out`, or as it was joined."""
         _, specs, _, _ = self._merged()
         spec = specs[side][k]
-        first = channels[spec[0][0]]
-        kept = self._joined[(side, k)] if out is None else None
+        parts, coefs = [channels[i] for i, _ in spec], [c for _, c in spec]
+        kept = self._joined[(side, k)] if out is None else None if _alike(parts) else join_slabs(parts, coefs)
         if out is None:
             out = empty((_packed_size(self.n_alpha, self.P),))
-        _, (na0, na1, d0, d1), st = first.source()
+        _, (na0, na1, d0, d1), st = parts[0].source()
         if kept is not None:
             P = self.P
             _lib.call("cc_stage3_pack_strided_f64", stream(), self.n_alpha, 1, d0, d1,
                       _lib.i64_array([P * P, 0, d1 * P, P, d1, 1]), ptr(kept), ptr(out))
         else:
-            _lib.call("cc_stage3_pack_sum_f64", stream(), len(spec),
-                      _lib.ptr_array([channels[i].source()[0].data_ptr() for i, _ in spec]),
-                      _lib.f64_array([c for _, c in spec]), na0, na1, d0, d1, _lib.i64_array(st), ptr(out))
+            _lib.call("cc_stage3_pack_sum_f64", stream(), len(spec), _lib.ptr_array([p.source()[0].data_ptr() for p in parts]),
+                      _lib.f64_array(coefs), na0, na1, d0, d1, _lib.i64_array(st), ptr(out))
         return out
 
     def refresh_fused_from(self, other):

@@ -51,3 +51,32 @@ def test_slab_matvec_of_a_kept_copy(gpu, table):
     other.snapshot()
     other.apply_flat(x, got)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("D0,D1,chi", [(2, 2, 5), (3, 4, 6)])
+def test_refresh_from_channels_of_other_layouts(gpu, D0, D1, chi):
+    """An operator whose sums add channels of one layout is refreshed from one where a channel of each sum lies with its
+    legs in another order."""
+    import torch
+    from carcassonne_amd.data import HipData, PermutedView
+    from carcassonne_amd.stage3 import Stage3Operator
+    op, x = _operator(D0, D1, chi, STAR, 5)
+    assert max(len(spec) for side in op._merged()[1] for spec in side) > 1
+    other, _ = _operator(D0, D1, chi, STAR, 6)
+    order = [3, 0, 1, 4, 2, 5]                  # leg p of the channel is leg order[p] of the stored tensor
+    moved = {}
+
+    def view(t):
+        if id(t) not in moved:
+            moved[id(t)] = PermutedView(t._t.permute([order.index(k) for k in range(6)]).contiguous(), order)
+        return moved[id(t)]
+
+    a_list, b_list = ([ch.t for ch in chans] for chans in other._channels()[:2])
+    terms = [(view(a) if a is a_list[1] else a, view(b) if b is b_list[2] else b, o) for a, b, o in other.terms]
+    mixed = Stage3Operator(terms, physical_dimension=2)
+    want, got = torch.empty_like(x), torch.empty_like(x)
+    other.apply_generic_flat(x, want)
+    op.apply_flat(x, got)
+    op.refresh_fused_from(mixed)
+    op.apply_flat(x, got)
+    assert float((got - want).norm() / want.norm()) < 1e-13
