@@ -334,7 +334,8 @@ class Stage3Operator:
                 # a channel by itself is kept with the channel, for every operator built from it
                 one = channels[side][spec[0][0]] if len(spec) == 1 and spec[0][1] == 1.0 else None
                 need_j = joined and (one._joined is None if one else (side, k) not in self._joined)
-                need_p = (side, k) not in self._packs and (one._packed is None if one else True)
+                # packed once: into _packs until _build_fused hands them to the plan, from then on never again
+                need_p = self._fused is None and (side, k) not in self._packs and (one._packed is None if one else True)
                 if need_p and not need_j and (side, k) in self._joined:
                     self._packs[(side, k)] = self._pack(side, k, channels[side])     # what was taken before
                 elif need_j or need_p:
@@ -345,7 +346,7 @@ class Stage3Operator:
                 jobs = [job for job in jobs if job not in alike]
                 self._take_alike(side, channels[side], sizes, alike)
             for k, spec in enumerate(specs[side]):
-                if (side, k) not in self._packs:
+                if self._fused is None and (side, k) not in self._packs:
                     self._packs[(side, k)] = channels[side][spec[0][0]]._packed
                 if joined and (side, k) not in self._joined:
                     self._joined[(side, k)] = channels[side][spec[0][0]]._t

@@ -80,3 +80,15 @@ def test_refresh_from_channels_of_other_layouts(gpu, D0, D1, chi):
     op.refresh_fused_from(mixed)
     op.apply_flat(x, got)
     assert float((got - want).norm() / want.norm()) < 1e-13
+
+
+def test_snapshot_of_an_applied_operator_joins_only(gpu):
+    """The plan of an operator that was applied holds its packed sums: a snapshot adds the joined ones and nothing else."""
+    import torch
+    op, x = _operator(4, 4, 12, STAR, 5)
+    op.apply_flat(x, torch.empty_like(x))
+    used = torch.cuda.memory_allocated()
+    op.snapshot()
+    sums = sum(len(specs) for specs in op._merged()[1])
+    assert op._packs == {}
+    assert torch.cuda.memory_allocated() - used <= sums * (12 * 12 * 16 * 16 * 8 + 512)
