@@ -38,12 +38,10 @@ class NormalizationFactor:
         self.n_env, self.d = P * Q, n_operator.d
         self._shape = (P, Q, n_operator.n_alpha, n_operator.d)
         self.version = 0    # counts refresh(): the environment held
-        self._form_work = empty((_lib.query("cc_form_work_size", 1, 1, n_operator.n_alpha, P, Q),))
         self.N_env = empty((self.n_env, self.n_env))
         self.L, self.W = empty(self.N_env.shape), empty(self.N_env.shape)
         self.Lt, self.Wt = empty(self.N_env.shape), empty(self.N_env.shape)
         self._info = torch.zeros(1, dtype=torch.int32, device=self.L.device)
-        self._lwork = empty((_lib.query("cc_linalg_work_size", self.n_env),))
         if not defer:
             self.refresh(n_operator)
 
@@ -53,7 +51,7 @@ class NormalizationFactor:
         one workgroup each) on the side stream, so that the caller's own setup kernels run meanwhile.
         Returns (factor, side stream); the caller joins the side stream before using the factor."""
         f = cls(n_operator, defer=True)    # buffers from the caller's stream
-        n_operator._A[0]._t, n_operator._B[0]._t   # the joined slabs too: nothing is allocated on the side stream
+        n_operator._A[0]._t, n_operator._B[0]._t   # the joined slabs too: the side stream allocates what it alone uses
         side = fork()
         with torch.cuda.stream(side):
             f.refresh(n_operator)
@@ -61,8 +59,9 @@ class NormalizationFactor:
 
     def refresh(self, n_operator):
         """Forms N_env, L, W and their transposes from a normalization operator of this factor's shape into
-        the factor's own buffers (kernels only, no allocation or host work, so the sequence can be captured
-        in a HIP graph and replayed for new environments)."""
+        the factor's own buffers (kernels only, and no host work, so the sequence can be captured in a HIP
+        graph and replayed for new environments).  The parts of the formation's split sums (107 MB at D = 6,
+        chi = 64) are the current stream's for the call, not each factor's for its life."""
         if len(n_operator._A) != 1 or n_operator._O[0] is not None:
             raise ValueError("the normalization operator must be a single identity term")
         if (n_operator.P, n_operator.Q, n_operator.n_alpha, n_operator.d) != self._shape:
@@ -71,11 +70,11 @@ class NormalizationFactor:
         A, B = n_operator._A[0], n_operator._B[0]
         P, Q, na, _ = self._shape
         # N_env[(p'q')][(pq)] = sum_alpha A[alpha][p'][p] B[alpha][q'][q]
+        work = empty((_lib.query("cc_form_work_size", 1, 1, na, P, Q),))
         _lib.call("cc_form_f64", stream(), 1, _lib.i32_array([0, 1]), _lib.ptr_array([A._t.data_ptr()]),
-                  _lib.ptr_array([B._t.data_ptr()]), na, P, Q, ptr(self.N_env), ptr(self._form_work))
+                  _lib.ptr_array([B._t.data_ptr()]), na, P, Q, ptr(self.N_env), ptr(work))
         self.L.copy_(self.N_env)
-        _lib.call("cc_cholesky_inverse_f64", stream(), self.n_env, ptr(self.L), ptr(self.W), ptr(self._info),
-                  ptr(self._lwork))
+        _lib.call("cc_cholesky_inverse_f64", stream(), self.n_env, ptr(self.L), ptr(self.W), ptr(self._info), None)
         self._checked = False   # the pivot flag is read by check() where the solver synchronizes anyway
         _lib.call("cc_transpose_f64", stream(), self.n_env, ptr(self.L), ptr(self.Lt))
         _lib.call("cc_transpose_f64", stream(), self.n_env, ptr(self.W), ptr(self.Wt))
@@ -202,14 +201,13 @@ class _DenseInverse:
     def __init__(self, matrix):
         n = matrix.shape[0]
         base = matrix.tensor()
-        work = empty((_lib.query("cc_linalg_work_size", n),))
         info = torch.zeros(1, dtype=torch.int32, device=base.device)
         self.W, self.Ninv, self.n = empty((n, n)), None, n
         for shift in (0.0, 1e-14, 1e-12, 1e-10):
             L = base.clone()
             if shift:
                 L.view(-1)[:: n + 1] += shift * abs(float(torch.diagonal(base).sum().item())) / n
-            _lib.call("cc_cholesky_inverse_f64", stream(), n, ptr(L), ptr(self.W), ptr(info), ptr(work))
+            _lib.call("cc_cholesky_inverse_f64", stream(), n, ptr(L), ptr(self.W), ptr(info), None)
             if int(info.item()) == 0:
                 break
         else:

@@ -180,3 +180,24 @@ def test_whitening_products(gpu, n, count):
     _lib.call("cc_whiten_f64", stream(), n, count, ptr(g), ptr(wt), ptr(K), ptr(work))
     bound = 2 * (n + 2) * np.finfo(float).eps * (abs(W) @ abs(G) @ abs(W.T))
     assert np.all(abs(K.cpu().numpy() - W @ G @ W.T) <= bound)
+
+
+@pytest.mark.parametrize("beside", [False, True])
+def test_factor_holds_its_matrices_alone(gpu, beside):
+    """N, L, W and two transposes; the sums' parts are given back, also where the factor was made on a side stream."""
+    from carcassonne_amd.device import join
+    from carcassonne_amd.solver import NormalizationFactor
+    _, N, _ = _operators(4, 16, "ising", 3)
+    if beside:
+        factor, side = NormalizationFactor.beside(N)
+        join(side)
+    else:
+        factor = NormalizationFactor(N)
+    factor.check()
+    held = sum(t.numel() * t.element_size() for t in vars(factor).values() if isinstance(t, torch.Tensor))
+    assert held <= 5 * 256 * 256 * 8 + 64
+    used = torch.cuda.memory_allocated()
+    factor.refresh(N)
+    assert torch.cuda.memory_allocated() == used
+    residual = factor.L @ factor.L.t() - factor.N_env
+    assert float(residual.norm() / factor.N_env.norm()) < 1e-14
