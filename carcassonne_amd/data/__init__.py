@@ -87,6 +87,13 @@ def _svd_work_size(m, n):
     return _lib.query("cc_svd_work_size", 1, m, n)
 
 
+def _check_legs(perm, ndim):
+    """Refuses a leg taken twice (as numpy's transpose does): the permuting kernel and the readers that take strides would
+    follow it past the data."""
+    if len({p % ndim for p in perm}) != len(perm):
+        raise ValueError("a leg is taken twice in {}".format(tuple(perm)))
+
+
 class HipData(Data):
     """A real FP64 tensor in device memory with the NDArrayData method surface."""
 
@@ -329,6 +336,7 @@ class HipData(Data):
         sh = self.shape
         if perm == list(range(len(sh))):
             return self._t
+        _check_legs(perm, len(sh))
         shape = [sh[p] for p in perm]
         st = _strides(sh)
         out = empty(shape)
@@ -613,6 +621,7 @@ class PermutedView(HipData):
         if not (isinstance(base, torch.Tensor) and base.is_contiguous() and base.dtype == torch.float64):
             raise TypeError("PermutedView needs a contiguous float64 device tensor")
         self._base, self._perm, self._mat = base, [int(p) for p in perm], None
+        _check_legs(self._perm, base.ndim)
         bs = base.shape
         self._shape = torch.Size([bs[p] for p in self._perm])
 

@@ -265,3 +265,18 @@ def test_strided_slab_packing_matches_join(gpu):
                           src_elems, ptr(base), ptr(sc1), ptr(got))
                 assert float(sc1[0]) == float(sc2[0]) == float(np.abs(joined).max())
                 assert torch.equal(got, ref)
+
+
+def test_a_leg_taken_twice_is_refused(gpu):
+    """Before anything is launched: the copy would read past the tensor (an axis counted from the end gives such leg lists
+    in absorbMatrixAt and normalizeAxis); legs counted from the end are fine where each is taken once."""
+    from carcassonne_amd.data import HipData, PermutedView
+    a = np.arange(24.0).reshape(2, 3, 4)
+    t = HipData.fromArray(a)
+    for bad in (lambda: t.transpose(0, 0, 1), lambda: t.transpose(0, 2, -1), lambda: t.join((0, 1), (1, 2)),
+                lambda: t.join(0, 1, 2, -1), lambda: t.absorbMatrixAt(-1, HipData.fromArray(np.ones((2, 4)))),
+                lambda: t.normalizeAxis(-1), lambda: t.permuted_lazily([1, 1, 0]), lambda: PermutedView(t._t, [0, 1, -3])):
+        with pytest.raises(ValueError):
+            bad()
+    np.testing.assert_array_equal(t.transpose(0, -1, 1).toArray(), a.transpose(0, -1, 1))
+    np.testing.assert_array_equal(t.permuted_lazily([-1, 0, 1]).toArray(), a.transpose(-1, 0, 1))
