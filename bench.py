@@ -8,10 +8,11 @@ stage 1/2 on the GPU, the stage-3 operators, the normalization factor (N_env = L
 eigensolve to a 1e-10 relative energy, and the FP64 Rayleigh quotient of the result; the energy is
 checked against the oracle's eigh energy (tests/golden).
 
-Two forms are timed on the same inputs:
+The forms are timed on the same inputs:
   * mixed (the headline `value`): the operator formed in FP64, FP32 copies of its whitened matrices inside the
-    Lanczos and the correction equation, FP64 Jacobi-Davidson refinement, FP64 Rayleigh-Ritz energy;
-  * fp64: the plain FP64 Lanczos form on the same formed operator (`plain_fp64_*` fields).
+    Lanczos and the correction equation (MixedSolver dtype "f32"), FP64 Jacobi-Davidson refinement, FP64
+    Rayleigh-Ritz energy; the same with FP16 products of the slabs inside (`mixed_f16_*` fields);
+  * fp64: the plain FP64 Lanczos form on the formed operator (`plain_fp64_*` fields).
 """
 import argparse
 import json
@@ -361,6 +362,10 @@ def main():
     if args.form in ("both", "mixed"):
         ms, r, kms, nl = run(lambda: pipeline.solve_mixed(corners, sides, op_center, x0, dtype="f16"),
                              args.steps, args.warmup)
+        out["mixed_f16"] = dict(ms=ms, err=abs(r["energy"] - e_ref) / abs(e_ref), iterations=r["iterations"],
+                                passes=r["info"]["fp64_passes"], product_ms=kms[1] / max(1, nl[1]))
+        ms, r, kms, nl = run(lambda: pipeline.solve_mixed(corners, sides, op_center, x0, dtype="f32"),
+                             args.steps, args.warmup)
         out["mixed"] = dict(ms=ms, energy=r["energy"], err=abs(r["energy"] - e_ref) / abs(e_ref),
                             iterations=r["iterations"], info=r["info"], product_ms=kms[2] / max(1, nl[2]), launches=nl[2])
     formation = isolated_formation(r["operator"])
@@ -375,7 +380,8 @@ def main():
         "metric": "ground-state solves/sec at D=6,chi=64 to 1e-10 rel. energy vs plain FP64 GPU",
         "value": 1e3 / head["ms"], "unit": "solves/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": head["ms"], "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "f64",
+        # mixed: products inside the eigensolve in FP32; refinement, Rayleigh-Ritz and everything else in FP64
+        "dtype": "f64+f32" if form == "mixed" else "f64",
         "data": "synthetic (seeded environment, carcassonne_amd.synthetic seed 0)",
         "config": {"workload": "2D TFIM h=3.0, D=6, chi=64, d=2, w=3; one solve = stage 1/2 + normalization "
                                "factor + eigensolve to 1e-10 rel. energy + FP64 Rayleigh quotient",
@@ -392,7 +398,10 @@ def main():
                     plain_fp64_energy_rel_err=f["err"], plain_fp64_lanczos_iterations=f["iterations"],
                     plain_fp64_product_ms=f["product_ms"], plain_fp64_product_gbs=f["gbs"])
     if "mixed" in out:
-        m = out["mixed"]
+        m, h = out["mixed"], out["mixed_f16"]
+        line.update(mixed_f16_solves_per_s=1e3 / h["ms"], mixed_f16_ms_per_solve=h["ms"], mixed_f16_energy_rel_err=h["err"],
+                    mixed_f16_lanczos_iterations=h["iterations"], mixed_f16_fp64_passes=h["passes"],
+                    mixed_f16_product_ms=h["product_ms"])
         line.update(mixed_lowprec_iterations=m["iterations"], mixed_info=m["info"], mixed_product_ms=m["product_ms"],
                     products_timed=m["launches"], products_timed_every=TIMING_EVERY)
         if "fp64" in out:

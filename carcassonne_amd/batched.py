@@ -6,15 +6,16 @@ slabs and plan) and runs the setup once eagerly.  `capture` records every system
 graph, each system on its own stream branch forked from the capture stream, so one `replay` launches every
 solve and the GPU overlaps the small systems' kernels.  With setup=True (the default) each branch first
 rebuilds its system's setup from the environment tensors into those buffers -- stage 1/2, the
-normalization factor, the FP64 and low-precision slabs -- so a replay is a whole solve of every system,
+normalization factor, the FP64 and low-precision slabs or formed matrices -- so a replay is a whole solve of every system,
 and `load_environments` + `replay` solves new environments of the same shapes; with setup=False only the
 eigensolves are recorded.  The eigensolve is the fixed-work mixed solve (low-precision Lanczos plus FP64
 Rayleigh-Ritz refinement, no host reads: MixedSolver.solve_fixed), which also writes a convergence record
 per system; `convergence` reads the records after a replay and `resolve_unconverged` solves the flagged
-systems again with the adaptive solve.  An autotuner picks, per shape bucket, the low-precision kernel's
-workgroup count by timing candidates on the bucket's first system, and the fixed work (Lanczos steps,
-refinement passes) from adaptive solves of every system of the bucket with a safety margin.  The plain
-FP64 solve of every system is the reference for the batched energies.
+systems again with the adaptive solve.  dtype "f16" and "bf16" run the low-precision slabs inside, "f32" the
+formed matrices (MixedSolver).  An autotuner picks, per shape bucket, the low-precision kernel's workgroup
+count by timing candidates on the bucket's first system, and the fixed work (Lanczos steps, refinement
+passes) from adaptive solves of every system of the bucket with a safety margin.  The plain FP64 solve of
+every system is the reference for the batched energies.
 """
 import time
 
