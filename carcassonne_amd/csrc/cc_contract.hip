@@ -42,6 +42,8 @@ struct ContractArgs {
   double* work;                  // splits > 1: splits partial results per output, M x N each
 };
 
+// Index i split into the group's legs, divisions by the invariant extents as a multiply-high and shifts (Granlund and
+// Montgomery, "Division by invariant integers using multiplication", 1994).
 __device__ __forceinline__ void leg_offsets(const LegGroup& g, uint32_t i, int& a, int& b) {
   a = b = 0;
   for (int l = g.rank - 1; l >= 0; --l) {
