@@ -432,6 +432,7 @@ class System(BaseSystem):
         i = direction
         # the two corners and their truncation bases and the gauge of the center are independent: the right corner and
         # the gauge on streams of their own (the eigen-decompositions run on one workgroup each)
+        self.state_center_data.tensor()     # a lazily permuted center is the caller's: carried out on the caller's stream
         (side, gauge), produced, gauged = fork_both(), [], []
         try:
             with torch.cuda.stream(side):

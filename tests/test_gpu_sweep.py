@@ -160,3 +160,31 @@ def test_fused_truncation_diagonalizes_the_gram_matrix(gpu, n, rank):
     assert np.abs(T.T @ T - np.diag(want[:rank] ** 2)).max(initial=0) <= 1e-10
     if rank == 0:
         assert not U.any()
+
+
+def test_fused_step_of_a_lazily_permuted_center(gpu, monkeypatch):
+    """A center whose leg permutation is still to be carried out gives the step of the plain one, and its data, which stay
+    with the caller's tensor, are made on the caller's stream."""
+    import torch
+    from carcassonne_amd import pipeline, synthetic as syn
+    from carcassonne_amd.data import HipData
+    from carcassonne_amd.system import System
+    c, s, st = syn.make_environment(3, 6, model="ising", seed=4)
+    corners, sides, opc = pipeline.device_environment(c, s, syn.operator_center("ising"))
+    plain = System(list(corners), list(sides), HipData.fromArray(st), opc)
+    plain.contractAndCompressTowards(1, 5)
+    moved = HipData.fromArray(np.ascontiguousarray(st.transpose(4, 3, 0, 1, 2)))
+    center = moved.permuted_lazily([2, 3, 4, 1, 0])
+    lazy = System(list(corners), list(sides), center, opc)
+    streams = []
+    permuted = HipData._permuted
+
+    def watched(self, perm):
+        if self._t is moved._t:
+            streams.append(torch.cuda.current_stream())
+        return permuted(self, perm)
+
+    monkeypatch.setattr(HipData, "_permuted", watched)
+    lazy.contractAndCompressTowards(1, 5)
+    assert streams == [torch.cuda.current_stream()]
+    np.testing.assert_array_equal(lazy.state_center_data.toArray(), plain.state_center_data.toArray())
